@@ -32,7 +32,7 @@ constexpr int kNf4StreamRowsPerExpert = 128;
 constexpr int kNf4StreamGatedRowsPerExpert = 384;
 constexpr int kNf4StreamTwoBlockRows = 20;
 
-// Any shape / any float type; plain FMA.
+// Any shape / any float type; fp32 matrix instruction.
 int gemm_generic(int mode, const void *a, const void *b, const void *m_sizes, int ms_i64, void *c, int64_t R, int N,
                  int K, int E, int in_dtype, int out_dtype, float alpha, int accumulate, hipStream_t stream);
 

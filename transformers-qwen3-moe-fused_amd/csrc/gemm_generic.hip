@@ -1,12 +1,16 @@
-// Shape- and type-generic grouped GEMM (plain FMA, fp32 accumulate).
+// Shape- and type-generic grouped GEMM on the fp32 matrix instruction (v_mfma_f32_16x16x4_f32: fp32 products, fp32
+// sums, at the rate of the vector ALU but without its operand traffic).
 //
-// This is the path for fp32 / fp16 inputs and for bf16 shapes the MFMA kernels do not
-// take (dimensions that are not multiples of 8, tiny experts): every dimension is
-// masked, nothing is assumed about alignment beyond the element size.
+// This is the path for fp32 / fp16 inputs and for bf16 shapes the bf16 kernels do not take (dimensions that are not
+// multiples of 8): every dimension is masked, nothing is assumed about alignment beyond the element size.
 //
 //   MODE_FWD : c[m, n]    = sum_k a[m, k] * b[e(m), n, k]     a = x (R,K),  b = w (E,N,K)
 //   MODE_DX  : c[m, n]    = sum_k a[m, k] * b[e(m), k, n]     a = dy (R,K), b = w (E,K,N)
 //   MODE_DW  : c[e, n, k] = sum_{m in e} a[m, n] * b[m, k]    a = dy (R,N), b = x (R,K)
+//
+// Operands go global -> registers (the next step's, while the present one is multiplied) -> LDS as fp32.  One LDS
+// stage and two barriers a step: what hides the loads is the number of workgroups on a CU (six of the 16-row tile,
+// 24 KiB each), not a second stage.
 #include "common.h"
 #include "gemm.h"
 
@@ -14,165 +18,308 @@ namespace mfl {
 
 namespace {
 
-constexpr int GT = 64;   // output tile edge
-constexpr int GK = 16;   // reduction step
-constexpr int GPAD = 4;  // LDS row padding (floats)
+constexpr int kThreads = 256;
+constexpr int kPad = 4;  // floats: rows stay 16-byte aligned and 16 consecutive rows start in 16 different bank quads
 
-// Loads a GT x GK operand tile into lds[k][i].
-//   red_contig  : element (i, r) lives at base[i * ld + r]
-//   !red_contig : element (i, r) lives at base[r * ld + i]
-template <typename TI, bool RED_CONTIG>
-__device__ __forceinline__ void load_tile(float (*lds)[GT + GPAD], const TI *base, int64_t ld, int i0,
-                                          int i_end, int r0, int r_end, int tid) {
-    if (RED_CONTIG) {
-        const int i = tid >> 2, rq = (tid & 3) * 4;
-        const bool iok = (i0 + i) < i_end;
-        const TI *p = base + (int64_t)(i0 + i) * ld + r0 + rq;
+// An operand tile of BI rows (output side) by BK reduction elements.
+//   RC (reduction-contiguous): element (i, r) at base[i * ld + r], in LDS at [i][r]
+//   RS (reduction-strided):    element (i, r) at base[r * ld + i], in LDS at [r][i]
+template <typename TI, int BI, int BK, bool RC, int VEC>
+struct Operand {
+    static constexpr int kRow = RC ? BK : BI;                  // contiguous elements of a tile row
+    static constexpr int kStride = kRow + kPad;                // floats
+    static constexpr int kFloats = (RC ? BI : BK) * kStride;
+    static constexpr int kGroups = BI * BK / 4;                // groups of four contiguous elements
+    static constexpr int kPerThread = (kGroups + kThreads - 1) / kThreads;
+    floatx4 v[kPerThread];
+
+    __device__ __forceinline__ void load(const TI *base, int64_t ld, int i0, int i_end, int r0, int r_end, int tid) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            float v = 0.f;
-            if (iok && (r0 + rq + u) < r_end) v = to_f32(p[u]);
-            lds[rq + u][i] = v;
-        }
-    } else {
-        const int r = tid >> 4, iq = (tid & 15) * 4;
-        const bool rok = (r0 + r) < r_end;
-        const TI *p = base + (int64_t)(r0 + r) * ld + i0 + iq;
+        for (int q = 0; q < kPerThread; ++q) {
+            const int g = q * kThreads + tid;
+            const int row = g / (kRow / 4), col = (g % (kRow / 4)) * 4;
+            const int i = i0 + (RC ? row : col), r = r0 + (RC ? col : row);
+            const TI *p = base + (RC ? (int64_t)i * ld + r : (int64_t)r * ld + i);
+            v[q] = floatx4{0.f, 0.f, 0.f, 0.f};
+            if (kGroups % kThreads != 0 && g >= kGroups) continue;
+            if constexpr (VEC == 4) {  // the contiguous dimension is a multiple of four: a group is inside or outside
+                if (i < i_end && r < r_end) {
+                    typedef __attribute__((ext_vector_type(4))) TI vec_t;
+                    const vec_t t = *(const vec_t *)p;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            float v = 0.f;
-            if (rok && (i0 + iq + u) < i_end) v = to_f32(p[u]);
-            lds[r][iq + u] = v;
+                    for (int u = 0; u < 4; ++u) v[q][u] = to_f32(t[u]);
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (i + (RC ? 0 : u) < i_end && r + (RC ? u : 0) < r_end) v[q][u] = to_f32(p[u]);
+            }
         }
     }
+    __device__ __forceinline__ void store(float *lds, int tid) const {
+#pragma unroll
+        for (int q = 0; q < kPerThread; ++q) {
+            const int g = q * kThreads + tid;
+            if (kGroups % kThreads != 0 && g >= kGroups) continue;
+            *(floatx4 *)(lds + (g / (kRow / 4)) * kStride + (g % (kRow / 4)) * 4) = v[q];
+        }
+    }
+    // The lane's values of four matrix instructions: reduction elements k + 4 * (lane / 16) + 0..3 of row i + lane % 16
+    // (which of the 16 elements of a chunk goes to which instruction is the same for both operands, so free).
+    __device__ static __forceinline__ floatx4 frag(const float *lds, int i, int k, int lane) {
+        const int row = i + (lane & 15), r = k + (lane >> 4) * 4;
+        if constexpr (RC) return *(const floatx4 *)(lds + row * kStride + r);
+        floatx4 f;  // four rows apart, the lane groups of a read lie 16 banks apart: no conflicts
+#pragma unroll
+        for (int u = 0; u < 4; ++u) f[u] = lds[(r + u) * kStride + row];
+        return f;
+    }
+};
+
+// (expert, first row, rows) of the slot-th tile of BM rows, by prefix sums over the experts 64 at a time.
+// false: the slot lies past the last tile.  Every wave does it for itself; the row counts come from the cache.
+template <int BM>
+__device__ __forceinline__ bool find_tile(const void *m_sizes, int ms_i64, int E, int slot, int lane, int &expert,
+                                          int &tile, int &m_start, int &m_size) {
+    int tiles_before = 0, rows_before = 0;
+    for (int e0 = 0; e0 < E; e0 += kWave) {
+        const int m = e0 + lane < E ? load_msize(m_sizes, ms_i64, e0 + lane) : 0;
+        const int tiles_to = tiles_before + wave_inclusive_scan(ceil_div(m, BM));
+        const int rows_to = rows_before + wave_inclusive_scan(m);
+        const uint64_t past = __ballot(tiles_to > slot);
+        if (past != 0) {
+            const int l = __builtin_ctzll(past);
+            expert = e0 + l;
+            m_size = __builtin_amdgcn_readlane(m, l);
+            m_start = __builtin_amdgcn_readlane(rows_to, l) - m_size;
+            tile = slot - (__builtin_amdgcn_readlane(tiles_to, l) - ceil_div(m_size, BM));
+            return true;
+        }
+        tiles_before = wave_last(tiles_to), rows_before = wave_last(rows_to);
+    }
+    return false;
 }
 
-template <typename TI, typename TO, int MODE>
-__global__ __launch_bounds__(256) void gemm_generic_kernel(const TI *__restrict__ a, const TI *__restrict__ b,
-                                                           const void *__restrict__ m_sizes, int ms_i64,
-                                                           TO *c, int64_t R, int N, int K, int E, float alpha,
-                                                           int accumulate) {
-    __shared__ float As[GK][GT + GPAD];
-    __shared__ float Bs[GK][GT + GPAD];
-    const int tid = threadIdx.x;
-    const int tx = tid & 15, ty = tid >> 4;
+// rows of the experts before e
+__device__ __forceinline__ int rows_before_expert(const void *m_sizes, int ms_i64, int e, int lane) {
+    int m = 0;
+    for (int q = lane; q < e; q += kWave) m += load_msize(m_sizes, ms_i64, q);
+    return wave_last(wave_inclusive_scan(m));
+}
+
+// WM x WN waves over the tile; WK > 1: the waves share the tile and split the reduction (partial sums meet in LDS).
+template <typename TI, typename TO, int MODE, int BM, int BN, int WM, int WN, int WK, int BK, int VEC>
+__global__ __launch_bounds__(kThreads) void gemm_generic_kernel(const TI *__restrict__ a, const TI *__restrict__ b,
+                                                                const void *__restrict__ m_sizes, int ms_i64, TO *c,
+                                                                int64_t R, int N, int K, int E, float alpha,
+                                                                int accumulate, int vec_out) {
+    static_assert(WM * WN * WK * kWave == kThreads && BK % (16 * WK) == 0, "four waves");
+    constexpr int TM = BM / WM / 16, TN = BN / WN / 16, KW = BK / WK;
+    // whether a lane ends with four consecutive columns of one row (16-byte stores) or with four rows of one column
+    // (consecutive lanes then store consecutive single elements, where rows are not aligned)
+    constexpr bool kRowLanes = VEC == 4;
+    typedef Operand<TI, BM, BK, MODE != MODE_DW, VEC> OpA;
+    typedef Operand<TI, BN, BK, MODE == MODE_FWD, VEC> OpB;
+    constexpr int kPartFloats = WM * WN * TM * TN * (WK - 1) * 4 * kWave;  // partial sums of the waves that share a tile
+    static_assert(kPartFloats <= OpA::kFloats + OpB::kFloats, "partial sums go where the stage was");
+    __shared__ __align__(16) float smem[OpA::kFloats + OpB::kFloats];
+    float *As = smem, *Bs = smem + OpA::kFloats;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave % WK, wn = wave / WK % WN, wm = wave / WK / WN;
 
     // Output tile [i0, i_end) x [j0, j_end), reduction range [r_begin, r_end).
     int i0, i_end, j0, j_end, r_begin, r_end;
-    const TI *a_base;
-    const TI *b_base;
+    const TI *b_base = b;
     int64_t lda, ldb, ldc;
-    TO *c_base;
-
+    TO *c_base = c;
     if (MODE == MODE_DW) {
         const int e = blockIdx.z;
-        int m_start = 0;
-        for (int q = 0; q < e; ++q) m_start += load_msize(m_sizes, ms_i64, q);
-        const int m_size = load_msize(m_sizes, ms_i64, e);
-        i0 = blockIdx.y * GT, i_end = N;
-        j0 = blockIdx.x * GT, j_end = K;
-        r_begin = m_start, r_end = m_start + m_size;
+        r_begin = rows_before_expert(m_sizes, ms_i64, e, lane);
+        r_end = r_begin + load_msize(m_sizes, ms_i64, e);
         if ((int64_t)r_end > R) r_end = (int)R;
-        a_base = a, lda = N;
-        b_base = b, ldb = K;
-        c_base = c + (int64_t)e * N * K, ldc = K;
+        i0 = blockIdx.y * BM, i_end = N;
+        j0 = blockIdx.x * BN, j_end = K;
+        lda = N, ldb = K, ldc = K;
+        c_base = c + (int64_t)e * N * K;
     } else {
-        // blockIdx.x enumerates (expert, m-tile) pairs in expert order; slots past the last
-        // real tile exit.
-        int slot = blockIdx.x, m_start = 0, e = 0, m_size = 0;
-        bool found = false;
-        for (; e < E; ++e) {
-            m_size = load_msize(m_sizes, ms_i64, e);
-            const int t = ceil_div(m_size, GT);
-            if (slot < t) {
-                found = true;
-                break;
-            }
-            slot -= t;
-            m_start += m_size;
-        }
-        if (!found) return;
-        i0 = m_start + slot * GT;
+        int e, tile, m_start, m_size;
+        if (!find_tile<BM>(m_sizes, ms_i64, E, blockIdx.x, lane, e, tile, m_start, m_size)) return;
+        i0 = m_start + tile * BM;
         i_end = m_start + m_size;
         if ((int64_t)i_end > R) i_end = (int)R;
-        j0 = blockIdx.y * GT, j_end = N;
+        j0 = blockIdx.y * BN, j_end = N;
         r_begin = 0, r_end = K;
-        a_base = a, lda = K;
+        lda = K, ldb = MODE == MODE_FWD ? K : N, ldc = N;
         b_base = b + (int64_t)e * N * K;
-        ldb = (MODE == MODE_FWD) ? K : N;
-        c_base = c, ldc = N;
     }
 
-    float acc[4][4];
+    floatx4 acc[TM][TN];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+        for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    for (int r0 = r_begin; r0 < r_end; r0 += GK) {
-        load_tile<TI, MODE != MODE_DW>(As, a_base, lda, i0, i_end, r0, r_end, tid);
-        load_tile<TI, MODE == MODE_FWD>(Bs, b_base, ldb, j0, j_end, r0, r_end, tid);
+    OpA ra;
+    OpB rb;
+    ra.load(a, lda, i0, i_end, r_begin, r_end, tid);
+    rb.load(b_base, ldb, j0, j_end, r_begin, r_end, tid);
+    for (int r0 = r_begin; r0 < r_end; r0 += BK) {
+        __syncthreads();  // the previous step's fragments have been read
+        ra.store(As, tid);
+        rb.store(Bs, tid);
         __syncthreads();
-#pragma unroll
-        for (int k = 0; k < GK; ++k) {
-            float av[4], bv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) av[i] = As[k][ty + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) bv[j] = Bs[k][tx + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
+        if (r0 + BK < r_end) {
+            ra.load(a, lda, i0, i_end, r0 + BK, r_end, tid);
+            rb.load(b_base, ldb, j0, j_end, r0 + BK, r_end, tid);
         }
+#pragma unroll
+        for (int kk = 0; kk < KW; kk += 16) {
+            const int k = wk * KW + kk;
+            if (r0 + k >= r_end) break;  // the rest of the stage is zeros
+            floatx4 fa[TM], fb[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) fa[i] = OpA::frag(As, (wm * TM + i) * 16, k, lane);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) fb[j] = OpB::frag(Bs, (wn * TN + j) * 16, k, lane);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = kRowLanes ? __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j][u], fa[i][u], acc[i][j], 0, 0, 0)
+                                              : __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i][u], fb[j][u], acc[i][j], 0, 0, 0);
+        }
+    }
+
+    if constexpr (WK > 1) {
+        // of the waves that share a tile, wave t % WK ends with output block t: the others' sums, in wave order
+        float *part = smem + (wave / WK) * TM * TN * (WK - 1) * kWave * 4 + lane * 4;
         __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TM * TN; ++t)
+            if (wk != t % WK)
+                *(floatx4 *)(part + (t * (WK - 1) + wk - (wk > t % WK)) * kWave * 4) = acc[t / TN][t % TN];
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TM * TN; ++t)
+            if (wk == t % WK)
+#pragma unroll
+                for (int s = 0; s < WK - 1; ++s)
+                    acc[t / TN][t % TN] += *(const floatx4 *)(part + (t * (WK - 1) + s) * kWave * 4);
     }
 
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = i0 + ty + 16 * i;
-        if (row >= i_end) continue;
+    for (int i = 0; i < TM; ++i) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int col = j0 + tx + 16 * j;
-            if (col >= j_end) continue;
+        for (int j = 0; j < TN; ++j) {
+            if (WK > 1 && wk != (i * TN + j) % WK) continue;
+            const int across = lane & 15, along = (lane >> 4) * 4;
+            const int row = i0 + (wm * TM + i) * 16 + (kRowLanes ? across : along);
+            const int col = j0 + (wn * TN + j) * 16 + (kRowLanes ? along : across);
             TO *p = c_base + (int64_t)row * ldc + col;
-            float v = alpha * acc[i][j];
-            if (accumulate) v += to_f32(*p);
-            *p = from_f32<TO>(v);
+            if (kRowLanes && vec_out) {
+                if (row >= i_end || col >= j_end) continue;
+                typedef __attribute__((ext_vector_type(4))) TO vec_t;
+                vec_t o;
+                if (accumulate) o = *(const vec_t *)p;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    float v = alpha * acc[i][j][u];
+                    if (accumulate) v += to_f32(o[u]);
+                    o[u] = from_f32<TO>(v);
+                }
+                *(vec_t *)p = o;
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (row + (kRowLanes ? 0 : u) >= i_end || col + (kRowLanes ? u : 0) >= j_end) continue;
+                    TO *q = p + (kRowLanes ? u : u * ldc);
+                    float v = alpha * acc[i][j][u];
+                    if (accumulate) v += to_f32(*q);
+                    *q = from_f32<TO>(v);
+                }
+            }
         }
     }
 }
 
-template <typename TI, typename TO>
-int launch_generic(int mode, const void *a, const void *b, const void *m_sizes, int ms_i64, void *c, int64_t R,
-                   int N, int K, int E, float alpha, int accumulate, hipStream_t stream) {
-    if (mode == MODE_DW) {
-        if (ceil_div(N, GT) > 65535 || E > 65535) return MFL_ERR_UNSUPPORTED;
-        dim3 grid(ceil_div(K, GT), ceil_div(N, GT), E);
-        gemm_generic_kernel<TI, TO, MODE_DW><<<grid, 256, 0, stream>>>((const TI *)a, (const TI *)b, m_sizes, ms_i64,
-                                                                       (TO *)c, R, N, K, E, alpha, accumulate);
+struct Args {
+    const void *a, *b, *m_sizes;
+    void *c;
+    int64_t R;
+    int ms_i64, N, K, E, accumulate, vec_out;
+    float alpha;
+    hipStream_t stream;
+};
+
+template <typename TI, typename TO, int MODE, int BM, int BN, int WM, int WN, int WK, int BK, int VEC>
+int launch_tile(const Args &g) {
+    dim3 grid;
+    if (MODE == MODE_DW) {
+        if (ceil_div(g.N, BM) > 65535 || g.E > 65535) return MFL_ERR_UNSUPPORTED;
+        grid = dim3(ceil_div(g.K, BN), ceil_div(g.N, BM), g.E);
     } else {
-        const int64_t slots = (R + GT - 1) / GT + E;
-        if (slots > 0x7fffffff || ceil_div(N, GT) > 65535) return MFL_ERR_UNSUPPORTED;
-        dim3 grid((unsigned)slots, ceil_div(N, GT), 1);
-        if (mode == MODE_FWD)
-            gemm_generic_kernel<TI, TO, MODE_FWD><<<grid, 256, 0, stream>>>(
-                (const TI *)a, (const TI *)b, m_sizes, ms_i64, (TO *)c, R, N, K, E, alpha, accumulate);
-        else
-            gemm_generic_kernel<TI, TO, MODE_DX><<<grid, 256, 0, stream>>>(
-                (const TI *)a, (const TI *)b, m_sizes, ms_i64, (TO *)c, R, N, K, E, alpha, accumulate);
+        const int64_t slots = (g.R + BM - 1) / BM + g.E;
+        if (slots > 0x7fffffff || ceil_div(g.N, BN) > 65535) return MFL_ERR_UNSUPPORTED;
+        grid = dim3((unsigned)slots, ceil_div(g.N, BN), 1);
     }
+    gemm_generic_kernel<TI, TO, MODE, BM, BN, WM, WN, WK, BK, VEC><<<grid, kThreads, 0, g.stream>>>(
+        (const TI *)g.a, (const TI *)g.b, g.m_sizes, g.ms_i64, (TO *)g.c, g.R, g.N, g.K, g.E, g.alpha, g.accumulate,
+        g.vec_out);
     return launch_status();
+}
+
+// Tiles, with fp32 times at 128 experts, K = 2048, N = 768 (us; the plain FMA kernel that stood here in brackets):
+// * up to 16 rows per expert the product streams the weights: 16-row tiles whose waves split the reduction, so that a
+//   step asks for 512 consecutive bytes of every weight row and 24 KiB workgroups keep 96 KiB a CU in flight: 150 us
+//   forward at 8 rows per expert = 5.4 TB/s (712), 168 dX (533); 64 x 64 tiles with the waves side by side: 285.
+// * up to 48, and where 64-row tiles would leave CUs without a second and third workgroup, 32 x 64 tiles: 191 us
+//   forward at 24 rows per expert (746; 64 x 64 tiles 275, 16-row tiles 295), 154 us at 8 experts of 512 rows (518;
+//   64 x 64 166).
+// * beyond, 64 x 64 tiles: 373 us at 64 rows per expert (1584; 128 x 128 tiles 392, whose 64 accumulators and 32
+//   registers in transit leave two workgroups a CU).
+// * the weight gradient writes more than it reads up to about 100 rows per expert: 64 x 128 tiles and 16-row steps,
+//   182 us at 8 rows per expert = 4.5 TB/s (294; with 32-row steps 225, the zeros of a half-empty stage cost as much
+//   as rows do); outputs with a side of at most 16 (adapter ranks) take 16-row tiles.
+template <typename TI, typename TO, int MODE, int VEC>
+int launch_mode(const Args &g) {
+    if (MODE == MODE_DW) {
+        if (g.N <= 16) return launch_tile<TI, TO, MODE, 16, 64, 1, 4, 1, 32, VEC>(g);
+        if (g.N >= 64 && g.K >= 128) return launch_tile<TI, TO, MODE, 64, 128, 2, 2, 1, 16, VEC>(g);
+        return launch_tile<TI, TO, MODE, 64, 64, 2, 2, 1, 32, VEC>(g);
+    }
+    if (g.R <= (int64_t)16 * g.E) return launch_tile<TI, TO, MODE, 16, 32, 1, 1, 4, 128, VEC>(g);
+    const int64_t tiles64 = (g.R / 64 + g.E) * ceil_div(g.N, 64);
+    if (g.R <= (int64_t)48 * g.E || tiles64 < 4 * device_info().cu_count)
+        return launch_tile<TI, TO, MODE, 32, 64, 1, 2, 2, 64, VEC>(g);
+    return launch_tile<TI, TO, MODE, 64, 64, 2, 1, 2, 64, VEC>(g);
+}
+
+template <typename TI, typename TO>
+int launch_generic(int mode, const Args &g) {
+    // groups of four elements: every contiguous dimension that is read has to be a multiple of four
+    const size_t align = 4 * sizeof(TI);
+    bool vec = aligned(g.a, align) && aligned(g.b, align) && g.K % 4 == 0 && (mode == MODE_FWD || g.N % 4 == 0);
+    if (vec) {
+        if (mode == MODE_FWD) return launch_mode<TI, TO, MODE_FWD, 4>(g);
+        if (mode == MODE_DX) return launch_mode<TI, TO, MODE_DX, 4>(g);
+        return launch_mode<TI, TO, MODE_DW, 4>(g);
+    }
+    if (mode == MODE_FWD) return launch_mode<TI, TO, MODE_FWD, 1>(g);
+    if (mode == MODE_DX) return launch_mode<TI, TO, MODE_DX, 1>(g);
+    return launch_mode<TI, TO, MODE_DW, 1>(g);
 }
 
 }  // namespace
 
 int gemm_generic(int mode, const void *a, const void *b, const void *m_sizes, int ms_i64, void *c, int64_t R, int N,
                  int K, int E, int in_dtype, int out_dtype, float alpha, int accumulate, hipStream_t stream) {
+    const int ldc = mode == MODE_DW ? K : N;
+    const int vec_out = ldc % 4 == 0 && aligned(c, 4 * dtype_size(out_dtype));
+    const Args g = {a, b, m_sizes, c, R, ms_i64, N, K, E, accumulate, vec_out, alpha, stream};
     int rc = MFL_ERR_DTYPE;
-    MFL_DISPATCH_FLOAT(in_dtype, TI, MFL_DISPATCH_FLOAT(out_dtype, TO, rc = (launch_generic<TI, TO>(
-        mode, a, b, m_sizes, ms_i64, c, R, N, K, E, alpha, accumulate, stream))));
+    MFL_DISPATCH_FLOAT(in_dtype, TI, MFL_DISPATCH_FLOAT(out_dtype, TO, rc = (launch_generic<TI, TO>(mode, g))));
     return rc;
 }
 
