@@ -255,6 +255,30 @@ MFL_API int mfl_glu_fwd_nf4_tiled(const void *x, int64_t src_rows, const int32_t
                           int m_sizes_dtype, void *h, void *e_out, void *g_out, int64_t R, int N, int K,
                           int E, int dtype, void *stream);
 
+/* A packed 4-bit matrix with its quantisation state.  Its scales are either fp32 (absmax, and optionally their
+ * tile-ordered copy) or quantised once more to 8 bits (absmax_u8 not NULL; the bitsandbytes default):
+ * scale b = code256[absmax_u8[b]] * absmax2[b / blocksize2] + *offset. */
+typedef struct mfl_nf4_weight {
+    const uint8_t *packed;
+    const float *code16;
+    const float *absmax, *absmax_tiled;
+    const uint8_t *absmax_u8;
+    const float *code256, *absmax2, *offset;
+    int blocksize, blocksize2;
+} mfl_nf4_weight;
+
+/* mfl_gemm_fwd_nf4_tiled / mfl_glu_fwd_nf4_tiled with each matrix as one (host) struct.  A double-quantised matrix
+ * is read as it is by the decode-sized kernels (blocks of 64, K a multiple of 128 and at most 64 * blocksize2, or a
+ * few rows per expert); beyond them the answer is MFL_ERR_UNSUPPORTED and the caller writes the scales out
+ * (mfl_nf4_unnest_absmax) first, as the reference does for every product (forward_4bit.py:149-152). */
+MFL_API int mfl_gemm_fwd_nf4_packed(const void *x_src, int64_t src_rows, const int32_t *row_idx, int idx_div,
+                            const mfl_nf4_weight *w, const void *m_sizes, int m_sizes_dtype, void *y, int64_t R,
+                            int N, int K, int E, int in_dtype, int out_dtype, void *stream);
+MFL_API int mfl_glu_fwd_nf4_packed(const void *x, int64_t src_rows, const int32_t *row_idx, int idx_div,
+                           const mfl_nf4_weight *gate, const mfl_nf4_weight *up, const void *m_sizes,
+                           int m_sizes_dtype, void *h, void *e_out, void *g_out, int64_t R, int N, int K, int E,
+                           int dtype, void *stream);
+
 /* ---- NF4 / blockwise dequantisation ----------------------------------------------- */
 
 /* out[i] = code16[nibble(i)] * absmax[i / blocksize], i < n (n even).  Stands in for the
@@ -267,6 +291,10 @@ MFL_API int mfl_nf4_dequant(const uint8_t *wq, const float *code16, const float 
  * qwen3_moe_fused/grouped_gemm/forward_4bit.py:149-152. */
 MFL_API int mfl_dequant_blockwise_u8(const uint8_t *v, const float *code256, const float *absmax2,
                              int blocksize2, float offset, float *out, int64_t n, void *stream);
+
+/* The same with the offset read on the device (offset: one float) and blocksize2 a power of two. */
+MFL_API int mfl_nf4_unnest_absmax(const uint8_t *v, const float *code256, const float *absmax2, int blocksize2,
+                          const float *offset, float *out, int64_t n, void *stream);
 
 /* Blockwise NF4 quantiser: absmax[b] = max|block b|, nibble = nearest code16 entry to
  * x / absmax (ties -> lower entry).  w has n elements of w_dtype, n % blocksize == 0.

@@ -1,0 +1,73 @@
+"""Double-quantised NF4 weights, whose 8-bit scales the decode-sized kernels read as they are: the same bits as with the
+scales written out in fp32 first (code256[q] * absmax2 rounded, then the offset added and rounded, in both)."""
+import pytest
+import torch
+
+from util import gen
+
+pytestmark = pytest.mark.gpu
+
+from qwen3_moe_fused.grouped_gemm.forward_4bit import grouped_gemm_forward_4bit  # noqa: E402
+from qwen3_moe_fused.grouped_gemm.fused import grouped_gemm_forward_4bit_gathered, grouped_glu_forward_4bit  # noqa: E402
+from qwen3_moe_fused.quantize.nf4 import Nf4QuantState, quantize_nf4, resolve_absmax  # noqa: E402
+
+
+def _weights(e, n, k, blocksize, seed):
+    w = (torch.randn((e, n, k), generator=gen(seed)) * 0.02).to(torch.bfloat16).cuda()
+    packed, nested = quantize_nf4(w, blocksize, "nf4", compress_statistics=True)
+    assert nested.nested
+    plain = Nf4QuantState(absmax=resolve_absmax(nested), shape=nested.shape, code=nested.code, blocksize=blocksize)
+    return packed, nested, plain
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 255, 256, 257, 4096, 100003])
+@pytest.mark.parametrize("blocksize2", [8, 256])
+def test_scales_written_out_are_the_formula(n, blocksize2):
+    from qwen3_moe_fused.quantize.nf4 import BlockwiseState
+
+    g = gen(n)
+    q = torch.randint(0, 256, (n,), generator=g, dtype=torch.uint8).cuda()
+    code = torch.randn(256, generator=g).cuda()
+    absmax2 = torch.rand((n + blocksize2 - 1) // blocksize2, generator=g).cuda()
+    offset = torch.tensor(0.0473).cuda()
+    state = Nf4QuantState(absmax=q, shape=(1,), code=code, offset=offset,
+                          state2=BlockwiseState(absmax=absmax2, code=code, blocksize=blocksize2))
+    want = code[q.long()] * absmax2.repeat_interleave(blocksize2)[:n] + offset
+    assert torch.equal(resolve_absmax(state), want)
+
+
+# (rows per expert, N, K, blocksize): the matrix-vector kernel (up to two rows per expert; rows of at most 1024, and of
+# more), the streaming kernel with 32-row and 64-row tiles; rows of the matrix that cross a border of the second-level
+# blocks (K = 768: 12 scales a row), column tiles that end past N, scales under blocks of 128, a row of more scales than a
+# second-level block (no kernel for it), and batches beyond the decode sizes
+CASES = [
+    ([1, 0, 1, 2, 0, 0, 0, 0, 0], 64, 2048, 64),
+    ([1, 0, 1, 0, 0], 96, 768, 64),
+    ([2, 1, 0, 2], 32, 1536, 64),
+    ([1, 1, 0], 32, 1024, 128),
+    ([5, 0, 3, 17], 200, 768, 64),
+    ([40, 1, 33], 128, 384, 64),
+    ([70, 0, 12], 72, 2048, 64),
+    ([9], 40, 16512, 64),
+    ([4, 9], 64, 256, 128),
+    ([600, 20], 64, 256, 64),
+]
+
+
+@pytest.mark.parametrize("sizes,n,k,blocksize", CASES)
+def test_products_on_double_quantised_weights_are_those_on_written_out_scales(sizes, n, k, blocksize):
+    e, rows = len(sizes), sum(sizes)
+    gate, gate_nested, gate_plain = _weights(e, n, k, blocksize, n + k)
+    up, up_nested, up_plain = _weights(e, n, k, blocksize, n + k + 1)
+    ms = torch.tensor(sizes, dtype=torch.int32).cuda()
+    src = torch.randn((rows, k), generator=gen(rows)).to(torch.bfloat16).cuda()
+    idx = torch.randperm(rows, generator=gen(rows + 1)).to(torch.int32).cuda()
+    for dtype in (torch.bfloat16, torch.float32):
+        assert torch.equal(grouped_gemm_forward_4bit(src, gate, gate_nested, ms, dtype),
+                           grouped_gemm_forward_4bit(src, gate, gate_plain, ms, dtype))
+    assert torch.equal(grouped_gemm_forward_4bit_gathered(src, idx, 1, gate, gate_nested, ms),
+                       grouped_gemm_forward_4bit_gathered(src, idx, 1, gate, gate_plain, ms))
+    got = grouped_glu_forward_4bit(src, gate, gate_nested, up, up_nested, ms, idx, 1, return_products=True)
+    want = grouped_glu_forward_4bit(src, gate, gate_plain, up, up_plain, ms, idx, 1, return_products=True)
+    for a, b in zip(got, want):
+        assert torch.isfinite(a).all() and torch.equal(a, b)

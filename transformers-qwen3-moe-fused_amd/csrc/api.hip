@@ -129,40 +129,70 @@ int mfl_gemm_dw_split(const void *x, const void *dy, const void *m_sizes, int m_
                          (hipStream_t)stream);
 }
 
-// The NF4 forward product, with or without gathered rows (row_idx null: x is (R, K)) and with or without the
-// tile-ordered copy of the scales.
-static int fwd_nf4(const void *x, int64_t src_rows, const int32_t *row_idx, int idx_div, const uint8_t *wq,
-                   const float *code16, const float *absmax, const float *absmax_tiled, int blocksize,
+namespace {
+
+bool blocksize_ok(int bs) { return bs >= 2 && (bs & (bs - 1)) == 0; }
+int log2_of(int v) {
+    int s = 0;
+    while ((1 << s) < v) ++s;
+    return s;
+}
+
+// (absmax_tiled only where the shape has such a copy)
+Nf4Matrix nf4_matrix(const uint8_t *wq, const float *code16, const float *absmax, const float *absmax_tiled, int blocksize,
+                     int N, int K, int E) {
+    Nf4Matrix m = {wq, code16, absmax, log2_of(blocksize)};
+    if (absmax_tiled != nullptr && nf4_tiled_absmax_floats(blocksize, N, K, E) != 0) m.absmax_tiled = absmax_tiled;
+    return m;
+}
+
+// The same from the public description; MFL_OK or an argument error.
+int nf4_matrix_of(const mfl_nf4_weight *w, int N, int K, int E, Nf4Matrix &m) {
+    if (!w || !w->packed || !w->code16) return MFL_ERR_NULL;
+    if (!blocksize_ok(w->blocksize) || K % 2 != 0 || ((int64_t)E * N * K) % w->blocksize != 0) return MFL_ERR_SHAPE;
+    if (w->absmax_u8 != nullptr) {
+        if (!w->code256 || !w->absmax2 || !w->offset) return MFL_ERR_NULL;
+        if (!blocksize_ok(w->blocksize2)) return MFL_ERR_SHAPE;
+        m = {w->packed, w->code16, nullptr, log2_of(w->blocksize)};
+        m.absmax_u8 = w->absmax_u8, m.code256 = w->code256, m.absmax2 = w->absmax2, m.offset = w->offset;
+        m.bs2_shift = log2_of(w->blocksize2);
+    } else {
+        if (!w->absmax) return MFL_ERR_NULL;
+        m = nf4_matrix(w->packed, w->code16, w->absmax, w->absmax_tiled, w->blocksize, N, K, E);
+    }
+    return MFL_OK;
+}
+
+}  // namespace
+
+// The NF4 forward product, with or without gathered rows (row_idx null: x is (R, K)).
+static int fwd_nf4(const void *x, int64_t src_rows, const int32_t *row_idx, int idx_div, const Nf4Matrix &w,
                    const void *m_sizes, int m_sizes_dtype, void *y, int64_t R, int N, int K, int E, int in_dtype,
                    int out_dtype, void *stream) {
     if (R < 0 || N <= 0 || K <= 0 || E <= 0 || R > 0x7fffffff) return MFL_ERR_SHAPE;
-    if (blocksize < 2 || (blocksize & (blocksize - 1)) != 0) return MFL_ERR_SHAPE;
-    if (K % 2 != 0 || ((int64_t)E * N * K) % blocksize != 0) return MFL_ERR_SHAPE;
+    if (K % 2 != 0 || (((int64_t)E * N * K) & ((1ll << w.bs_shift) - 1)) != 0) return MFL_ERR_SHAPE;
     if (!dtype_ok(in_dtype) || !dtype_ok(out_dtype) || !itype_ok(m_sizes_dtype)) return MFL_ERR_DTYPE;
-    if (!wq || !code16 || !absmax || !m_sizes || (R > 0 && (!x || !y))) return MFL_ERR_NULL;
+    if (!w.wq || !w.code16 || (!w.absmax && !w.nested()) || !m_sizes || (R > 0 && (!x || !y))) return MFL_ERR_NULL;
     if (R == 0) return MFL_OK;
     if (in_dtype != MFL_BF16) return MFL_ERR_UNSUPPORTED;
-    if (absmax_tiled != nullptr && nf4_tiled_absmax_floats(blocksize, N, K, E) == 0) absmax_tiled = nullptr;
     const int ms_i64 = m_sizes_dtype == MFL_I64;
-    GemmFusion fu = {row_idx, idx_div, src_rows, nullptr, nullptr, nullptr, 0, nullptr, nullptr};
-    fu.absmax_tiled = absmax_tiled;
-    const GemmFusion *pf = (row_idx != nullptr || absmax_tiled != nullptr) ? &fu : nullptr;
-    int rc = gemm_nf4_decode(x, wq, code16, absmax, blocksize, m_sizes, ms_i64, y, R, N, K, E, out_dtype,
-                             (hipStream_t)stream, pf);
-    if (rc != MFL_ERR_UNSUPPORTED) return rc;
-    pf = row_idx != nullptr ? &fu : nullptr;
-    rc = gemm_nf4_pipe(x, wq, code16, absmax, blocksize, m_sizes, ms_i64, y, R, N, K, E, out_dtype,
-                       (hipStream_t)stream, pf);
+    int rc = gemm_nf4_decode(x, row_idx, idx_div, w, w, false, m_sizes, ms_i64, y, nullptr, nullptr, R, N, K, E, out_dtype,
+                             (hipStream_t)stream);
+    if (rc != MFL_ERR_UNSUPPORTED || w.nested()) return rc;
+    const GemmFusion fu = {row_idx, idx_div, src_rows, nullptr, nullptr, nullptr, 0, nullptr, nullptr};
+    rc = gemm_nf4_pipe(x, w.wq, w.code16, w.absmax, 1 << w.bs_shift, m_sizes, ms_i64, y, R, N, K, E, out_dtype,
+                       (hipStream_t)stream, row_idx != nullptr ? &fu : nullptr);
     if (rc != MFL_ERR_UNSUPPORTED || row_idx != nullptr) return rc;
-    return gemm_nf4_mfma(x, wq, code16, absmax, blocksize, m_sizes, ms_i64, y, R, N, K, E, out_dtype,
+    return gemm_nf4_mfma(x, w.wq, w.code16, w.absmax, 1 << w.bs_shift, m_sizes, ms_i64, y, R, N, K, E, out_dtype,
                          (hipStream_t)stream);
 }
 
 int mfl_gemm_fwd_nf4(const void *x, const uint8_t *wq, const float *code16, const float *absmax, int blocksize,
                      const void *m_sizes, int m_sizes_dtype, void *y, int64_t R, int N, int K, int E, int in_dtype,
                      int out_dtype, void *stream) {
-    return fwd_nf4(x, 0, nullptr, 1, wq, code16, absmax, nullptr, blocksize, m_sizes, m_sizes_dtype, y, R, N, K, E,
-                   in_dtype, out_dtype, stream);
+    if (!blocksize_ok(blocksize)) return MFL_ERR_SHAPE;
+    return fwd_nf4(x, 0, nullptr, 1, nf4_matrix(wq, code16, absmax, nullptr, blocksize, N, K, E), m_sizes, m_sizes_dtype, y, R,
+                   N, K, E, in_dtype, out_dtype, stream);
 }
 
 int64_t mfl_nf4_tiled_absmax_floats(int blocksize, int N, int K, int E) {
@@ -190,8 +220,20 @@ int mfl_gemm_fwd_nf4_tiled(const void *x_src, int64_t src_rows, const int32_t *r
         const int rc = check_fused(src_rows, row_idx, idx_div, m_sizes, m_sizes_dtype, R, N, K, E, in_dtype, out_dtype);
         if (rc) return rc;
     }
-    return fwd_nf4(x_src, src_rows, row_idx, idx_div, wq, code16, absmax, absmax_tiled, blocksize, m_sizes,
+    if (!blocksize_ok(blocksize)) return MFL_ERR_SHAPE;
+    return fwd_nf4(x_src, src_rows, row_idx, idx_div, nf4_matrix(wq, code16, absmax, absmax_tiled, blocksize, N, K, E), m_sizes,
                    m_sizes_dtype, y, R, N, K, E, in_dtype, out_dtype, stream);
+}
+
+int mfl_gemm_fwd_nf4_packed(const void *x_src, int64_t src_rows, const int32_t *row_idx, int idx_div,
+                            const mfl_nf4_weight *w, const void *m_sizes, int m_sizes_dtype, void *y, int64_t R, int N,
+                            int K, int E, int in_dtype, int out_dtype, void *stream) {
+    int rc = check_fused(src_rows, row_idx, idx_div, m_sizes, m_sizes_dtype, R, N, K, E, in_dtype, out_dtype);
+    if (rc) return rc;
+    Nf4Matrix m;
+    rc = nf4_matrix_of(w, N, K, E, m);
+    if (rc) return rc;
+    return fwd_nf4(x_src, src_rows, row_idx, idx_div, m, m_sizes, m_sizes_dtype, y, R, N, K, E, in_dtype, out_dtype, stream);
 }
 
 int mfl_gemm_dx_nf4(const void *dy, const uint8_t *wq, const float *code16, const float *absmax, int blocksize,
@@ -364,18 +406,10 @@ int mfl_gemm_fwd_nf4_gather(const void *x_src, int64_t src_rows, const int32_t *
                             void *stream) {
     int rc = check_fused(src_rows, row_idx, idx_div, m_sizes, m_sizes_dtype, R, N, K, E, in_dtype, out_dtype);
     if (rc) return rc;
-    if (blocksize < 2 || (blocksize & (blocksize - 1)) != 0) return MFL_ERR_SHAPE;
-    if (K % 2 != 0 || ((int64_t)E * N * K) % blocksize != 0) return MFL_ERR_SHAPE;
-    if (!wq || !code16 || !absmax || (R > 0 && (!x_src || !row_idx || !y))) return MFL_ERR_NULL;
-    if (R == 0) return MFL_OK;
-    if (in_dtype != MFL_BF16) return MFL_ERR_UNSUPPORTED;
-    const GemmFusion fu = {row_idx, idx_div, src_rows, nullptr, nullptr, nullptr, 0, nullptr, nullptr};
-    const int ms_i64 = m_sizes_dtype == MFL_I64;
-    rc = gemm_nf4_decode(x_src, wq, code16, absmax, blocksize, m_sizes, ms_i64, y, R, N, K, E, out_dtype,
-                         (hipStream_t)stream, &fu);
-    if (rc != MFL_ERR_UNSUPPORTED) return rc;
-    return gemm_nf4_pipe(x_src, wq, code16, absmax, blocksize, m_sizes, ms_i64, y, R, N, K, E, out_dtype,
-                         (hipStream_t)stream, &fu);
+    if (!blocksize_ok(blocksize)) return MFL_ERR_SHAPE;
+    if (R > 0 && !row_idx) return MFL_ERR_NULL;
+    return fwd_nf4(x_src, src_rows, row_idx, idx_div, nf4_matrix(wq, code16, absmax, nullptr, blocksize, N, K, E), m_sizes,
+                   m_sizes_dtype, y, R, N, K, E, in_dtype, out_dtype, stream);
 }
 
 int mfl_glu_fwd(const void *x, int64_t src_rows, const int32_t *row_idx, int idx_div, const void *w_gate,
@@ -406,6 +440,22 @@ int mfl_glu_fwd_lora(const void *x, const void *w_gate, const void *w_up, const 
                           (hipStream_t)stream, &fu);
 }
 
+static int glu_fwd_nf4(const void *x, int64_t src_rows, const int32_t *row_idx, int idx_div, const Nf4Matrix &gate,
+                       const Nf4Matrix &up, const void *m_sizes, int m_sizes_dtype, void *h, void *e_out, void *g_out,
+                       int64_t R, int N, int K, int E, int dtype, void *stream) {
+    if (R > 0 && (!x || !h)) return MFL_ERR_NULL;
+    if (R == 0) return MFL_OK;
+    if (dtype != MFL_BF16) return MFL_ERR_UNSUPPORTED;
+    const int ms_i64 = m_sizes_dtype == MFL_I64;
+    const int rc = gemm_nf4_decode(x, row_idx, idx_div, gate, up, true, m_sizes, ms_i64, h, e_out, g_out, R, N, K, E,
+                                   MFL_BF16, (hipStream_t)stream);
+    if (rc != MFL_ERR_UNSUPPORTED || gate.nested() || up.nested()) return rc;
+    const GemmFusion fu = {row_idx,   idx_div,           src_rows, up.wq, up.code16, up.absmax,
+                           1 << up.bs_shift, e_out, g_out};
+    return gemm_nf4_pipe(x, gate.wq, gate.code16, gate.absmax, 1 << gate.bs_shift, m_sizes, ms_i64, h, R, N, K, E, MFL_BF16,
+                         (hipStream_t)stream, &fu);
+}
+
 int mfl_glu_fwd_nf4_tiled(const void *x, int64_t src_rows, const int32_t *row_idx, int idx_div, const uint8_t *wq_gate,
                           const float *code16_gate, const float *absmax_gate, const float *absmax_tiled_gate,
                           int blocksize_gate, const uint8_t *wq_up, const float *code16_up, const float *absmax_up,
@@ -413,27 +463,25 @@ int mfl_glu_fwd_nf4_tiled(const void *x, int64_t src_rows, const int32_t *row_id
                           void *h, void *e_out, void *g_out, int64_t R, int N, int K, int E, int dtype, void *stream) {
     int rc = check_fused(src_rows, row_idx, idx_div, m_sizes, m_sizes_dtype, R, N, K, E, dtype, dtype);
     if (rc) return rc;
-    for (int bs : {blocksize_gate, blocksize_up}) {
-        if (bs < 2 || (bs & (bs - 1)) != 0 || ((int64_t)E * N * K) % bs != 0) return MFL_ERR_SHAPE;
-    }
+    for (int bs : {blocksize_gate, blocksize_up})
+        if (!blocksize_ok(bs) || ((int64_t)E * N * K) % bs != 0) return MFL_ERR_SHAPE;
     if (K % 2 != 0) return MFL_ERR_SHAPE;
-    if (!wq_gate || !code16_gate || !absmax_gate || !wq_up || !code16_up || !absmax_up || (R > 0 && (!x || !h)))
-        return MFL_ERR_NULL;
-    if (R == 0) return MFL_OK;
-    if (dtype != MFL_BF16) return MFL_ERR_UNSUPPORTED;
-    GemmFusion fu = {row_idx, idx_div, src_rows, wq_up, code16_up, absmax_up, blocksize_up, e_out, g_out};
-    // the tile-ordered scales serve where both matrices have them
-    if (absmax_tiled_gate != nullptr && absmax_tiled_up != nullptr &&
-        nf4_tiled_absmax_floats(blocksize_gate, N, K, E) != 0 && nf4_tiled_absmax_floats(blocksize_up, N, K, E) != 0) {
-        fu.absmax_tiled = absmax_tiled_gate;
-        fu.absmax_tiled_2 = absmax_tiled_up;
-    }
-    const int ms_i64 = m_sizes_dtype == MFL_I64;
-    rc = gemm_nf4_decode(x, wq_gate, code16_gate, absmax_gate, blocksize_gate, m_sizes, ms_i64, h, R, N, K, E, MFL_BF16,
-                         (hipStream_t)stream, &fu);
-    if (rc != MFL_ERR_UNSUPPORTED) return rc;
-    return gemm_nf4_pipe(x, wq_gate, code16_gate, absmax_gate, blocksize_gate, m_sizes, ms_i64, h, R, N, K, E, MFL_BF16,
-                         (hipStream_t)stream, &fu);
+    if (!wq_gate || !code16_gate || !absmax_gate || !wq_up || !code16_up || !absmax_up) return MFL_ERR_NULL;
+    return glu_fwd_nf4(x, src_rows, row_idx, idx_div,
+                       nf4_matrix(wq_gate, code16_gate, absmax_gate, absmax_tiled_gate, blocksize_gate, N, K, E),
+                       nf4_matrix(wq_up, code16_up, absmax_up, absmax_tiled_up, blocksize_up, N, K, E), m_sizes,
+                       m_sizes_dtype, h, e_out, g_out, R, N, K, E, dtype, stream);
+}
+
+int mfl_glu_fwd_nf4_packed(const void *x, int64_t src_rows, const int32_t *row_idx, int idx_div, const mfl_nf4_weight *gate,
+                           const mfl_nf4_weight *up, const void *m_sizes, int m_sizes_dtype, void *h, void *e_out,
+                           void *g_out, int64_t R, int N, int K, int E, int dtype, void *stream) {
+    int rc = check_fused(src_rows, row_idx, idx_div, m_sizes, m_sizes_dtype, R, N, K, E, dtype, dtype);
+    if (rc) return rc;
+    Nf4Matrix mg, mu;
+    if ((rc = nf4_matrix_of(gate, N, K, E, mg)) != 0 || (rc = nf4_matrix_of(up, N, K, E, mu)) != 0) return rc;
+    return glu_fwd_nf4(x, src_rows, row_idx, idx_div, mg, mu, m_sizes, m_sizes_dtype, h, e_out, g_out, R, N, K, E, dtype,
+                       stream);
 }
 
 int mfl_glu_fwd_nf4(const void *x, int64_t src_rows, const int32_t *row_idx, int idx_div, const uint8_t *wq_gate,
@@ -460,6 +508,13 @@ int mfl_dequant_blockwise_u8(const uint8_t *v, const float *code256, const float
     if (n < 0 || blocksize2 <= 0) return MFL_ERR_SHAPE;
     if (n > 0 && (!v || !code256 || !absmax2 || !out)) return MFL_ERR_NULL;
     return dequant_blockwise_u8(v, code256, absmax2, blocksize2, offset, out, n, (hipStream_t)stream);
+}
+
+int mfl_nf4_unnest_absmax(const uint8_t *v, const float *code256, const float *absmax2, int blocksize2,
+                          const float *offset, float *out, int64_t n, void *stream) {
+    if (n < 0 || !blocksize_ok(blocksize2)) return MFL_ERR_SHAPE;
+    if (n > 0 && (!v || !code256 || !absmax2 || !offset || !out)) return MFL_ERR_NULL;
+    return nf4_unnest_absmax(v, code256, absmax2, blocksize2, offset, out, n, (hipStream_t)stream);
 }
 
 int mfl_nf4_quant(const void *w, int w_dtype, int64_t n, int blocksize, const float *code16, uint8_t *wq, float *absmax,

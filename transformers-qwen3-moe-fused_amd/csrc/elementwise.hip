@@ -373,6 +373,36 @@ __global__ __launch_bounds__(256) void dequant_u8_kernel(const uint8_t *__restri
         out[i] = code[v[i]] * absmax2[i / blocksize2] + offset;
 }
 
+// The fp32 scales of a double-quantised matrix, offset included, 16 at a time: 16 bytes in and 64 out per lane.  Two
+// launches of a byte per lane each (scales, then the offset) took 10.0 + 6.6 us for 3.1 M scales.
+__global__ __launch_bounds__(256) void nf4_unnest_kernel(const uint8_t *__restrict__ v, const float *__restrict__ code256,
+                                                         const float *__restrict__ absmax2, int bs2_shift,
+                                                         const float *__restrict__ offset, float *__restrict__ out,
+                                                         int64_t n, int vec_ok) {
+    __shared__ float code[256];
+    code[threadIdx.x] = code256[threadIdx.x];
+    const float off = *offset;
+    __syncthreads();
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (vec_ok) {
+        const int64_t nv = n / 16;
+        for (int64_t q = i; q < nv; q += stride) {
+            const uint4_t b = ((const uint4_t *)v)[q];
+            const float am = absmax2[(q * 16) >> bs2_shift];
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                floatx4 o;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) o[u] = code[(b[d] >> (8 * u)) & 0xffu] * am + off;
+                ((floatx4 *)out)[q * 4 + d] = o;
+            }
+        }
+        i += nv * 16;
+    }
+    for (; i < n; i += stride) out[i] = code[v[i]] * absmax2[i >> bs2_shift] + off;
+}
+
 // One wave per quantisation block.
 template <typename T>
 __global__ __launch_bounds__(256) void nf4_quant_kernel(const T *__restrict__ w, int64_t nblocks, int blocksize,
@@ -497,6 +527,16 @@ int dequant_blockwise_u8(const uint8_t *v, const float *code256, const float *ab
                          float *out, int64_t n, hipStream_t stream) {
     if (n == 0) return MFL_OK;
     dequant_u8_kernel<<<stream_grid(n), 256, 0, stream>>>(v, code256, absmax2, blocksize2, offset, out, n);
+    return launch_status();
+}
+
+int nf4_unnest_absmax(const uint8_t *v, const float *code256, const float *absmax2, int blocksize2, const float *offset,
+                      float *out, int64_t n, hipStream_t stream) {
+    if (n == 0) return MFL_OK;
+    const int shift = log2_exact(blocksize2);
+    const int vec_ok = aligned(v, 16) && aligned(out, 16) && blocksize2 >= 16;
+    nf4_unnest_kernel<<<stream_grid(vec_ok ? n / 16 + 1 : n), 256, 0, stream>>>(v, code256, absmax2, shift, offset, out, n,
+                                                                                vec_ok);
     return launch_status();
 }
 

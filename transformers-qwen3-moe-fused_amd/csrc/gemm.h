@@ -62,8 +62,6 @@ struct GemmFusion {
     int kt;
     // the same with the gated unit (w2 given, x2 not): thin weights of the second matrix; xt is shared
     const void *wt2;
-    // NF4: tile-ordered copies of the scales of w and w2 (see Nf4Matrix), or null
-    const float *absmax_tiled, *absmax_tiled_2;
     // DX with the backward of the gated unit in its epilogue (bw_e given): the product dh = dy w is not stored;
     // de, dg (and h = silu(e) g where bw_h is given) are computed from it and the forward products e, g (all
     // (R, N) bf16; de may be e and dg may be g) as silu_mul_bwd computes them from a stored dh
@@ -104,6 +102,11 @@ struct Nf4Matrix {
     // The scales once more in the order in which the streaming kernel's waves consume them (nf4_tile_absmax),
     // or null: [expert][32-column tile][128-wide reduction stage][column of the tile][half of the stage].
     const float *absmax_tiled = nullptr;
+    // Double quantisation, instead of absmax: scale b = code256[absmax_u8[b]] * absmax2[b >> bs2_shift] + *offset.
+    const uint8_t *absmax_u8 = nullptr;
+    const float *code256 = nullptr, *absmax2 = nullptr, *offset = nullptr;
+    int bs2_shift = 0;
+    __host__ __device__ bool nested() const { return absmax_u8 != nullptr; }
 };
 
 // Writes the tile-ordered copy of an (E, N, K) matrix's scales: E * ceil(N / 32) * (K / 128) * 64 floats
@@ -124,11 +127,11 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
                   bool glu, const void *m_sizes, int ms_i64, void *y, void *e_out, void *g_out, int64_t R, int N,
                   int K, int E, int out_dtype, hipStream_t stream);
 
-// Forward with NF4 weights for decode-sized batches (at most 32 rows per expert on average):
-// weights decoded in registers, no LDS stage.
-int gemm_nf4_decode(const void *x, const uint8_t *wq, const float *code16, const float *absmax, int blocksize,
-                    const void *m_sizes, int ms_i64, void *y, int64_t R, int N, int K, int E, int out_dtype,
-                    hipStream_t stream, const GemmFusion *fusion = nullptr);
+// Forward with NF4 weights for decode-sized batches: the matrix-vector, streaming or register-decoding kernel.  glu:
+// w0 is the gate and w1 the up projection (else w1 is not read).  A double-quantised matrix is taken by the first two.
+int gemm_nf4_decode(const void *x, const int32_t *row_idx, int idx_div, const Nf4Matrix &w0, const Nf4Matrix &w1, bool glu,
+                    const void *m_sizes, int ms_i64, void *y, void *e_out, void *g_out, int64_t R, int N, int K, int E,
+                    int out_dtype, hipStream_t stream);
 
 // Pipelined forward with NF4 weights decoded into LDS one step ahead of the multiply.
 int gemm_nf4_pipe(const void *x, const uint8_t *wq, const float *code16, const float *absmax, int blocksize,

@@ -284,44 +284,18 @@ __global__ __launch_bounds__(256) void nf4_decode_kernel(const bf16_t *__restric
 
 }  // namespace
 
-int gemm_nf4_decode(const void *x, const uint8_t *wq, const float *code16, const float *absmax, int blocksize,
-                    const void *m_sizes, int ms_i64, void *y, int64_t R, int N, int K, int E, int out_dtype,
-                    hipStream_t stream, const GemmFusion *fusion) {
+int gemm_nf4_decode(const void *x, const int32_t *row_idx, int idx_div, const Nf4Matrix &w0, const Nf4Matrix &w1_, bool glu,
+                    const void *m_sizes, int ms_i64, void *y, void *e_out, void *g_out, int64_t R, int N, int K, int E,
+                    int out_dtype, hipStream_t stream) {
     // up to where the streaming kernel (64-row tiles) is ahead of the pipelined one: with more rows per expert every
     // row tile streams and decodes the weights again
-    const bool gated = fusion != nullptr && fusion->w2 != nullptr;
     if (R <= 0) return MFL_OK;
-    if (R > (int64_t)(gated ? kNf4StreamGatedRowsPerExpert : kNf4StreamRowsPerExpert) * E) return MFL_ERR_UNSUPPORTED;
-    int shift = 0;
-    while ((1 << shift) < blocksize) ++shift;
-    if (K % 64 != 0 || N % 8 != 0 || N < 8 || blocksize < 8) return MFL_ERR_UNSUPPORTED;
-    if (!aligned(x, 16) || !aligned(wq, 16) || !aligned(y, 16)) return MFL_ERR_UNSUPPORTED;
-    if (out_dtype != MFL_BF16 && out_dtype != MFL_F32) return MFL_ERR_UNSUPPORTED;
-    Nf4Matrix w0 = {wq, code16, absmax, shift};
-    if (fusion != nullptr) w0.absmax_tiled = fusion->absmax_tiled;
-    Nf4Matrix w1 = w0;
-    const int32_t *row_idx = nullptr;
-    int idx_div = 1;
-    void *e_out = nullptr, *g_out = nullptr;
-    bool glu = false;
-    if (fusion != nullptr) {
-        if (fusion->row_idx != nullptr) {
-            if (fusion->idx_div <= 0 || fusion->src_rows <= 0) return MFL_ERR_UNSUPPORTED;
-            row_idx = fusion->row_idx;
-            idx_div = fusion->idx_div;
-        }
-        if (fusion->w2 != nullptr) {
-            int shift2 = 0;
-            while ((1 << shift2) < fusion->blocksize_2) ++shift2;
-            if (out_dtype != MFL_BF16 || fusion->blocksize_2 < 8 || !fusion->code16_2 || !fusion->absmax_2 ||
-                !aligned(fusion->w2, 16) || !aligned(fusion->e_out, 8) || !aligned(fusion->g_out, 8))
-                return MFL_ERR_UNSUPPORTED;
-            glu = true;
-            w1 = Nf4Matrix{(const uint8_t *)fusion->w2, fusion->code16_2, fusion->absmax_2, shift2, fusion->absmax_tiled_2};
-            e_out = fusion->e_out;
-            g_out = fusion->g_out;
-        }
-    }
+    if (R > (int64_t)(glu ? kNf4StreamGatedRowsPerExpert : kNf4StreamRowsPerExpert) * E) return MFL_ERR_UNSUPPORTED;
+    const Nf4Matrix &w1 = glu ? w1_ : w0;
+    if (K % 64 != 0 || N % 8 != 0 || N < 8 || w0.bs_shift < 3 || w1.bs_shift < 3) return MFL_ERR_UNSUPPORTED;
+    if (!aligned(x, 16) || !aligned(w0.wq, 16) || !aligned(w1.wq, 16) || !aligned(y, 16)) return MFL_ERR_UNSUPPORTED;
+    if (out_dtype != MFL_BF16 && (glu || out_dtype != MFL_F32)) return MFL_ERR_UNSUPPORTED;
+    if (!aligned(e_out, 8) || !aligned(g_out, 8)) return MFL_ERR_UNSUPPORTED;
     // 128 columns per workgroup: the most workgroups per expert (two blocks per wave: slower)
     const int tiles_n = ceil_div(N, 128);
     const int64_t row_tiles = R / 32 + (R < E ? R : E);  // upper bound on sum over experts of ceil(m / 32)
@@ -339,6 +313,7 @@ int gemm_nf4_decode(const void *x, const uint8_t *wq, const float *code16, const
         if (rc != MFL_ERR_UNSUPPORTED) return rc;
     }
     if (R > (int64_t)kNf4DecodeRowsPerExpert * E) return MFL_ERR_UNSUPPORTED;  // 32-row tiles from here on
+    if (w0.nested() || w1.nested()) return MFL_ERR_UNSUPPORTED;
     const bool wide = K % 256 == 0;  // 64 packed bytes per lane and super-step
     const bool am1 = w0.bs_shift >= 5 && w1.bs_shift >= 5;  // one scale per lane and step
     const bool xstage = R > 2 * (int64_t)E;                   // rows change hands in LDS

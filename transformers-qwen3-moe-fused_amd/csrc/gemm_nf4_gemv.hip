@@ -88,8 +88,19 @@ __device__ __forceinline__ void lookup4(uint32_t (&pr)[4], uint32_t a0, uint32_t
         : "v"(a0), "v"(a1), "v"(a2), "v"(a3));
 }
 
+// the same with a fifth read of its own address
+__device__ __forceinline__ void lookup5(uint32_t (&pr)[4], float &f, uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3,
+                                        uint32_t af) {
+    asm volatile(
+        "ds_read_b32 %4, %9\n\tds_read_b32 %0, %5\n\tds_read_b32 %1, %6\n\tds_read_b32 %2, %7\n\tds_read_b32 %3, %8\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(pr[0]), "=&v"(pr[1]), "=&v"(pr[2]), "=&v"(pr[3]), "=&v"(f)
+        : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "v"(af));
+}
+
 constexpr int kGemvThreads = 1024;
 constexpr int kGemvTable = 65536;
+constexpr int kGemvScales = 2048;  // scales by 8-bit value, of either matrix (double-quantised matrices)
 
 
 // The LDS address of the pair of packed byte `B` of w: 256 * byte + lane_copy (the lane's copy of the table, one
@@ -101,7 +112,7 @@ __device__ __forceinline__ uint32_t pair_address(uint32_t w, uint32_t lane_copy)
 }
 
 // NL: loads per column (K <= 512 NL); ROWS: rows per group; D: columns whose loads a wave keeps in flight
-template <int NL, int ROWS, int D, bool GLU, bool EXACT, bool HALF, typename TO>
+template <int NL, int ROWS, int D, bool GLU, bool EXACT, bool HALF, bool NESTED, typename TO>
 __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__restrict__ x,
                                                                 const int32_t *__restrict__ row_idx, int idx_div,
                                                                 Nf4Matrix w0, Nf4Matrix w1,
@@ -120,7 +131,7 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
     static_assert(D % CB == 0, "the matrix of a ring slot is fixed");
     extern __shared__ __attribute__((aligned(256))) unsigned char smem[];
     unsigned char *const table = smem;                      // kGemvTable bytes
-    int *const grp_e = (int *)(smem + kGemvTable);          // expert | rows << 16
+    int *const grp_e = (int *)(smem + kGemvTable + (NESTED ? kGemvScales : 0));          // expert | rows << 16
     int *const grp_r = grp_e + max_groups;                  // first row
     int *const n_groups_s = grp_r + max_groups;
     int *const ms_s = n_groups_s + 1;                       // the E counts
@@ -155,6 +166,8 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
             for (int j = 0; j < 4; ++j) dst[j] = v;
         }
     }
+    if constexpr (NESTED)
+        if (tid < 256 * CB) ((float *)(table + kGemvTable))[tid] = (tid < 256 ? w0 : w1).code256[tid & 255];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int e = tid + j * kGemvThreads;
@@ -211,7 +224,13 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
 
     // ---- the ring of columns ahead
     uint32_t ring_w[D][COLS][NL];  // a slot: the wave's columns of a unit
-    float ring_a[D][COLS][NL];
+    float ring_a[D][COLS][NL];     // the scale; double-quantised: its second-level factor,
+    uint32_t ring_q[NESTED ? D : 1][COLS][NL];  // and its 8-bit value
+    float q_off[CB];
+    if constexpr (NESTED) {
+        q_off[0] = *w0.offset;
+        if constexpr (CB == 2) q_off[1] = *w1.offset;
+    }
     // Cursor of the loads: the wave's column of unit ic of group ig.  The pointers move on by 16 columns per unit
     // (N % 16 == 0: every unit is whole) and are set up afresh when the group changes: a handful of scalar
     // instructions per column instead of the 64-bit products, which with 16 waves to a CU are what the scalar
@@ -221,13 +240,20 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
     int i_units_left = (int)(u_end - u_begin);
     const uint32_t *i_wp[CB];
     const float *i_ap[CB];
+    const uint8_t *i_qp[CB];
+    int64_t i_b[CB];  // double-quantised: number of the first scale behind i_qp
     auto point_loads = [&]() {
         const int expert = __builtin_amdgcn_readfirstlane(grp_e[ig]) & 0xffff;
         const int64_t base = ((int64_t)expert * N + ic * UCOLS + wave) * K;
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
             i_wp[cb] = (const uint32_t *)(mat[cb].wq + (base >> 1));
-            i_ap[cb] = mat[cb].absmax + (base >> mat[cb].bs_shift);
+            if constexpr (NESTED) {
+                i_b[cb] = base >> mat[cb].bs_shift;
+                i_qp[cb] = mat[cb].absmax_u8 + i_b[cb];
+            } else {
+                i_ap[cb] = mat[cb].absmax + (base >> mat[cb].bs_shift);
+            }
         }
     };
     point_loads();
@@ -243,10 +269,21 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
             ring_w[d][0][i] = i_wp[cb][w_idx];
             // (computed here: a register per load and matrix less)
             const uint32_t a_off = (x_off[i] >> mat[cb].bs_shift) + (HALF ? (lane >> 5) * a_step[cb] : 0);
-            ring_a[d][0][i] = i_ap[cb][a_off];
+            // (E N K / 64 scales: their numbers fit 32 bits, which the launcher checks)
+            if constexpr (NESTED) {
+                ring_q[d][0][i] = i_qp[cb][a_off];
+                ring_a[d][0][i] = mat[cb].absmax2[((uint32_t)i_b[cb] + a_off) >> mat[cb].bs2_shift];
+            } else {
+                ring_a[d][0][i] = i_ap[cb][a_off];
+            }
             if constexpr (COLS == 2) {
                 ring_w[d][1][i] = i_wp[cb][w_step + w_idx];
-                ring_a[d][1][i] = i_ap[cb][a_step[cb] + a_off];
+                if constexpr (NESTED) {
+                    ring_q[d][1][i] = i_qp[cb][a_step[cb] + a_off];
+                    ring_a[d][1][i] = mat[cb].absmax2[((uint32_t)i_b[cb] + a_step[cb] + a_off) >> mat[cb].bs2_shift];
+                } else {
+                    ring_a[d][1][i] = i_ap[cb][a_step[cb] + a_off];
+                }
             }
         }
         // past the end the cursor stays on the last unit: loads that nobody uses
@@ -260,7 +297,12 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
 #pragma unroll
                 for (int c2 = 0; c2 < CB; ++c2) {
                     i_wp[c2] += (UCOLS / 16) * w_step;
-                    i_ap[c2] += (UCOLS / 16) * a_step[c2];
+                    if constexpr (NESTED) {
+                        i_b[c2] += (UCOLS / 16) * a_step[c2];
+                        i_qp[c2] += (UCOLS / 16) * a_step[c2];
+                    } else {
+                        i_ap[c2] += (UCOLS / 16) * a_step[c2];
+                    }
                 }
             }
         }
@@ -317,15 +359,25 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
 #pragma unroll
                     for (int c = 0; c < COLS; ++c) {
                         uint32_t pr[4];
-                        lookup4(pr, pair_address<0>(ring_w[d][c][i], lane_copy), pair_address<1>(ring_w[d][c][i], lane_copy),
-                                pair_address<2>(ring_w[d][c][i], lane_copy), pair_address<3>(ring_w[d][c][i], lane_copy));
+                        const uint32_t w = ring_w[d][c][i];
+                        float scale = ring_a[d][c][i];
+                        if constexpr (NESTED) {
+                            float q;
+                            lookup5(pr, q, pair_address<0>(w, lane_copy), pair_address<1>(w, lane_copy),
+                                    pair_address<2>(w, lane_copy), pair_address<3>(w, lane_copy),
+                                    ring_q[d][c][i] * 4 + (kGemvTable + cb * 1024));
+                            scale = q * scale + q_off[cb];
+                        } else {
+                            lookup4(pr, pair_address<0>(w, lane_copy), pair_address<1>(w, lane_copy),
+                                    pair_address<2>(w, lane_copy), pair_address<3>(w, lane_copy));
+                        }
 #pragma unroll
                         for (int r = 0; r < rn; ++r) {
                             float s = dot2_bf16(pr[0], xr[r][i][0], 0.f);
                             s = dot2_bf16(pr[1], xr[r][i][1], s);
                             s = dot2_bf16(pr[2], xr[r][i][2], s);
                             s = dot2_bf16(pr[3], xr[r][i][3], s);
-                            acc[c][r] = __builtin_fmaf(ring_a[d][c][i], s, acc[c][r]);
+                            acc[c][r] = __builtin_fmaf(scale, s, acc[c][r]);
                         }
                     }
                 }
@@ -393,13 +445,13 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
         if (d < rest) column(d, false);
 }
 
-template <int NL, int ROWS, int D, bool GLU, bool EXACT, bool HALF, typename TO>
+template <int NL, int ROWS, int D, bool GLU, bool EXACT, bool HALF, bool NESTED, typename TO>
 int launch_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf4Matrix &w0, const Nf4Matrix &w1,
                 const void *m_sizes, int ms_i64, TO *y, TO *e_out, TO *g_out, int64_t R, int N, int K, int E,
                 hipStream_t stream) {
     const int64_t max_groups = R / ROWS + (R < E ? R : E);  // upper bound on sum over experts of ceil(m / ROWS)
-    const int lds = kGemvTable + (int)max_groups * 8 + 16 + E * 4;
-    auto *kernel = nf4_gemv_kernel<NL, ROWS, D, GLU, EXACT, HALF, TO>;
+    const int lds = kGemvTable + kGemvScales + (int)max_groups * 8 + 16 + E * 4;
+    auto *kernel = nf4_gemv_kernel<NL, ROWS, D, GLU, EXACT, HALF, NESTED, TO>;
     static PerDeviceOnce attr;
     // The table lookups take the dynamic LDS to start at address 0; static LDS in this kernel would move it, so
     // such a build is left to the kernels that decode in registers.
@@ -409,7 +461,7 @@ int launch_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf4M
         const hipError_t e1 = hipFuncGetAttributes(&fa, (const void *)kernel);
         if (e1 != hipSuccess) return e1;
         static_lds.store((int)fa.sharedSizeBytes, std::memory_order_release);
-        return hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kGemvTable + 4096 * 8 + 16 + 2048 * 4);
+        return hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kGemvTable + kGemvScales + 4096 * 8 + 16 + 2048 * 4);
     });
     if (e != hipSuccess) return (int)e;
     if (static_lds.load(std::memory_order_acquire) != 0) return MFL_ERR_UNSUPPORTED;
@@ -425,8 +477,10 @@ int dispatch_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
                   int K, int E, int out_dtype, hipStream_t stream) {
     const bool exact = !HALF && K % 512 == 0;
 #define MFL_GEMV(GLU, EXACT, TO, Y, EO, GO)                                                                         \
-    launch_gemv<NL, ROWS, ((GLU || HALF) ? 4 : 2), GLU, (EXACT && !HALF), HALF, TO>(x, row_idx, idx_div, w0, w1, m_sizes, \
-                                                                                 ms_i64, Y, EO, GO, R, N, K, E, stream)
+    (w0.nested() ? launch_gemv<NL, ROWS, ((GLU || HALF) ? 4 : 2), GLU, (EXACT && !HALF), HALF, true, TO>(              \
+                       x, row_idx, idx_div, w0, w1, m_sizes, ms_i64, Y, EO, GO, R, N, K, E, stream)                 \
+                 : launch_gemv<NL, ROWS, ((GLU || HALF) ? 4 : 2), GLU, (EXACT && !HALF), HALF, false, TO>(             \
+                       x, row_idx, idx_div, w0, w1, m_sizes, ms_i64, Y, EO, GO, R, N, K, E, stream))
     if (glu)
         return exact ? MFL_GEMV(true, true, bf16_t, (bf16_t *)y, (bf16_t *)e_out, (bf16_t *)g_out)
                      : MFL_GEMV(true, false, bf16_t, (bf16_t *)y, (bf16_t *)e_out, (bf16_t *)g_out);
@@ -457,6 +511,8 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
         // a lane's 8 weights under one scale, and every column starts a quantisation block
         if (m.bs_shift < 3 || (K & ((1 << m.bs_shift) - 1)) != 0) return MFL_ERR_UNSUPPORTED;
         if (!aligned(m.absmax, 4) || !aligned(m.wq, 4)) return MFL_ERR_UNSUPPORTED;
+        if (m.nested() != w0.nested() || (m.nested() && (((int64_t)E * N * K) >> m.bs_shift) > 0x7fffffff))
+            return MFL_ERR_UNSUPPORTED;
     }
     if (!aligned(x, 16)) return MFL_ERR_UNSUPPORTED;
 #define MFL_GEMV_D(NL, ROWS, HALF) \

@@ -57,6 +57,12 @@ __device__ __forceinline__ void copy4_to_lds(const void *src, unsigned char *dst
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(lds_addr) : "memory");
 }
 
+// Two bytes per lane, zero-extended to the lane's dword of LDS.
+__device__ __forceinline__ void copy2_to_lds(const void *src, unsigned char *dst) {
+    const uint32_t lds_addr = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void_ptr)dst);
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_ushort %0, off" : : "v"(src), "s"(lds_addr) : "memory");
+}
+
 // (byte `B` of w) << 2: the LDS byte offset of the pair-table entry of two packed weights, in one instruction.
 template <int B>
 __device__ __forceinline__ uint32_t byte_times_4(uint32_t w) {
@@ -73,18 +79,25 @@ __device__ __forceinline__ uint32_t byte_times_4(uint32_t w) {
     return r;
 }
 
-template <bool GLU, int MR, int RING_>
+// Where the scales come from: each column's own run of fp32 values, the tile-ordered copy, or the 8-bit values of a
+// double-quantised matrix.
+enum { SC_PLAIN = 0, SC_TILED = 1, SC_NESTED = 2 };
+
+template <bool GLU, int SC, int MR, int RING_>
 struct StreamShape {
     static constexpr int CB = GLU ? 2 : 1;     // weight matrices per wave
     static constexpr int RING = RING_;         // stages in LDS; all but one of them in flight
     static constexpr int kX = MR * 32 * 256;   // rows of a stage: MR blocks of 32
     static constexpr int kW = 32 * 64;         // packed weights of a stage, per wave and matrix
-    static constexpr int kA = 32 * 2 * 4;      // scales of a stage, per wave and matrix
+    // scales of a stage, per wave and matrix: two floats per column, or one dword with two 8-bit values
+    static constexpr int kA = SC == SC_NESTED ? 32 * 4 : 32 * 2 * 4;
     static constexpr int kStage = kX + 4 * CB * (kW + kA);
     static constexpr int kTable = CB * 256 * 4;
+    static constexpr int kTables = kTable * (SC == SC_NESTED ? 2 : 1);  // pairs of weights; scales by 8-bit value
     // RING 3, MR 1: 53248, three workgroups per CU; gated: 81920, two.  RING 2, MR 2: 52224, three; gated: 71680, two.
-    static constexpr int kLds = RING * kStage + kTable;
-    static constexpr int kWOps = 2 * CB + CB;  // copies of weights and scales per wave and stage (the rows: up to 2 MR more)
+    // (8-bit scales: 52736, 80896, 52224 and 71680: the same residency)
+    static constexpr int kLds = RING * kStage + kTables;
+    static constexpr int kWOps = 2 * CB + (SC == SC_NESTED ? 1 : CB);  // copies of weights and scales per wave and stage (the rows: up to 2 MR more)
 };
 
 // at most OPS + xc (xc = 0 .. XMAX, wave-uniform) vector-memory operations outstanding
@@ -98,7 +111,7 @@ __device__ __forceinline__ void wait_stage_ops(int xc) {
     }
 }
 
-template <bool GLU, bool TILED, int MR, int RING_, typename TO>
+template <bool GLU, int SC, int MR, int RING_, typename TO>
 __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restrict__ x,
                                                          const int32_t *__restrict__ row_idx, int idx_div,
                                                          Nf4Matrix w0, Nf4Matrix w1,
@@ -106,13 +119,13 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
                                                          TO *__restrict__ y, TO *__restrict__ e_out,
                                                          TO *__restrict__ g_out, int64_t R, int N, int K, int E,
                                                          int tiles_n) {
-    using S = StreamShape<GLU, MR, RING_>;
+    using S = StreamShape<GLU, SC, MR, RING_>;
     constexpr int CB = S::CB, RING = S::RING, TR = 32 * MR;  // TR: rows of a workgroup's tile
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     // the pair table first, at LDS address 0 (the kernel has no static LDS, which the launcher checks): a lookup's address is then the shifted
     // byte itself plus a constant that fits the instruction's offset field, no add
     unsigned char *const table = smem;
-    unsigned char *const ring = smem + S::kTable;
+    unsigned char *const ring = smem + S::kTables;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, h = lane >> 5;
@@ -130,6 +143,7 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
             pr.e[0] = (bf16_t)mats[cb]->code16[tid >> 4];
             pr.e[1] = (bf16_t)mats[cb]->code16[tid & 15];
             ((uint32_t *)table)[cb * 256 + tid] = pr.u;
+            if constexpr (SC == SC_NESTED) ((float *)(table + S::kTable))[cb * 256 + tid] = mats[cb]->code256[tid];
         }
     }
 
@@ -190,6 +204,26 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
         if (col >= N) col = N - 1;
         a_el[cb] = ((int64_t)expert * N + col) * K + (lane & 1) * 64;
     }
+    // 8-bit scales: lane i brings the two bytes of a stage of column i & 31, of the gate projection's in lanes 0..31
+    // and of the up projection's in lanes 32..63; 32 columns' runs are one run of memory.  The scales of a row
+    // of the matrix (at most 1 << bs2_shift of them) lie under one or two second-level factors.
+    const uint8_t *q_src = nullptr;
+    float q_lo[CB], q_hi[CB], q_off[CB];
+    int q_turn = 0;  // first scale of the column under the second factor
+    if constexpr (SC == SC_NESTED) {
+        int col = j0 + n;
+        if (col >= N) col = N - 1;
+        const int64_t b0 = (((int64_t)expert * N + col) * K) >> 6;
+        q_src = (GLU && h ? w1 : w0).absmax_u8 + b0;
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+            const int sh = mat[cb].bs2_shift;
+            q_lo[cb] = mat[cb].absmax2[b0 >> sh];
+            q_hi[cb] = mat[cb].absmax2[(b0 + (K >> 6) - 1) >> sh];
+            q_off[cb] = *mat[cb].offset;
+        }
+        q_turn = (int)((((b0 >> mat[0].bs2_shift) + 1) << mat[0].bs2_shift) - b0);
+    }
     const bf16_t *x_src[2 * MR];  // copy j: rows 32 (j / 2) + 8 wave + 4 (j % 2) .. + 3, sixteen lanes to a row
 #pragma unroll
     for (int j = 0; j < 2 * MR; ++j) {
@@ -223,10 +257,13 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
                 copy16_to_lds(w_src[cb][j] + (int64_t)stg * 64, base + S::kX + (wave * CB + cb) * S::kW + j * 1024);
             // the wave's 64 scales of the stage: 256 consecutive bytes of the tile-ordered copy where the caller
             // brought one (two lines per copy), else two neighbours out of each column's own run (32 lines)
-            const float *a_src = TILED ? mat[cb].absmax_tiled + ((((int64_t)expert * tiles32 + a_tile) * NS + stg) * 64 + lane)
+            if constexpr (SC == SC_NESTED) continue;
+            const float *a_src = SC == SC_TILED ? mat[cb].absmax_tiled + ((((int64_t)expert * tiles32 + a_tile) * NS + stg) * 64 + lane)
                                        : mat[cb].absmax + ((a_el[cb] + (int64_t)stg * 128) >> mat[cb].bs_shift);
             copy4_to_lds(a_src, base + S::kX + 4 * CB * S::kW + (wave * CB + cb) * S::kA);
         }
+        if constexpr (SC == SC_NESTED)
+            if (GLU || lane < 32) copy2_to_lds(q_src + 2 * stg, base + S::kX + 4 * CB * S::kW + wave * CB * S::kA);
     };
     // ---- where this lane reads a stage: its 16 bytes of packed weights of step s2, its 16 bytes of row n for
     // MFMA ks of step s2
@@ -266,7 +303,11 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb) {
                 wl2[s2][cb] = *(const uint4_t *)(base + S::kX + (wave * CB + cb) * S::kW + w_rd[s2]);
-                am2[s2][cb] = *(const float *)(base + S::kX + 4 * CB * S::kW + (wave * CB + cb) * S::kA + (n * 2 + s2) * 4);
+                const unsigned char *const a_rd = base + S::kX + 4 * CB * S::kW + (wave * CB + cb) * S::kA;
+                if constexpr (SC == SC_NESTED)
+                    am2[s2][cb] = *(const float *)(table + S::kTable + cb * 1024 + a_rd[n * 4 + s2] * 4);
+                else
+                    am2[s2][cb] = *(const float *)(a_rd + (n * 2 + s2) * 4);
             }
         issue(q + RING - 1 < NS ? q + RING - 1 : NS - 1);
         // The eight MFMA steps of the stage in one sequence, the operands of a step (16 bytes of the rows, four
@@ -321,6 +362,11 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
                         blk[m][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa.v, wf.v, blk[m][cb], 0, 0, 0);
                     }
                 }
+                if (SC == SC_NESTED && ks == 3 && m == 0) {
+#pragma unroll
+                    for (int cb = 0; cb < CB; ++cb)
+                        am2[s2][cb] = am2[s2][cb] * (2 * q + s2 < q_turn ? q_lo[cb] : q_hi[cb]) + q_off[cb];
+                }
                 if (ks == 3) {
 #pragma unroll
                     for (int cb = 0; cb < CB; ++cb)
@@ -354,17 +400,17 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
         }
 }
 
-template <bool GLU, bool TILED, int MR, int RING_, typename TO>
+template <bool GLU, int SC, int MR, int RING_, typename TO>
 int launch_stream(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf4Matrix &w0, const Nf4Matrix &w1,
                   const void *m_sizes, int ms_i64, TO *y, TO *e_out, TO *g_out, int64_t R, int N, int K, int E,
                   hipStream_t stream) {
-    using S = StreamShape<GLU, MR, RING_>;
+    using S = StreamShape<GLU, SC, MR, RING_>;
     constexpr int kLds = S::kLds;
     const int tiles_n = ceil_div(N, 128);
     const int64_t row_tiles = R / (32 * MR) + (R < E ? R : E);  // upper bound on sum over experts of ceil(m / (32 MR))
     const int64_t grid = (row_tiles + 7) / 8 * 8 * tiles_n;  // row tiles in eights: one per XCD
     if (grid > 0x7fffffff) return MFL_ERR_UNSUPPORTED;
-    auto *kernel = nf4_stream_kernel<GLU, TILED, MR, RING_, TO>;
+    auto *kernel = nf4_stream_kernel<GLU, SC, MR, RING_, TO>;
     static PerDeviceOnce attr;
     // The kernel's table lookups take the dynamic LDS to start at address 0: any static LDS in this kernel
     // (a later __shared__ variable, an inlined helper that brings one) would move it, so the launcher asks the
@@ -425,7 +471,16 @@ int gemm_nf4_stream(const bf16_t *x, const int32_t *row_idx, int idx_div, const 
                     int K, int E, int out_dtype, hipStream_t stream) {
     // a 64-wide step must lie inside one quantisation block, and the scales are copied four bytes at a time
     if (K % 128 != 0 || w0.bs_shift < 6 || w1.bs_shift < 6) return MFL_ERR_UNSUPPORTED;
-    if (!aligned(w0.absmax, 4) || !aligned(w1.absmax, 4)) return MFL_ERR_UNSUPPORTED;
+    // 8-bit scales: two bytes a stage, so blocks of exactly 64, and a row of the matrix under at most two factors
+    const bool nested = w0.nested();
+    if (nested != w1.nested()) return MFL_ERR_UNSUPPORTED;
+    if (nested) {
+        if (w0.bs_shift != 6 || w1.bs_shift != 6 || w0.bs2_shift != w1.bs2_shift || K / 64 > (1 << w0.bs2_shift) ||
+            !aligned(w0.absmax_u8, 2) || !aligned(w1.absmax_u8, 2))
+            return MFL_ERR_UNSUPPORTED;
+    } else if (!aligned(w0.absmax, 4) || !aligned(w1.absmax, 4)) {
+        return MFL_ERR_UNSUPPORTED;
+    }
     // the tile-ordered scales are used where the caller brought them for every matrix of the product
     const bool tiled = w0.absmax_tiled != nullptr && (!glu || w1.absmax_tiled != nullptr) &&
                        aligned(w0.absmax_tiled, 4) && (!glu || aligned(w1.absmax_tiled, 4));
@@ -435,15 +490,19 @@ int gemm_nf4_stream(const bf16_t *x, const int32_t *row_idx, int idx_div, const 
     // more than a second stage in flight (plain product, 40 rows per expert: 43 us against 55 with three stages
     // and two workgroups per CU, 59 with 32-row tiles).  The bits are the same whatever the tile height.
     const bool two = R > (int64_t)kNf4StreamTwoBlockRows * E;
-#define MFL_STREAM_MR(GLU, MR, RG, TO, Y, EO, GO)                                                                              \
-    (tiled ? launch_stream<GLU, true, MR, RG, TO>(x, row_idx, idx_div, w0, w1, m_sizes, ms_i64, Y, EO, GO, R, N, K, E, stream) \
-           : launch_stream<GLU, false, MR, RG, TO>(x, row_idx, idx_div, w0, w1, m_sizes, ms_i64, Y, EO, GO, R, N, K, E, stream))
+#define MFL_STREAM_SC(GLU, SC, MR, RG, TO, Y, EO, GO) \
+    launch_stream<GLU, SC, MR, RG, TO>(x, row_idx, idx_div, w0, w1, m_sizes, ms_i64, Y, EO, GO, R, N, K, E, stream)
+#define MFL_STREAM_MR(GLU, MR, RG, TO, Y, EO, GO)                            \
+    (nested  ? MFL_STREAM_SC(GLU, SC_NESTED, MR, RG, TO, Y, EO, GO)          \
+     : tiled ? MFL_STREAM_SC(GLU, SC_TILED, MR, RG, TO, Y, EO, GO)           \
+             : MFL_STREAM_SC(GLU, SC_PLAIN, MR, RG, TO, Y, EO, GO))
 #define MFL_STREAM(GLU, TO, Y, EO, GO) (two ? MFL_STREAM_MR(GLU, 2, 2, TO, Y, EO, GO) : MFL_STREAM_MR(GLU, 1, 3, TO, Y, EO, GO))
     if (glu) return MFL_STREAM(true, bf16_t, (bf16_t *)y, (bf16_t *)e_out, (bf16_t *)g_out);
     if (out_dtype == MFL_BF16) return MFL_STREAM(false, bf16_t, (bf16_t *)y, nullptr, nullptr);
     return MFL_STREAM(false, float, (float *)y, nullptr, nullptr);
 #undef MFL_STREAM
 #undef MFL_STREAM_MR
+#undef MFL_STREAM_SC
 }
 
 }  // namespace mfl

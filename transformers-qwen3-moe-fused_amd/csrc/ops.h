@@ -19,6 +19,8 @@ int nf4_dequant(const uint8_t *wq, const float *code16, const float *absmax, int
                 int out_dtype, hipStream_t stream);
 int dequant_blockwise_u8(const uint8_t *v, const float *code256, const float *absmax2, int blocksize2, float offset,
                          float *out, int64_t n, hipStream_t stream);
+int nf4_unnest_absmax(const uint8_t *v, const float *code256, const float *absmax2, int blocksize2, const float *offset,
+                      float *out, int64_t n, hipStream_t stream);
 int nf4_quant(const void *w, int w_dtype, int64_t n, int blocksize, const float *code16, uint8_t *wq, float *absmax,
               hipStream_t stream);
 

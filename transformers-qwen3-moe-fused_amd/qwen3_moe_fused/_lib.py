@@ -24,6 +24,17 @@ _ITYPES = {torch.int32: I32, torch.int64: I64}
 
 _vp, _i, _i64, _f, _sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float, ctypes.c_size_t
 
+
+
+class Nf4Weight(ctypes.Structure):
+    """``mfl_nf4_weight``: a packed 4-bit matrix with its quantisation state, as device pointers."""
+
+    _fields_ = [("packed", _vp), ("code16", _vp), ("absmax", _vp), ("absmax_tiled", _vp), ("absmax_u8", _vp),
+                ("code256", _vp), ("absmax2", _vp), ("offset", _vp), ("blocksize", _i), ("blocksize2", _i)]
+
+
+_nf4p = ctypes.POINTER(Nf4Weight)
+
 # name -> (restype, argtypes); mirrors include/moe_fused_linear.h
 _SIGNATURES = {
     "mfl_abi_version": (_i, []),
@@ -54,8 +65,11 @@ _SIGNATURES = {
                                     _i, _vp]),
     "mfl_glu_fwd_nf4_tiled": (_i, [_vp, _i64, _vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _i, _vp, _i, _vp,
                                    _vp, _vp, _i64, _i, _i, _i, _i, _vp]),
+    "mfl_gemm_fwd_nf4_packed": (_i, [_vp, _i64, _vp, _i, _nf4p, _vp, _i, _vp, _i64, _i, _i, _i, _i, _i, _vp]),
+    "mfl_glu_fwd_nf4_packed": (_i, [_vp, _i64, _vp, _i, _nf4p, _nf4p, _vp, _i, _vp, _vp, _vp, _i64, _i, _i, _i, _i, _vp]),
     "mfl_nf4_dequant": (_i, [_vp, _vp, _vp, _i, _vp, _i64, _i, _vp]),
     "mfl_dequant_blockwise_u8": (_i, [_vp, _vp, _vp, _i, _f, _vp, _i64, _vp]),
+    "mfl_nf4_unnest_absmax": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _i64, _vp]),
     "mfl_nf4_quant": (_i, [_vp, _i, _i64, _i, _vp, _vp, _vp, _vp]),
     "mfl_route_softmax_topk": (_i, [_vp, _i, _i64, _i, _i, _i, _vp, _vp, _i, _vp, _vp]),
     "mfl_route_softmax_topk_bwd": (_i, [_vp, _i, _i64, _i, _i, _i, _vp, _vp, _vp, _i, _vp, _vp]),

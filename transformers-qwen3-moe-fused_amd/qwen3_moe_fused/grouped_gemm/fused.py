@@ -23,12 +23,10 @@ import torch
 from .. import _lib
 from ..kernels.routing import _gather as gather_kernel
 from ..kernels.silu_mul import silu_mul_forward
-from ..quantize.nf4 import resolve_absmax, tiled_absmax
+from ..quantize.nf4 import packed_weight, resolve_absmax
 from ._common import check_operands, is_int_tensor
 from .forward import grouped_gemm_forward
-from .forward_4bit import grouped_gemm_forward_4bit
-
-UNSUPPORTED = -6  # MFL_ERR_UNSUPPORTED
+from .forward_4bit import UNSUPPORTED, check_packed, grouped_gemm_forward_4bit
 
 
 def _gather(x_src: torch.Tensor, row_idx: torch.Tensor, idx_div: int) -> torch.Tensor:
@@ -46,20 +44,8 @@ def _check_gather(x_src: torch.Tensor, row_idx: Optional[torch.Tensor], idx_div:
 
 
 def _nf4_args(w_quant: torch.Tensor, state, x: torch.Tensor, k: int):
-    assert state.quant_type in ("nf4", "fp4")
-    blocksize = int(state.blocksize)
-    assert blocksize > 0 and blocksize & (blocksize - 1) == 0, "blocksize must be a power of two"
-    code = state.code
-    assert code.dtype == torch.float32
-    absmax = resolve_absmax(state)
-    for t in (w_quant, code, absmax):
-        assert t.device == x.device and t.is_contiguous()
-    assert is_int_tensor(w_quant) and len(state.shape) == 3
-    experts, n, k_w = state.shape
-    assert k_w == k and k % 2 == 0
-    total = experts * n * k
-    assert total % blocksize == 0 and w_quant.numel() == total // 2 and absmax.numel() == total // blocksize
-    return code, absmax, blocksize, experts, n
+    experts, n = check_packed(x, w_quant, state, k)
+    return state.code, resolve_absmax(state), int(state.blocksize), experts, n
 
 
 def grouped_gemm_forward_gathered(x_src: torch.Tensor, row_idx: torch.Tensor, idx_div: int, w: torch.Tensor,
@@ -88,26 +74,21 @@ def grouped_gemm_forward_4bit_gathered(x_src: torch.Tensor, row_idx: torch.Tenso
     assert x_src.is_cuda and x_src.is_contiguous() and m_sizes.is_contiguous() and is_int_tensor(m_sizes)
     rows = _check_gather(x_src, row_idx, idx_div)
     k = x_src.shape[1]
-    code, absmax, blocksize, experts, n = _nf4_args(w_quant, w_quant_state, x_src, k)
+    experts, n = check_packed(x_src, w_quant, w_quant_state, k)
     assert m_sizes.numel() == experts
     y = torch.empty((rows, n), device=x_src.device, dtype=x_src.dtype if dtype is None else dtype)
     ms = _lib.as_index_tensor(m_sizes)
-    tiled = tiled_absmax(w_quant_state, absmax, rows)
-    if tiled is not None:
-        rc = _lib.lib().mfl_gemm_fwd_nf4_tiled(_lib.ptr(x_src), x_src.shape[0], _lib.ptr(row_idx), idx_div,
-                                               _lib.ptr(w_quant), _lib.ptr(code), _lib.ptr(absmax), _lib.ptr(tiled),
-                                               blocksize, _lib.ptr(ms), _lib.itype_code(ms.dtype), _lib.ptr(y), rows,
-                                               n, k, experts, _lib.dtype_code(x_src.dtype),
-                                               _lib.dtype_code(y.dtype), _lib.stream())
-    else:
-        rc = _lib.lib().mfl_gemm_fwd_nf4_gather(_lib.ptr(x_src), x_src.shape[0], _lib.ptr(row_idx), idx_div,
-                                                _lib.ptr(w_quant), _lib.ptr(code), _lib.ptr(absmax), blocksize,
-                                                _lib.ptr(ms), _lib.itype_code(ms.dtype), _lib.ptr(y), rows, n, k,
+    for unnested in (False, True):
+        w, _keep = packed_weight(w_quant, w_quant_state, rows, unnested)
+        rc = _lib.lib().mfl_gemm_fwd_nf4_packed(x_src.data_ptr(), x_src.shape[0], row_idx.data_ptr(), idx_div, w,
+                                                ms.data_ptr(), _lib.itype_code(ms.dtype), y.data_ptr(), rows, n, k,
                                                 experts, _lib.dtype_code(x_src.dtype), _lib.dtype_code(y.dtype),
                                                 _lib.stream())
+        if rc != UNSUPPORTED or w.absmax_u8 is None:
+            break
     if rc == UNSUPPORTED:
         return grouped_gemm_forward_4bit(_gather(x_src, row_idx, idx_div), w_quant, w_quant_state, m_sizes, dtype)
-    _lib.check(rc, "mfl_gemm_fwd_nf4_gather")
+    _lib.check(rc, "mfl_gemm_fwd_nf4_packed")
     return y
 
 
@@ -146,27 +127,27 @@ def grouped_glu_forward_4bit(x: torch.Tensor, gate_quant: torch.Tensor, gate_sta
     assert x.is_cuda and x.is_contiguous() and m_sizes.is_contiguous() and is_int_tensor(m_sizes)
     rows = _check_gather(x, row_idx, idx_div)
     k = x.shape[1]
-    code_g, absmax_g, bs_g, experts, n = _nf4_args(gate_quant, gate_state, x, k)
-    code_u, absmax_u, bs_u, experts_u, n_u = _nf4_args(up_quant, up_state, x, k)
-    assert (experts_u, n_u) == (experts, n) and m_sizes.numel() == experts
+    experts, n = check_packed(x, gate_quant, gate_state, k)
+    assert check_packed(x, up_quant, up_state, k) == (experts, n) and m_sizes.numel() == experts
     h = torch.empty((rows, n), device=x.device, dtype=x.dtype)
     e = torch.empty_like(h) if return_products else None
     g = torch.empty_like(h) if return_products else None
     ms = _lib.as_index_tensor(m_sizes)
-    tiled_g, tiled_u = tiled_absmax(gate_state, absmax_g, rows), tiled_absmax(up_state, absmax_u, rows)
-    rc = _lib.lib().mfl_glu_fwd_nf4_tiled(_lib.ptr(x), x.shape[0], _lib.ptr(row_idx), idx_div,
-                                          _lib.ptr(gate_quant), _lib.ptr(code_g), _lib.ptr(absmax_g), _lib.ptr(tiled_g),
-                                          bs_g, _lib.ptr(up_quant), _lib.ptr(code_u), _lib.ptr(absmax_u),
-                                          _lib.ptr(tiled_u), bs_u, _lib.ptr(ms), _lib.itype_code(ms.dtype), _lib.ptr(h),
-                                          _lib.ptr(e), _lib.ptr(g), rows, n, k, experts, _lib.dtype_code(x.dtype),
-                                          _lib.stream())
+    for unnested in (False, True):
+        gate, _keep_gate = packed_weight(gate_quant, gate_state, rows, unnested)
+        up, _keep_up = packed_weight(up_quant, up_state, rows, unnested)
+        rc = _lib.lib().mfl_glu_fwd_nf4_packed(x.data_ptr(), x.shape[0], _lib.ptr(row_idx), idx_div, gate, up, ms.data_ptr(),
+                                               _lib.itype_code(ms.dtype), h.data_ptr(), _lib.ptr(e), _lib.ptr(g), rows, n, k,
+                                               experts, _lib.dtype_code(x.dtype), _lib.stream())
+        if rc != UNSUPPORTED or (gate.absmax_u8 is None and up.absmax_u8 is None):
+            break
     if rc == UNSUPPORTED:
         xg = x if row_idx is None else _gather(x, row_idx, idx_div)
         e = grouped_gemm_forward_4bit(xg, gate_quant, gate_state, m_sizes)
         g = grouped_gemm_forward_4bit(xg, up_quant, up_state, m_sizes)
         h = silu_mul_forward(e, g)
     else:
-        _lib.check(rc, "mfl_glu_fwd_nf4_tiled")
+        _lib.check(rc, "mfl_glu_fwd_nf4_packed")
     return (h, e, g) if return_products else h
 
 

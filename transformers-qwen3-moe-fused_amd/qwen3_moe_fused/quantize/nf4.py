@@ -148,26 +148,51 @@ class BlockwiseState:
     dtype: torch.dtype = torch.float32
 
 
+def _second_level(quant_state):
+    """(uint8 scales, 256-entry code, second-level factors, their block size, offset) of a double-quantised state, all
+    on the scales' device; the offset as a one-element fp32 tensor, never read on the host."""
+    st2 = quant_state.state2
+    absmax = quant_state.absmax.contiguous()
+    code2 = st2.code.to(device=absmax.device, dtype=torch.float32).contiguous()
+    absmax2 = st2.absmax.to(torch.float32).contiguous()
+    offset = quant_state.offset
+    if not torch.is_tensor(offset):
+        offset = torch.tensor(0.0 if offset is None else float(offset), dtype=torch.float32, device=absmax.device)
+    return absmax, code2, absmax2, int(st2.blocksize), offset.to(device=absmax.device, dtype=torch.float32)
+
+
 def resolve_absmax(quant_state) -> torch.Tensor:
     """fp32 absmax of an NF4 state, un-nesting a double-quantised one:
     ``dequantize_blockwise(absmax_u8, state2) + offset`` (forward_4bit.py:149-152)."""
     absmax = quant_state.absmax
     if getattr(quant_state, "nested", False):
-        st2 = quant_state.state2
+        absmax, code2, absmax2, blocksize2, offset = _second_level(quant_state)
         out = torch.empty(absmax.numel(), device=absmax.device, dtype=torch.float32)
-        code2 = st2.code.to(device=absmax.device, dtype=torch.float32).contiguous()
-        absmax2 = st2.absmax.to(torch.float32).contiguous()
-        rc = _lib.lib().mfl_dequant_blockwise_u8(_lib.ptr(absmax.contiguous()), _lib.ptr(code2), _lib.ptr(absmax2),
-                                                 int(st2.blocksize), 0.0, _lib.ptr(out), absmax.numel(),
-                                                 _lib.stream())
-        _lib.check(rc, "mfl_dequant_blockwise_u8")
-        offset = quant_state.offset
-        if offset is not None:
-            # the offset is a device scalar: add it on the device, never read it on the host
-            out += offset.to(device=out.device, dtype=torch.float32) if torch.is_tensor(offset) else float(offset)
+        if blocksize2 & (blocksize2 - 1):
+            rc = _lib.lib().mfl_dequant_blockwise_u8(_lib.ptr(absmax), _lib.ptr(code2), _lib.ptr(absmax2), blocksize2, 0.0,
+                                                     _lib.ptr(out), absmax.numel(), _lib.stream())
+            _lib.check(rc, "mfl_dequant_blockwise_u8")
+            return out.add_(offset)
+        rc = _lib.lib().mfl_nf4_unnest_absmax(_lib.ptr(absmax), _lib.ptr(code2), _lib.ptr(absmax2), blocksize2,
+                                              _lib.ptr(offset), _lib.ptr(out), absmax.numel(), _lib.stream())
+        _lib.check(rc, "mfl_nf4_unnest_absmax")
         return out
     assert absmax.dtype == torch.float32
     return absmax.contiguous()
+
+
+def packed_weight(w_quant: torch.Tensor, quant_state, rows: int, unnested: bool = False):
+    """(``_lib.Nf4Weight``, the tensors it points into) for a call with ``rows`` rows.  A double-quantised state is
+    described as it is, for the kernels that read it so, or with ``unnested`` by its fp32 scales, written out."""
+    code, blocksize = quant_state.code, int(quant_state.blocksize)
+    if not unnested and getattr(quant_state, "nested", False):
+        absmax, code2, absmax2, blocksize2, offset = keep = _second_level(quant_state)
+        return _lib.Nf4Weight(w_quant.data_ptr(), code.data_ptr(), None, None, absmax.data_ptr(), code2.data_ptr(),
+                              absmax2.data_ptr(), offset.data_ptr(), blocksize, blocksize2), keep
+    absmax = resolve_absmax(quant_state)
+    tiled = tiled_absmax(quant_state, absmax, rows)  # decode-sized batches: scales in the order of consumption
+    return _lib.Nf4Weight(w_quant.data_ptr(), code.data_ptr(), absmax.data_ptr(), _lib.ptr(tiled), None, None, None, None,
+                          blocksize, 0), (absmax, tiled)
 
 
 # rows per expert up to which the library's NF4 products run on the kernels that read tile-ordered scales (the plain
