@@ -411,6 +411,35 @@ MFL_API int mfl_silu_mul_fwd(const void *e, const void *g, void *h, int64_t n, i
 MFL_API int mfl_silu_mul_bwd(const void *dh, const void *e, const void *g, void *de, void *dg, void *h_out,
                      int64_t n, int dtype, void *stream);
 
+/* ---- the sparse MoE block after its router projection, as one call ------------------- */
+
+/* softmax + top-k of the logits, expert sort, gate / up / SiLU-mul, down projection, routing-weighted sum
+ * (modular_qwen3_moe_fused.py:87-115): the kernels and results of the entry points above, enqueued one behind the
+ * other with all intermediates in one workspace.  Weights (E,I,H), (E,I,H), (E,H,I) of `dtype`, or packed (q_gate,
+ * q_up, q_down; then the dense pointers are ignored, dtype is MFL_BF16 and training 0).  logits (T,E), tokens (T,H),
+ * T > 0. */
+typedef struct mfl_moe_block {
+    const void *tokens, *logits, *w_gate, *w_up, *w_down;
+    const mfl_nf4_weight *q_gate, *q_up, *q_down;
+    int64_t T;
+    int E, k, H, I, renorm, dtype, logits_dtype;
+    int training; /* keep what the backward call needs in the workspace */
+} mfl_moe_block;
+
+/* out (T,H).  workspace: mfl_moe_block_workspace(b) bytes (0: the arguments are invalid), 256-byte aligned; it begins
+ * with the T * k expert ids (int64).  MFL_ERR_UNSUPPORTED: a shape the fused kernels do not take on packed weights (what
+ * was enqueued before is harmless); the caller then makes the separate calls. */
+MFL_API size_t mfl_moe_block_workspace(const mfl_moe_block *b);
+MFL_API int mfl_moe_block_fwd(const mfl_moe_block *b, void *out, void *workspace, size_t ws_bytes, void *stream);
+
+/* Gradients of mfl_moe_block_fwd with training set, dense weights: d_tokens (T,H), d_logits (T,E; of logits_dtype),
+ * d_gate, d_up (E,I,H), d_down (E,H,I); NULL for those that are not wanted.  saved: the forward call's workspace, which
+ * is only read. */
+MFL_API size_t mfl_moe_block_bwd_workspace(const mfl_moe_block *b);
+MFL_API int mfl_moe_block_bwd(const mfl_moe_block *b, const void *dout, const void *saved, void *d_tokens,
+                      void *d_logits, void *d_gate, void *d_up, void *d_down, void *workspace,
+                      size_t ws_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

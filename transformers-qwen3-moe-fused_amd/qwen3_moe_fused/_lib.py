@@ -35,6 +35,17 @@ class Nf4Weight(ctypes.Structure):
 
 _nf4p = ctypes.POINTER(Nf4Weight)
 
+
+class MoeBlock(ctypes.Structure):
+    """``mfl_moe_block``: the sparse block after its router projection."""
+
+    _fields_ = [("tokens", _vp), ("logits", _vp), ("w_gate", _vp), ("w_up", _vp), ("w_down", _vp), ("q_gate", _nf4p),
+                ("q_up", _nf4p), ("q_down", _nf4p), ("T", _i64), ("E", _i), ("k", _i), ("H", _i), ("I", _i), ("renorm", _i),
+                ("dtype", _i), ("logits_dtype", _i), ("training", _i)]
+
+
+_blockp = ctypes.POINTER(MoeBlock)
+
 # name -> (restype, argtypes); mirrors include/moe_fused_linear.h
 _SIGNATURES = {
     "mfl_abi_version": (_i, []),
@@ -85,6 +96,10 @@ _SIGNATURES = {
     "mfl_rows_dot": (_i, [_vp, _vp, _vp, _vp, _i64, _i, _i, _i, _vp]),
     "mfl_silu_mul_fwd": (_i, [_vp, _vp, _vp, _i64, _i, _vp]),
     "mfl_silu_mul_bwd": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i, _vp]),
+    "mfl_moe_block_workspace": (_sz, [_blockp]),
+    "mfl_moe_block_fwd": (_i, [_blockp, _vp, _vp, _sz, _vp]),
+    "mfl_moe_block_bwd_workspace": (_sz, [_blockp]),
+    "mfl_moe_block_bwd": (_i, [_blockp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
 }
 
 # the entry points declared in include/moe_fused_linear.h: the library exports these and nothing else
@@ -140,8 +155,15 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+# the current stream's handle without building a Stream object for it (4 us of every call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None or _device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_device())
 
 
 def as_index_tensor(m_sizes: torch.Tensor) -> torch.Tensor:

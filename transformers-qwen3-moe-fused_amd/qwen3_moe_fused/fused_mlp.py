@@ -9,15 +9,19 @@ re-gathers the token rows instead of keeping a (rows, hidden) copy alive.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
+from . import _lib
 from .grouped_gemm.backward_dw import grouped_gemm_backward_dw
 from .grouped_gemm.forward import grouped_gemm_forward
 from .grouped_gemm.fused import (grouped_gemm_forward_transposed_dual, grouped_gemm_forward_transposed_silu_bwd,
                                  grouped_glu_forward, grouped_glu_forward_4bit)
 from .kernels.routing import _combine, _gather, _scatter
 from .kernels.silu_mul import silu_mul_backward
-from .grouped_gemm.forward_4bit import grouped_gemm_forward_transposed_4bit
+from .grouped_gemm.forward_4bit import UNSUPPORTED, check_packed, grouped_gemm_forward_transposed_4bit
+from .quantize.nf4 import packed_weight
 
 
 class _GluGathered(torch.autograd.Function):
@@ -140,3 +144,82 @@ def moe_fused_glu_4bit(tokens: torch.Tensor, gate_weight: torch.Tensor, up_weigh
     assert not gate_weight.requires_grad and not up_weight.requires_grad
     return _GluGathered4bit.apply(tokens, gate_weight.data, gate_weight.quant_state, up_weight.data,
                                   up_weight.quant_state, m_sizes, sort_idx, inv_sort_idx, num_selected)
+
+
+class _MoeBlock(torch.autograd.Function):
+    """The block after its router projection as one node of the graph and one library call each way.  All intermediates
+    of the forward lie in one buffer, which is what is kept for the backward."""
+
+    @staticmethod
+    def forward(ctx, tokens, logits, w_gate, w_up, w_down, k, renorm):
+        b = _dense_block(tokens, logits, w_gate, w_up, w_down, k, renorm, True)
+        out, ws = _run_block(b, tokens)
+        ctx.save_for_backward(tokens, logits, w_gate, w_up, w_down, ws)
+        ctx.k, ctx.renorm = k, renorm
+        ctx.mark_non_differentiable(ws)
+        ctx.set_materialize_grads(False)
+        return out, ws
+
+    @staticmethod
+    def backward(ctx, dout, _):
+        if dout is None:
+            return (None,) * 7
+        tokens, logits, w_gate, w_up, w_down, saved = ctx.saved_tensors
+        dout = dout.contiguous()
+        b = _dense_block(tokens, logits, w_gate, w_up, w_down, ctx.k, ctx.renorm, True)
+        grads = [torch.empty_like(t) if need else None
+                 for t, need in zip((tokens, logits, w_gate, w_up, w_down), ctx.needs_input_grad)]
+        lib = _lib.lib()
+        n = lib.mfl_moe_block_bwd_workspace(b)
+        ws = torch.empty(n, device=tokens.device, dtype=torch.uint8)
+        rc = lib.mfl_moe_block_bwd(b, dout.data_ptr(), saved.data_ptr(), *(_lib.ptr(g) for g in grads), ws.data_ptr(), n,
+                                   _lib.stream())
+        _lib.check(rc, "mfl_moe_block_bwd")
+        return (*grads, None, None)
+
+
+def _dense_block(tokens, logits, w_gate, w_up, w_down, k, renorm, training):
+    experts, inter, hidden = w_gate.shape
+    return _lib.MoeBlock(tokens.data_ptr(), logits.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), w_down.data_ptr(), None,
+                         None, None, tokens.shape[0], experts, k, hidden, inter, int(bool(renorm)),
+                         _lib.dtype_code(tokens.dtype), _lib.dtype_code(logits.dtype), int(training))
+
+
+def _run_block(b, tokens):
+    lib = _lib.lib()
+    n = lib.mfl_moe_block_workspace(b)
+    ws = torch.empty(n, device=tokens.device, dtype=torch.uint8)
+    out = torch.empty_like(tokens)
+    rc = lib.mfl_moe_block_fwd(b, out.data_ptr(), ws.data_ptr(), n, _lib.stream())
+    if rc == UNSUPPORTED:
+        return None, None
+    _lib.check(rc, "mfl_moe_block_fwd")
+    return out, ws
+
+
+def moe_block(tokens: torch.Tensor, logits: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
+              num_selected: int, renorm: bool):
+    """Everything of the sparse block that follows the router projection (modular_qwen3_moe_fused.py:87-115):
+    ``tokens`` (T, hidden), ``logits`` (T, E), the three expert matrices in the tokens' type.  Returns (output (T, hidden),
+    workspace, whose first T * num_selected int64 are the expert ids).  Differentiable in all five tensors."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in (tokens, logits, w_gate, w_up, w_down)):
+        return _MoeBlock.apply(tokens, logits, w_gate, w_up, w_down, num_selected, renorm)
+    return _run_block(_dense_block(tokens, logits, w_gate, w_up, w_down, num_selected, renorm, False), tokens)
+
+
+def moe_block_4bit(tokens: torch.Tensor, logits: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor,
+                   w_down: torch.Tensor, num_selected: int, renorm: bool):
+    """``moe_block`` on packed 4-bit weights carrying a ``quant_state``, without gradients; (None, None) for shapes the
+    fused kernels do not take."""
+    hidden = tokens.shape[1]
+    experts, inter = check_packed(tokens, w_gate, w_gate.quant_state, hidden)
+    assert check_packed(tokens, w_up, w_up.quant_state, hidden) == (experts, inter)
+    assert check_packed(tokens, w_down, w_down.quant_state, inter) == (experts, hidden)
+    rows = tokens.shape[0] * num_selected
+    (gate, _kg), (up, _ku), (down, _kd) = (packed_weight(w, w.quant_state, rows) for w in (w_gate, w_up, w_down))
+    if any(w.absmax_u8 and w.blocksize2 & (w.blocksize2 - 1) for w in (gate, up, down)):
+        return None, None
+    b = _lib.MoeBlock(tokens.data_ptr(), logits.data_ptr(), None, None, None, ctypes.pointer(gate), ctypes.pointer(up),
+                      ctypes.pointer(down), tokens.shape[0], experts, num_selected, hidden, inter, int(bool(renorm)),
+                      _lib.dtype_code(tokens.dtype), _lib.dtype_code(logits.dtype), 0)
+    return _run_block(b, tokens)

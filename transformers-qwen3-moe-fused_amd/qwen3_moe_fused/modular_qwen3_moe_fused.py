@@ -48,10 +48,11 @@ class MoeFusedLinear(nn.Module):
         return f"in_features={self.in_features}, out_features={self.out_features}, num_experts={self.num_experts}"
 
 
-def route_tokens(block, hidden_2d: torch.Tensor):
+def route_tokens(block, hidden_2d: torch.Tensor, router_logits: Optional[torch.Tensor] = None):
     """Router half of the block, shared with the fast-LoRA forward: returns
     (router_logits, routing_weights (T,k), m_sizes, sort_idx, inv_sort_idx)."""
-    router_logits = block.gate(hidden_2d)
+    if router_logits is None:
+        router_logits = block.gate(hidden_2d)
     routing_weights, selected, m_sizes, sort_idx, inv_sort_idx = route_and_sort(
         router_logits.contiguous(), block.num_selected, block.norm_topk_prob, hidden_2d.dtype, block.num_experts)
     if getattr(block, "keep_routing", False):
@@ -129,10 +130,57 @@ class Qwen3MoeFusedSparseMoeBlock(nn.Module):
         return moe_fused_mlp(tokens, self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, m_sizes,
                              sort_idx, inv_sort_idx, self.num_selected)
 
+    def _one_call(self, tokens: torch.Tensor, logits: torch.Tensor) -> Optional[torch.Tensor]:
+        """Everything behind the router projection as one library call, where the three projections are plain expert
+        matrices in the tokens' type (both ways), or plain packed ones (without gradients)."""
+        from .fused_mlp import moe_block, moe_block_4bit
+        from .quantize.layer import MoeFusedLinear4bit
+
+        gate, up, down = self.gate_proj, self.up_proj, self.down_proj
+        kind = type(gate)
+        if kind not in (MoeFusedLinear, MoeFusedLinear4bit) or type(up) is not kind or type(down) is not kind:
+            return None
+        if tokens.shape[0] == 0 or self.num_experts > 1024:
+            return None
+        if down._forward_hooks or down._forward_pre_hooks or down._backward_hooks or down._backward_pre_hooks:
+            return None  # (a hook on the down projection fires on the separate steps)
+        assert logits.shape == (tokens.shape[0], self.num_experts)
+        weights = (gate.weight, up.weight, down.weight)
+        if kind is MoeFusedLinear:
+            if tokens.dtype not in (torch.bfloat16, torch.float32):
+                return None
+            for w in weights:
+                if w.dtype != tokens.dtype or not w.is_contiguous() or w.device != tokens.device:
+                    return None
+            out, ws = moe_block(tokens, logits, *weights, self.num_selected, self.norm_topk_prob)
+        else:
+            if tokens.dtype != torch.bfloat16 or (torch.is_grad_enabled() and (tokens.requires_grad or logits.requires_grad)):
+                return None
+            for proj in (gate, up, down):
+                if getattr(proj.weight, "quant_state", None) is None or proj.compute_dtype not in (None, torch.bfloat16):
+                    return None
+            if not down.compute_type_is_set:  # as its own forward does on the first call
+                down.set_compute_type(tokens)
+                down.compute_type_is_set = True
+            out, ws = moe_block_4bit(tokens, logits, *weights, self.num_selected, self.norm_topk_prob)
+        if out is not None and self.keep_routing:
+            n, k = tokens.shape[0], self.num_selected
+            self.last_selected = ws[:n * k * 8].view(torch.int64).view(n, k)
+        return out
+
     def forward(self, hidden_states: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         batch, seq, hidden = hidden_states.shape
         tokens = hidden_states.reshape(batch * seq, hidden).contiguous()
-        router_logits, routing_weights, m_sizes, sort_idx, inv_sort_idx = route_tokens(self, tokens)
+        if self.fuse_front and not self.fuse_backward:
+            router_logits = self.gate(tokens)
+            out = self._one_call(tokens, router_logits.contiguous())
+            if out is not None:
+                return out.view(batch, seq, hidden), router_logits
+            # (the separate steps take the logits as they are: the router is not called twice)
+            routed = route_tokens(self, tokens, router_logits)
+        else:
+            routed = route_tokens(self, tokens)
+        router_logits, routing_weights, m_sizes, sort_idx, inv_sort_idx = routed
 
         y = self._fused_mlp(tokens, m_sizes, sort_idx, inv_sort_idx) if self.fuse_front else None
         if y is None:
