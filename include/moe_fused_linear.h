@@ -334,7 +334,7 @@ MFL_API int mfl_route_sort_small(const void *logits, int logits_dtype, int64_t T
                          int32_t *counts, int32_t *sort_idx, int32_t *inv_sort_idx, void *stream);
 
 /* mfl_route_softmax_topk followed by mfl_expert_sort of its T * k selections, for any T: one launch
- * up to 64 tokens (mfl_route_sort_small), otherwise two (the top-k kernel leaves a histogram of
+ * up to 32 tokens (mfl_route_sort_small), otherwise two (the top-k kernel leaves a histogram of
  * experts per 256 selections, which is the counting pass of the sort), three where the two-launch
  * form does not apply (E > 512, more than 1024 * 256 selections).  Same outputs as the separate
  * calls, bit for bit; both index arrays are required.  workspace: mfl_route_sort_workspace(T, E, k)

@@ -175,8 +175,13 @@ __global__ __launch_bounds__(256) void scatter_rows_kernel(const T *src, const i
     }
 }
 
-// One wave per token; fp32 accumulation over the k selected rows.
-template <typename T>
+// A wave per token and slice of columns; fp32 accumulation over the k selected rows.  A lane owns CC chunks of V columns,
+// 64 * V apart, so that a wave reads whole pieces of rows, U rows at a time before they are added (in order: the sum is
+// the same as one row after the other).  Every row is read exactly once: streaming loads, which leave the caches to
+// the writes.  Many tokens: CC = 4, the whole row of 2048 by one wave, 27 us at 4096 tokens x 8 rows of 2048 (a 1 KiB piece
+// of each of 8 rows per pass with ordinary loads: 55).  Few tokens leave most of the chip idle and the wave waits
+// out one latency per pass: CC = 1, a slice of 512 columns per wave and all eight rows in flight.
+template <typename T, int CC, int U>
 __global__ __launch_bounds__(256) void combine_rows_kernel(const T *src, const int32_t *pos, const T *weights,
                                                            T *dst, int64_t Tn, int k, int H, int vec_ok) {
     constexpr int V = Vec<T>::N;
@@ -186,14 +191,7 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(const T *src, const i
     const int32_t *p = pos + t * k;
     T *d = dst + t * H;
     if (vec_ok) {
-        // A lane owns CC chunks of V columns, 64 * V apart, so that the wave reads whole rows (a
-        // row is one contiguous run in memory): U rows at a time, all chunks of a row together,
-        // before they are added (in order: the sum is the same as one row after the other).
-        // Every row is read exactly once: streaming loads, which leave the caches to the writes.
-        // (Measured at 4096 tokens x 8 rows of 2048: a 1 KiB piece of each of 8 rows per pass
-        // with ordinary loads, 55 us; this, 27 us.)
-        constexpr int CC = 4, U = 4;
-        for (int c0 = lane * V; c0 < H; c0 += CC * 64 * V) {
+        for (int c0 = (blockIdx.y * CC * 64 + lane) * V; c0 < H; c0 += gridDim.y * CC * 64 * V) {
             float acc[CC][V];
 #pragma unroll
             for (int cc = 0; cc < CC; ++cc)
@@ -230,7 +228,7 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(const T *src, const i
             }
         }
     } else {
-        for (int c = lane; c < H; c += 64) {
+        for (int c = blockIdx.y * 64 + lane; c < H; c += gridDim.y * 64) {
             float acc = 0.f;
             for (int j = 0; j < k; ++j) {
                 const float w = weights ? to_f32(weights[t * k + j]) : 1.0f;
@@ -373,8 +371,8 @@ __global__ __launch_bounds__(256) void dequant_u8_kernel(const uint8_t *__restri
         out[i] = code[v[i]] * absmax2[i / blocksize2] + offset;
 }
 
-// The fp32 scales of a double-quantised matrix, offset included, 16 at a time: 16 bytes in and 64 out per lane.  Two
-// launches of a byte per lane each (scales, then the offset) took 10.0 + 6.6 us for 3.1 M scales.
+// The fp32 scales of a double-quantised matrix, offset included.  3.1 M scales: two launches of a byte per lane each
+// (scales, then the offset) took 10.0 + 6.6 us, 16 bytes in and 64 out per lane 8.3 us (a store touched every line).
 __global__ __launch_bounds__(256) void nf4_unnest_kernel(const uint8_t *__restrict__ v, const float *__restrict__ code256,
                                                          const float *__restrict__ absmax2, int bs2_shift,
                                                          const float *__restrict__ offset, float *__restrict__ out,
@@ -386,19 +384,31 @@ __global__ __launch_bounds__(256) void nf4_unnest_kernel(const uint8_t *__restri
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (vec_ok) {
-        const int64_t nv = n / 16;
-        for (int64_t q = i; q < nv; q += stride) {
-            const uint4_t b = ((const uint4_t *)v)[q];
-            const float am = absmax2[(q * 16) >> bs2_shift];
+        // a lane takes four scales: four bytes in, sixteen out, both contiguous over the wave
+        constexpr int U = 4;
+        const int64_t nv = n / 4;
+        const int lane = threadIdx.x & 63;
+        for (int64_t base = (i >> 6) * (64 * U); base < nv; base += (stride >> 6) * (64 * U)) {
+            uint32_t b[U];
+            float am[U];
 #pragma unroll
-            for (int d = 0; d < 4; ++d) {
+            for (int u = 0; u < U; ++u) {
+                const int64_t q = base + u * 64 + lane;
+                if (q >= nv) continue;
+                b[u] = ((const uint32_t *)v)[q];
+                am[u] = absmax2[(q * 4) >> bs2_shift];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int64_t q = base + u * 64 + lane;
+                if (q >= nv) continue;
                 floatx4 o;
 #pragma unroll
-                for (int u = 0; u < 4; ++u) o[u] = code[(b[d] >> (8 * u)) & 0xffu] * am + off;
-                ((floatx4 *)out)[q * 4 + d] = o;
+                for (int d = 0; d < 4; ++d) o[d] = code[(b[u] >> (8 * d)) & 0xffu] * am[u] + off;
+                ((floatx4 *)out)[q] = o;
             }
         }
-        i += nv * 16;
+        i += nv * 4;
     }
     for (; i < n; i += stride) out[i] = code[v[i]] * absmax2[i >> bs2_shift] + off;
 }
@@ -496,8 +506,14 @@ int combine_rows(const void *src, const int32_t *pos, const void *weights, void 
     const size_t es = dtype_size(dtype);
     const int vec_ok = aligned(src, 16) && aligned(dst, 16) && ((size_t)H * es) % 16 == 0;
     const unsigned grid = (unsigned)((T_ + 3) / 4);
-    MFL_DISPATCH_FLOAT(dtype, T, (combine_rows_kernel<T><<<grid, 256, 0, stream>>>(
-                                     (const T *)src, pos, (const T *)weights, (T *)dst, T_, k, H, vec_ok)));
+    if (T_ <= 512) {  // (3.1 against 4.0 us at 1 token, 3.8 against 5.1 at 256, even at 512 and 1024, behind from 2048 on)
+        const unsigned slices = (unsigned)((H * es + 1023) / 1024 < 64 ? (H * es + 1023) / 1024 : 64);
+        MFL_DISPATCH_FLOAT(dtype, T, (combine_rows_kernel<T, 1, 8><<<dim3(grid, slices), 256, 0, stream>>>(
+                                         (const T *)src, pos, (const T *)weights, (T *)dst, T_, k, H, vec_ok)));
+    } else {
+        MFL_DISPATCH_FLOAT(dtype, T, (combine_rows_kernel<T, 4, 4><<<grid, 256, 0, stream>>>(
+                                         (const T *)src, pos, (const T *)weights, (T *)dst, T_, k, H, vec_ok)));
+    }
     return launch_status();
 }
 
@@ -534,7 +550,7 @@ int nf4_unnest_absmax(const uint8_t *v, const float *code256, const float *absma
                       float *out, int64_t n, hipStream_t stream) {
     if (n == 0) return MFL_OK;
     const int shift = log2_exact(blocksize2);
-    const int vec_ok = aligned(v, 16) && aligned(out, 16) && blocksize2 >= 16;
+    const int vec_ok = aligned(v, 4) && aligned(out, 16) && blocksize2 >= 4;
     nf4_unnest_kernel<<<stream_grid(vec_ok ? n / 16 + 1 : n), 256, 0, stream>>>(v, code256, absmax2, shift, offset, out, n,
                                                                                 vec_ok);
     return launch_status();

@@ -35,7 +35,25 @@ __device__ __forceinline__ float wave_max_f32(float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
 }
 
-// One wave per token.  Lane l holds experts l, l+64, l+128, ... (VPL of them).
+// The same for integers: the moves fold into the maxima, and lanes without a source meet the identity.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ int dpp_max_step(int x) {
+    const int y = __builtin_amdgcn_update_dpp((int)0x80000000, x, CTRL, ROW_MASK, 0xf, false);
+    return x > y ? x : y;
+}
+__device__ __forceinline__ int wave_max_i32(int x) {
+    x = dpp_max_step<0xb1, 0xf>(x);
+    x = dpp_max_step<0x4e, 0xf>(x);
+    x = dpp_max_step<0x124, 0xf>(x);
+    x = dpp_max_step<0x128, 0xf>(x);
+    x = dpp_max_step<0x142, 0xa>(x);
+    x = dpp_max_step<0x143, 0xc>(x);
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
+// One wave per token.  Lane l holds experts l, l+64, l+128, ... (VPL of them).  The k rounds of "maximum of the wave, its
+// owner, retire it" are most of the work: on the bit patterns of the probabilities (non-negative floats order like
+// integers), which halves a round's instructions against float maxima.
 template <typename TI, typename TC, int VPL>
 __device__ __forceinline__ int topk_one_token(const TI *__restrict__ logits, int64_t t, int E, int k, int renorm,
                                                float *__restrict__ w_f32, TC *__restrict__ w_cast,
@@ -68,36 +86,38 @@ __device__ __forceinline__ int topk_one_token(const TI *__restrict__ logits, int
 
     float my_w = 0.f, wsum = 0.f;
     int my_i = 0;
+    int key[VPL];  // -1: not selectable (past E, retired, NaN)
+#pragma unroll
+    for (int v = 0; v < VPL; ++v) key[v] = p[v] >= 0.f ? __builtin_bit_cast(int, p[v]) : -1;
     for (int j = 0; j < k; ++j) {
         // lane-local best: larger p, then lower expert id (v ascending = id ascending)
-        float bp = -2.0f;
-        int bi = 0x7fffffff;
+        int bk = -1, bi = 0x7fffffff;
 #pragma unroll
         for (int v = 0; v < VPL; ++v) {
-            if (p[v] > bp) {
-                bp = p[v];
+            if (key[v] > bk) {
+                bk = key[v];
                 bi = lane + 64 * v;
             }
         }
         // the wave's best: the maximum, then its owner; several lanes with the same value (rare)
         // settle for the lowest expert id the slow way
-        const float m = wave_max_f32(bp);
-        const uint64_t owners = __ballot(bp == m);
+        const int m = wave_max_i32(bk);
+        const uint64_t owners = __ballot(bk == m);
         if (__popcll(owners) == 1) {
             bi = __builtin_amdgcn_readlane(bi, __ffsll((unsigned long long)owners) - 1);
         } else {
-            if (bp != m) bi = 0x7fffffff;
+            if (bk != m) bi = 0x7fffffff;
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) {
                 const int oi = __shfl_xor(bi, off);
                 if (oi < bi) bi = oi;
             }
         }
-        bp = m;
+        const float bp = m < 0 ? -2.0f : __builtin_bit_cast(float, m);  // (nothing left: a row of NaN)
         // the owner retires the winner
 #pragma unroll
         for (int v = 0; v < VPL; ++v)
-            if (bi == lane + 64 * v) p[v] = -1.0f;
+            if (bi == lane + 64 * v) key[v] = -1;
         if (lane == j) {
             my_w = bp;
             my_i = bi;
@@ -399,7 +419,11 @@ __global__ __launch_bounds__(1024) void sort_single_kernel(const void *__restric
 
 // Decode-sized batches: softmax + top-k of every token and the stable expert sort of the T * k
 // selections in ONE launch of one workgroup (three launches otherwise, each a few microseconds of
-// work): the waves take the tokens round robin, then sort what they wrote.
+// work): the waves take the tokens round robin, then sort what they selected.  It is a chain of latencies, so the
+// selections and ranks never leave the workgroup on their way (through memory, with a fence and two reads back, the
+// kernel took 10.5 us for one token and 15.7 for 32), and few tokens take few waves.
+constexpr int kSmallBatches = 8;  // batches of 64 selections per wave, at most (8192 selections, 16 waves)
+
 template <typename TI, typename TC, int VPL>
 __global__ __launch_bounds__(1024) void route_sort_small_kernel(const TI *__restrict__ logits, int64_t T, int E,
                                                                 int k, int renorm, float *__restrict__ w_f32,
@@ -407,13 +431,74 @@ __global__ __launch_bounds__(1024) void route_sort_small_kernel(const TI *__rest
                                                                 int key_bits, int32_t *__restrict__ counts,
                                                                 int32_t *__restrict__ sort_idx,
                                                                 int32_t *__restrict__ inv_sort_idx) {
-    extern __shared__ int lds[];
+    extern __shared__ int lds[];  // counts per wave and expert [n_waves][E], rows before the expert [E], selections [R]
     const int lane = threadIdx.x & 63, n_waves = blockDim.x >> 6;
-    for (int64_t t = threadIdx.x >> 6; t < T; t += n_waves)
-        topk_one_token<TI, TC, VPL>(logits, t, E, k, renorm, w_f32, w_cast, idx, lane);
-    __threadfence();  // the selections are read back from memory by other waves of the workgroup
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int *const table = lds, *const first = lds + n_waves * E;
+    uint16_t *const keys = (uint16_t *)(first + E);
+    for (int i = threadIdx.x; i < n_waves * E; i += blockDim.x) table[i] = 0;
+    for (int t = wave; t < (int)T; t += n_waves) {
+        const int sel = topk_one_token<TI, TC, VPL>(logits, t, E, k, renorm, w_f32, w_cast, idx, lane);
+        // (a row of NaN selects no expert: an id outside [0, E), which is neither counted nor placed)
+        if (lane < k) keys[t * k + lane] = (unsigned)sel < (unsigned)E ? (uint16_t)sel : (uint16_t)0xffff;
+    }
     __syncthreads();
-    sort_single_body(idx, 1, T * k, E, key_bits, counts, sort_idx, inv_sort_idx, lds);
+    // ranks of the wave's consecutive batches within the wave's selections of the same expert
+    const int R = (int)T * k;
+    const int per_wave = ceil_div(ceil_div(R, 64), n_waves);
+    const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    int *const hist = table + wave * E;
+    int key[kSmallBatches], rank[kSmallBatches];
+#pragma unroll
+    for (int u = 0; u < kSmallBatches; ++u) {
+        key[u] = 0xffff, rank[u] = 0;
+        if (u >= per_wave) continue;
+        const int j = (wave * per_wave + u) * 64 + lane;
+        if (j < R) key[u] = keys[j];
+        const bool valid = key[u] != 0xffff;
+        uint64_t same = __ballot(valid);
+        if (same == 0) continue;
+        for (int b = 0; b < key_bits; ++b) {
+            const uint64_t bal = __ballot((key[u] >> b) & 1);
+            same &= ((key[u] >> b) & 1) ? bal : ~bal;
+        }
+        if (valid) {
+            const int before = hist[key[u]];
+            rank[u] = before + __popcll(same & lt_mask);
+            // the last lane of each group of equal ids publishes the new running count
+            if ((same >> lane) == 1ull) hist[key[u]] = before + __popcll(same);
+        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < E; e += blockDim.x) {
+        int run = 0;
+        for (int w = 0; w < n_waves; ++w) {
+            const int c = table[w * E + e];
+            table[w * E + e] = run;
+            run += c;
+        }
+        first[e] = run;
+        counts[e] = run;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        int carry = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int v = e0 + lane < E ? first[e0 + lane] : 0;
+            const int inc = wave_inclusive_scan(v);
+            if (e0 + lane < E) first[e0 + lane] = carry + inc - v;
+            carry += wave_last(inc);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kSmallBatches; ++u) {
+        if (u >= per_wave || key[u] == 0xffff) continue;
+        const int j = (wave * per_wave + u) * 64 + lane;
+        const int pos = rank[u] + hist[key[u]] + first[key[u]];
+        inv_sort_idx[j] = pos;
+        sort_idx[pos] = j;
+    }
 }
 
 // Multi-workgroup path: count -> scan -> scatter, table in global workspace.
@@ -854,8 +939,8 @@ int launch_route_sort_small(const void *logits, int64_t T, int E, int k, int ren
                             hipStream_t stream) {
     int key_bits = 0;
     while ((1 << key_bits) < E) ++key_bits;
-    const int n_waves = 16;
-    const size_t lds = (size_t)(n_waves + 1) * E * 4;
+    const int n_waves = T <= 4 ? 4 : T <= 8 ? 8 : 16;
+    const size_t lds = (size_t)(n_waves + 1) * E * 4 + (size_t)T * k * 2;  // at most 51200 bytes
     const int vpl = ceil_div(E, 64);
 #define MFL_RS(V)                                                                                              \
     route_sort_small_kernel<TI, TC, V><<<1, n_waves * 64, lds, stream>>>(                                      \
@@ -878,7 +963,7 @@ int route_sort_small(const void *logits, int logits_dtype, int64_t T, int E, int
                      void *w_cast, int cast_dtype, int64_t *idx, int32_t *counts, int32_t *sort_idx,
                      int32_t *inv_sort_idx, hipStream_t stream) {
     // one workgroup does everything: worth it only while the tokens are few
-    if (T > 128 || T * k > 8192 || E > 512 || inv_sort_idx == nullptr || sort_idx == nullptr)
+    if (T > 128 || T * k > 64 * 16 * kSmallBatches || E > 512 || inv_sort_idx == nullptr || sort_idx == nullptr)
         return MFL_ERR_UNSUPPORTED;
     if (T == 0) return MFL_ERR_UNSUPPORTED;  // the separate entry points define the empty case
     int rc = MFL_OK;
@@ -932,8 +1017,9 @@ size_t route_sort_workspace(int64_t T, int E, int k) {
 int route_sort(const void *logits, int logits_dtype, int64_t T, int E, int k, int renorm, float *w_f32, void *w_cast,
                int cast_dtype, int64_t *idx, int32_t *counts, int32_t *sort_idx, int32_t *inv_sort_idx,
                void *workspace, size_t ws_bytes, hipStream_t stream) {
-    // up to 64 tokens one workgroup does it all in one launch (above, its single workgroup is the slower way)
-    int rc = T <= 64 ? route_sort_small(logits, logits_dtype, T, E, k, renorm, w_f32, w_cast, cast_dtype, idx, counts,
+    // up to 32 tokens one workgroup does it all in one launch (4.7 us at 1 token, 8.6 against 9.3 at 32, 14.3 against 10.0
+    // at 64: a wave takes one token after the other)
+    int rc = T <= 32 ? route_sort_small(logits, logits_dtype, T, E, k, renorm, w_f32, w_cast, cast_dtype, idx, counts,
                                         sort_idx, inv_sort_idx, stream)
                      : MFL_ERR_UNSUPPORTED;
     if (rc != MFL_ERR_UNSUPPORTED) return rc;

@@ -81,7 +81,7 @@ def _round256(n: int) -> int:
 
 
 def _route_and_sort_raw(logits: torch.Tensor, k: int, renorm: bool, out_dtype: Optional[torch.dtype]):
-    """One library call (``mfl_route_sort``: one launch up to 64 tokens, two above) and ONE allocation, of which
+    """One library call (``mfl_route_sort``: one launch up to 32 tokens, two above) and ONE allocation, of which
     the outputs and the call's scratch are views.  Returns (w32, weights, idx, m_sizes, sort_idx, inv_sort_idx)."""
     assert logits.is_cuda and logits.ndim == 2 and logits.is_contiguous()
     T, E = logits.shape
