@@ -302,6 +302,18 @@ MFL_API int mfl_nf4_unnest_absmax(const uint8_t *v, const float *code256, const 
 MFL_API int mfl_nf4_quant(const void *w, int w_dtype, int64_t n, int blocksize, const float *code16,
                   uint8_t *wq, float *absmax, void *stream);
 
+/* ---- the router projection (modular_qwen3_moe_fused.py:85) -------------------------- */
+
+/* logits (T,E) = x (T,H) w (E,H)^T, bf16 operands, out_dtype bf16 or fp32.  H a multiple of 64
+ * (MFL_ERR_UNSUPPORTED otherwise). */
+MFL_API int mfl_router_fwd(const void *x, const void *w, void *logits, int64_t T, int H, int E, int out_dtype,
+                   void *stream);
+/* dw (E,H) = dlogits (T,E)^T x (T,H), all bf16, T > 0; H and E multiples of 8 (MFL_ERR_UNSUPPORTED otherwise; the
+ * workspace is then 0 bytes). */
+MFL_API size_t mfl_router_dw_workspace(int64_t T, int H, int E);
+MFL_API int mfl_router_dw(const void *x, const void *dlogits, void *dw, int64_t T, int H, int E, void *workspace,
+                  size_t ws_bytes, void *stream);
+
 /* ---- routing ---------------------------------------------------------------------- */
 
 /* p = softmax_fp32(logits[t, :]); top-k of p, descending, equal values -> lower expert id

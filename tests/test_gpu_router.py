@@ -1,0 +1,51 @@
+"""The router projection and its gradients against float64 products.  Tolerance: fp32 sums of L products in any order are
+within L * 2^-24 * sum |a b| of the exact ones, plus one bf16 rounding (2^-8 of the value)."""
+import pytest
+import torch
+
+from util import gen
+
+pytestmark = pytest.mark.gpu
+
+from qwen3_moe_fused.kernels.routing import router_linear  # noqa: E402
+from qwen3_moe_fused.modular_qwen3_moe_fused import Qwen3MoeFusedRouter  # noqa: E402
+
+
+def _near(got, a, b, length, ulp=2.0 ** -8):
+    exact, bound = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    room = length * 2.0 ** -24 * bound + ulp * exact.abs()
+    assert torch.isfinite(got).all() and ((got.double().cpu() - exact).abs() <= room + 1e-30).all()
+
+
+# tokens around the blocks of 16 and 64 of the forward, the steps of 32 and parts of 256 of the weight gradient; experts
+# around the blocks of 16 and 128; hidden sizes of one piece, of pieces that do not divide among eight waves, of a last
+# column tile that is not whole
+@pytest.mark.parametrize("t,h,e", [(1, 2048, 128), (15, 64, 8), (16, 576, 16), (17, 1024, 136), (33, 512, 60), (64, 192, 8),
+                                   (255, 264, 128), (257, 2048, 120), (511, 640, 264), (512, 264, 128), (513, 2048, 120), (769, 136, 264), (3001, 128, 64)])
+def test_router_projection_and_gradients(t, h, e):
+    g = gen(t + h + e)
+    x, w, d = (torch.randn(s, generator=g).to(torch.bfloat16) for s in ((t, h), (e, h), (t, e)))
+    xd, wd = x.cuda().requires_grad_(), w.cuda().requires_grad_()
+    y = router_linear(xd, wd)
+    _near(y, x, w.t(), h)
+    with torch.no_grad():
+        assert torch.equal(router_linear(xd, wd), y)
+    y.backward(d.cuda())
+    _near(wd.grad, d.t(), x, t)
+    _near(xd.grad, d, w, e)
+
+
+def test_fp32_logits_and_other_kinds_of_input():
+    from qwen3_moe_fused import _lib
+
+    x, w = (torch.randn(s, generator=gen(s[0])).to(torch.bfloat16) for s in ((530, 256), (72, 256)))
+    xd, wd = x.cuda(), w.cuda()
+    out = torch.empty((530, 72), device="cuda")
+    for t in (530, 40):
+        _lib.check(_lib.lib().mfl_router_fwd(xd.data_ptr(), wd.data_ptr(), out.data_ptr(), t, 256, 72, _lib.F32, _lib.stream()),
+                   "mfl_router_fwd")
+        _near(out[:t], x[:t], w.t(), 256, 2.0 ** -23)
+    assert router_linear(xd.float(), wd) is None and router_linear(xd[:, :64], wd[:, :64]) is None
+    gate = Qwen3MoeFusedRouter(256, 72, bias=False).cuda()
+    z = torch.randn((3, 5, 256)).cuda()
+    assert torch.equal(gate(z), torch.nn.functional.linear(z, gate.weight))

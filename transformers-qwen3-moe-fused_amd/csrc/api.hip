@@ -525,6 +525,25 @@ int mfl_nf4_quant(const void *w, int w_dtype, int64_t n, int blocksize, const fl
     return nf4_quant(w, w_dtype, n, blocksize, code16, wq, absmax, (hipStream_t)stream);
 }
 
+int mfl_router_fwd(const void *x, const void *w, void *logits, int64_t T, int H, int E, int out_dtype, void *stream) {
+    if (T < 0 || H <= 0 || E <= 0) return MFL_ERR_SHAPE;
+    if (!dtype_ok(out_dtype)) return MFL_ERR_DTYPE;
+    if (T == 0) return MFL_OK;
+    if (!x || !w || !logits) return MFL_ERR_NULL;
+    return router_fwd(x, w, logits, T, H, E, out_dtype, (hipStream_t)stream);
+}
+
+size_t mfl_router_dw_workspace(int64_t T, int H, int E) {
+    return T > 0 && H > 0 && E > 0 ? router_dw_workspace(T, H, E) : 0;
+}
+
+int mfl_router_dw(const void *x, const void *dlogits, void *dw, int64_t T, int H, int E, void *workspace, size_t ws_bytes,
+                  void *stream) {
+    if (T <= 0 || H <= 0 || E <= 0) return MFL_ERR_SHAPE;
+    if (!x || !dlogits || !dw) return MFL_ERR_NULL;
+    return router_dw(x, dlogits, dw, T, H, E, workspace, ws_bytes, (hipStream_t)stream);
+}
+
 int mfl_route_softmax_topk(const void *logits, int logits_dtype, int64_t T, int E, int k, int renorm, float *weights_f32,
                            void *weights_cast, int cast_dtype, int64_t *idx, void *stream) {
     if (T < 0 || E <= 0 || k <= 0 || k > E || k > 64) return MFL_ERR_SHAPE;

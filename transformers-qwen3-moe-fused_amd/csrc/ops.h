@@ -24,6 +24,10 @@ int nf4_unnest_absmax(const uint8_t *v, const float *code256, const float *absma
 int nf4_quant(const void *w, int w_dtype, int64_t n, int blocksize, const float *code16, uint8_t *wq, float *absmax,
               hipStream_t stream);
 
+int router_fwd(const void *x, const void *w, void *logits, int64_t T, int H, int E, int out_dtype, hipStream_t stream);
+size_t router_dw_workspace(int64_t T, int H, int E);
+int router_dw(const void *x, const void *dlogits, void *dw, int64_t T, int H, int E, void *workspace, size_t ws_bytes,
+              hipStream_t stream);
 int route_softmax_topk(const void *logits, int logits_dtype, int64_t T, int E, int k, int renorm, float *w_f32,
                        void *w_cast, int cast_dtype, int64_t *idx, hipStream_t stream);
 // d logits of the routing weights (recomputes the softmax; idx and w_f32 as route_softmax_topk wrote them)

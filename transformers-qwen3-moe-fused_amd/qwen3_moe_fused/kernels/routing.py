@@ -14,6 +14,62 @@ import torch
 from .. import _lib
 
 
+# Tokens up to which the router projection runs on the library's own kernel (as fast as the stock product on the device,
+# and 14 us less of the host's time), and from which its weight gradient does (9.5 against 9.3 us at 512 tokens, 19
+# against 67 at 8192).
+_ROUTER_FWD_TOKENS = 512
+_ROUTER_DW_TOKENS = 512
+
+
+def _router_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    tokens, hidden = x.shape
+    if tokens <= _ROUTER_FWD_TOKENS and hidden % 64 == 0:
+        out = torch.empty((tokens, w.shape[0]), device=x.device, dtype=x.dtype)
+        rc = _lib.lib().mfl_router_fwd(x.data_ptr(), w.data_ptr(), out.data_ptr(), tokens, hidden, w.shape[0], _lib.BF16,
+                                       _lib.stream())
+        if rc != -6:  # MFL_ERR_UNSUPPORTED
+            _lib.check(rc, "mfl_router_fwd")
+            return out
+    return torch.nn.functional.linear(x, w)
+
+
+class _RouterLinear(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(x, w)
+        return _router_logits(x, w)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dlogits):
+        x, w = ctx.saved_tensors
+        dlogits = dlogits.contiguous()
+        dx = dlogits @ w if ctx.needs_input_grad[0] else None
+        dw = None
+        if ctx.needs_input_grad[1]:
+            tokens, hidden = x.shape
+            n = _lib.lib().mfl_router_dw_workspace(tokens, hidden, w.shape[0]) if tokens >= _ROUTER_DW_TOKENS else 0
+            if n == 0:
+                return dx, dlogits.t() @ x
+            dw, ws = torch.empty_like(w), torch.empty(n, device=x.device, dtype=torch.uint8)
+            rc = _lib.lib().mfl_router_dw(x.data_ptr(), dlogits.data_ptr(), dw.data_ptr(), tokens, hidden, w.shape[0],
+                                          ws.data_ptr(), n, _lib.stream())
+            _lib.check(rc, "mfl_router_dw")
+        return dx, dw
+
+
+def router_linear(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """``torch.nn.functional.linear(x, w)`` for a bf16 router, x (T, hidden), w (E, hidden), both contiguous on one GPU;
+    differentiable once.  ``None`` for anything else."""
+    if (x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda or x.device != w.device or x.ndim != 2
+            or x.shape[0] == 0 or not x.is_contiguous() or not w.is_contiguous() or torch.is_autocast_enabled("cuda")
+            or x.data_ptr() % 16 or w.data_ptr() % 16):
+        return None
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+        return _RouterLinear.apply(x, w)
+    return _router_logits(x, w)
+
+
 def softmax_topk_raw(logits: torch.Tensor, k: int, renorm: bool,
                      out_dtype: Optional[torch.dtype] = None) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Returns (weights fp32 (T,k), weights cast to ``out_dtype`` (T,k), expert ids int64 (T,k)).

@@ -15,7 +15,7 @@ import torch
 from torch import nn
 
 from .functional import moe_fused_linear
-from .kernels.routing import combine_rows, gather_rows, route_and_sort
+from .kernels.routing import combine_rows, gather_rows, route_and_sort, router_linear
 from .kernels.silu_mul import silu_mul
 
 
@@ -65,6 +65,10 @@ class Qwen3MoeFusedRouter(nn.Linear):
     reference) under a class name of its own, so that transformers releases that collect
     ``router_logits`` with a forward hook on the router module (instead of from the block's return
     value, as the reference's release did) have a class to hook: its output is the raw logits."""
+
+    def forward(self, input: torch.Tensor) -> torch.Tensor:
+        out = router_linear(input, self.weight) if self.bias is None else None
+        return super().forward(input) if out is None else out
 
 
 class Qwen3MoeFusedSparseMoeBlock(nn.Module):
