@@ -102,3 +102,18 @@ def test_block_call_on_two_streams_and_with_a_hook():
         assert torch.equal(blk(xs[0])[0], want[0]) and len(seen) == 1
         handle.remove()
     assert type(blk.down_proj) is MoeFusedLinear
+
+
+def test_block_call_leaves_hooks_forward_mode_and_the_routing_alone():
+    blk, _ = _block(8, 2, 64, 64, "fp32", 5)
+    blk.keep_routing = True
+    x = torch.randn((1, 40, 64), generator=gen(5)).cuda()
+    with torch.no_grad():
+        want = blk(x)[0]
+        assert blk.last_selected.untyped_storage().nbytes() == 40 * 2 * 8
+        seen = []
+        handle = blk.up_proj.register_forward_hook(lambda m, a, o: seen.append(o.shape))
+        assert torch.equal(blk(x)[0], want) and len(seen) == 1
+        handle.remove()
+        with torch.autograd.forward_ad.dual_level(), pytest.raises(Exception):  # no kernel here has a forward-mode rule
+            blk(torch.autograd.forward_ad.make_dual(x, x))

@@ -49,3 +49,29 @@ def test_fp32_logits_and_other_kinds_of_input():
     gate = Qwen3MoeFusedRouter(256, 72, bias=False).cuda()
     z = torch.randn((3, 5, 256)).cuda()
     assert torch.equal(gate(z), torch.nn.functional.linear(z, gate.weight))
+
+
+def test_router_gradients_of_gradients_and_forward_mode():
+    """What the stock projection takes: a penalty on its gradients, and tangents."""
+    t, h, e = 600, 128, 16
+    x, w, d = (torch.randn(s, generator=gen(7)).to(torch.bfloat16).cuda() for s in ((t, h), (e, h), (t, e)))
+    gate = Qwen3MoeFusedRouter(h, e, bias=False).to("cuda", torch.bfloat16)
+    got = []
+    for f in (gate, lambda z: torch.nn.functional.linear(z, gate.weight)):
+        xr = x.clone().requires_grad_()
+        gate.weight.data.copy_(w)
+        (dx,) = torch.autograd.grad((f(xr) * d).sum(), xr, create_graph=True)
+        got.append(torch.autograd.grad(dx.float().square().sum(), gate.weight)[0])
+        with torch.autograd.forward_ad.dual_level(), torch.no_grad():
+            dual = f(torch.autograd.forward_ad.make_dual(x, x))
+            got.append(torch.autograd.forward_ad.unpack_dual(dual).tangent)
+    assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[3])
+
+
+def test_router_weight_gradient_keeps_an_infinity_of_the_last_token():
+    t, h, e = 513, 128, 16
+    x, d = torch.ones((t, h)).to(torch.bfloat16).cuda(), torch.ones((t, e)).to(torch.bfloat16).cuda()
+    w = torch.zeros((e, h), device="cuda", dtype=torch.bfloat16).requires_grad_()
+    x[-1, 5] = float("inf")
+    router_linear(x, w).backward(d)
+    assert torch.isinf(w.grad[:, 5]).all() and (torch.cat((w.grad[:, :5], w.grad[:, 6:]), 1) == 512).all()  # 513 in bf16

@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void router_dw_kernel(const bf16_t *__restrict
         off_x[q] = lane_src_offset<kDwTile, kDwStep, false>(load, lane, H, h_lim);
     }
     const int steps = ceil_div(t_end - t_begin, kDwStep);
-    // rows past the last token: zeros in the left operand, the last token's row again in the right one
+    // rows past the last token: zeros in both operands (an infinity of a row read again would turn into NaN)
     auto issue = [&](int s) {
         unsigned char *const base = smem + (s % kDwRing) * 2 * DwStage::kBytes;
         const int t0 = t_begin + s * kDwStep;
@@ -103,9 +103,8 @@ __global__ __launch_bounds__(256) void router_dw_kernel(const bf16_t *__restrict
             const bool in = t0 + row[q] < t_end;
             const unsigned char *const pd = in ? (const unsigned char *)(d + (int64_t)t0 * E + e0) + off_d[q]
                                                : (const unsigned char *)&g_zero_chunk;
-            const int back = in ? 0 : t0 + row[q] - (t_end - 1);
-            const unsigned char *const px =
-                (const unsigned char *)(x + (int64_t)t0 * H + h0) + off_x[q] - (int64_t)back * H * 2;
+            const unsigned char *const px = in ? (const unsigned char *)(x + (int64_t)t0 * H + h0) + off_x[q]
+                                               : (const unsigned char *)&g_zero_chunk;
             copy_to_lds<0, true>(pd, base + (wave * LOADS + q) * 1024);
             copy_to_lds<0, true>(px, base + DwStage::kBytes + (wave * LOADS + q) * 1024);
         }

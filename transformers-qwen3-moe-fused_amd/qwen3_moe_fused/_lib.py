@@ -11,6 +11,7 @@ import os
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmoe_fused_linear.so")
@@ -167,6 +168,14 @@ def stream() -> int:
     if _raw_stream is None or _device is None:
         return torch.cuda.current_stream().cuda_stream
     return _raw_stream(_device())
+
+
+def plain_call() -> bool:
+    """Whether a call that passes autograd by, or stands in for a stock operator, may do so: no forward-mode level, no
+    functorch transform and no dispatch mode (counters, fake tensors, selective checkpointing) that would have to see
+    the operators, and nobody tracing."""
+    return (forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None)
 
 
 def as_index_tensor(m_sizes: torch.Tensor) -> torch.Tensor:

@@ -19,6 +19,7 @@ from .. import _lib
 # against 67 at 8192).
 _ROUTER_FWD_TOKENS = 512
 _ROUTER_DW_TOKENS = 512
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _router_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -40,9 +41,11 @@ class _RouterLinear(torch.autograd.Function):
         return _router_logits(x, w)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, dlogits):
         x, w = ctx.saved_tensors
+        if torch.is_grad_enabled():  # a graph of the gradients is asked for (create_graph): stock products have one
+            return (dlogits @ w if ctx.needs_input_grad[0] else None,
+                    dlogits.t() @ x if ctx.needs_input_grad[1] else None)
         dlogits = dlogits.contiguous()
         dx = dlogits @ w if ctx.needs_input_grad[0] else None
         dw = None
@@ -54,14 +57,16 @@ class _RouterLinear(torch.autograd.Function):
             dw, ws = torch.empty_like(w), torch.empty(n, device=x.device, dtype=torch.uint8)
             rc = _lib.lib().mfl_router_dw(x.data_ptr(), dlogits.data_ptr(), dw.data_ptr(), tokens, hidden, w.shape[0],
                                           ws.data_ptr(), n, _lib.stream())
+            if rc == -6:  # MFL_ERR_UNSUPPORTED: a gradient that is not aligned
+                return dx, dlogits.t() @ x
             _lib.check(rc, "mfl_router_dw")
         return dx, dw
 
 
 def router_linear(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
-    """``torch.nn.functional.linear(x, w)`` for a bf16 router, x (T, hidden), w (E, hidden), both contiguous on one GPU;
-    differentiable once.  ``None`` for anything else."""
-    if (x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda or x.device != w.device or x.ndim != 2
+    """``torch.nn.functional.linear(x, w)`` for a bf16 router, x (T, hidden), w (E, hidden), both contiguous on one GPU.
+    ``None`` for anything else: other types and forms, tensor subclasses, and calls that a transform has to see."""
+    if (type(x) not in _PLAIN or type(w) not in _PLAIN or not _lib.plain_call() or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda or x.device != w.device or x.ndim != 2
             or x.shape[0] == 0 or not x.is_contiguous() or not w.is_contiguous() or torch.is_autocast_enabled("cuda")
             or x.data_ptr() % 16 or w.data_ptr() % 16):
         return None

@@ -14,6 +14,7 @@ from typing import Optional, Tuple
 import torch
 from torch import nn
 
+from . import _lib
 from .functional import moe_fused_linear
 from .kernels.routing import combine_rows, gather_rows, route_and_sort, router_linear
 from .kernels.silu_mul import silu_mul
@@ -146,8 +147,12 @@ class Qwen3MoeFusedSparseMoeBlock(nn.Module):
             return None
         if tokens.shape[0] == 0 or self.num_experts > 1024:
             return None
-        if down._forward_hooks or down._forward_pre_hooks or down._backward_hooks or down._backward_pre_hooks:
-            return None  # (a hook on the down projection fires on the separate steps)
+        for proj in (gate, up, down):  # hooks and replaced forwards run on the separate steps
+            if (proj._forward_hooks or proj._forward_pre_hooks or proj._backward_hooks or proj._backward_pre_hooks
+                    or "forward" in proj.__dict__):
+                return None
+        if torch.nn.modules.module._has_any_global_hook() or not _lib.plain_call():
+            return None
         assert logits.shape == (tokens.shape[0], self.num_experts)
         weights = (gate.weight, up.weight, down.weight)
         if kind is MoeFusedLinear:
@@ -169,7 +174,7 @@ class Qwen3MoeFusedSparseMoeBlock(nn.Module):
             out, ws = moe_block_4bit(tokens, logits, *weights, self.num_selected, self.norm_topk_prob)
         if out is not None and self.keep_routing:
             n, k = tokens.shape[0], self.num_selected
-            self.last_selected = ws[:n * k * 8].view(torch.int64).view(n, k)
+            self.last_selected = ws[:n * k * 8].view(torch.int64).view(n, k).clone()  # (not the whole workspace)
         return out
 
     def forward(self, hidden_states: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
