@@ -410,6 +410,16 @@ MFL_API int mfl_combine_rows(const void *src, const int32_t *pos, const void *we
 MFL_API int mfl_rows_dot(const void *a, const void *b, const int32_t *pos, void *dots, int64_t T, int k,
                  int H, int dtype, void *stream);
 
+/* Copies of `blocks` runs of `bytes` bytes each, run b from src + b * src_stride (NULL: zeros) to dst + b * dst_stride:
+ * joining and splitting the thin matrices of two LoRA adapters.  Up to 8 copies, in no order, in one launch; bytes,
+ * strides and pointers multiples of 16 (else MFL_ERR_UNSUPPORTED).  jobs is read on the host, before the call returns. */
+typedef struct mfl_block_copy {
+    const void *src;
+    void *dst;
+    int64_t blocks, bytes, src_stride, dst_stride;
+} mfl_block_copy;
+MFL_API int mfl_copy_blocks(const mfl_block_copy *jobs, int n, void *stream);
+
 /* ---- SiLU-mul --------------------------------------------------------------------- */
 
 /* h = T(f32(e) * sigmoid(f32(e))) * g.  Replaces silu_mul_forward,

@@ -634,6 +634,12 @@ int mfl_combine_rows(const void *src, const int32_t *pos, const void *weights, v
     return combine_rows(src, pos, weights, dst, T, k, H, dtype, (hipStream_t)stream);
 }
 
+int mfl_copy_blocks(const mfl_block_copy *jobs, int n, void *stream) {
+    if (n < 0) return MFL_ERR_SHAPE;
+    if (n > 0 && !jobs) return MFL_ERR_NULL;
+    return copy_blocks(jobs, n, (hipStream_t)stream);
+}
+
 int mfl_rows_dot(const void *a, const void *b, const int32_t *pos, void *dots, int64_t T, int k, int H, int dtype,
                  void *stream) {
     if (T < 0 || H <= 0 || k <= 0) return MFL_ERR_SHAPE;

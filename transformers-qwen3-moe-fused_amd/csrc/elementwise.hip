@@ -299,6 +299,36 @@ __global__ __launch_bounds__(256) void rows_dot_kernel(const T *a, const T *b, c
     }
 }
 
+// ---------------------------------------------------------------- blocks copied between layouts
+
+// Up to kMaxCopies strided copies in one launch: workgroups are dealt out over the copies by their size, a lane
+// moves kCopyUnroll pieces of 16 bytes, neighbouring lanes neighbouring pieces.
+constexpr int kMaxCopies = 8, kCopyUnroll = 4;
+struct CopyJobs {
+    mfl_block_copy job[kMaxCopies];
+    uint32_t first_block[kMaxCopies];
+    int n;
+};
+__global__ __launch_bounds__(256) void copy_blocks_kernel(CopyJobs c) {
+    int q = 0;
+    while (q + 1 < c.n && blockIdx.x >= c.first_block[q + 1]) ++q;
+    const mfl_block_copy &j = c.job[q];
+    const uint32_t inner = (uint32_t)(j.bytes / 16), total = (uint32_t)j.blocks * inner;
+    const uint32_t i0 = (blockIdx.x - c.first_block[q]) * (256 * kCopyUnroll) + threadIdx.x;
+    uint4_t v[kCopyUnroll];
+    int64_t to[kCopyUnroll];
+#pragma unroll
+    for (int u = 0; u < kCopyUnroll; ++u) {
+        const uint32_t i = i0 + u * 256, b = i / inner, at = (i - b * inner) * 16;
+        to[u] = i < total ? b * j.dst_stride + at : -1;
+        v[u] = uint4_t{0u, 0u, 0u, 0u};
+        if (i < total && j.src != nullptr) v[u] = *(const uint4_t *)((const char *)j.src + b * j.src_stride + at);
+    }
+#pragma unroll
+    for (int u = 0; u < kCopyUnroll; ++u)
+        if (to[u] >= 0) *(uint4_t *)((char *)j.dst + to[u]) = v[u];
+}
+
 // ---------------------------------------------------------------- NF4
 
 // Vector path (blocksize >= 8, aligned pointers): a lane decodes one packed dword (8 elements that
@@ -527,6 +557,27 @@ int rows_dot(const void *a, const void *b, const int32_t *pos, void *dots, int64
     const unsigned grid = (unsigned)((T_ * ceil_div(k, 4) + 3) / 4);
     MFL_DISPATCH_FLOAT(dtype, T, (rows_dot_kernel<T><<<grid, 256, 0, stream>>>((const T *)a, (const T *)b, pos,
                                                                                (T *)dots, T_, k, H, vec_ok)));
+    return launch_status();
+}
+
+int copy_blocks(const mfl_block_copy *jobs, int n, hipStream_t stream) {
+    if (n > kMaxCopies) return MFL_ERR_UNSUPPORTED;
+    CopyJobs c = {};
+    int64_t grid = 0;
+    for (int q = 0; q < n; ++q) {
+        const mfl_block_copy &j = jobs[q];
+        if (j.blocks < 0 || j.bytes < 0) return MFL_ERR_SHAPE;
+        if (j.blocks == 0 || j.bytes == 0) continue;
+        if (!j.dst) return MFL_ERR_NULL;
+        if (j.bytes % 16 != 0 || j.dst_stride % 16 != 0 || !aligned(j.dst, 16)) return MFL_ERR_UNSUPPORTED;
+        if (j.src != nullptr && (j.src_stride % 16 != 0 || !aligned(j.src, 16))) return MFL_ERR_UNSUPPORTED;
+        if (j.blocks > 0x7fffffff || j.bytes / 16 > 0x7fffffff / j.blocks) return MFL_ERR_UNSUPPORTED;
+        c.job[c.n] = j;
+        c.first_block[c.n++] = (uint32_t)grid;
+        grid += (j.blocks * (j.bytes / 16) + 256 * kCopyUnroll - 1) / (256 * kCopyUnroll);
+    }
+    if (grid == 0) return MFL_OK;
+    copy_blocks_kernel<<<(unsigned)grid, 256, 0, stream>>>(c);
     return launch_status();
 }
 

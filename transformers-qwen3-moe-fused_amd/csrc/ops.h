@@ -13,6 +13,7 @@ int gather_rows(const void *src, const int32_t *idx, int idx_div, const void *ro
                 int H, int dtype, hipStream_t stream);
 int combine_rows(const void *src, const int32_t *pos, const void *weights, void *dst, int64_t T, int k, int H,
                  int dtype, hipStream_t stream);
+int copy_blocks(const mfl_block_copy *jobs, int n, hipStream_t stream);
 int rows_dot(const void *a, const void *b, const int32_t *pos, void *dots, int64_t T, int k, int H, int dtype,
              hipStream_t stream);
 int nf4_dequant(const uint8_t *wq, const float *code16, const float *absmax, int blocksize, void *out, int64_t n,

@@ -47,6 +47,13 @@ class MoeBlock(ctypes.Structure):
 
 _blockp = ctypes.POINTER(MoeBlock)
 
+
+class BlockCopy(ctypes.Structure):
+    """``mfl_block_copy``: a strided copy of runs of bytes."""
+
+    _fields_ = [("src", _vp), ("dst", _vp), ("blocks", _i64), ("bytes", _i64), ("src_stride", _i64), ("dst_stride", _i64)]
+
+
 # name -> (restype, argtypes); mirrors include/moe_fused_linear.h
 _SIGNATURES = {
     "mfl_abi_version": (_i, []),
@@ -97,6 +104,7 @@ _SIGNATURES = {
     "mfl_gather_rows": (_i, [_vp, _vp, _i, _vp, _vp, _i64, _i, _i, _vp]),
     "mfl_scatter_rows": (_i, [_vp, _vp, _i, _vp, _vp, _i64, _i, _i, _vp]),
     "mfl_combine_rows": (_i, [_vp, _vp, _vp, _vp, _i64, _i, _i, _i, _vp]),
+    "mfl_copy_blocks": (_i, [ctypes.POINTER(BlockCopy), _i, _vp]),
     "mfl_rows_dot": (_i, [_vp, _vp, _vp, _vp, _i64, _i, _i, _i, _vp]),
     "mfl_silu_mul_fwd": (_i, [_vp, _vp, _vp, _i64, _i, _vp]),
     "mfl_silu_mul_bwd": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i, _vp]),
