@@ -51,6 +51,11 @@ CASES = [
     ([9], 40, 16512, 64),
     ([4, 9], 64, 256, 128),
     ([600, 20], 64, 256, 64),
+    # stages that do not divide by eight or two, and more of them than the registers hold at once, at both tile heights
+    ([5, 30], 160, 2176, 64),
+    ([5, 30], 72, 4224, 64),
+    ([50, 3], 96, 4096, 64),
+    ([40, 30], 40, 2432, 64),
 ]
 
 

@@ -10,7 +10,7 @@
 // both matrices in the gated linear unit) for all of the rows.
 //   stage = rows     32 MR x 128 bf16 (8 KiB a block of 32, shared by the four waves; chunk c of row r at c ^ (r & 15))
 //         + weights  per wave and matrix 32 columns x 64 packed bytes (2 KiB; chunk c of row r at c ^ ((r >> 2) & 3))
-//         + scales   per wave and matrix 32 columns x 2 floats (one per 64 reduction elements)
+//         + scales   per wave and matrix 32 columns x 2 floats (one per 64 reduction elements; 8-bit ones in registers)
 //   One barrier per stage: it publishes the rows that the other waves copied and frees the slot of the
 //   stage before for the next copies.  Three stages of 32-row tiles are 52 KiB, two stages of 64-row tiles 51 KiB:
 //   three workgroups share a CU (two of the gated form), and what counts is how many workgroups of the launch
@@ -57,12 +57,6 @@ __device__ __forceinline__ void copy4_to_lds(const void *src, unsigned char *dst
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(lds_addr) : "memory");
 }
 
-// Two bytes per lane, zero-extended to the lane's dword of LDS.
-__device__ __forceinline__ void copy2_to_lds(const void *src, unsigned char *dst) {
-    const uint32_t lds_addr = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void_ptr)dst);
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_ushort %0, off" : : "v"(src), "s"(lds_addr) : "memory");
-}
-
 // (byte `B` of w) << 2: the LDS byte offset of the pair-table entry of two packed weights, in one instruction.
 template <int B>
 __device__ __forceinline__ uint32_t byte_times_4(uint32_t w) {
@@ -89,15 +83,15 @@ struct StreamShape {
     static constexpr int RING = RING_;         // stages in LDS; all but one of them in flight
     static constexpr int kX = MR * 32 * 256;   // rows of a stage: MR blocks of 32
     static constexpr int kW = 32 * 64;         // packed weights of a stage, per wave and matrix
-    // scales of a stage, per wave and matrix: two floats per column, or one dword with two 8-bit values
-    static constexpr int kA = SC == SC_NESTED ? 32 * 4 : 32 * 2 * 4;
+    // scales of a stage, per wave and matrix: two floats per column (8-bit ones stay in registers)
+    static constexpr int kA = SC == SC_NESTED ? 0 : 32 * 2 * 4;
     static constexpr int kStage = kX + 4 * CB * (kW + kA);
     static constexpr int kTable = CB * 256 * 4;
     static constexpr int kTables = kTable * (SC == SC_NESTED ? 2 : 1);  // pairs of weights; scales by 8-bit value
     // RING 3, MR 1: 53248, three workgroups per CU; gated: 81920, two.  RING 2, MR 2: 52224, three; gated: 71680, two.
-    // (8-bit scales: 52736, 80896, 52224 and 71680: the same residency)
+    // (8-bit scales: 51200, 77824, 51200 and 69632: the same residency)
     static constexpr int kLds = RING * kStage + kTables;
-    static constexpr int kWOps = 2 * CB + (SC == SC_NESTED ? 1 : CB);  // copies of weights and scales per wave and stage (the rows: up to 2 MR more)
+    static constexpr int kWOps = 2 * CB + (SC == SC_NESTED ? 0 : CB);  // copies of weights and scales per wave and stage (the rows: up to 2 MR more)
 };
 
 // at most OPS + xc (xc = 0 .. XMAX, wave-uniform) vector-memory operations outstanding
@@ -112,7 +106,7 @@ __device__ __forceinline__ void wait_stage_ops(int xc) {
 }
 
 template <bool GLU, int SC, int MR, int RING_, typename TO>
-__global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restrict__ x,
+__global__ __launch_bounds__(256, GLU && !(SC == SC_NESTED && MR == 1) ? 2 : 3) void nf4_stream_kernel(const bf16_t *__restrict__ x,
                                                          const int32_t *__restrict__ row_idx, int idx_div,
                                                          Nf4Matrix w0, Nf4Matrix w1,
                                                          const void *__restrict__ m_sizes, int ms_i64,
@@ -204,25 +198,63 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
         if (col >= N) col = N - 1;
         a_el[cb] = ((int64_t)expert * N + col) * K + (lane & 1) * 64;
     }
-    // 8-bit scales: lane i brings the two bytes of a stage of column i & 31, of the gate projection's in lanes 0..31
-    // and of the up projection's in lanes 32..63; 32 columns' runs are one run of memory.  The scales of a row
-    // of the matrix (at most 1 << bs2_shift of them) lie under one or two second-level factors.
-    const uint8_t *q_src = nullptr;
+    const int NS = K / 128, tiles32 = (N + 31) / 32;
+    // 8-bit scales: a lane keeps its column's values of 16 stages in eight registers per matrix, two bytes a stage, read
+    // in one go before the first copies (and again every 16 stages, which waits for the copies in flight).  Copied like
+    // the rest, two bytes a stage and column, they cost every stage one more copy, in 32 pieces, and the second-level
+    // factors, loaded but not waited for before the loop, a wait for all copies in flight in every stage
+    // (16 rows per expert on 128 experts, N = 768 gated / 2048 plain: 70.8 / 42.2 us, now 67.7 / 40.6).  The scales of
+    // a row of the matrix (at most 1 << bs2_shift of them) lie under one or two second-level factors.
+    constexpr int QW = GLU && MR == 2 ? 4 : 8;  // (four, 8 stages, where eight would pass 256 registers)
+    uint32_t qw[CB][QW];
+    const uint8_t *q_run[CB];
     float q_lo[CB], q_hi[CB], q_off[CB];
     int q_turn = 0;  // first scale of the column under the second factor
+    auto load_scales = [&](int stg) {
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+            // (past the last stage: the last ones again, which nobody uses)
+            if (NS % 8 == 0 && ((uintptr_t)mat[cb].absmax_u8 & 15) == 0) {
+#pragma unroll
+                for (int i = 0; i < QW; i += 4) {
+                    const int s = stg + 2 * i < NS - 8 ? stg + 2 * i : NS - 8;
+                    const uint4_t v = *(const uint4_t *)(q_run[cb] + 2 * s);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) qw[cb][i + u] = v[u];
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < QW; ++i) {
+                    const int s = stg + 2 * i < NS - 1 ? stg + 2 * i : NS - 1, t = s + 1 < NS - 1 ? s + 1 : NS - 1;
+                    qw[cb][i] = *(const uint16_t *)(q_run[cb] + 2 * s) | (uint32_t) * (const uint16_t *)(q_run[cb] + 2 * t) << 16;
+                }
+            }
+        }
+    };
+    // what was loaded into registers is waited for here and not where it is used: a wait that the compiler puts into
+    // the loop would be one for all copies in flight, in every stage
+    auto scales_landed = [&]() {
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+#pragma unroll
+            for (int i = 0; i < QW; ++i) asm volatile("" : "+v"(qw[cb][i]));
+            asm volatile("" : "+v"(q_lo[cb]), "+v"(q_hi[cb]), "+v"(q_off[cb]));
+        }
+    };
     if constexpr (SC == SC_NESTED) {
         int col = j0 + n;
         if (col >= N) col = N - 1;
         const int64_t b0 = (((int64_t)expert * N + col) * K) >> 6;
-        q_src = (GLU && h ? w1 : w0).absmax_u8 + b0;
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
             const int sh = mat[cb].bs2_shift;
+            q_run[cb] = mat[cb].absmax_u8 + b0;
             q_lo[cb] = mat[cb].absmax2[b0 >> sh];
             q_hi[cb] = mat[cb].absmax2[(b0 + (K >> 6) - 1) >> sh];
             q_off[cb] = *mat[cb].offset;
         }
         q_turn = (int)((((b0 >> mat[0].bs2_shift) + 1) << mat[0].bs2_shift) - b0);
+        load_scales(0);
     }
     const bf16_t *x_src[2 * MR];  // copy j: rows 32 (j / 2) + 8 wave + 4 (j % 2) .. + 3, sixteen lanes to a row
 #pragma unroll
@@ -233,7 +265,6 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
         if (row_idx != nullptr) src_row = (uint32_t)row_idx[src_row] / (uint32_t)idx_div;
         x_src[j] = x + src_row * K + c * 8;
     }
-    const int NS = K / 128, tiles32 = (N + 31) / 32;
     // a wave whose 32 columns all lie past N (N not a multiple of 128) takes the scales of the last tile of its
     // expert: copied, multiplied, never stored, and inside the array also for the last expert
     const int a_tile = j0 / 32 < tiles32 ? j0 / 32 : tiles32 - 1;
@@ -262,8 +293,6 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
                                        : mat[cb].absmax + ((a_el[cb] + (int64_t)stg * 128) >> mat[cb].bs_shift);
             copy4_to_lds(a_src, base + S::kX + 4 * CB * S::kW + (wave * CB + cb) * S::kA);
         }
-        if constexpr (SC == SC_NESTED)
-            if (GLU || lane < 32) copy2_to_lds(q_src + 2 * stg, base + S::kX + 4 * CB * S::kW + wave * CB * S::kA);
     };
     // ---- where this lane reads a stage: its 16 bytes of packed weights of step s2, its 16 bytes of row n for
     // MFMA ks of step s2
@@ -286,9 +315,15 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
     // Every wave issues the same number of copies per stage (S::kWOps and the row copies it does not leave out),
     // unconditionally (past the end they repeat the last stage, into a slot that is free), so "at most RING - 2
     // stages' worth of my copies outstanding" means that the stage about to be read has landed.
+    if constexpr (SC == SC_NESTED) scales_landed();
 #pragma unroll
     for (int q = 0; q < RING - 1; ++q) issue(q < NS ? q : NS - 1);
     for (int q = 0; q < NS; ++q) {
+        if constexpr (SC == SC_NESTED)
+            if (q != 0 && q % (2 * QW) == 0) {
+                load_scales(q);
+                scales_landed();
+            }
         // at most (RING - 2) stages' worth of this wave's copies outstanding
         if constexpr (RING == 3) wait_stage_ops<S::kWOps, 2 * MR>(x_copies);
         else wait_vmcnt<0>();
@@ -303,11 +338,19 @@ __global__ __launch_bounds__(256) void nf4_stream_kernel(const bf16_t *__restric
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb) {
                 wl2[s2][cb] = *(const uint4_t *)(base + S::kX + (wave * CB + cb) * S::kW + w_rd[s2]);
-                const unsigned char *const a_rd = base + S::kX + 4 * CB * S::kW + (wave * CB + cb) * S::kA;
-                if constexpr (SC == SC_NESTED)
-                    am2[s2][cb] = *(const float *)(table + S::kTable + cb * 1024 + a_rd[n * 4 + s2] * 4);
-                else
-                    am2[s2][cb] = *(const float *)(a_rd + (n * 2 + s2) * 4);
+                if constexpr (SC == SC_NESTED) {
+                    const uint32_t value = (qw[cb][0] >> (16 * (q & 1) + 8 * s2)) & 0xff;
+                    am2[s2][cb] = *(const float *)(table + S::kTable + cb * 1024 + value * 4);
+                } else {
+                    am2[s2][cb] = *(const float *)(base + S::kX + 4 * CB * S::kW + (wave * CB + cb) * S::kA + (n * 2 + s2) * 4);
+                }
+            }
+        if constexpr (SC == SC_NESTED)
+            if (q & 1) {
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                    for (int i = 0; i + 1 < QW; ++i) qw[cb][i] = qw[cb][i + 1];
             }
         issue(q + RING - 1 < NS ? q + RING - 1 : NS - 1);
         // The eight MFMA steps of the stage in one sequence, the operands of a step (16 bytes of the rows, four
