@@ -89,7 +89,7 @@ struct StreamShape {
     static constexpr int kTable = CB * 256 * 4;
     static constexpr int kTables = kTable * (SC == SC_NESTED ? 2 : 1);  // pairs of weights; scales by 8-bit value
     // RING 3, MR 1: 53248, three workgroups per CU; gated: 81920, two.  RING 2, MR 2: 52224, three; gated: 71680, two.
-    // (8-bit scales: 51200, 77824, 51200 and 69632: the same residency)
+    // (8-bit scales: 51200, 77824, 51200 and 69632: the same residency; RING 2, MR 1: 34816, four; gated: 53248, three)
     static constexpr int kLds = RING * kStage + kTables;
     static constexpr int kWOps = 2 * CB + (SC == SC_NESTED ? 0 : CB);  // copies of weights and scales per wave and stage (the rows: up to 2 MR more)
 };
@@ -533,13 +533,23 @@ int gemm_nf4_stream(const bf16_t *x, const int32_t *row_idx, int idx_div, const 
     // more than a second stage in flight (plain product, 40 rows per expert: 43 us against 55 with three stages
     // and two workgroups per CU, 59 with 32-row tiles).  The bits are the same whatever the tile height.
     const bool two = R > (int64_t)kNf4StreamTwoBlockRows * E;
+    // 8-bit scales take no room in the stages, and two stages of 32-row tiles are small enough for one workgroup more on
+    // a CU (three of the gated form, four of the plain one).  Taken where the launch has more workgroups than stay
+    // resident with three stages: 61.6 against 67.7 us gated (768 workgroups, all resident instead of 512) and 36.6
+    // against 40.6 plain (2048) at 16 rows per expert; the block from 40 to 320 tokens 5 to 7 % faster, even where all
+    // workgroups are resident either way or nearly (8 to 16 experts).
+    const int64_t workgroups = (R / 32 + (R < E ? R : E)) * ceil_div(N, 128);
+    const bool shallow = nested && !two && workgroups > (int64_t)device_info().cu_count * (glu ? 2 : 3);
 #define MFL_STREAM_SC(GLU, SC, MR, RG, TO, Y, EO, GO) \
     launch_stream<GLU, SC, MR, RG, TO>(x, row_idx, idx_div, w0, w1, m_sizes, ms_i64, Y, EO, GO, R, N, K, E, stream)
 #define MFL_STREAM_MR(GLU, MR, RG, TO, Y, EO, GO)                            \
     (nested  ? MFL_STREAM_SC(GLU, SC_NESTED, MR, RG, TO, Y, EO, GO)          \
      : tiled ? MFL_STREAM_SC(GLU, SC_TILED, MR, RG, TO, Y, EO, GO)           \
              : MFL_STREAM_SC(GLU, SC_PLAIN, MR, RG, TO, Y, EO, GO))
-#define MFL_STREAM(GLU, TO, Y, EO, GO) (two ? MFL_STREAM_MR(GLU, 2, 2, TO, Y, EO, GO) : MFL_STREAM_MR(GLU, 1, 3, TO, Y, EO, GO))
+#define MFL_STREAM(GLU, TO, Y, EO, GO)                                    \
+    (two       ? MFL_STREAM_MR(GLU, 2, 2, TO, Y, EO, GO)                  \
+     : shallow ? MFL_STREAM_SC(GLU, SC_NESTED, 1, 2, TO, Y, EO, GO)       \
+               : MFL_STREAM_MR(GLU, 1, 3, TO, Y, EO, GO))
     if (glu) return MFL_STREAM(true, bf16_t, (bf16_t *)y, (bf16_t *)e_out, (bf16_t *)g_out);
     if (out_dtype == MFL_BF16) return MFL_STREAM(false, bf16_t, (bf16_t *)y, nullptr, nullptr);
     return MFL_STREAM(false, float, (float *)y, nullptr, nullptr);
