@@ -32,6 +32,18 @@ def test_join_pad_and_split(e, ra, rb, h, dtype):
         assert all(torch.equal(x, y) and x.is_contiguous() for x, y in zip(halves, parts))
 
 
+def test_strided_and_mixed_operands():
+    g = gen(3)
+    a, b = (torch.randn((5, 24, 16), generator=g).bfloat16().cuda().transpose(1, 2) for _ in range(2))
+    p = torch.randn((5, 16, 24), generator=g).bfloat16().cuda().transpose(1, 2)
+    f = torch.randn((5, 16, 24), generator=g).cuda()
+    pieces = []
+    got = [_joined(a, b, 1, pieces), _padded(p, 2, 0, 32, pieces), _joined(a, f, 1, pieces)]
+    _copy_pieces(pieces, True)
+    want = [torch.cat((a, b), 1), torch.cat((p, torch.zeros_like(p)), 2), torch.cat((a, f), 1)]
+    assert all(torch.equal(x, y) and x.dtype == y.dtype for x, y in zip(got, want))
+
+
 def test_copy_blocks_refuses_what_it_cannot_copy():
     buf = torch.zeros(256, device="cuda", dtype=torch.uint8)
     at = buf.data_ptr()

@@ -113,7 +113,8 @@ def _copy_pieces(pieces: Sequence[_Piece], join: bool) -> None:
 
 def _joined(a: torch.Tensor, b: torch.Tensor, dim: int, pieces: List[_Piece]) -> torch.Tensor:
     """Room for ``torch.cat((a, b), dim)``; what fills it is added to ``pieces``."""
-    assert a.is_contiguous() and b.is_contiguous() and a.dtype == b.dtype
+    dtype = torch.promote_types(a.dtype, b.dtype)  # (any strides and types, as the concatenation takes them)
+    a, b = a.to(dtype).contiguous(), b.to(dtype).contiguous()
     shape = list(a.shape)
     na, nb = a.shape[dim], b.shape[dim]
     shape[dim] = na + nb
@@ -124,6 +125,7 @@ def _joined(a: torch.Tensor, b: torch.Tensor, dim: int, pieces: List[_Piece]) ->
 
 def _padded(b: torch.Tensor, dim: int, first: int, total: int, pieces: List[_Piece]) -> torch.Tensor:
     """Room for ``b`` in the columns from ``first`` on of ``total``, zeros in the others (one side of it)."""
+    b = b.contiguous()
     size = b.shape[dim]
     shape = list(b.shape)
     shape[dim] = total
