@@ -117,3 +117,17 @@ def test_block_call_leaves_hooks_forward_mode_and_the_routing_alone():
         handle.remove()
         with torch.autograd.forward_ad.dual_level(), pytest.raises(Exception):  # no kernel here has a forward-mode rule
             blk(torch.autograd.forward_ad.make_dual(x, x))
+
+
+@pytest.mark.parametrize("kind", ["bf16", "nf4dq"])
+def test_rows_beyond_one_call(kind, monkeypatch):
+    """The same bits on both sides of the row count that ends the one call."""
+    blk, dtype = _block(8, 4, 256, 128, kind, 4)
+    hidden = torch.randn((1, 33, 256), generator=gen(4)).to(dtype).cuda()
+    got = []
+    for rows in (33 * 4, 33 * 4 - 1):
+        monkeypatch.setattr(blk, "_ONE_CALL_ROWS", rows, raising=False)
+        with torch.no_grad():
+            assert (blk._one_call(hidden[0], blk.gate(hidden[0])) is None) == (rows < 33 * 4)
+            got.append(blk(hidden))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])

@@ -135,6 +135,11 @@ class Qwen3MoeFusedSparseMoeBlock(nn.Module):
         return moe_fused_mlp(tokens, self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, m_sizes,
                              sort_idx, inv_sort_idx, self.num_selected)
 
+    # Rows up to which the block is one library call: beyond, the kernels hide the host's time (131072 rows on packed
+    # weights: 1638 us either way) and the one buffer of all intermediates, 740 MB there, costs a first pass more than the
+    # steps' own tensors do, which find their room in what the allocator holds (1870 against 1733 us).
+    _ONE_CALL_ROWS = 65536
+
     def _one_call(self, tokens: torch.Tensor, logits: torch.Tensor) -> Optional[torch.Tensor]:
         """Everything behind the router projection as one library call, where the three projections are plain expert
         matrices in the tokens' type (both ways), or plain packed ones (without gradients)."""
@@ -146,6 +151,8 @@ class Qwen3MoeFusedSparseMoeBlock(nn.Module):
         if kind not in (MoeFusedLinear, MoeFusedLinear4bit) or type(up) is not kind or type(down) is not kind:
             return None
         if tokens.shape[0] == 0 or self.num_experts > 1024:
+            return None
+        if tokens.shape[0] * self.num_selected > self._ONE_CALL_ROWS:
             return None
         for proj in (gate, up, down):  # hooks and replaced forwards run on the separate steps
             if (proj._forward_hooks or proj._forward_pre_hooks or proj._backward_hooks or proj._backward_pre_hooks
