@@ -65,10 +65,15 @@ class _RouterLinear(torch.autograd.Function):
 
 def router_linear(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
     """``torch.nn.functional.linear(x, w)`` for a bf16 router, x (T, hidden), w (E, hidden), both contiguous on one GPU.
-    ``None`` for anything else: other types and forms, tensor subclasses, and calls that a transform has to see."""
-    if (type(x) not in _PLAIN or type(w) not in _PLAIN or not _lib.plain_call() or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda or x.device != w.device or x.ndim != 2
-            or x.shape[0] == 0 or not x.is_contiguous() or not w.is_contiguous() or torch.is_autocast_enabled("cuda")
-            or x.data_ptr() % 16 or w.data_ptr() % 16):
+    ``None`` for anything else: other types and forms, tensor subclasses, calls that a transform has to see, and rows of
+    another width than the weight's, which the stock operator refuses."""
+    if type(x) not in _PLAIN or type(w) not in _PLAIN or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+        return None
+    if not x.is_cuda or x.device != w.device or x.ndim != 2 or w.ndim != 2 or x.shape[1] != w.shape[1] or x.shape[0] == 0:
+        return None
+    if not _lib.plain_call() or torch.is_autocast_enabled("cuda"):
+        return None
+    if not x.is_contiguous() or not w.is_contiguous() or x.data_ptr() % 16 or w.data_ptr() % 16:
         return None
     if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
         return _RouterLinear.apply(x, w)
