@@ -37,3 +37,67 @@ def test_router_refuses_rows_of_another_width(no_kernels, width, grad):
     with pytest.raises(RuntimeError, match="cannot be multiplied"):
         out = routing.router_linear(x, w)
         torch.nn.functional.linear(x, w) if out is None else out
+
+
+def _dense(t=6, e=4, h=32, i=16, dtype=torch.bfloat16):
+    g = torch.Generator().manual_seed(1)
+    return [torch.randn(s, generator=g).to(dtype) for s in ((t, h), (t, e), (e, i, h), (e, i, h), (e, h, i))]
+
+
+# position of the tensor that does not fit (tokens, logits, gate, up, down) and what stands there instead
+MISFITS = [(0, (6, 16)), (0, (6, 48)), (0, (5, 32)), (1, (6, 3)), (1, (6, 5)), (1, (7, 4)), (2, (3, 16, 32)), (2, (4, 8, 32)),
+           (3, (4, 8, 32)), (3, (4, 24, 32)), (3, (5, 16, 32)), (4, (4, 16, 32)), (4, (3, 32, 16)), (4, (4, 40, 16)),
+           (2, (64, 32))]
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("which,shape", MISFITS)
+def test_block_call_refuses_operands_that_do_not_fit(no_kernels, which, shape, grad):
+    from qwen3_moe_fused.fused_mlp import moe_block
+
+    args = _dense()
+    with pytest.raises(LibraryCalled):
+        moe_block(*args, 2, True)
+    args[which] = torch.zeros(shape, dtype=torch.bfloat16)
+    args[4].requires_grad_(grad)
+    with pytest.raises(AssertionError):
+        moe_block(*args, 2, True)
+
+
+def _strided(t):
+    return torch.empty((*t.shape[:-1], t.shape[-1] + 1), dtype=t.dtype)[..., :-1]
+
+
+@pytest.mark.parametrize("which", range(5))
+@pytest.mark.parametrize("how", [_strided, torch.Tensor.double, lambda t: t.to("meta")], ids=["strided", "type", "device"])
+def test_block_call_refuses_strides_types_and_devices(no_kernels, which, how):
+    from qwen3_moe_fused.fused_mlp import moe_block
+
+    args = _dense()
+    args[which] = how(args[which])
+    with pytest.raises((AssertionError, TypeError)):
+        moe_block(*args, 2, True)
+
+
+@pytest.mark.parametrize("e", [3, 5])
+def test_block_call_on_packed_weights_refuses_logits_of_other_experts(no_kernels, e):
+    from qwen3_moe_fused import fused_mlp
+
+    tokens, _, gate, up, down = _packed_block()
+    with pytest.raises(AssertionError):
+        fused_mlp.moe_block_4bit(tokens, torch.zeros((6, e), dtype=torch.bfloat16), gate, up, down, 2, True)
+    with pytest.raises(LibraryCalled):
+        fused_mlp.moe_block_4bit(tokens, torch.zeros((6, 4), dtype=torch.bfloat16), gate, up, down, 2, True)
+
+
+def _packed_block(t=6, e=4, h=128, i=64):
+    from qwen3_moe_fused.quantize.layer import Nf4Params
+    from qwen3_moe_fused.quantize.nf4 import BlockwiseState, Nf4QuantState, code_of
+
+    def packed(n, k):
+        state = Nf4QuantState(absmax=torch.ones(e * n * k // 64, dtype=torch.uint8), shape=(e, n, k), code=code_of("nf4", "cpu"),
+                              blocksize=64, quant_type="nf4", dtype=torch.bfloat16, offset=torch.zeros(()),
+                              state2=BlockwiseState(absmax=torch.ones(e * n * k // 64 // 4), code=torch.zeros(256), blocksize=4))
+        return Nf4Params(torch.zeros((e * n * k // 2, 1), dtype=torch.uint8), quant_state=state)
+
+    return _bf16(t, h), None, packed(i, h), packed(i, h), packed(h, i)

@@ -197,11 +197,23 @@ def _run_block(b, tokens):
     return out, ws
 
 
+def _check_rows(tokens, logits, experts, hidden):
+    """The block's rows against its experts: the library gets sizes from one operand and pointers to all."""
+    assert tokens.ndim == 2 and tokens.shape[1] == hidden and logits.shape == (tokens.shape[0], experts)
+    assert tokens.is_contiguous() and logits.is_contiguous() and logits.device == tokens.device
+
+
 def moe_block(tokens: torch.Tensor, logits: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
               num_selected: int, renorm: bool):
     """Everything of the sparse block that follows the router projection (modular_qwen3_moe_fused.py:87-115):
     ``tokens`` (T, hidden), ``logits`` (T, E), the three expert matrices in the tokens' type.  Returns (output (T, hidden),
     workspace, whose first T * num_selected int64 are the expert ids).  Differentiable in all five tensors."""
+    assert w_gate.ndim == 3
+    experts, inter, hidden = w_gate.shape
+    assert w_up.shape == w_gate.shape and w_down.shape == (experts, hidden, inter)
+    _check_rows(tokens, logits, experts, hidden)
+    for w in (w_gate, w_up, w_down):
+        assert w.dtype == tokens.dtype and w.device == tokens.device and w.is_contiguous()
     if torch.is_grad_enabled() and any(t.requires_grad for t in (tokens, logits, w_gate, w_up, w_down)):
         return _MoeBlock.apply(tokens, logits, w_gate, w_up, w_down, num_selected, renorm)
     return _run_block(_dense_block(tokens, logits, w_gate, w_up, w_down, num_selected, renorm, False), tokens)
@@ -215,6 +227,7 @@ def moe_block_4bit(tokens: torch.Tensor, logits: torch.Tensor, w_gate: torch.Ten
     experts, inter = check_packed(tokens, w_gate, w_gate.quant_state, hidden)
     assert check_packed(tokens, w_up, w_up.quant_state, hidden) == (experts, inter)
     assert check_packed(tokens, w_down, w_down.quant_state, inter) == (experts, hidden)
+    _check_rows(tokens, logits, experts, hidden)
     rows = tokens.shape[0] * num_selected
     (gate, _kg), (up, _ku), (down, _kd) = (packed_weight(w, w.quant_state, rows) for w in (w_gate, w_up, w_down))
     if any(w.absmax_u8 and w.blocksize2 & (w.blocksize2 - 1) for w in (gate, up, down)):
