@@ -101,3 +101,23 @@ def _packed_block(t=6, e=4, h=128, i=64):
         return Nf4Params(torch.zeros((e * n * k // 2, 1), dtype=torch.uint8), quant_state=state)
 
     return _bf16(t, h), None, packed(i, h), packed(i, h), packed(h, i)
+
+
+def test_nothing_on_the_host_reaches_the_block_kernels(monkeypatch):
+    """A block on the CPU was refused by the checks of the separate steps: as one call it is as well."""
+    from types import SimpleNamespace
+
+    from qwen3_moe_fused.modular_qwen3_moe_fused import Qwen3MoeFusedSparseMoeBlock
+
+    monkeypatch.setattr(_lib, "lib", lambda: _StandIn())
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    block = Qwen3MoeFusedSparseMoeBlock(SimpleNamespace(
+        num_experts=4, num_experts_per_tok=2, norm_topk_prob=True, hidden_size=32, moe_intermediate_size=16,
+        hidden_act="silu"))
+    with pytest.raises(AssertionError):
+        block(torch.zeros((1, 3, 32)))
+    from qwen3_moe_fused.fused_mlp import moe_block_4bit
+
+    tokens, _, gate, up, down = _packed_block()
+    with pytest.raises(AssertionError):
+        moe_block_4bit(tokens, torch.zeros((6, 4), dtype=torch.bfloat16), gate, up, down, 2, True)

@@ -201,6 +201,7 @@ def _check_rows(tokens, logits, experts, hidden):
     """The block's rows against its experts: the library gets sizes from one operand and pointers to all."""
     assert tokens.ndim == 2 and tokens.shape[1] == hidden and logits.shape == (tokens.shape[0], experts)
     assert tokens.is_contiguous() and logits.is_contiguous() and logits.device == tokens.device
+    assert tokens.is_cuda, "the block runs on the GPU only"
 
 
 def moe_block(tokens: torch.Tensor, logits: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
