@@ -318,7 +318,8 @@ MFL_API int mfl_router_dw(const void *x, const void *dlogits, void *dw, int64_t 
 
 /* p = softmax_fp32(logits[t, :]); top-k of p, descending, equal values -> lower expert id
  * first; if renorm, weights /= sum(weights).  weights_f32 (T,k) and/or weights_cast (T,k) of
- * cast_dtype may be NULL; idx (T,k) int64 is required.
+ * cast_dtype may be NULL; idx (T,k) int64 is required.  A token whose probabilities are NaN selects
+ * no expert: its ids are 0x7fffffff, its weights NaN.
  * Replaces qwen3_moe_fused/modular_qwen3_moe_fused.py:87-93 (= fast_lora.py:52-58). */
 MFL_API int mfl_route_softmax_topk(const void *logits, int logits_dtype, int64_t T, int E, int k,
                            int renorm, float *weights_f32, void *weights_cast, int cast_dtype,
@@ -362,8 +363,8 @@ MFL_API int mfl_route_sort(const void *logits, int logits_dtype, int64_t T, int 
  *   counts[e]        = #{j : sel[j] == e}
  *   sort_idx[i]      = j of the i-th row in the stable ascending order
  *   inv_sort_idx[j]  = position of row j in that order
- * sort_idx and inv_sort_idx may both be NULL (counts only).  Ids outside [0, E) are a
- * caller error (they are ignored by the counts and leave their slots unwritten).
+ * sort_idx and inv_sort_idx may both be NULL (counts only).  Ids outside [0, E) are not counted
+ * and come behind all others, in order: both arrays are permutations of 0 .. R-1 in any case.
  * workspace: mfl_expert_sort_workspace(R, E) bytes of device memory, contents ignored.
  * Replaces get_expert_counts_and_idx / get_expert_counts,
  * qwen3_moe_fused/kernels/indexing.py:18-23,48-65. */

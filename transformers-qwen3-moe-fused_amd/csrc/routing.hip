@@ -113,7 +113,8 @@ __device__ __forceinline__ int topk_one_token(const TI *__restrict__ logits, int
                 if (oi < bi) bi = oi;
             }
         }
-        const float bp = m < 0 ? -2.0f : __builtin_bit_cast(float, m);  // (nothing left: a row of NaN)
+        // (nothing left: a row of NaN, whose weights say so; its selections are the id 0x7fffffff)
+        const float bp = m < 0 ? __builtin_nanf("") : __builtin_bit_cast(float, m);
         // the owner retires the winner
 #pragma unroll
         for (int v = 0; v < VPL; ++v)
@@ -276,6 +277,15 @@ __device__ __forceinline__ int64_t load_key(const void *sel, int is_i64, int64_t
     return is_i64 ? ((const int64_t *)sel)[j] : (int64_t)((const int32_t *)sel)[j];
 }
 
+struct NoExpert {  // whether selection j names no expert
+    const void *sel;
+    int is_i64, E;
+    __device__ __forceinline__ bool operator()(int64_t j) const {
+        const int64_t k = load_key(sel, is_i64, j);
+        return k < 0 || k >= E;
+    }
+};
+
 // Phase 1 for one wave: walk its segment [seg_begin, seg_end) in batches of 64 in order,
 // count keys into the wave-private histogram `hist` (LDS, E ints, zeroed by the caller) and,
 // when `local_rank` is given, store each row's rank among the rows of the same key seen so
@@ -320,11 +330,40 @@ __device__ __forceinline__ void wave_count(const void *sel, int is_i64, int E, i
     }
 }
 
+// Selections that name no expert (those of a token whose logits are NaN) come behind all others, in order: every
+// position and index is written and in range, so that what reads or writes rows by them stays inside its tensors.
+// A wave places those of its segment [sb, se); it asks no_expert(j) of all R selections, which only a wave that has met
+// such a selection comes to.
+template <typename F>
+__device__ __forceinline__ void place_rest(F &&no_expert, int64_t R, int64_t sb, int64_t se, int32_t *sort_idx,
+                                           int32_t *inv_sort_idx, int lane) {
+    int all = 0, before = 0;
+    for (int64_t j = lane; j < R; j += 64)
+        if (no_expert(j)) {
+            ++all;
+            if (j < sb) ++before;
+        }
+    int64_t pos = R - wave_last(wave_inclusive_scan(all)) + wave_last(wave_inclusive_scan(before));
+    const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    for (int64_t j0 = sb; j0 < se; j0 += 64) {
+        const int64_t j = j0 + lane;
+        const bool mine = j < se && no_expert(j);
+        const uint64_t those = __ballot(mine);
+        if (mine) {
+            const int at = (int)(pos + __popcll(those & lt_mask));
+            if (inv_sort_idx) inv_sort_idx[j] = at;
+            if (sort_idx) sort_idx[at] = (int32_t)j;
+        }
+        pos += __popcll(those);
+    }
+}
+
 // Phase 3 for one wave: final position = rank within the wave's segment + global offset of
 // (wave, key); writes inv_sort_idx in place of the rank and scatters sort_idx.
-__device__ __forceinline__ void wave_scatter(const void *sel, int is_i64, int E, int64_t seg_begin, int64_t seg_end,
-                                             const int *offsets, const int *offsets2, int32_t *sort_idx,
-                                             int32_t *rank_io, int lane) {
+__device__ __forceinline__ void wave_scatter(const void *sel, int is_i64, int64_t R, int E, int64_t seg_begin,
+                                             int64_t seg_end, const int *offsets, const int *offsets2,
+                                             int32_t *sort_idx, int32_t *rank_io, int lane) {
+    bool rest = false;
     for (int64_t chunk = seg_begin; chunk < seg_end; chunk += 64 * kSortChunk) {
         int keys[kSortChunk], ranks[kSortChunk];
 #pragma unroll
@@ -346,9 +385,12 @@ __device__ __forceinline__ void wave_scatter(const void *sel, int is_i64, int E,
                 const int pos = ranks[u] + offsets[keys[u]] + (offsets2 ? offsets2[keys[u]] : 0);
                 rank_io[j] = pos;
                 if (sort_idx) sort_idx[pos] = (int32_t)j;
+            } else if (j < seg_end) {
+                rest = true;
             }
         }
     }
+    if (__ballot(rest) != 0) place_rest(NoExpert{sel, is_i64, E}, R, seg_begin, seg_end, sort_idx, rank_io, lane);
 }
 
 __device__ __forceinline__ void segment_of(int w, int n_waves, int64_t R, int64_t &b, int64_t &e) {
@@ -406,7 +448,7 @@ __device__ __forceinline__ void sort_single_body(const void *__restrict__ sel, i
         }
     }
     __syncthreads();
-    wave_scatter(sel, is_i64, E, sb, se, table + wave * E, totals, sort_idx, inv_sort_idx, lane);
+    wave_scatter(sel, is_i64, R, E, sb, se, table + wave * E, totals, sort_idx, inv_sort_idx, lane);
 }
 
 __global__ __launch_bounds__(1024) void sort_single_kernel(const void *__restrict__ sel, int is_i64, int64_t R,
@@ -439,7 +481,7 @@ __global__ __launch_bounds__(1024) void route_sort_small_kernel(const TI *__rest
     for (int i = threadIdx.x; i < n_waves * E; i += blockDim.x) table[i] = 0;
     for (int t = wave; t < (int)T; t += n_waves) {
         const int sel = topk_one_token<TI, TC, VPL>(logits, t, E, k, renorm, w_f32, w_cast, idx, lane);
-        // (a row of NaN selects no expert: an id outside [0, E), which is neither counted nor placed)
+        // (a row of NaN selects no expert: an id outside [0, E), which is not counted and placed behind all others)
         if (lane < k) keys[t * k + lane] = (unsigned)sel < (unsigned)E ? (uint16_t)sel : (uint16_t)0xffff;
     }
     __syncthreads();
@@ -491,13 +533,22 @@ __global__ __launch_bounds__(1024) void route_sort_small_kernel(const TI *__rest
         }
     }
     __syncthreads();
+    bool rest = false;
 #pragma unroll
     for (int u = 0; u < kSmallBatches; ++u) {
-        if (u >= per_wave || key[u] == 0xffff) continue;
+        if (u >= per_wave) continue;
         const int j = (wave * per_wave + u) * 64 + lane;
+        if (key[u] == 0xffff) {
+            rest |= j < R;
+            continue;
+        }
         const int pos = rank[u] + hist[key[u]] + first[key[u]];
         inv_sort_idx[j] = pos;
         sort_idx[pos] = j;
+    }
+    if (__ballot(rest) != 0) {
+        const int sb = wave * per_wave * 64, se = sb + per_wave * 64;
+        place_rest([&](int64_t j) { return keys[j] == 0xffff; }, R, sb, se < R ? se : R, sort_idx, inv_sort_idx, lane);
     }
 }
 
@@ -565,7 +616,7 @@ __global__ __launch_bounds__(256) void sort_scatter_kernel(const void *__restric
     if (wave >= n_waves) return;
     int64_t sb, se;
     segment_of(wave, n_waves, R, sb, se);
-    wave_scatter(sel, is_i64, E, sb, se, table + (int64_t)wave * E, nullptr, sort_idx, inv_sort_idx, lane);
+    wave_scatter(sel, is_i64, R, E, sb, se, table + (int64_t)wave * E, nullptr, sort_idx, inv_sort_idx, lane);
 }
 
 // ---- two-kernel sort (E <= 512) ------------------------------------------------------------
@@ -703,18 +754,23 @@ __global__ __launch_bounds__(1024) void fast_scatter_kernel(const void *__restri
     }
     int64_t sb, se;
     segment_of(wave, n_waves, R, sb, se);
+    bool rest = false;
     for (int64_t c = sb; c < se; c += 64 * kFastBatches) {
         int keys[kFastBatches], ranks[kFastBatches];
         wave_rank_chunk<kFastBatches>(sel, is_i64, E, key_bits, c, se, hist, keys, ranks, lane);
 #pragma unroll
         for (int u = 0; u < kFastBatches; ++u) {
-            if (keys[u] < 0) continue;
             const int64_t j = c + u * 64 + lane;
+            if (keys[u] < 0) {
+                rest |= j < se;
+                continue;
+            }
             const int pos = ranks[u] + my_off[keys[u]];
             if (inv_sort_idx) inv_sort_idx[j] = pos;
             if (sort_idx) sort_idx[pos] = (int32_t)j;
         }
     }
+    if (__ballot(rest) != 0) place_rest(NoExpert{sel, is_i64, E}, R, sb, se, sort_idx, inv_sort_idx, lane);
 }
 
 // ---- routing in two launches: softmax + top-k that also counts, then the scatter
@@ -736,8 +792,8 @@ __global__ __launch_bounds__(1024) void route_count_kernel(const TI *__restrict_
         const int64_t t = (int64_t)blockIdx.x * tokens_per_seg + tt;
         if (t >= T) break;
         const int sel = topk_one_token<TI, TC, VPL>(logits, t, E, k, renorm, w_f32, w_cast, idx, lane);
-        // a row of NaN (or of -inf throughout) selects nothing: its lanes keep the "no expert" id, which the
-        // scatter pass skips like any key outside [0, E); it must not reach the histogram either
+        // a row of NaN (or of -inf throughout) selects nothing: its lanes keep the "no expert" id, which the scatter
+        // pass places behind all others like any key outside [0, E); it must not reach the histogram
         if (lane < k && (unsigned)sel < (unsigned)E) atomicAdd(&lds[sel], 1);
     }
     __syncthreads();
@@ -872,12 +928,14 @@ __global__ __launch_bounds__(1024) void route_scatter_kernel(const int64_t *__re
     if (seg >= n_segs) return;
     const int *my_off = offs + wib * E;
     const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    bool rest = false;
 #pragma unroll
     for (int u = 0; u < kFastBatches; ++u) {
         const int key = keys[u];
         const bool valid = key >= 0;
+        rest |= !valid && sb + u * 64 + lane < se;
         uint64_t same = __ballot(valid);
-        if (same == 0) continue;  // past the end of the segment
+        if (same == 0) continue;  // past the end of the segment, or rows of NaN throughout
         for (int b = 0; b < key_bits; ++b) {
             const uint64_t bal = __ballot((key >> b) & 1);
             same &= ((key >> b) & 1) ? bal : ~bal;
@@ -891,6 +949,7 @@ __global__ __launch_bounds__(1024) void route_scatter_kernel(const int64_t *__re
             if (sort_idx) sort_idx[pos] = (int32_t)j;
         }
     }
+    if (__ballot(rest) != 0) place_rest(NoExpert{sel, 1, E}, R, sb, se, sort_idx, inv_sort_idx, lane);
 }
 
 inline int fast_waves(int64_t R) {
