@@ -257,7 +257,7 @@ MFL_API int mfl_glu_fwd_nf4_tiled(const void *x, int64_t src_rows, const int32_t
 
 /* A packed 4-bit matrix with its quantisation state.  Its scales are either fp32 (absmax, and optionally their
  * tile-ordered copy) or quantised once more to 8 bits (absmax_u8 not NULL; the bitsandbytes default):
- * scale b = code256[absmax_u8[b]] * absmax2[b / blocksize2] + *offset. */
+ * scale b = code256[absmax_u8[b]] * absmax2[b / blocksize2] + *offset, blocksize2 a power of two, 2 at least. */
 typedef struct mfl_nf4_weight {
     const uint8_t *packed;
     const float *code16;

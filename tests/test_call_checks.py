@@ -121,3 +121,55 @@ def test_nothing_on_the_host_reaches_the_block_kernels(monkeypatch):
     tokens, _, gate, up, down = _packed_block()
     with pytest.raises(AssertionError):
         moe_block_4bit(tokens, torch.zeros((6, 4), dtype=torch.bfloat16), gate, up, down, 2, True)
+
+
+class _Recorder:
+    """Stands for the library: notes the packed matrices that a product is given and answers as told."""
+
+    def __init__(self, answers):
+        self.seen, self.answers = [], answers
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.seen.append((name, [(a.absmax_u8 is not None, a.blocksize2) for a in args if isinstance(a, _lib.Nf4Weight)]))
+            return self.answers.get(name, 0)
+
+        return call
+
+
+def _with_blocksize2(w, blocksize2):
+    st = w.quant_state
+    st.state2.blocksize = blocksize2
+    st.state2.absmax = torch.ones(-(-st.absmax.numel() // blocksize2))
+    return w
+
+
+# A second level in blocks that are not a power of two, or of one scale each, has no kernel of its own: the scales are
+# written out first, as they were for every product.
+@pytest.mark.parametrize("blocksize2", [1, 3, 100])
+def test_other_second_level_blocks_are_written_out(monkeypatch, blocksize2):
+    from qwen3_moe_fused import fused_mlp
+    from qwen3_moe_fused.grouped_gemm import forward_4bit, fused
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    tokens, _, gate, up, down = (t if i < 2 else _with_blocksize2(t, blocksize2) for i, t in enumerate(_packed_block()))
+    sizes, rows = torch.full((4,), 3, dtype=torch.int32), torch.zeros(12, dtype=torch.int32)
+    products = {
+        "mfl_gemm_fwd_nf4_packed": [
+            lambda: forward_4bit.grouped_gemm_forward_4bit(_bf16(12, 128), gate, gate.quant_state, sizes),
+            lambda: fused.grouped_gemm_forward_4bit_gathered(tokens, rows, 2, gate, gate.quant_state, sizes)],
+        "mfl_glu_fwd_nf4_packed": [
+            lambda: fused.grouped_glu_forward_4bit(tokens, gate, gate.quant_state, up, up.quant_state, sizes, rows, 2)]}
+    for name, calls in products.items():
+        for call in calls:
+            lib = _Recorder({})
+            monkeypatch.setattr(_lib, "lib", lambda: lib)
+            call()
+            given = [w for n, w in lib.seen if n == name]
+            assert given and not any(nested for ws in given for nested, _ in ws)
+            assert any(n == "mfl_dequant_blockwise_u8" for n, _ in lib.seen)
+    lib = _Recorder({})
+    fused_mlp.moe_block_4bit(tokens, torch.zeros((6, 4), dtype=torch.bfloat16), gate, up, down, 2, True)
+    names = [n for n, _ in lib.seen]
+    assert names[-1] == "mfl_moe_block_fwd" and names.count("mfl_dequant_blockwise_u8") == 3

@@ -76,3 +76,33 @@ def test_products_on_double_quantised_weights_are_those_on_written_out_scales(si
     want = grouped_glu_forward_4bit(src, gate, gate_plain, up, up_plain, ms, idx, 1, return_products=True)
     for a, b in zip(got, want):
         assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("blocksize2", [1, 3, 100])
+def test_second_level_blocks_of_any_size(blocksize2):
+    from qwen3_moe_fused.fused_mlp import moe_block_4bit
+    from qwen3_moe_fused.quantize.layer import Nf4Params
+    from qwen3_moe_fused.quantize.nf4 import _quantize_absmax
+
+    e, k, n, rows = 3, 128, 64, 10
+    states = []
+    for seed, shape in enumerate(((e, n, k), (e, n, k), (e, k, n))):
+        packed, state = quantize_nf4((torch.randn(shape, generator=gen(seed)) * 0.02).to(torch.bfloat16).cuda(), 64)
+        q, state2, offset = _quantize_absmax(state.absmax, blocksize2)
+        nested = Nf4QuantState(absmax=q, shape=shape, code=state.code, blocksize=64, offset=offset, state2=state2)
+        want = state2.code[q.long()] * state2.absmax.repeat_interleave(blocksize2)[:q.numel()] + offset
+        plain = Nf4QuantState(absmax=want, shape=shape, code=state.code, blocksize=64)
+        assert torch.equal(resolve_absmax(nested), want)
+        states.append((packed, nested, plain))
+    x = torch.randn((rows, k), generator=gen(9)).to(torch.bfloat16).cuda()
+    ms = torch.tensor([4, 0, 6], dtype=torch.int32).cuda()
+    idx = torch.randperm(rows, generator=gen(8)).to(torch.int32).cuda()
+    (g, g8, g32), (u, u8, u32), (d, d8, d32) = states
+    assert torch.equal(grouped_gemm_forward_4bit(x, g, g8, ms), grouped_gemm_forward_4bit(x, g, g32, ms))
+    assert torch.equal(grouped_gemm_forward_4bit_gathered(x, idx, 1, g, g8, ms),
+                       grouped_gemm_forward_4bit_gathered(x, idx, 1, g, g32, ms))
+    assert torch.equal(grouped_glu_forward_4bit(x, g, g8, u, u8, ms, idx, 1), grouped_glu_forward_4bit(x, g, g32, u, u32, ms, idx, 1))
+    logits = torch.randn((rows, e), generator=gen(7)).to(torch.bfloat16).cuda()
+    outs = [moe_block_4bit(x, logits, *(Nf4Params(p, quant_state=s) for p, s in zip((g, u, d), which)), 2, True)[0]
+            for which in ((g8, u8, d8), (g32, u32, d32))]
+    assert torch.equal(*outs)

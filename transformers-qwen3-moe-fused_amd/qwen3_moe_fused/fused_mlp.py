@@ -231,8 +231,6 @@ def moe_block_4bit(tokens: torch.Tensor, logits: torch.Tensor, w_gate: torch.Ten
     _check_rows(tokens, logits, experts, hidden)
     rows = tokens.shape[0] * num_selected
     (gate, _kg), (up, _ku), (down, _kd) = (packed_weight(w, w.quant_state, rows) for w in (w_gate, w_up, w_down))
-    if any(w.absmax_u8 and w.blocksize2 & (w.blocksize2 - 1) for w in (gate, up, down)):
-        return None, None
     b = _lib.MoeBlock(tokens.data_ptr(), logits.data_ptr(), None, None, None, ctypes.pointer(gate), ctypes.pointer(up),
                       ctypes.pointer(down), tokens.shape[0], experts, num_selected, hidden, inter, int(bool(renorm)),
                       _lib.dtype_code(tokens.dtype), _lib.dtype_code(logits.dtype), 0)

@@ -161,6 +161,11 @@ def _second_level(quant_state):
     return absmax, code2, absmax2, int(st2.blocksize), offset.to(device=absmax.device, dtype=torch.float32)
 
 
+def _is_shift(blocksize2: int) -> bool:
+    """Whether the kernels that read 8-bit scales find a scale's second-level factor by a shift of its number."""
+    return blocksize2 >= 2 and blocksize2 & (blocksize2 - 1) == 0
+
+
 def resolve_absmax(quant_state) -> torch.Tensor:
     """fp32 absmax of an NF4 state, un-nesting a double-quantised one:
     ``dequantize_blockwise(absmax_u8, state2) + offset`` (forward_4bit.py:149-152)."""
@@ -168,7 +173,7 @@ def resolve_absmax(quant_state) -> torch.Tensor:
     if getattr(quant_state, "nested", False):
         absmax, code2, absmax2, blocksize2, offset = _second_level(quant_state)
         out = torch.empty(absmax.numel(), device=absmax.device, dtype=torch.float32)
-        if blocksize2 & (blocksize2 - 1):
+        if not _is_shift(blocksize2):
             rc = _lib.lib().mfl_dequant_blockwise_u8(_lib.ptr(absmax), _lib.ptr(code2), _lib.ptr(absmax2), blocksize2, 0.0,
                                                      _lib.ptr(out), absmax.numel(), _lib.stream())
             _lib.check(rc, "mfl_dequant_blockwise_u8")
@@ -183,9 +188,10 @@ def resolve_absmax(quant_state) -> torch.Tensor:
 
 def packed_weight(w_quant: torch.Tensor, quant_state, rows: int, unnested: bool = False):
     """(``_lib.Nf4Weight``, the tensors it points into) for a call with ``rows`` rows.  A double-quantised state is
-    described as it is, for the kernels that read it so, or with ``unnested`` by its fp32 scales, written out."""
+    described as it is, for the kernels that read it so, or by its fp32 scales, written out: with ``unnested``, and where
+    its second-level blocks are not a power of two."""
     code, blocksize = quant_state.code, int(quant_state.blocksize)
-    if not unnested and getattr(quant_state, "nested", False):
+    if not unnested and getattr(quant_state, "nested", False) and _is_shift(int(quant_state.state2.blocksize)):
         absmax, code2, absmax2, blocksize2, offset = keep = _second_level(quant_state)
         return _lib.Nf4Weight(w_quant.data_ptr(), code.data_ptr(), None, None, absmax.data_ptr(), code2.data_ptr(),
                               absmax2.data_ptr(), offset.data_ptr(), blocksize, blocksize2), keep
