@@ -173,3 +173,23 @@ def test_other_second_level_blocks_are_written_out(monkeypatch, blocksize2):
     fused_mlp.moe_block_4bit(tokens, torch.zeros((6, 4), dtype=torch.bfloat16), gate, up, down, 2, True)
     names = [n for n, _ in lib.seen]
     assert names[-1] == "mfl_moe_block_fwd" and names.count("mfl_dequant_blockwise_u8") == 3
+
+
+@pytest.mark.parametrize("nested", [False, True])
+def test_strided_scales_are_taken(monkeypatch, nested):
+    """A state's scales may lie apart (a view of more): they are made contiguous for the kernels."""
+    from qwen3_moe_fused.grouped_gemm import forward_4bit
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    tokens, _, gate, _, _ = _packed_block()
+    st = gate.quant_state
+    if not nested:
+        st.absmax, st.state2, st.offset = torch.ones(st.absmax.numel()), None, None
+    assert st.nested == nested
+    st.absmax = torch.stack((st.absmax, st.absmax), dim=1)[:, 0]
+    assert not st.absmax.is_contiguous()
+    lib = _Recorder({})
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    forward_4bit.grouped_gemm_forward_4bit(tokens, gate, st, torch.tensor([6, 0, 0, 0], dtype=torch.int32))
+    assert lib.seen[-1] == ("mfl_gemm_fwd_nf4_packed", [(nested, 4 if nested else 0)])

@@ -29,7 +29,8 @@ def check_packed(x: torch.Tensor, w_quant: torch.Tensor, w_quant_state, k: int):
     code, absmax = w_quant_state.code, w_quant_state.absmax
     assert code.dtype == torch.float32
     for t in (w_quant, code, absmax):
-        assert t.device == x.device and t.is_contiguous()
+        assert t.device == x.device
+    assert w_quant.is_contiguous() and code.is_contiguous()  # (the scales are made so)
     assert is_int_tensor(w_quant) and len(w_quant_state.shape) == 3
     experts, n, k_w = w_quant_state.shape
     assert k_w == k and k % 2 == 0
