@@ -193,3 +193,20 @@ def test_strided_scales_are_taken(monkeypatch, nested):
     monkeypatch.setattr(_lib, "lib", lambda: lib)
     forward_4bit.grouped_gemm_forward_4bit(tokens, gate, st, torch.tensor([6, 0, 0, 0], dtype=torch.int32))
     assert lib.seen[-1] == ("mfl_gemm_fwd_nf4_packed", [(nested, 4 if nested else 0)])
+
+
+@pytest.mark.parametrize("offset", [None, 0.25, torch.tensor(0.25), torch.tensor([0.25], dtype=torch.float64)])
+def test_an_offset_of_any_kind_is_made_on_the_device(monkeypatch, offset):
+    """None and plain numbers become a one-element tensor by a fill, which a stream capture takes; a copy from the host
+    (what ``torch.tensor(value, device=...)`` does) it refuses."""
+    from qwen3_moe_fused.quantize import nf4
+
+    state = _packed_block()[2].quant_state
+    state.offset = offset
+
+    def from_host(*args, **kwargs):
+        raise AssertionError("a copy from the host")
+
+    monkeypatch.setattr(torch, "tensor", from_host)
+    off = nf4._second_level(state)[4]
+    assert off.numel() == 1 and off.dtype == torch.float32 and float(off) == (0.0 if offset is None else 0.25)

@@ -157,7 +157,8 @@ def _second_level(quant_state):
     absmax2 = st2.absmax.to(torch.float32).contiguous()
     offset = quant_state.offset
     if not torch.is_tensor(offset):
-        offset = torch.tensor(0.0 if offset is None else float(offset), dtype=torch.float32, device=absmax.device)
+        # (a fill and not a copy from the host, which would wait for the device and end a stream capture)
+        offset = torch.full((), 0.0 if offset is None else float(offset), dtype=torch.float32, device=absmax.device)
     return absmax, code2, absmax2, int(st2.blocksize), offset.to(device=absmax.device, dtype=torch.float32)
 
 
