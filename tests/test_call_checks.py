@@ -210,3 +210,28 @@ def test_an_offset_of_any_kind_is_made_on_the_device(monkeypatch, offset):
     monkeypatch.setattr(torch, "tensor", from_host)
     off = nf4._second_level(state)[4]
     assert off.numel() == 1 and off.dtype == torch.float32 and float(off) == (0.0 if offset is None else 0.25)
+
+
+def _lora_args(rows=4096, e=2, h=16, m=16, r=8, rb=None):
+    """Operands of the fast-LoRA function; ``rb``: another rank in the B matrices of gate and up."""
+    a, b = (_bf16(e, r, h), _bf16(e, m, rb or r))
+    return [_bf16(rows, h), _bf16(e, m, h), None, a, b, 1.0, _bf16(e, m, h), None, a.clone(), b.clone(), 1.0, _bf16(e, h, m), None,
+            _bf16(e, r, m), _bf16(e, h, r), 1.0, torch.tensor([rows - 1, 1], dtype=torch.int32)]
+
+
+@pytest.mark.parametrize("rb", [4, 12, 16, 24])
+def test_thin_matrices_of_unequal_rank_are_refused(monkeypatch, rb):
+    from qwen3_moe_fused.kernels.fast_lora import fast_lora
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    for args, fits in ((_lora_args(), True), (_lora_args(rb=rb), False)):
+        lib = _Recorder({})
+        monkeypatch.setattr(_lib, "lib", lambda: lib)
+        if fits:
+            fast_lora(*args)
+            assert lib.seen[0][0] == "mfl_copy_blocks"
+        else:
+            with pytest.raises(AssertionError):
+                fast_lora(*args)
+            assert not lib.seen

@@ -115,6 +115,7 @@ def _joined(a: torch.Tensor, b: torch.Tensor, dim: int, pieces: List[_Piece]) ->
     """Room for ``torch.cat((a, b), dim)``; what fills it is added to ``pieces``."""
     dtype = torch.promote_types(a.dtype, b.dtype)  # (any strides and types, as the concatenation takes them)
     a, b = a.to(dtype).contiguous(), b.to(dtype).contiguous()
+    assert a.shape[:dim] == b.shape[:dim] and a.shape[dim + 1:] == b.shape[dim + 1:]
     shape = list(a.shape)
     na, nb = a.shape[dim], b.shape[dim]
     shape[dim] = na + nb
@@ -127,6 +128,7 @@ def _padded(b: torch.Tensor, dim: int, first: int, total: int, pieces: List[_Pie
     """Room for ``b`` in the columns from ``first`` on of ``total``, zeros in the others (one side of it)."""
     b = b.contiguous()
     size = b.shape[dim]
+    assert 0 <= first <= total - size
     shape = list(b.shape)
     shape[dim] = total
     wide = torch.empty(shape, device=b.device, dtype=b.dtype)
@@ -166,6 +168,7 @@ class FastLora(torch.autograd.Function):
                           and Bg.shape == Bu.shape)
             if one_launch:
                 # each matrix's thin weights are its adapter's B over its own columns of ucat and zeros over the other's
+                assert Bg.shape[2] == r, "an adapter's A and B have one rank"
                 bg, bu = _padded(Bg, 2, 0, 2 * r, pieces), _padded(Bu, 2, r, 2 * r, pieces)
             _copy_pieces(pieces, True)
             ucat = _fwd(x, acat, m_sizes, alpha=Sg)
