@@ -235,3 +235,19 @@ def test_thin_matrices_of_unequal_rank_are_refused(monkeypatch, rb):
             with pytest.raises(AssertionError):
                 fast_lora(*args)
             assert not lib.seen
+
+
+@pytest.mark.parametrize("elsewhere", [(), (3, 8), (4, 9), (3,), (8,), (9,)])
+def test_thin_matrices_on_another_device_never_reach_the_copies(monkeypatch, elsewhere):
+    """Operands on the host, or on another device than the rows, are refused by the products; the copies that join the
+    thin matrices come before those.  (): all of them on the host."""
+    from qwen3_moe_fused.kernels.fast_lora import fast_lora
+
+    if elsewhere:
+        monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    lib = _Recorder({})
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    with pytest.raises((AssertionError, RuntimeError)):
+        fast_lora(*(t.to("meta") if i in elsewhere else t for i, t in enumerate(_lora_args())))
+    assert not lib.seen

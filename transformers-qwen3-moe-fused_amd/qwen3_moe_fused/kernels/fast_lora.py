@@ -162,6 +162,7 @@ class FastLora(torch.autograd.Function):
         if Sg == Su and Ag.shape == Au.shape and x.shape[0] >= _WIDE_ROWS:
             # one pass over x for both adapters' rank-r activations
             r = Ag.shape[1]
+            assert x.is_cuda and all(t.device == x.device for t in (Ag, Bg, Au, Bu))  # (the copies come before the products)
             pieces = []
             acat = _joined(Ag, Au, 1, pieces)
             one_launch = (Gqs is None and Uqs is None and dt == torch.bfloat16 and Gq.dtype == dt and Uq.dtype == dt
