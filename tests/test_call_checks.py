@@ -251,3 +251,27 @@ def test_thin_matrices_on_another_device_never_reach_the_copies(monkeypatch, els
     with pytest.raises((AssertionError, RuntimeError)):
         fast_lora(*(t.to("meta") if i in elsewhere else t for i, t in enumerate(_lora_args())))
     assert not lib.seen
+
+
+def _router_and_rows():
+    from qwen3_moe_fused.modular_qwen3_moe_fused import Qwen3MoeFusedRouter
+
+    return Qwen3MoeFusedRouter(64, 8, bias=False), torch.randn(3, 64)
+
+
+def _compiled(m, x):
+    return torch.compile(m, fullgraph=True, backend="eager")
+
+
+# the router is a linear layer to whoever records or compiles it
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("how", [lambda m, x: torch.jit.script(m), lambda m, x: torch.jit.trace(m, (x,)), _compiled,
+                                 lambda m, x: torch.fx.symbolic_trace(m),
+                                 lambda m, x: torch.export.export(m, (x,)).module(),
+                                 lambda m, x: torch.export.export(m, (x,), strict=True).module()],
+                         ids=["script", "trace", "compile", "fx", "export", "export-strict"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_router_is_recorded_as_a_linear_layer(how, dtype):
+    m, x = _router_and_rows()
+    m, x = m.to(dtype), x.to(dtype)
+    assert torch.equal(how(m, x)(x), torch.nn.functional.linear(x, m.weight))

@@ -75,3 +75,24 @@ def test_router_weight_gradient_keeps_an_infinity_of_the_last_token():
     x[-1, 5] = float("inf")
     router_linear(x, w).backward(d)
     assert torch.isinf(w.grad[:, 5]).all() and (torch.cat((w.grad[:, :5], w.grad[:, 6:]), 1) == 512).all()  # 513 in bf16
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_router_compiles_as_a_whole(grad):
+    gate = Qwen3MoeFusedRouter(128, 16, bias=False).to("cuda", torch.bfloat16)
+    x = torch.randn((40, 128), generator=gen(1)).to(torch.bfloat16).cuda().requires_grad_(grad)
+    with torch.set_grad_enabled(grad):
+        out = torch.compile(gate, fullgraph=True, backend="eager")(x)
+        assert torch.equal(out, torch.nn.functional.linear(x, gate.weight))
+
+
+def test_block_compiles_around_its_kernels():
+    from test_gpu_block_call import _block
+
+    blk, dtype = _block(8, 2, 64, 64, "bf16", 3)
+    x = torch.randn((1, 40, 64), generator=gen(1)).to(dtype).cuda()
+    with torch.no_grad():
+        want = blk(x)
+        got = torch.compile(blk, backend="eager")(x)
+    for a, b in zip(got, want):
+        assert (a.float() - b.float()).abs().max() <= 2e-2 * b.float().abs().max()

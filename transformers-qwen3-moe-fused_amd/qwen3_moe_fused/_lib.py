@@ -181,8 +181,8 @@ def stream() -> int:
 def plain_call() -> bool:
     """Whether a call that passes autograd by, or stands in for a stock operator, may do so: no forward-mode level, no
     functorch transform and no dispatch mode (counters, fake tensors, selective checkpointing) that would have to see
-    the operators, and nobody tracing."""
-    return (forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+    the operators, and nobody tracing or compiling (asked first: a compiler cannot look into the others)."""
+    return (not torch.compiler.is_compiling() and forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None)
 
 

@@ -68,8 +68,11 @@ class Qwen3MoeFusedRouter(nn.Linear):
     value, as the reference's release did) have a class to hook: its output is the raw logits."""
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:
-        out = router_linear(input, self.weight) if self.bias is None else None
-        return super().forward(input) if out is None else out
+        if torch.jit.is_scripting():  # (compiled from source, where neither the kernel nor super() can be called)
+            return nn.functional.linear(input, self.weight, self.bias)
+        else:
+            out = router_linear(input, self.weight) if self.bias is None else None
+            return super().forward(input) if out is None else out
 
 
 class Qwen3MoeFusedSparseMoeBlock(nn.Module):
