@@ -275,3 +275,28 @@ def test_router_is_recorded_as_a_linear_layer(how, dtype):
     m, x = _router_and_rows()
     m, x = m.to(dtype), x.to(dtype)
     assert torch.equal(how(m, x)(x), torch.nn.functional.linear(x, m.weight))
+
+
+@pytest.mark.parametrize("tokens", [4, 600])
+def test_router_gradients_batched_and_under_modes_are_the_stock_products(monkeypatch, tokens):
+    """Several gradients at once (``is_grads_batched``, vectorised Jacobians) run the backward on batched tensors, which have
+    no address; an operator counter around the backward sees its products."""
+    from torch.utils.flop_counter import FlopCounterMode
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    monkeypatch.setattr(routing, "_router_logits", torch.nn.functional.linear)
+    lib = _Recorder({})
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    g = torch.Generator().manual_seed(tokens)
+    x, w, d = (torch.randn(s, generator=g).to(torch.bfloat16) for s in ((tokens, 64), (8, 64), (3, tokens, 8)))
+    x.requires_grad_(), w.requires_grad_()
+    y = routing.router_linear(x, w)
+    assert type(y.grad_fn).__name__ == "_RouterLinearBackward"
+    got = torch.autograd.grad(y, (x, w), d, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        for a, b in zip(got, torch.autograd.grad(torch.nn.functional.linear(x, w), (x, w), d[i])):
+            assert torch.allclose(a[i].float(), b.float(), rtol=2 ** -7, atol=1e-2)
+    with FlopCounterMode(display=False) as count:
+        torch.autograd.grad(y, (x, w), d[0])
+    assert count.get_total_flops() == 2 * 2 * tokens * 64 * 8 and not lib.seen

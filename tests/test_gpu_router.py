@@ -96,3 +96,12 @@ def test_block_compiles_around_its_kernels():
         got = torch.compile(blk, backend="eager")(x)
     for a, b in zip(got, want):
         assert (a.float() - b.float()).abs().max() <= 2e-2 * b.float().abs().max()
+
+
+def test_router_gradients_several_at_once():
+    x, w, d = (torch.randn(s, generator=gen(5)).to(torch.bfloat16).cuda() for s in ((600, 128), (16, 128), (2, 600, 16)))
+    x.requires_grad_(), w.requires_grad_()
+    got = torch.autograd.grad(router_linear(x, w), (x, w), d, is_grads_batched=True)
+    for i in range(2):
+        _near(got[0][i], d[i].cpu(), w.detach().cpu(), 16)
+        _near(got[1][i], d[i].t().cpu(), x.detach().cpu(), 600)

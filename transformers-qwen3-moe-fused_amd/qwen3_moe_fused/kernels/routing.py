@@ -43,7 +43,9 @@ class _RouterLinear(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dlogits):
         x, w = ctx.saved_tensors
-        if torch.is_grad_enabled():  # a graph of the gradients is asked for (create_graph): stock products have one
+        # a graph of the gradients is asked for (create_graph), several gradients at once (batched tensors have no address)
+        # or somebody watches the operators: stock products have the one, take the other and are seen
+        if torch.is_grad_enabled() or not _lib.plain_call() or torch._C._functorch.is_legacy_batchedtensor(dlogits):
             return (dlogits @ w if ctx.needs_input_grad[0] else None,
                     dlogits.t() @ x if ctx.needs_input_grad[1] else None)
         dlogits = dlogits.contiguous()
