@@ -300,3 +300,38 @@ def test_router_gradients_batched_and_under_modes_are_the_stock_products(monkeyp
     with FlopCounterMode(display=False) as count:
         torch.autograd.grad(y, (x, w), d[0])
     assert count.get_total_flops() == 2 * 2 * tokens * 64 * 8 and not lib.seen
+
+
+def _small_block(kind="bf16"):
+    from types import SimpleNamespace
+
+    from qwen3_moe_fused.modular_qwen3_moe_fused import Qwen3MoeFusedSparseMoeBlock
+    from qwen3_moe_fused.quantize.layer import MoeFusedLinear4bit
+
+    block = Qwen3MoeFusedSparseMoeBlock(SimpleNamespace(
+        num_experts=4, num_experts_per_tok=2, norm_topk_prob=True, hidden_size=128, moe_intermediate_size=64,
+        hidden_act="silu")).to(torch.bfloat16)
+    if kind == "nf4":
+        for name, w in zip(("gate_proj", "up_proj", "down_proj"), _packed_block()[2:]):
+            proj = MoeFusedLinear4bit(*w.quant_state.shape[:0:-1], 4, device="meta")
+            proj._parameters["weight"] = w
+            setattr(block, name, proj)
+    return block
+
+
+@pytest.mark.parametrize("kind", ["bf16", "nf4"])
+@pytest.mark.parametrize("how", ["class", "instance", "hook"])
+def test_block_call_steps_aside_for_replaced_forwards(no_kernels, monkeypatch, kind, how):
+    block = _small_block(kind)
+    tokens, logits = _bf16(3, 128), _bf16(3, 4)
+    with torch.no_grad():
+        with pytest.raises(LibraryCalled):
+            block._one_call(tokens, logits)
+        if how == "class":
+            plain = type(block.down_proj).forward
+            monkeypatch.setattr(type(block.down_proj), "forward", lambda self, *a: plain(self, *a))
+        elif how == "instance":
+            block.down_proj.forward = block.down_proj.forward
+        else:
+            block.down_proj.register_forward_hook(lambda m, a, o: None)
+        assert block._one_call(tokens, logits) is None

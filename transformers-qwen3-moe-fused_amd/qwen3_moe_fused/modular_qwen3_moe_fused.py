@@ -48,6 +48,9 @@ class MoeFusedLinear(nn.Module):
     def extra_repr(self) -> str:
         return f"in_features={self.in_features}, out_features={self.out_features}, num_experts={self.num_experts}"
 
+    # what the block's one call stands in for: a class whose forward has been replaced runs on the separate steps
+    _own_forward = forward
+
 
 def route_tokens(block, hidden_2d: torch.Tensor, router_logits: Optional[torch.Tensor] = None):
     """Router half of the block, shared with the fast-LoRA forward: returns
@@ -157,7 +160,11 @@ class Qwen3MoeFusedSparseMoeBlock(nn.Module):
             return None
         if tokens.shape[0] * self.num_selected > self._ONE_CALL_ROWS:
             return None
-        for proj in (gate, up, down):  # hooks and replaced forwards run on the separate steps
+        # Hooks and replaced forwards run on the separate steps.  (In bf16 and on packed weights those call the down
+        # projection; what gate and up do is the fused front's, which calls neither unless ``fuse_front`` is off.)
+        if kind.forward is not kind._own_forward:
+            return None
+        for proj in (gate, up, down):
             if (proj._forward_hooks or proj._forward_pre_hooks or proj._backward_hooks or proj._backward_pre_hooks
                     or "forward" in proj.__dict__):
                 return None

@@ -189,3 +189,5 @@ class MoeFusedLinear4bit(MoeFusedLinear):
         if self.compute_dtype is not None:
             x = x.to(self.compute_dtype)
         return moe_fused_linear_4bit(x, self.weight, m_sizes).to(in_dtype)
+
+    _own_forward = forward
