@@ -335,3 +335,25 @@ def test_block_call_steps_aside_for_replaced_forwards(no_kernels, monkeypatch, k
         else:
             block.down_proj.register_forward_hook(lambda m, a, o: None)
         assert block._one_call(tokens, logits) is None
+
+
+def test_router_is_seen_by_function_modes(no_kernels):
+    from torch.overrides import TorchFunctionMode
+
+    class Seen(TorchFunctionMode):
+        names = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.names.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    gate, x = _router_and_rows()
+    gate, x = gate.to(torch.bfloat16), x.to(torch.bfloat16)
+    with torch.no_grad():
+        with pytest.raises(LibraryCalled):
+            gate(x)
+        with torch.device("cpu"), pytest.raises(LibraryCalled):  # a default device watches nothing
+            gate(x)
+        with Seen(), torch.device("cpu"):
+            gate(x)
+    assert "linear" in Seen.names

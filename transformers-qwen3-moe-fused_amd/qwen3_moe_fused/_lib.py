@@ -12,6 +12,7 @@ from typing import Optional
 
 import torch
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmoe_fused_linear.so")
@@ -180,10 +181,13 @@ def stream() -> int:
 
 def plain_call() -> bool:
     """Whether a call that passes autograd by, or stands in for a stock operator, may do so: no forward-mode level, no
-    functorch transform and no dispatch mode (counters, fake tensors, selective checkpointing) that would have to see
-    the operators, and nobody tracing or compiling (asked first: a compiler cannot look into the others)."""
+    functorch transform, no dispatch mode (counters, fake tensors, selective checkpointing) and no function mode (but for
+    default devices, which watch nothing) that would have to see the operators, and nobody tracing or compiling (asked first: a compiler cannot look into the others)."""
     return (not torch.compiler.is_compiling() and forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None)
+            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None
+            and (torch._C._len_torch_function_stack() == 0
+                 or all(isinstance(torch._C._get_function_stack_at(i), DeviceContext)
+                        for i in range(torch._C._len_torch_function_stack()))))
 
 
 def as_index_tensor(m_sizes: torch.Tensor) -> torch.Tensor:
