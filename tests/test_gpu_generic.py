@@ -80,3 +80,17 @@ def test_generic_products_within_the_bound_of_their_sums(sizes, n, k, dtype, out
             res.copy_(old)
         got = fn(*args, out, out=res, alpha=alpha, accumulate=accumulate)
         _check(got, exact[i], bound[i], length, alpha, old, fn.__name__)
+
+
+@pytest.mark.parametrize("n", [65535 * 32, 65535 * 32 + 1, 65535 * 64])
+def test_outputs_of_more_column_tiles_than_a_grid_has_rows(n):
+    """The narrowest tiles are left to the wider ones where their number would pass 65535: one row, 4 to 8 products each."""
+    g = gen(n)
+    ms = torch.tensor([1], dtype=torch.int32, device="cuda")
+    for k, fn in ((4, grouped_gemm_forward), (3, grouped_gemm_forward_transposed)):
+        a = torch.randn((1, k), generator=g).cuda()
+        w = torch.randn((1, n, k) if fn is grouped_gemm_forward else (1, k, n), generator=g).cuda()
+        got = fn(a, w, ms, torch.float32)
+        w64 = w[0].double().t() if fn is grouped_gemm_forward else w[0].double()
+        room = k * 2.0 ** -24 * (a.double().abs() @ w64.abs()) + 2.0 ** -23 * (a.double() @ w64).abs()
+        assert ((got.double() - a.double() @ w64).abs() <= room).all()

@@ -289,7 +289,8 @@ int launch_mode(const Args &g) {
         if (g.N >= 64 && g.K >= 128) return launch_tile<TI, TO, MODE, 64, 128, 2, 2, 1, 16, VEC>(g);
         return launch_tile<TI, TO, MODE, 64, 64, 2, 2, 1, 32, VEC>(g);
     }
-    if (g.R <= (int64_t)16 * g.E) return launch_tile<TI, TO, MODE, 16, 32, 1, 1, 4, 128, VEC>(g);
+    // (their 32 columns would be more tiles than a grid has rows past two million outputs)
+    if (g.R <= (int64_t)16 * g.E && ceil_div(g.N, 32) <= 65535) return launch_tile<TI, TO, MODE, 16, 32, 1, 1, 4, 128, VEC>(g);
     const int64_t tiles64 = (g.R / 64 + g.E) * ceil_div(g.N, 64);
     if (g.R <= (int64_t)48 * g.E || tiles64 < 4 * device_info().cu_count)
         return launch_tile<TI, TO, MODE, 32, 64, 1, 2, 2, 64, VEC>(g);
