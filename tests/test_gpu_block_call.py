@@ -131,3 +131,31 @@ def test_rows_beyond_one_call(kind, monkeypatch):
             assert (blk._one_call(hidden[0], blk.gate(hidden[0])) is None) == (rows < 33 * 4)
             got.append(blk(hidden))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+def _apart(t):
+    """The same values with the last dimension's elements two apart."""
+    return torch.stack((t, torch.zeros_like(t)), dim=-1)[..., 0]
+
+
+def _shifted(t):
+    """The same values one element past where an allocation starts."""
+    out = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    return out.copy_(t)
+
+
+@pytest.mark.parametrize("unpack", [_apart, _shifted])
+@pytest.mark.parametrize("kind", ["bf16", "fp32"])
+def test_block_call_with_saved_tensors_handed_back_elsewhere(unpack, kind):
+    """Saved-tensor hooks (offloading, packing into one buffer) hand back equal tensors, not the same ones."""
+    blk, dtype = _block(8, 2, 64, 64, kind, 6)
+    grads = []
+    for hooks in ((lambda t: t, lambda t: t), (lambda t: t.clone(), unpack)):
+        x = torch.randn((1, 700, 64), generator=gen(6)).to(dtype).cuda().requires_grad_()
+        blk.zero_grad(set_to_none=True)
+        with torch.autograd.graph.saved_tensors_hooks(*hooks):
+            out, logits = blk(x)
+        (out.float().square().sum() + logits.float().sum()).backward()
+        grads.append([x.grad] + [p.grad for p in blk.parameters()])
+    for a, b in zip(*grads):
+        assert float((a.float() - b.float()).abs().max()) <= (1e-5 if kind == "fp32" else 2e-2) * float(a.float().abs().max())

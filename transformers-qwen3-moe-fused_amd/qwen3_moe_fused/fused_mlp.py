@@ -164,7 +164,10 @@ class _MoeBlock(torch.autograd.Function):
     def backward(ctx, dout, _):
         if dout is None:
             return (None,) * 7
-        tokens, logits, w_gate, w_up, w_down, saved = ctx.saved_tensors
+        # (a saved-tensor hook may hand back equal tensors in other strides and places)
+        tokens, logits, w_gate, w_up, w_down, saved = (t.contiguous() for t in ctx.saved_tensors)
+        if saved.data_ptr() % 256:
+            saved = saved.clone()
         dout = dout.contiguous()
         b = _dense_block(tokens, logits, w_gate, w_up, w_down, ctx.k, ctx.renorm, True)
         grads = [torch.empty_like(t) if need else None

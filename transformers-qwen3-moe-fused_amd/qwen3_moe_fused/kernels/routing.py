@@ -48,7 +48,7 @@ class _RouterLinear(torch.autograd.Function):
         if torch.is_grad_enabled() or not _lib.plain_call() or torch._C._functorch.is_legacy_batchedtensor(dlogits):
             return (dlogits @ w if ctx.needs_input_grad[0] else None,
                     dlogits.t() @ x if ctx.needs_input_grad[1] else None)
-        dlogits = dlogits.contiguous()
+        dlogits, x = dlogits.contiguous(), x.contiguous()  # (a saved-tensor hook may hand x back in other strides)
         dx = dlogits @ w if ctx.needs_input_grad[0] else None
         dw = None
         if ctx.needs_input_grad[1]:
@@ -56,7 +56,7 @@ class _RouterLinear(torch.autograd.Function):
             n = _lib.lib().mfl_router_dw_workspace(tokens, hidden, w.shape[0]) if tokens >= _ROUTER_DW_TOKENS else 0
             if n == 0:
                 return dx, dlogits.t() @ x
-            dw, ws = torch.empty_like(w), torch.empty(n, device=x.device, dtype=torch.uint8)
+            dw, ws = w.new_empty(w.shape), torch.empty(n, device=x.device, dtype=torch.uint8)
             rc = _lib.lib().mfl_router_dw(x.data_ptr(), dlogits.data_ptr(), dw.data_ptr(), tokens, hidden, w.shape[0],
                                           ws.data_ptr(), n, _lib.stream())
             if rc == -6:  # MFL_ERR_UNSUPPORTED: a gradient that is not aligned
