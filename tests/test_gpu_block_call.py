@@ -159,3 +159,20 @@ def test_block_call_with_saved_tensors_handed_back_elsewhere(unpack, kind):
         grads.append([x.grad] + [p.grad for p in blk.parameters()])
     for a, b in zip(*grads):
         assert float((a.float() - b.float()).abs().max()) <= (1e-5 if kind == "fp32" else 2e-2) * float(a.float().abs().max())
+
+
+# one side as thin as an adapter's rank, the other a multiple of 256, 16384 rows and more: the rows are dealt out evenly
+@pytest.mark.parametrize("t,k,h,i", [(8192, 2, 256, 32), (5500, 3, 512, 64), (16500, 1, 16, 256)])
+def test_block_call_deals_the_rows_of_thin_weight_gradients_out(t, k, h, i):
+    """The same bits as the separate steps, whose weight gradients take the kernel with even shares."""
+    blk, dtype = _block(8, k, h, i, "bf16", 2)
+    with torch.no_grad():
+        blk.gate.weight[0] += 0.1  # one popular expert
+    x, dout = (torch.randn((1, t, h), generator=gen(s)).abs().to(dtype).cuda() for s in (1, 2))
+    grads = []
+    for fused in (True, False):
+        blk.zero_grad(set_to_none=True)
+        blk._ONE_CALL_ROWS = 65536 if fused else 0
+        blk(x)[0].backward(dout)
+        grads.append([getattr(blk, n).weight.grad for n in PROJ])
+    assert all(torch.equal(a, b) for a, b in zip(*grads))

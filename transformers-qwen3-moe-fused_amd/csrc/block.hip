@@ -145,8 +145,32 @@ int down(const mfl_moe_block &b, char *ws, const Layout &l, void *stream) {
 // What the backward needs besides the forward's buffer: the output gradient's rows (then, in their place, the input
 // gradient's), the tokens' rows, dh, de and dg
 struct BackLayout {
-    size_t dy, x, dh, de, dg, dw, total;
+    size_t dy, x, dh, de, dg, dw, split, total;
 };
+
+// Scratch of a weight gradient (E, N, K) with one thin side (8 to 64) whose rows are dealt out evenly over the workgroups;
+// 0: the general kernel, whose launch under skewed routing lasts as long as its largest expert.  A step, hidden 2048,
+// general against even shares, routing uniform / Zipf 1.25 / Zipf 4:
+//   16 experts, side 32, 65536 rows: 815 / 1193 / 1437 against 809 / 810 / 805 us; 16384 rows: 271 / 357 / 405 against
+//   292 / 302 / 298; 8192 rows: 263 / 259 / 278 against 285 / 283 / 281 (nothing left to even out);
+//   128 experts, side 32, 32768 rows: 477 / 496 / 455 against 441 / 478 / 519;
+//   side 64, which leaves the even shares fewer stages: 16 experts, 65536 rows 845 / 1298 / 1607 against 876 / 888 / 874, but
+//   128 experts 843 / 865 / 854 against 856 / 971 / 930: from 1024 rows per expert on.
+size_t split_bytes(const mfl_moe_block &b, int N, int K) {
+    const int64_t R = b.T * b.k;
+    if (b.dtype != MFL_BF16 || R < 16384 || ((N < K ? N : K) > 32 && R < (int64_t)1024 * b.E)) return 0;
+    return mfl_gemm_dw_split_workspace(R, N, K, b.E);
+}
+
+int weight_grad(const mfl_moe_block &b, const void *x, const void *dy, const int32_t *ms, void *dw, int N, int K, void *scratch,
+                void *stream) {
+    const int64_t R = b.T * b.k;
+    const size_t bytes = split_bytes(b, N, K);
+    if (bytes != 0 && aligned(dw, 16))
+        return mfl_gemm_dw_split(x, dy, ms, MFL_I32, dw, R, N, K, b.E, b.dtype, b.dtype, 1.0f, scratch, bytes, stream);
+    return mfl_gemm_dw(x, dy, ms, MFL_I32, dw, R, N, K, b.E, b.dtype, b.dtype, 1.0f, 0, stream);
+}
+
 BackLayout back_layout(const mfl_moe_block &b) {
     const size_t R = (size_t)b.T * b.k, es = dtype_size(b.dtype);
     BackLayout l;
@@ -156,7 +180,9 @@ BackLayout back_layout(const mfl_moe_block &b) {
     l.de = l.dh + up256(R * b.I * es);
     l.dg = l.de + up256(R * b.I * es);
     l.dw = l.dg + up256(R * b.I * es);
-    l.total = l.dw + up256(R * es);
+    l.split = l.dw + up256(R * es);
+    const size_t down = split_bytes(b, b.H, b.I), front = split_bytes(b, b.I, b.H);
+    l.total = l.split + up256(down > front ? down : front);
     return l;
 }
 
@@ -211,7 +237,7 @@ int mfl_moe_block_bwd(const mfl_moe_block *b, const void *dout, const void *save
     if (d_tokens == nullptr && d_gate == nullptr && d_up == nullptr && d_down == nullptr) return MFL_OK;
     MFL_TRY(spread_rows(*b, dout, fw, l, fw + l.weights, ws + t.dy, stream));
     if (d_down != nullptr)
-        MFL_TRY(mfl_gemm_dw(fw + l.h, ws + t.dy, ms, MFL_I32, d_down, R, b->H, b->I, b->E, dt, dt, 1.0f, 0, stream));
+        MFL_TRY(weight_grad(*b, fw + l.h, ws + t.dy, ms, d_down, b->H, b->I, ws + t.split, stream));
     if (d_tokens == nullptr && d_gate == nullptr && d_up == nullptr) return MFL_OK;
     MFL_TRY(mfl_gemm_dx(ws + t.dy, b->w_down, ms, MFL_I32, ws + t.dh, R, b->I, b->H, b->E, dt, dt, 1.0f, 0, stream));
     MFL_TRY(mfl_silu_mul_bwd(ws + t.dh, fw + l.e, fw + l.g, ws + t.de, ws + t.dg, nullptr, R * b->I, dt, stream));
@@ -229,9 +255,9 @@ int mfl_moe_block_bwd(const mfl_moe_block *b, const void *dout, const void *save
         // the replicated, sorted rows again: the forward pass did not keep them
         MFL_TRY(spread_rows(*b, b->tokens, fw, l, nullptr, ws + t.x, stream));
         if (d_gate != nullptr)
-            MFL_TRY(mfl_gemm_dw(ws + t.x, ws + t.de, ms, MFL_I32, d_gate, R, b->I, b->H, b->E, dt, dt, 1.0f, 0, stream));
+            MFL_TRY(weight_grad(*b, ws + t.x, ws + t.de, ms, d_gate, b->I, b->H, ws + t.split, stream));
         if (d_up != nullptr)
-            MFL_TRY(mfl_gemm_dw(ws + t.x, ws + t.dg, ms, MFL_I32, d_up, R, b->I, b->H, b->E, dt, dt, 1.0f, 0, stream));
+            MFL_TRY(weight_grad(*b, ws + t.x, ws + t.dg, ms, d_up, b->I, b->H, ws + t.split, stream));
     }
     return MFL_OK;
 }
