@@ -357,3 +357,21 @@ def test_router_is_seen_by_function_modes(no_kernels):
         with Seen(), torch.device("cpu"):
             gate(x)
     assert "linear" in Seen.names
+
+
+# tokens of 8 selections each, 128 experts, hidden 2048, intermediate 768: the gated product reads 8-bit scales up to 384
+# rows per expert, the plain one up to 128; with K = 96, or second-level blocks shorter than a row, neither does
+@pytest.mark.parametrize("tokens,inter,blocksize2,slots", [(1, 768, 256, 0), (256, 768, 256, 0), (2048, 768, 256, 0),
+                                                           (2049, 768, 256, 1), (6144, 768, 256, 1), (6145, 768, 256, 2),
+                                                           (1, 96, 256, 1), (1, 768, 16, 2)])
+def test_block_workspace_has_room_for_written_out_scales_only_where_they_are(tokens, inter, blocksize2, slots):
+    import ctypes
+
+    def size(nested):
+        at = 1 << 20  # (an address that is compared with alignments, never followed)
+        w = _lib.Nf4Weight(at, at, None if nested else at, None, at if nested else None, at, at, at, 64, blocksize2)
+        p = ctypes.pointer(w)
+        b = _lib.MoeBlock(at, at, None, None, None, p, p, p, tokens, 128, 8, 2048, inter, 1, _lib.BF16, _lib.BF16, 0)
+        return _lib.lib().mfl_moe_block_workspace(b)
+
+    assert size(True) - size(False) == slots * 128 * 2048 * inter // 64 * 4

@@ -20,7 +20,17 @@ bool front_is_one_kernel(const mfl_moe_block &b) {
 
 struct Layout {
     size_t idx, w32, sort, inv, counts, weights, route, e, g, h, y, scales, total, route_bytes, scale_bytes;
+    int scale_slots;  // written-out scales there is room for: gate and up's, or one after the other the three matrices'
 };
+
+// Whether a product (R rows, reduction length K) on these weights needs no room for written-out scales: they are not
+// double-quantised, or a decode-sized kernel reads them as they are.  By the sizes: should that kernel refuse the call all
+// the same, the block does, and the caller makes the separate calls.
+bool scales_as_they_are(const mfl_moe_block &b, const mfl_nf4_weight &w, int K, int rows_per_expert) {
+    if (w.absmax_u8 == nullptr) return true;
+    return w.blocksize == 64 && K % 128 == 0 && K / 64 <= w.blocksize2 && b.H % 8 == 0 && b.I % 8 == 0 &&
+           b.T * b.k <= (int64_t)rows_per_expert * b.E && aligned(w.absmax_u8, 2) && aligned(w.packed, 16) && aligned(b.tokens, 16);
+}
 
 Layout layout(const mfl_moe_block &b) {
     const size_t R = (size_t)b.T * b.k, es = dtype_size(b.dtype);
@@ -45,15 +55,20 @@ Layout layout(const mfl_moe_block &b) {
     }
     l.h = take(R * b.I * es);
     l.y = take(R * b.H * es);
-    if (b.q_gate != nullptr) {  // room for the written-out scales of a double-quantised matrix, two at a time
+    if (b.q_gate != nullptr) {
+        const mfl_nf4_weight &gate = *b.q_gate, &up = *b.q_up, &down = *b.q_down;
+        const bool alike = (gate.absmax_u8 != nullptr) == (up.absmax_u8 != nullptr) && gate.blocksize2 == up.blocksize2;
+        const bool front_ok = scales_as_they_are(b, gate, b.H, kNf4StreamGatedRowsPerExpert) &&
+                              scales_as_they_are(b, up, b.H, kNf4StreamGatedRowsPerExpert) &&
+                              (alike || (gate.absmax_u8 == nullptr && up.absmax_u8 == nullptr));
+        l.scale_slots = !front_ok ? 2 : scales_as_they_are(b, down, b.I, kNf4StreamRowsPerExpert) ? 0 : 1;
         size_t most = 0;
-        for (const mfl_nf4_weight *w : {b.q_gate, b.q_up, b.q_down})
-            if (w->absmax_u8 != nullptr) {
-                const size_t bytes = (size_t)((int64_t)b.E * b.H * b.I / w->blocksize) * 4;
-                most = bytes > most ? bytes : most;
-            }
+        for (const mfl_nf4_weight *w : {b.q_gate, b.q_up, b.q_down}) {
+            const size_t bytes = (size_t)((int64_t)b.E * b.H * b.I / w->blocksize) * 4;
+            most = bytes > most ? bytes : most;
+        }
         l.scale_bytes = up256(most);
-        l.scales = take(2 * l.scale_bytes);
+        l.scales = take(l.scale_slots * l.scale_bytes);
     }
     l.total = o;
     return l;
@@ -105,7 +120,7 @@ int front(const mfl_moe_block &b, char *ws, const Layout &l, void *stream) {
     if (b.q_gate != nullptr) {
         int rc = mfl_glu_fwd_nf4_packed(b.tokens, b.T, sort, b.k, b.q_gate, b.q_up, ms, MFL_I32, h, e, g, R, b.I, b.H, b.E,
                                         b.dtype, stream);
-        if (rc == MFL_ERR_UNSUPPORTED && (b.q_gate->absmax_u8 != nullptr || b.q_up->absmax_u8 != nullptr)) {
+        if (rc == MFL_ERR_UNSUPPORTED && (b.q_gate->absmax_u8 != nullptr || b.q_up->absmax_u8 != nullptr) && l.scale_slots == 2) {
             mfl_nf4_weight gate, up;
             MFL_TRY(write_out_scales(b, b.q_gate, (float *)(ws + l.scales), gate, stream));
             MFL_TRY(write_out_scales(b, b.q_up, (float *)(ws + l.scales + l.scale_bytes), up, stream));
@@ -133,7 +148,7 @@ int down(const mfl_moe_block &b, char *ws, const Layout &l, void *stream) {
         return mfl_gemm_fwd(ws + l.h, b.w_down, ms, MFL_I32, ws + l.y, R, b.H, b.I, b.E, b.dtype, b.dtype, 1.0f, 0, stream);
     int rc = mfl_gemm_fwd_nf4_packed(ws + l.h, 0, nullptr, 1, b.q_down, ms, MFL_I32, ws + l.y, R, b.H, b.I, b.E, b.dtype,
                                      b.dtype, stream);
-    if (rc == MFL_ERR_UNSUPPORTED && b.q_down->absmax_u8 != nullptr) {
+    if (rc == MFL_ERR_UNSUPPORTED && b.q_down->absmax_u8 != nullptr && l.scale_slots != 0) {
         mfl_nf4_weight w;
         MFL_TRY(write_out_scales(b, b.q_down, (float *)(ws + l.scales), w, stream));
         rc = mfl_gemm_fwd_nf4_packed(ws + l.h, 0, nullptr, 1, &w, ms, MFL_I32, ws + l.y, R, b.H, b.I, b.E, b.dtype, b.dtype,
