@@ -375,3 +375,17 @@ def test_block_workspace_has_room_for_written_out_scales_only_where_they_are(tok
         return _lib.lib().mfl_moe_block_workspace(b)
 
     assert size(True) - size(False) == slots * 128 * 2048 * inter // 64 * 4
+
+
+def test_block_workspace_on_packed_weights_never_holds_the_two_products():
+    """More than 512 experts: the dense form keeps gate's and up's products for a separate SiLU-mul, the packed kernels do
+    not need them."""
+    import ctypes
+
+    def size(experts):
+        at = 1 << 20
+        p = ctypes.pointer(_lib.Nf4Weight(at, at, at, None, None, None, None, None, 64, 0))
+        b = _lib.MoeBlock(at, at, None, None, None, p, p, p, 16, experts, 8, 512, 256, 1, _lib.BF16, _lib.BF16, 0)
+        return _lib.lib().mfl_moe_block_workspace(b)
+
+    assert size(513) - size(512) < 16 * 8 * 256 * 2

@@ -49,7 +49,7 @@ Layout layout(const mfl_moe_block &b) {
     l.weights = take(R * es);
     l.route_bytes = mfl_route_sort_workspace(b.T, b.E, b.k);
     l.route = take(l.route_bytes);
-    if (b.training || !front_is_one_kernel(b)) {
+    if (b.training || (b.q_gate == nullptr && !front_is_one_kernel(b))) {
         l.e = take(R * b.I * es);
         l.g = take(R * b.I * es);
     }
