@@ -148,18 +148,28 @@ class BlockwiseState:
     dtype: torch.dtype = torch.float32
 
 
+def _fp32_on(t: torch.Tensor, device: torch.device) -> torch.Tensor:
+    # (asked first: the two conversions cost a microsecond and a half of every call where there is nothing to convert)
+    if t.dtype is torch.float32 and t.device == device:
+        return t
+    return t.to(device=device, dtype=torch.float32)
+
+
 def _second_level(quant_state):
     """(uint8 scales, 256-entry code, second-level factors, their block size, offset) of a double-quantised state, all
     on the scales' device; the offset as a one-element fp32 tensor, never read on the host."""
     st2 = quant_state.state2
     absmax = quant_state.absmax.contiguous()
-    code2 = st2.code.to(device=absmax.device, dtype=torch.float32).contiguous()
-    absmax2 = st2.absmax.to(torch.float32).contiguous()
+    device = absmax.device
+    code2 = _fp32_on(st2.code, device).contiguous()
+    absmax2 = _fp32_on(st2.absmax, device).contiguous()
     offset = quant_state.offset
-    if not torch.is_tensor(offset):
+    if torch.is_tensor(offset):
+        offset = _fp32_on(offset, device)
+    else:
         # (a fill and not a copy from the host, which would wait for the device and end a stream capture)
-        offset = torch.full((), 0.0 if offset is None else float(offset), dtype=torch.float32, device=absmax.device)
-    return absmax, code2, absmax2, int(st2.blocksize), offset.to(device=absmax.device, dtype=torch.float32)
+        offset = torch.full((), 0.0 if offset is None else float(offset), dtype=torch.float32, device=device)
+    return absmax, code2, absmax2, int(st2.blocksize), offset
 
 
 def _is_shift(blocksize2: int) -> bool:
