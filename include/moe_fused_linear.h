@@ -218,7 +218,8 @@ MFL_API int mfl_glu_fwd_lora(const void *x, const void *w_gate, const void *w_up
                      int m_sizes_dtype, void *h, void *e_out, void *g_out, int64_t R, int N, int K,
                      int E, int dtype, void *stream);
 
-/* The same with NF4 weights, each matrix with its own quantisation state. */
+/* The same with NF4 weights, each matrix with its own quantisation state.  (This one, mfl_gemm_fwd_nf4_gather and the
+ * two _tiled entry points are for callers that hold the pieces of a state one by one; the _packed ones take a struct.) */
 MFL_API int mfl_glu_fwd_nf4(const void *x, int64_t src_rows, const int32_t *row_idx, int idx_div,
                     const uint8_t *wq_gate, const float *code16_gate, const float *absmax_gate,
                     int blocksize_gate, const uint8_t *wq_up, const float *code16_up,
@@ -304,8 +305,8 @@ MFL_API int mfl_nf4_quant(const void *w, int w_dtype, int64_t n, int blocksize, 
 
 /* ---- the router projection (modular_qwen3_moe_fused.py:85) -------------------------- */
 
-/* logits (T,E) = x (T,H) w (E,H)^T, bf16 operands, out_dtype bf16 or fp32.  H a multiple of 64
- * (MFL_ERR_UNSUPPORTED otherwise). */
+/* logits (T,E) = x (T,H) w (E,H)^T, bf16 operands, out_dtype bf16 or fp32 (for callers that route on unrounded
+ * logits).  H a multiple of 64 (MFL_ERR_UNSUPPORTED otherwise). */
 MFL_API int mfl_router_fwd(const void *x, const void *w, void *logits, int64_t T, int H, int E, int out_dtype,
                    void *stream);
 /* dw (E,H) = dlogits (T,E)^T x (T,H), all bf16, T > 0; H and E multiples of 8 (MFL_ERR_UNSUPPORTED otherwise; the

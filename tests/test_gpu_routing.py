@@ -237,7 +237,7 @@ def _check_route_outputs(logits, k, E, w, sel, m_sizes, sort_idx, inv):
     assert np.array_equal(inv.cpu().numpy(), i_o)
 
 
-# one launch up to 64 tokens; two launches (top-k that counts, scatter) above; three where the two-launch form
+# one launch up to 32 tokens; two launches (top-k that counts, scatter) above; three where the two-launch form
 # does not apply: more than 512 experts, more than 1024 segments of 256 selections
 @pytest.mark.parametrize("T,E,k,dtype", [(16, 128, 8, torch.float32), (1, 128, 8, torch.bfloat16), (64, 128, 8, torch.bfloat16),
                                          (7, 11, 3, torch.float32), (60, 512, 6, torch.float32), (33, 60, 1, torch.float32),
@@ -256,7 +256,7 @@ def test_route_and_sort_equals_the_separate_calls(T, E, k, dtype):
 @pytest.mark.parametrize("T", [200, 4096])
 def test_route_and_sort_with_a_row_of_nan(T):
     """A token whose logits are all NaN selects no expert (no probability compares greater than another): its
-    k selections are left out of the counts and of the sort, and every other token is routed as without it.
+    k selections are left out of the counts and sorted behind all others, and every other token is routed as without it.
     The histogram pass of the two-launch form must not count the row's "no expert" id."""
     from qwen3_moe_fused.kernels.routing import route_and_sort
 
@@ -281,7 +281,7 @@ def test_route_and_sort_with_a_row_of_nan(T):
 
 @pytest.mark.parametrize("T,E,k", [(128, 128, 8), (100, 512, 6), (65, 40, 5)])
 def test_one_launch_entry_point_up_to_its_own_limit(T, E, k):
-    # mfl_route_sort uses the one-workgroup form up to 64 tokens; the entry point itself takes up to 128
+    # mfl_route_sort uses the one-workgroup form up to 32 tokens; the entry point itself takes up to 128
     from qwen3_moe_fused import _lib
 
     logits = randn((T, E), gen(T), 2.0).to(DEV)

@@ -281,7 +281,8 @@ int launch_tile(const Args &g) {
 //   registers in transit leave two workgroups a CU).
 // * the weight gradient writes more than it reads up to about 100 rows per expert: 64 x 128 tiles and 16-row steps,
 //   182 us at 8 rows per expert = 4.5 TB/s (294; with 32-row steps 225, the zeros of a half-empty stage cost as much
-//   as rows do); outputs with a side of at most 16 (adapter ranks) take 16-row tiles.
+//   as rows do); outputs of at most 16 rows per expert (N: the rank in the gradient of an adapter's A) take
+//   16-row tiles.
 template <typename TI, typename TO, int MODE, int VEC>
 int launch_mode(const Args &g) {
     if (MODE == MODE_DW) {

@@ -141,9 +141,10 @@ class Qwen3MoeFusedSparseMoeBlock(nn.Module):
         return moe_fused_mlp(tokens, self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight, m_sizes,
                              sort_idx, inv_sort_idx, self.num_selected)
 
-    # Rows up to which the block is one library call: beyond, the kernels hide the host's time (131072 rows on packed
-    # weights: 1638 us either way) and the one buffer of all intermediates, 740 MB there, costs a first pass more than the
-    # steps' own tensors do, which find their room in what the allocator holds (1870 against 1733 us).
+    # Rows up to which the block is one library call.  Beyond, the kernels hide the host's time (131072 rows on packed
+    # weights: 1638 us either way), and the one buffer of all intermediates, 740 MB there, once cost a new state's first pass
+    # more than the steps' own tensors (1870 against 1733 us).  Measured again at hidden 1024 to 4096 it did not (1730 either
+    # way; buffers of 96 MB to 1.4 GB even or up to 3 % ahead), so the line is one of rows, not of the buffer's bytes.
     _ONE_CALL_ROWS = 65536
 
     def _one_call(self, tokens: torch.Tensor, logits: torch.Tensor) -> Optional[torch.Tensor]:

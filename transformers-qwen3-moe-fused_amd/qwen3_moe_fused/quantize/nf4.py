@@ -149,7 +149,7 @@ class BlockwiseState:
 
 
 def _fp32_on(t: torch.Tensor, device: torch.device) -> torch.Tensor:
-    # (asked first: the two conversions cost a microsecond and a half of every call where there is nothing to convert)
+    # (asked first: the two conversions cost about a microsecond of every call where there is nothing to convert)
     if t.dtype is torch.float32 and t.device == device:
         return t
     return t.to(device=device, dtype=torch.float32)
