@@ -389,3 +389,27 @@ def test_block_workspace_on_packed_weights_never_holds_the_two_products():
         return _lib.lib().mfl_moe_block_workspace(b)
 
     assert size(513) - size(512) < 16 * 8 * 256 * 2
+
+
+# (tokens, hidden, experts): where the router's own kernel takes the projection, and where the stock product is ahead of it
+@pytest.mark.parametrize("t,h,e,own", [(1, 64, 1, True), (512, 4096, 128, True), (513, 2048, 8, False), (1, 4160, 8, False),
+                                       (256, 64, 256, True), (257, 64, 256, False), (512, 64, 129, False)])
+def test_router_projection_takes_its_own_kernel_where_that_is_ahead(no_kernels, t, h, e, own):
+    if own:
+        with pytest.raises(LibraryCalled):
+            routing.router_linear(_bf16(t, h), _bf16(e, h))
+    else:
+        assert routing.router_linear(_bf16(t, h), _bf16(e, h)).shape == (t, e)
+
+
+@pytest.mark.parametrize("t,h,e,own", [(512, 4096, 512, True), (512, 4104, 512, False), (511, 64, 8, False)])
+def test_router_weight_gradient_takes_its_own_kernel_where_that_is_ahead(no_kernels, monkeypatch, t, h, e, own):
+    monkeypatch.setattr(routing, "_router_logits", torch.nn.functional.linear)
+    w = _bf16(e, h).requires_grad_()
+    y = routing.router_linear(_bf16(t, h), w)
+    if own:
+        with pytest.raises(LibraryCalled):
+            y.backward(_bf16(t, e))
+    else:
+        y.backward(_bf16(t, e))
+        assert w.grad.shape == (e, h)

@@ -14,17 +14,21 @@ import torch
 from .. import _lib
 
 
-# Tokens up to which the router projection runs on the library's own kernel (as fast as the stock product on the device,
-# and 14 us less of the host's time), and from which its weight gradient does (9.5 against 9.3 us at 512 tokens, 19
-# against 67 at 8192).
-_ROUTER_FWD_TOKENS = 512
-_ROUTER_DW_TOKENS = 512
+# Where the router projection runs on the library's own kernel: as fast as the stock product on the device there (hidden
+# 4096: 8.7 against 7.8 us) with 14 us less of the host's time.  Its workgroups take 16 tokens x 16 experts and the whole
+# reduction: with longer rows (hidden 7168: 15.6 against 7.4 us) or more of them than CUs (160 experts, 512 tokens, hidden 2048:
+# 8.8 against 6.1; 512 experts 16.0 against 7.0) the stock product is ahead.
+_ROUTER_FWD_TOKENS, _ROUTER_FWD_HIDDEN, _ROUTER_FWD_WORKGROUPS = 512, 4096, 256
+# Tokens from which its weight gradient does (9.5 against 9.3 us at 512 tokens, 19 against 67 at 8192), and the largest
+# weight: beyond, the stock product has workgroups enough (512 experts, hidden 7168, 4096 tokens: 49 against 44 us).
+_ROUTER_DW_TOKENS, _ROUTER_DW_WEIGHTS = 512, 1 << 21
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _router_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     tokens, hidden = x.shape
-    if tokens <= _ROUTER_FWD_TOKENS and hidden % 64 == 0:
+    if (tokens <= _ROUTER_FWD_TOKENS and hidden % 64 == 0 and hidden <= _ROUTER_FWD_HIDDEN
+            and -(-tokens // 16) * -(-w.shape[0] // 16) <= _ROUTER_FWD_WORKGROUPS):
         out = torch.empty((tokens, w.shape[0]), device=x.device, dtype=x.dtype)
         rc = _lib.lib().mfl_router_fwd(x.data_ptr(), w.data_ptr(), out.data_ptr(), tokens, hidden, w.shape[0], _lib.BF16,
                                        _lib.stream())
@@ -53,7 +57,8 @@ class _RouterLinear(torch.autograd.Function):
         dw = None
         if ctx.needs_input_grad[1]:
             tokens, hidden = x.shape
-            n = _lib.lib().mfl_router_dw_workspace(tokens, hidden, w.shape[0]) if tokens >= _ROUTER_DW_TOKENS else 0
+            own = tokens >= _ROUTER_DW_TOKENS and w.numel() <= _ROUTER_DW_WEIGHTS
+            n = _lib.lib().mfl_router_dw_workspace(tokens, hidden, w.shape[0]) if own else 0
             if n == 0:
                 return dx, dlogits.t() @ x
             dw, ws = w.new_empty(w.shape), torch.empty(n, device=x.device, dtype=torch.uint8)
