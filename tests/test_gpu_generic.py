@@ -82,15 +82,45 @@ def test_generic_products_within_the_bound_of_their_sums(sizes, n, k, dtype, out
         _check(got, exact[i], bound[i], length, alpha, old, fn.__name__)
 
 
+# short reductions (a step of 16, up to it, past it; aligned outputs and odd ones), up to 128 with tiles enough to fill the
+# chip, fp16 in odd sizes, weight gradients of a few rows (n x k as outputs: on both sides of the tiles' columns)
+SHORT = [
+    ([5, 0, 30], 132, 16),
+    ([5, 0, 30], 129, 15),
+    ([70, 60], 200, 17),
+    ([70, 60], 201, 32),
+    ([700, 300], 4160, 4),
+    ([700, 300], 4161, 16),
+    ([700, 300], 4161, 31),
+    ([700, 300], 4164, 33),
+    ([700, 320], 4161, 128),
+    ([3000, 1100], 2049, 131),
+    ([1], 130, 260),
+    ([3, 0, 1, 2], 65, 129),
+    ([16, 0], 128, 128),
+]
+
+
+@pytest.mark.parametrize("sizes,n,k", SHORT)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_short_reductions_and_few_rows_within_the_bound(sizes, n, k, dtype):
+    for length in ((n, k), (k, n)):  # the forward's short reduction, then the input gradient's
+        test_generic_products_within_the_bound_of_their_sums(sizes, *length, dtype, torch.float32, 0.5, True)
+
+
 @pytest.mark.parametrize("n", [65535 * 32, 65535 * 32 + 1, 65535 * 64])
 def test_outputs_of_more_column_tiles_than_a_grid_has_rows(n):
-    """The narrowest tiles are left to the wider ones where their number would pass 65535: one row, 4 to 8 products each."""
-    g = gen(n)
+    """The narrowest tiles are left to the wider ones where their number would pass 65535: one row, short and longer sums."""
     ms = torch.tensor([1], dtype=torch.int32, device="cuda")
-    for k, fn in ((4, grouped_gemm_forward), (3, grouped_gemm_forward_transposed)):
-        a = torch.randn((1, k), generator=g).cuda()
-        w = torch.randn((1, n, k) if fn is grouped_gemm_forward else (1, k, n), generator=g).cuda()
-        got = fn(a, w, ms, torch.float32)
-        w64 = w[0].double().t() if fn is grouped_gemm_forward else w[0].double()
-        room = k * 2.0 ** -24 * (a.double().abs() @ w64.abs()) + 2.0 ** -23 * (a.double() @ w64).abs()
-        assert ((got.double() - a.double() @ w64).abs() <= room).all()
+    torch.manual_seed(n)
+    for k, fn in ((4, grouped_gemm_forward), (3, grouped_gemm_forward_transposed), (36, grouped_gemm_forward),
+                  (35, grouped_gemm_forward_transposed)):
+        a = torch.randn((1, k), device="cuda")
+        w = torch.randn((1, n, k) if fn is grouped_gemm_forward else (1, k, n), device="cuda")
+        got = fn(a, w, ms, torch.float32)[0].double()
+        exact, bound = torch.zeros_like(got), torch.zeros_like(got)
+        for j in range(k):
+            term = a[0, j].double() * (w[0, :, j] if fn is grouped_gemm_forward else w[0, j]).double()
+            exact += term
+            bound += term.abs()
+        assert ((got - exact).abs() <= k * 2.0 ** -24 * bound + 2.0 ** -23 * exact.abs()).all()

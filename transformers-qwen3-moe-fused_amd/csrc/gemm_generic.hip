@@ -283,19 +283,36 @@ int launch_tile(const Args &g) {
 //   182 us at 8 rows per expert = 4.5 TB/s (294; with 32-row steps 225, the zeros of a half-empty stage cost as much
 //   as rows do); outputs of at most 16 rows per expert (N: the rank in the gradient of an adapter's A) take
 //   16-row tiles.
+// * short reductions (adapter ranks, toy sizes) leave most of a 64- or 128-wide step empty: 16-wide steps.  16000 rows of 8
+//   experts, 1500 outputs, reduction 8 / 32 / 64 / 128: 64 x 64 tiles 22.0 / 31.0 / 46 / 75 us (64-wide steps 34.9 / 44.5 / 54 /
+//   84, the kernel before 28.5 / 57 / 100 / 182); few rows 32 x 64 tiles (128 experts of 8 rows, 2048 outputs, reduction 16: 10.5
+//   us, 16-row tiles 23.9).  Where the output's rows are not aligned either, the stores decide: operands loaded one by one leave
+//   a lane with four rows of a column, and a store's lanes next to each other (8000 rows, 1001 outputs, reduction 8: 11.3 against
+//   22.4 us, 13.8 before; at 32 on 32 x 64 tiles 18.3 against 24.7).
+// * fp16 in odd sizes is bound by its single two-byte loads: 32 x 64 tiles, waves side by side (11311 rows of 8 experts, 1161 x
+//   793: 507 us; 64 x 64 588; before 530).
+// * weight gradients of a few rows per expert only store: smaller tiles, more of them (1 expert of 4 rows, 4096 x 4096: 15.6
+//   against 19.5 us, 16.6 before; 128 experts, 64 rows, 768 x 2048: 139 against 191).
 template <typename TI, typename TO, int MODE, int VEC>
 int launch_mode(const Args &g) {
     if (MODE == MODE_DW) {
         if (g.N <= 16) return launch_tile<TI, TO, MODE, 16, 64, 1, 4, 1, 32, VEC>(g);
-        if (g.N >= 64 && g.K >= 128) return launch_tile<TI, TO, MODE, 64, 128, 2, 2, 1, 16, VEC>(g);
+        const bool few = g.R <= (int64_t)4 * g.E || (g.R <= (int64_t)16 * g.E && (int64_t)g.E * g.N * g.K <= 1 << 25);
+        if (g.N >= 64 && g.K >= 128 && !few) return launch_tile<TI, TO, MODE, 64, 128, 2, 2, 1, 16, VEC>(g);
+        if (g.N >= 64 && g.K >= 128) return launch_tile<TI, TO, MODE, 64, 64, 2, 2, 1, 16, VEC>(g);
         return launch_tile<TI, TO, MODE, 64, 64, 2, 2, 1, 32, VEC>(g);
+    } else {
+        const bool few_tiles = (g.R / 64 + g.E) * ceil_div(g.N, 64) < 4 * device_info().cu_count;
+        const bool few = g.R <= (int64_t)48 * g.E || few_tiles;
+        if (VEC == 1 && !g.vec_out && g.K > 16 && g.K <= 32) return launch_tile<TI, TO, MODE, 32, 64, 2, 2, 1, 32, VEC>(g);
+        if (g.K <= 32 && few) return launch_tile<TI, TO, MODE, 32, 64, 2, 2, 1, 16, VEC>(g);
+        if (g.K <= 128 && !few) return launch_tile<TI, TO, MODE, 64, 64, 2, 2, 1, 16, VEC>(g);
+        // (their 32 columns would be more tiles than a grid has rows past two million outputs)
+        if (g.R <= (int64_t)16 * g.E && ceil_div(g.N, 32) <= 65535) return launch_tile<TI, TO, MODE, 16, 32, 1, 1, 4, 128, VEC>(g);
+        if (VEC == 1 && sizeof(TI) == 2 && !few_tiles) return launch_tile<TI, TO, MODE, 32, 64, 2, 2, 1, 32, VEC>(g);
+        if (few) return launch_tile<TI, TO, MODE, 32, 64, 1, 2, 2, 64, VEC>(g);
+        return launch_tile<TI, TO, MODE, 64, 64, 2, 1, 2, 64, VEC>(g);
     }
-    // (their 32 columns would be more tiles than a grid has rows past two million outputs)
-    if (g.R <= (int64_t)16 * g.E && ceil_div(g.N, 32) <= 65535) return launch_tile<TI, TO, MODE, 16, 32, 1, 1, 4, 128, VEC>(g);
-    const int64_t tiles64 = (g.R / 64 + g.E) * ceil_div(g.N, 64);
-    if (g.R <= (int64_t)48 * g.E || tiles64 < 4 * device_info().cu_count)
-        return launch_tile<TI, TO, MODE, 32, 64, 1, 2, 2, 64, VEC>(g);
-    return launch_tile<TI, TO, MODE, 64, 64, 2, 1, 2, 64, VEC>(g);
 }
 
 template <typename TI, typename TO>
@@ -303,6 +320,7 @@ int launch_generic(int mode, const Args &g) {
     // groups of four elements: every contiguous dimension that is read has to be a multiple of four
     const size_t align = 4 * sizeof(TI);
     bool vec = aligned(g.a, align) && aligned(g.b, align) && g.K % 4 == 0 && (mode == MODE_FWD || g.N % 4 == 0);
+    if (mode != MODE_DW && g.K <= 32 && !g.vec_out) vec = false;  // short reductions: the stores decide
     if (vec) {
         if (mode == MODE_FWD) return launch_mode<TI, TO, MODE_FWD, 4>(g);
         if (mode == MODE_DX) return launch_mode<TI, TO, MODE_DX, 4>(g);
