@@ -179,15 +179,32 @@ def stream() -> int:
     return _raw_stream(_device())
 
 
+# (bound once: the questions are asked in every call, and in a backward pass on another core than the forward's)
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_transforms, _tracing_state = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+_batched = torch._C._functorch.is_legacy_batchedtensor
+
+
+def plain_gradient(grad: torch.Tensor) -> bool:
+    """Whether a backward pass may hand this gradient's address to a kernel: no graph of the gradients is asked for, no
+    transform or mode is watching, and it is not several gradients at once (batched tensors have no address)."""
+    return not torch.is_grad_enabled() and _dispatch_modes() == 0 and _transforms() is None and not _batched(grad)
+
+
 def plain_call() -> bool:
     """Whether a call that passes autograd by, or stands in for a stock operator, may do so: no forward-mode level, no
     functorch transform, no dispatch mode (counters, fake tensors, selective checkpointing) and no function mode (but for
     default devices, which watch nothing) that would have to see the operators, and nobody tracing or compiling (asked first: a compiler cannot look into the others)."""
-    return (not torch.compiler.is_compiling() and forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None
-            and (torch._C._len_torch_function_stack() == 0
-                 or all(isinstance(torch._C._get_function_stack_at(i), DeviceContext)
-                        for i in range(torch._C._len_torch_function_stack()))))
+    return (not torch.compiler.is_compiling() and forward_ad._current_level < 0 and _dispatch_modes() == 0
+            and _transforms() is None and _tracing_state() is None
+            and (_function_modes() == 0 or all(isinstance(torch._C._get_function_stack_at(i), DeviceContext)
+                                               for i in range(_function_modes()))))
+
+
+def dense(t: torch.Tensor) -> torch.Tensor:
+    """``t.contiguous()``, asked first: the call gives the interpreter's lock away, and in a backward pass another thread
+    wants it (up to 5 us each until it is back)."""
+    return t if t.is_contiguous() else t.contiguous()
 
 
 def as_index_tensor(m_sizes: torch.Tensor) -> torch.Tensor:

@@ -165,10 +165,10 @@ class _MoeBlock(torch.autograd.Function):
         if dout is None:
             return (None,) * 7
         # (a saved-tensor hook may hand back equal tensors in other strides and places)
-        tokens, logits, w_gate, w_up, w_down, saved = (t.contiguous() for t in ctx.saved_tensors)
+        tokens, logits, w_gate, w_up, w_down, saved = map(_lib.dense, ctx.saved_tensors)
         if saved.data_ptr() % 256:
             saved = saved.clone()
-        dout = dout.contiguous()
+        dout = _lib.dense(dout)
         b = _dense_block(tokens, logits, w_gate, w_up, w_down, ctx.k, ctx.renorm, True)
         grads = [torch.empty_like(t) if need else None
                  for t, need in zip((tokens, logits, w_gate, w_up, w_down), ctx.needs_input_grad)]

@@ -47,20 +47,15 @@ class _RouterLinear(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dlogits):
         x, w = ctx.saved_tensors
-        # a graph of the gradients is asked for (create_graph), several gradients at once (batched tensors have no address)
-        # or somebody watches the operators: stock products have the one, take the other and are seen
-        if torch.is_grad_enabled() or not _lib.plain_call() or torch._C._functorch.is_legacy_batchedtensor(dlogits):
-            return (dlogits @ w if ctx.needs_input_grad[0] else None,
-                    dlogits.t() @ x if ctx.needs_input_grad[1] else None)
-        dlogits, x = dlogits.contiguous(), x.contiguous()  # (a saved-tensor hook may hand x back in other strides)
         dx = dlogits @ w if ctx.needs_input_grad[0] else None
         dw = None
         if ctx.needs_input_grad[1]:
             tokens, hidden = x.shape
-            own = tokens >= _ROUTER_DW_TOKENS and w.numel() <= _ROUTER_DW_WEIGHTS
+            own = tokens >= _ROUTER_DW_TOKENS and w.numel() <= _ROUTER_DW_WEIGHTS and _lib.plain_gradient(dlogits)
             n = _lib.lib().mfl_router_dw_workspace(tokens, hidden, w.shape[0]) if own else 0
             if n == 0:
                 return dx, dlogits.t() @ x
+            dlogits, x = _lib.dense(dlogits), _lib.dense(x)  # (a saved-tensor hook may hand x back in other strides)
             dw, ws = w.new_empty(w.shape), torch.empty(n, device=x.device, dtype=torch.uint8)
             rc = _lib.lib().mfl_router_dw(x.data_ptr(), dlogits.data_ptr(), dw.data_ptr(), tokens, hidden, w.shape[0],
                                           ws.data_ptr(), n, _lib.stream())
