@@ -392,8 +392,9 @@ def test_block_workspace_on_packed_weights_never_holds_the_two_products():
 
 
 # (tokens, hidden, experts): where the router's own kernel takes the projection, and where the stock product is ahead of it
-@pytest.mark.parametrize("t,h,e,own", [(1, 64, 1, True), (512, 4096, 128, True), (513, 2048, 8, False), (1, 4160, 8, False),
-                                       (256, 64, 256, True), (257, 64, 256, False), (512, 64, 129, False)])
+@pytest.mark.parametrize("t,h,e,own", [(1, 64, 1, True), (512, 4096, 128, True), (513, 2048, 8, False), (1, 5184, 8, False),
+                                       (512, 64, 256, True), (512, 64, 257, False), (512, 2048, 256, True), (512, 2112, 256, False),
+                                       (512, 4096, 129, False), (192, 5120, 272, True), (193, 5120, 272, False)])
 def test_router_projection_takes_its_own_kernel_where_that_is_ahead(no_kernels, t, h, e, own):
     if own:
         with pytest.raises(LibraryCalled):
@@ -413,3 +414,19 @@ def test_router_weight_gradient_takes_its_own_kernel_where_that_is_ahead(no_kern
     else:
         y.backward(_bf16(t, e))
         assert w.grad.shape == (e, h)
+
+
+@pytest.mark.parametrize("tokens,grad,frozen,own", [(1, True, True, True), (512, False, False, True), (513, True, False, False),
+                                                    (2047, True, False, False), (2048, True, False, True), (2048, True, True, False),
+                                                    (2048, False, False, False)])
+def test_router_module_is_the_stock_node_where_no_kernel_of_its_own_runs(monkeypatch, tokens, grad, frozen, own):
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    seen = []
+    from qwen3_moe_fused import modular_qwen3_moe_fused as mod
+
+    monkeypatch.setattr(mod, "router_linear", lambda x, w: seen.append(1))
+    gate = mod.Qwen3MoeFusedRouter(64, 8, bias=False).to(torch.bfloat16)
+    gate.weight.requires_grad_(not frozen)
+    with torch.set_grad_enabled(grad):
+        gate(_bf16(tokens, 64))
+    assert bool(seen) == own

@@ -165,7 +165,7 @@ class _MoeBlock(torch.autograd.Function):
         if dout is None:
             return (None,) * 7
         # (a saved-tensor hook may hand back equal tensors in other strides and places)
-        tokens, logits, w_gate, w_up, w_down, saved = map(_lib.dense, ctx.saved_tensors)
+        tokens, logits, w_gate, w_up, w_down, saved = [t if t.is_contiguous() else t.contiguous() for t in ctx.saved_tensors]
         if saved.data_ptr() % 256:
             saved = saved.clone()
         dout = _lib.dense(dout)
@@ -212,12 +212,17 @@ def moe_block(tokens: torch.Tensor, logits: torch.Tensor, w_gate: torch.Tensor, 
     """Everything of the sparse block that follows the router projection (modular_qwen3_moe_fused.py:87-115):
     ``tokens`` (T, hidden), ``logits`` (T, E), the three expert matrices in the tokens' type.  Returns (output (T, hidden),
     workspace, whose first T * num_selected int64 are the expert ids).  Differentiable in all five tensors."""
+    for w in (w_gate, w_up, w_down):
+        assert w.dtype == tokens.dtype and w.device == tokens.device and w.is_contiguous()
+    return moe_block_of(tokens, logits, w_gate, w_up, w_down, num_selected, renorm)
+
+
+def moe_block_of(tokens, logits, w_gate, w_up, w_down, num_selected, renorm):
+    """``moe_block`` on weights that are known to be dense and of the tokens' type and device."""
     assert w_gate.ndim == 3
     experts, inter, hidden = w_gate.shape
     assert w_up.shape == w_gate.shape and w_down.shape == (experts, hidden, inter)
     _check_rows(tokens, logits, experts, hidden)
-    for w in (w_gate, w_up, w_down):
-        assert w.dtype == tokens.dtype and w.device == tokens.device and w.is_contiguous()
     if torch.is_grad_enabled() and any(t.requires_grad for t in (tokens, logits, w_gate, w_up, w_down)):
         return _MoeBlock.apply(tokens, logits, w_gate, w_up, w_down, num_selected, renorm)
     return _run_block(_dense_block(tokens, logits, w_gate, w_up, w_down, num_selected, renorm, False), tokens)

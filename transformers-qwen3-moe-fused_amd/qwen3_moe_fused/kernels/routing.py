@@ -14,11 +14,13 @@ import torch
 from .. import _lib
 
 
-# Where the router projection runs on the library's own kernel: as fast as the stock product on the device there (hidden
-# 4096: 8.7 against 7.8 us) with 14 us less of the host's time.  Its workgroups take 16 tokens x 16 experts and the whole
-# reduction: with longer rows (hidden 7168: 15.6 against 7.4 us) or more of them than CUs (160 experts, 512 tokens, hidden 2048:
-# 8.8 against 6.1; 512 experts 16.0 against 7.0) the stock product is ahead.
-_ROUTER_FWD_TOKENS, _ROUTER_FWD_HIDDEN, _ROUTER_FWD_WORKGROUPS = 512, 4096, 256
+# Where the router projection runs on the library's own kernel: a few us slower on the device with long rows (hidden 4096:
+# 8.7 against 7.8), but its launches follow the block's others without a gap and cost 14 us less of the host's time: a pass of
+# the block is 3 to 6 us shorter (66 against 72 us at 1 token of hidden 4096, 262 against 266 at 256 on 256 experts).  Its
+# workgroups take 16 tokens x 16 experts and the whole reduction: with longer rows (hidden 7168: 2 to 6 us behind at any number
+# of tokens) or more of them (320 of hidden 4096: 382 against 377 us, 800 of hidden 2048: 191 against 187, 1024 of hidden 7168:
+# 405 against 367) the stock product is ahead.
+_ROUTER_FWD_TOKENS, _ROUTER_FWD_HIDDEN, _ROUTER_FWD_WORKGROUPS, _ROUTER_FWD_WORK = 512, 5120, 512, 1 << 20
 # Tokens from which its weight gradient does (9.5 against 9.3 us at 512 tokens, 19 against 67 at 8192), and the largest
 # weight: beyond, the stock product has workgroups enough (512 experts, hidden 7168, 4096 tokens: 49 against 44 us).
 _ROUTER_DW_TOKENS, _ROUTER_DW_WEIGHTS = 512, 1 << 21
@@ -27,8 +29,9 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 def _router_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     tokens, hidden = x.shape
+    workgroups = -(-tokens // 16) * -(-w.shape[0] // 16)
     if (tokens <= _ROUTER_FWD_TOKENS and hidden % 64 == 0 and hidden <= _ROUTER_FWD_HIDDEN
-            and -(-tokens // 16) * -(-w.shape[0] // 16) <= _ROUTER_FWD_WORKGROUPS):
+            and workgroups <= _ROUTER_FWD_WORKGROUPS and workgroups * hidden <= _ROUTER_FWD_WORK):
         out = torch.empty((tokens, w.shape[0]), device=x.device, dtype=x.dtype)
         rc = _lib.lib().mfl_router_fwd(x.data_ptr(), w.data_ptr(), out.data_ptr(), tokens, hidden, w.shape[0], _lib.BF16,
                                        _lib.stream())
@@ -63,6 +66,20 @@ class _RouterLinear(torch.autograd.Function):
                 return dx, dlogits.t() @ x
             _lib.check(rc, "mfl_router_dw")
         return dx, dw
+
+
+# Tokens from which a training step gains from the weight gradient's kernel: a node of the graph written in Python costs
+# the step up to 13 us of host time against the stock one, and below the gradient takes about as long either way (1024
+# tokens: 10.5 against 12.3 us; 4096: 16 against 34).
+_ROUTER_STEP_TOKENS = 2048
+
+
+def router_has_a_kernel(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether one of the router's own kernels would run for these rows, forward or backward."""
+    if type(x) not in _PLAIN or x.ndim != 2:  # (the type first: a tracer's stand-in has no size to decide on)
+        return False
+    tokens = x.shape[0]
+    return tokens <= _ROUTER_FWD_TOKENS or (tokens >= _ROUTER_STEP_TOKENS and torch.is_grad_enabled() and w.requires_grad)
 
 
 def router_linear(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:

@@ -16,7 +16,7 @@ from torch import nn
 
 from . import _lib
 from .functional import moe_fused_linear
-from .kernels.routing import combine_rows, gather_rows, route_and_sort, router_linear
+from .kernels.routing import combine_rows, gather_rows, route_and_sort, router_has_a_kernel, router_linear
 from .kernels.silu_mul import silu_mul
 
 
@@ -74,7 +74,9 @@ class Qwen3MoeFusedRouter(nn.Linear):
         if torch.jit.is_scripting():  # (compiled from source, where neither the kernel nor super() can be called)
             return nn.functional.linear(input, self.weight, self.bias)
         else:
-            out = router_linear(input, self.weight) if self.bias is None else None
+            out = None
+            if self.bias is None and router_has_a_kernel(input, self.weight):
+                out = router_linear(input, self.weight)
             return super().forward(input) if out is None else out
 
 
@@ -150,7 +152,7 @@ class Qwen3MoeFusedSparseMoeBlock(nn.Module):
     def _one_call(self, tokens: torch.Tensor, logits: torch.Tensor) -> Optional[torch.Tensor]:
         """Everything behind the router projection as one library call, where the three projections are plain expert
         matrices in the tokens' type (both ways), or plain packed ones (without gradients)."""
-        from .fused_mlp import moe_block, moe_block_4bit
+        from .fused_mlp import moe_block_4bit, moe_block_of
         from .quantize.layer import MoeFusedLinear4bit
 
         gate, up, down = self.gate_proj, self.up_proj, self.down_proj
@@ -171,7 +173,7 @@ class Qwen3MoeFusedSparseMoeBlock(nn.Module):
                 return None
         if torch.nn.modules.module._has_any_global_hook() or not _lib.plain_call():
             return None
-        assert logits.shape == (tokens.shape[0], self.num_experts)
+        assert logits.shape[-1] == self.num_experts
         weights = (gate.weight, up.weight, down.weight)
         if kind is MoeFusedLinear:
             if tokens.dtype not in (torch.bfloat16, torch.float32):
@@ -179,7 +181,7 @@ class Qwen3MoeFusedSparseMoeBlock(nn.Module):
             for w in weights:
                 if w.dtype != tokens.dtype or not w.is_contiguous() or w.device != tokens.device:
                     return None
-            out, ws = moe_block(tokens, logits, *weights, self.num_selected, self.norm_topk_prob)
+            out, ws = moe_block_of(tokens, logits, *weights, self.num_selected, self.norm_topk_prob)
         else:
             if tokens.dtype != torch.bfloat16 or (torch.is_grad_enabled() and (tokens.requires_grad or logits.requires_grad)):
                 return None
