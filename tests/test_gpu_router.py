@@ -105,3 +105,14 @@ def test_router_gradients_several_at_once():
     for i in range(2):
         _near(got[0][i], d[i].cpu(), w.detach().cpu(), 16)
         _near(got[1][i], d[i].t().cpu(), x.detach().cpu(), 600)
+
+
+@pytest.mark.parametrize("t,h,e", [(511, 640, 264), (33, 7168, 40), (530, 64, 520)])
+def test_projection_kernel_beyond_where_the_module_takes_it(t, h, e):
+    from qwen3_moe_fused import _lib
+
+    x, w = (torch.randn(s, generator=gen(t)).to(torch.bfloat16) for s in ((t, h), (e, h)))
+    xd, wd, out = x.cuda(), w.cuda(), torch.empty((t, e), dtype=torch.bfloat16, device="cuda")
+    _lib.check(_lib.lib().mfl_router_fwd(xd.data_ptr(), wd.data_ptr(), out.data_ptr(), t, h, e, _lib.BF16, _lib.stream()),
+               "mfl_router_fwd")
+    _near(out, x, w.t(), h)
