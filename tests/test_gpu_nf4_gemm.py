@@ -357,3 +357,35 @@ def test_nf4_forward_falls_back_for_inputs_without_a_fused_kernel(R, N, K, E, bl
     assert y.dtype == dtype
     tol = 1e-4 if dtype == torch.float32 else 1e-2
     check_close(y, oracle.linear_fwd(to_np32(x), w_deq, oracle.sel_from_m_sizes(ms.numpy())), tol, tol, "fallback forward")
+
+
+from qwen3_moe_fused.grouped_gemm.fused import (grouped_gemm_forward_4bit_lora,  # noqa: E402
+                                                grouped_gemm_forward_transposed_4bit_lora)
+
+
+# the 160 x 128 tiles: borders of a tile's rows and row blocks, empty experts, experts of several tiles, columns that end
+# inside a tile and inside a wave's part of it, one reduction step and an odd number of them, small quantisation blocks
+@pytest.mark.parametrize("m_sizes,N,K,blocksize", [([160, 161, 0, 159, 1], 128, 64, 64), ([32, 33, 31, 64, 96, 97], 160, 192, 64),
+                                                   ([0, 500, 3], 224, 128, 32), ([128] * 7, 96, 320, 16),
+                                                   ([1000], 256, 128, 64)])
+def test_packed_160_row_tiles(m_sizes, N, K, blocksize):
+    E, R, r = len(m_sizes), sum(m_sizes), 16
+    packed, state, w_deq = _quantised(E, N, K, blocksize, R + N)
+    g = gen(R)
+    ms = torch.tensor(m_sizes)
+    sel = oracle.sel_from_m_sizes(ms.numpy())
+    x, dy = randn((R, K), g, 1.0, torch.bfloat16), randn((R, N), g, 1.0, torch.bfloat16)
+    u, b, a = (randn(s, g, 0.1, torch.bfloat16) for s in ((R, r), (E, N, r), (E, r, K)))
+    up, bp, ap = to_np32(u), to_np32(b), to_np32(a)
+    ms = ms.to(DEV)
+    y = grouped_gemm_forward_4bit_lora(x.to(DEV), packed, state, u.to(DEV), b.to(DEV), ms)
+    check_close(y, oracle.linear_fwd(to_np32(x), w_deq, sel) + oracle.linear_fwd(up, bp, sel), what="forward")
+    ref = oracle.linear_bwd_input(to_np32(dy), w_deq, sel)
+    dx = grouped_gemm_forward_transposed_4bit_lora(dy.to(DEV), packed, state, u.to(DEV), a.to(DEV), ms)
+    check_close(dx, ref + oracle.linear_bwd_input(up, ap, sel), what="input gradient")
+    dx32 = grouped_gemm_forward_transposed_4bit(dy.to(DEV), packed, state, ms, torch.float32)
+    check_close(dx32, ref, 1e-4, 1e-4, "input gradient, fp32 output")
+    out0 = randn((R, K), g, 1.0, torch.bfloat16)
+    out = out0.to(DEV).clone()
+    grouped_gemm_forward_transposed_4bit(dy.to(DEV), packed, state, ms, out=out, accumulate=True)
+    check_close(out, to_np32(out0) + ref, what="input gradient, accumulated")

@@ -86,8 +86,19 @@ struct FwdFusion {
 // matrices with thin weights of its own, against one thin left operand; 4 the input gradient with the gated unit's
 // backward in its epilogue (a kernel of its own: its epilogue holds pieces of e and g in registers beside the
 // accumulators, which the plain input gradient has no room for).
+// Waves a SIMD has to hold: the workgroup's, and of two workgroups where two fit a CU's LDS (left to itself the compiler
+// gives a workgroup of four waves registers for itself alone: 267 in the packed 160 x 128 tile, one workgroup a CU).
+constexpr int lds_bytes(int MB, int NB, int BK, int S) {
+    // stages | two NF4 code tables | three per-expert prefix tables
+    return S * (MB + NB) * 32 * BK * 2 + 128 + 3 * (kMaxTableExperts + 1) * 4;
+}
+constexpr int workgroups_per_cu(int MB, int NB, int BK, int S) { return lds_bytes(MB, NB, BK, S) <= 80 * 1024 ? 2 : 1; }
+constexpr int min_waves(int MB, int NB, int BK, int S, int waves) {
+    return waves == 4 ? workgroups_per_cu(MB, NB, BK, S) : 1;
+}
+
 template <int MB, int NB, int BK, int S, int WGM, int WGN, int MODE, bool NF4, int FUSE, typename TO>
-__global__ __launch_bounds__(WGM *WGN * 64) void gemm_pipe_kernel(const bf16_t *__restrict__ a,
+__global__ __launch_bounds__(WGM *WGN * 64, min_waves(MB, NB, BK, S, WGM *WGN)) void gemm_pipe_kernel(const bf16_t *__restrict__ a,
                                                                   const bf16_t *__restrict__ b,
                                                                   const void *__restrict__ m_sizes, int ms_i64,
                                                                   TO *__restrict__ c, int64_t R, int N, int K, int E,
@@ -964,13 +975,12 @@ int launch_pipe(int mode, const void *a, const void *b, const void *m_sizes, int
     constexpr int STAGE_BYTES = (MB + NB) * 32 * BK * 2;
     constexpr int EP_BYTES = WGM * WGN * 32 * ((NB / WGN) * 64 + 16);
     static_assert(EP_BYTES <= S * STAGE_BYTES, "the output staging reuses the stages");
-    // stages | two NF4 code tables | three per-expert prefix tables
-    constexpr int LDS_BYTES = S * STAGE_BYTES + 128 + 3 * (kMaxTableExperts + 1) * 4;
+    constexpr int LDS_BYTES = lds_bytes(MB, NB, BK, S);
     static_assert(LDS_BYTES <= 160 * 1024, "LDS capacity of a CDNA4 compute unit");
     const bf16_t *pa = (const bf16_t *)a, *pb = (const bf16_t *)b;
     TO *pc = (TO *)c;
     // one persistent workgroup per CU, two where two fit (the small rings of the thin products)
-    constexpr int PER_CU = LDS_BYTES <= 80 * 1024 ? 2 : 1;
+    constexpr int PER_CU = workgroups_per_cu(MB, NB, BK, S);
     const int grid = device_info().cu_count / kXcd * kXcd * PER_CU;
     const Nf4Params none = {nullptr, nullptr, 0};
     const FwdFusion no_fusion = {nullptr, 1, nullptr, none, nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr};
@@ -1095,7 +1105,19 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
             // packed weights with an output of 1024 columns and more that is a multiple of 256 wide, up to 232 rows per
             // expert: 256 x 256 tiles as well (8 column slices an expert instead of 11 of 192 columns)
             const bool nf4_wide = nf4 != nullptr && N % 256 == 0 && N >= 1024 && R <= (int64_t)232 * E;
+            // packed weights, up to 128 rows per expert on average (few experts then hold more than 160), or as long as the
+            // smaller tiles are all resident at once (512 on 256 CUs): 160 x 128 tiles of four waves, two workgroups a CU.
+            // A step with packed weights is a chain (copies land, codes are looked up, stage written, barrier) that one
+            // workgroup a CU leaves the chip waiting on; two run theirs side by side.  us, 128 experts, N x K of the
+            // weights, against the tiles below, with the thin last term, forward 768 x 2048: 83 / 87 / 98 against 108 /
+            // 96 / 105 at 48 / 96 / 128 rows per expert (142 against 113 at 160), 2048 x 768: 106 against 115 at 128;
+            // input gradient 96 against 109 and 91 against 95 at 128.  Skewed routing (Zipf 1.2) at 64 rows per expert
+            // 101 against 165 and 97 against 112.  8 experts of 512 rows 46 against 68, of 1024 rows 61 against 69; 16
+            // experts of 1024 rows (708 tiles) 102 against 75.  The sums are the same bits.
+            const bool nf4_pair = nf4 != nullptr && (R <= (int64_t)128 * E ||
+                                                     (R / 160 + E) * (int64_t)ceil_div(N, 128) <= 2 * device_info().cu_count);
             cfg = (N <= 64 && nf4 == nullptr) ? 10
+                  : nf4_pair ? 5
                   : (R <= (int64_t)kFlatTileRowsPerExpert * E && nf4 == nullptr) ? 15
                   : (R >= (int64_t)512 * E || nf4_wide) ? 8 : 3;
         }
@@ -1109,6 +1131,8 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
             return MFL_LAUNCH(10, 6, 64, 2, 4, 2, 31);
         case 4:
             return MFL_LAUNCH(10, 4, 64, 2, 4, 2, 7);
+        case 5:  // 160 x 128 tiles, two stages of 36 KiB, two workgroups of four waves a CU
+            return MFL_LAUNCH(5, 4, 64, 2, 2, 2, 19);
         case 15:  // a few rows per expert (decode): the weights are all the traffic; flat 64 x 128 tiles,
                   // 3 stages of 24 KiB, two workgroups per CU (one with 6 stages: 85 instead of 77 us for
                   // 2048 rows over 128 experts, N = 768, K = 2048)
