@@ -510,3 +510,33 @@ def test_glu_with_lora_terms_equals_the_separate_products(R, N, K, E, r):
         check_close(e, to_np32(e_ref), what="gate product")
         check_close(gg, to_np32(g_ref), what="up product")
         assert torch.equal(h, silu_mul_forward(e, gg))
+
+
+# few experts or narrow outputs: 64 x 128 tiles, and 160 x 128 where those are too many to be resident at once (the
+# last three); borders of tiles and row blocks, experts without rows, columns that end inside a tile, odd numbers of steps
+@pytest.mark.parametrize("m_sizes,N,K", [([64, 65, 0, 63], 136, 64), ([0, 200, 50], 320, 192), ([49], 128, 320),
+                                         ([321, 0], 256, 128), ([3900, 161], 1936, 64), ([2900, 1100, 7], 1920, 128),
+                                         ([160, 159, 161, 0, 320] * 3, 760, 64)])
+def test_few_large_tiles(m_sizes, N, K):
+    E, R, r = len(m_sizes), sum(m_sizes), 8
+    g = gen(R + N)
+    ms = torch.tensor(m_sizes)
+    sel = oracle.sel_from_m_sizes(ms.numpy())
+    x, x2, u = (randn((R, n), g, 1.0, torch.bfloat16) for n in (K, K, r))
+    w, w2, b = (randn((E, N, k), g, 0.05, torch.bfloat16) for k in (K, K, r))
+    ms, on = ms.to(DEV), lambda *t: [v.to(DEV) for v in t]
+    e, g2 = (oracle.linear_fwd(to_np32(x), to_np32(v), sel).astype(np.float64) for v in (w, w2))
+    check_close(grouped_gemm_forward(*on(x, w), ms), e, what="forward")
+    term = oracle.linear_fwd(to_np32(u), to_np32(b), sel)
+    check_close(grouped_gemm_forward_lora(*on(x, w, u, b), ms), e + term, what="forward, rank-r term")
+    h, pe, pg = grouped_glu_forward(*on(x, w, w2), ms, return_products=True)
+    check_close(pe, e, what="gate")
+    check_close(pg, g2, what="up")
+    assert torch.equal(h, silu_mul_forward(pe, pg))
+    # input gradients: weights of (E, K, N), so that the output has the N columns again
+    wt, wt2, bt = (v.transpose(1, 2).contiguous() for v in (w, w2, b))
+    check_close(grouped_gemm_forward_transposed(*on(x, wt), ms), e, what="input gradient")
+    both = e + oracle.linear_fwd(to_np32(x2), to_np32(w2), sel)
+    check_close(grouped_gemm_forward_transposed_dual(*on(x, wt, x2, wt2), ms), both, what="input gradient, two terms")
+    check_close(grouped_gemm_forward_transposed_lora(*on(x, wt, u, bt), ms, dy2=x2.to(DEV), w2=wt2.to(DEV)), both + term,
+                what="input gradient, two terms and the rank-r one")

@@ -32,6 +32,33 @@ constexpr int kNf4StreamRowsPerExpert = 128;
 constexpr int kNf4StreamGatedRowsPerExpert = 384;
 constexpr int kNf4StreamTwoBlockRows = 20;
 
+// Outputs of at least 1024 columns that are a multiple of 256 wide: rows per expert up to which the four-wave kernel takes
+// 192 x 256 and 256 x 256 tiles (the times are at its dispatch).
+constexpr int kWideOutRowsPerExpert = 152, kWideMidRowsPerExpert = 232;
+
+// Tiles of BM x BN rows and columns, on average over routings: an expert's last row tile is half full.
+inline int64_t expected_tiles(int64_t R, int N, int E, int BM, int BN) {
+    const int64_t row_tiles = R / BM + E / 2;
+    return (row_tiles > E ? row_tiles : E) * ceil_div(N, BN);
+}
+
+// A row-grouped bf16 product (two: the gated unit's, half as many columns of each matrix in a tile) whose large tiles would
+// leave at least half of the CUs without one: with few experts, or narrow outputs, a launch then takes as long as one such
+// tile.  It runs on 64 x 128 tiles, or 160 x 128 where those are not all resident at once, two workgroups a CU either way
+// (the rule is in gemm_bf16_pipe.hip).  us at N x K = 768 x 2048 (8 experts of 64 / 128 / 256 / 512 rows, large tiles in brackets): forward 17 /
+// 19 / 20 / 33 (26 / 38 / 46 / 49), input gradient 11 / 16 / 17 / 26 (18 / 21 / 24 / 27; of two terms 18 / 27 / 29 / 41
+// against 33 / 36 / 39 / 43), gated 21 / 21 / 32 / 44 (37 / 40 / 51 / 57).  Where the large tiles occupy more than half of
+// the CUs they are ahead: 16 experts of 128 rows, 192 tiles: input gradient 28 against 34; 8 experts of 512 rows, 144 tiles:
+// 40 against 54.  The sums are the same bits on all of them.
+inline bool few_large_tiles(int64_t R, int N, int E, bool gated) {
+    int bm = 320, bn = 192;
+    if (R >= (int64_t)512 * E)
+        bm = 256, bn = 256;
+    else if (!gated && N % 256 == 0 && N >= 1024 && R <= (int64_t)kWideMidRowsPerExpert * E)
+        bm = R <= (int64_t)kWideOutRowsPerExpert * E ? 192 : 256, bn = 256;
+    return 2 * expected_tiles(R, N, E, bm, gated ? bn / 2 : bn) <= device_info().cu_count;
+}
+
 // Any shape / any float type; fp32 matrix instruction.
 int gemm_generic(int mode, const void *a, const void *b, const void *m_sizes, int ms_i64, void *c, int64_t R, int N,
                  int K, int E, int in_dtype, int out_dtype, float alpha, int accumulate, hipStream_t stream);

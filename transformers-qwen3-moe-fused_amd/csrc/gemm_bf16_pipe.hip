@@ -1096,8 +1096,19 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
     // Products with the GLU epilogue (bit 3): the configurations whose waves along N split in two halves.
     const bool glu = fusion != nullptr && fusion->b2 != nullptr && fusion->a2 == nullptr;
     int cfg = g_pipe_config;
+    // few experts or narrow outputs (few_large_tiles()): 64 x 128 tiles as long as they are all resident at once (512 on
+    // 256 CUs), 160 x 128 beyond (8 experts, input gradient at N = 2048: 16 / 24 us at 128 / 256 rows per expert on the
+    // former, 17 / 17 on the latter; forward at N = 768, 512 rows: 33 against 34)
+    const int small_cfg = !few_large_tiles(R, N, E, glu)                                                ? 0
+                          : expected_tiles(R, N, E, 64, glu ? 64 : 128) <= 2 * device_info().cu_count ? 15
+                                                                                                        : 5;
     if (glu && (cfg == 0 || nf4 != nullptr)) {
-        cfg = R >= (int64_t)512 * E ? 8 : (R <= (int64_t)kFlatTileRowsPerExpert * E && nf4 == nullptr) ? 15 : 3;
+        if (nf4 == nullptr)
+            cfg = R <= (int64_t)kFlatTileRowsPerExpert * E ? 15 : small_cfg ? small_cfg : R >= (int64_t)512 * E ? 8 : 3;
+        else
+            // packed: 160 x 128 tiles (64 columns of either matrix) as long as they are all resident at once; 8 experts of
+            // 512 rows, N = 768, K = 2048: 60 us against 68 (N = 1280, K = 2176, 672 tiles: 104 against 73)
+            cfg = (R / 160 + E) * (int64_t)ceil_div(N, 64) <= 2 * device_info().cu_count ? 5 : R >= (int64_t)512 * E ? 8 : 3;
     } else if (cfg == 0 || nf4 != nullptr) {
         if (mode == MODE_DW)
             cfg = (N <= 64 || K <= 64) ? 11 : 8;
@@ -1119,6 +1130,7 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
             cfg = (N <= 64 && nf4 == nullptr) ? 10
                   : nf4_pair ? 5
                   : (R <= (int64_t)kFlatTileRowsPerExpert * E && nf4 == nullptr) ? 15
+                  : (small_cfg && nf4 == nullptr) ? small_cfg
                   : (R >= (int64_t)512 * E || nf4_wide) ? 8 : 3;
         }
     }
@@ -1132,7 +1144,7 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
         case 4:
             return MFL_LAUNCH(10, 4, 64, 2, 4, 2, 7);
         case 5:  // 160 x 128 tiles, two stages of 36 KiB, two workgroups of four waves a CU
-            return MFL_LAUNCH(5, 4, 64, 2, 2, 2, 19);
+            return MFL_LAUNCH(5, 4, 64, 2, 2, 2, 27);
         case 15:  // a few rows per expert (decode): the weights are all the traffic; flat 64 x 128 tiles,
                   // 3 stages of 24 KiB, two workgroups per CU (one with 6 stages: 85 instead of 77 us for
                   // 2048 rows over 128 experts, N = 768, K = 2048)

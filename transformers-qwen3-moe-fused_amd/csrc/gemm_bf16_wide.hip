@@ -29,8 +29,6 @@ namespace mfl {
 
 namespace {
 
-constexpr int kWideOutRowsPerExpert = 152, kWideMidRowsPerExpert = 232;
-
 // Tuning builds can take parts of the kernel out (timing experiments only; the results are then wrong).
 #ifdef MFL_TUNING_BUILD
 #ifndef MFL_X_NO_STORE
@@ -955,6 +953,7 @@ int gemm_bf16_wide(int mode, const void *a, const void *b, const void *m_sizes, 
         return launch_wide<MODE_DW, 8, 8, 32, 4>(a, b, m_sizes, ms_i64, c, R, N, K, E, stream);
     }
     if (K % 64 != 0 || K < 64 || R <= 0) return R <= 0 ? MFL_OK : MFL_ERR_UNSUPPORTED;
+    if (few_large_tiles(R, N, E, false)) return MFL_ERR_UNSUPPORTED;  // smaller tiles: gemm_bf16_pipe.hip
     // 320 x 192 tiles (an expert of up to 320 rows is one tile per column slice) up to about 512 rows per expert,
     // 256 x 256 beyond (fewer bytes per flop).  Outputs that are wide and a multiple of 256 columns, up to 152 rows
     // per expert on average (few experts then hold more than 192 rows): 192 x 256 tiles, a quarter fewer tiles and
