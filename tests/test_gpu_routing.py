@@ -336,3 +336,22 @@ def test_routing_weight_gradient_bf16_logits_through_route_and_sort():
     (w64 * dw.double()).sum().backward()
     assert ld.grad.dtype == torch.bfloat16
     check_close(ld.grad, l64.grad.numpy(), rtol=1e-2, atol=1e-2 * float(l64.grad.abs().max()), what="d logits (bf16)")
+
+
+def test_routing_whose_weights_get_no_gradient():
+    from qwen3_moe_fused.kernels.routing import route_and_sort
+
+    # the index outputs are given no zeros to go with; a step behind that returns no gradient leaves zeros in the logits'
+    class NoGradient(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, w):
+            return w.sum()
+
+        @staticmethod
+        def backward(ctx, dout):
+            return None
+
+    for routed in (lambda v: route_and_sort(v, 2, True, torch.float32, 8)[0], lambda v: softmax_topk(v, 2, True)[0]):
+        logits = torch.randn((5, 8), device="cuda").requires_grad_()
+        (NoGradient.apply(routed(logits)) + 0.0 * logits.sum()).backward()
+        assert torch.equal(logits.grad, torch.zeros_like(logits))

@@ -126,12 +126,14 @@ class _SoftmaxTopk(torch.autograd.Function):
         ctx.save_for_backward(logits, idx, w32)
         ctx.renorm = renorm
         ctx.mark_non_differentiable(idx)
+        ctx.set_materialize_grads(False)  # (else the engine fills zeros for the ids)
         return wc, idx
 
     @staticmethod
     def backward(ctx, dw, _didx):
         # Not on the hot path (a (T, E) problem; the frozen-router LoRA recipes never reach it).
         logits, idx, w32 = ctx.saved_tensors
+        dw = torch.zeros_like(w32) if dw is None else dw
         return _softmax_topk_backward(logits, idx, w32, ctx.renorm, dw), None, None, None
 
 
@@ -212,11 +214,14 @@ class _RouteAndSort(torch.autograd.Function):
         ctx.save_for_backward(logits, idx, w32)
         ctx.renorm = renorm
         ctx.mark_non_differentiable(idx, m_sizes, sort_idx, inv)
+        # else the engine allocates and fills zeros for the four index outputs: four launches of 4 us each a step
+        ctx.set_materialize_grads(False)
         return wc, idx, m_sizes, sort_idx, inv
 
     @staticmethod
     def backward(ctx, dw, *_unused):
         logits, idx, w32 = ctx.saved_tensors
+        dw = torch.zeros_like(w32) if dw is None else dw
         return _softmax_topk_backward(logits, idx, w32, ctx.renorm, dw), None, None, None, None
 
 
