@@ -540,3 +540,26 @@ def test_few_large_tiles(m_sizes, N, K):
     check_close(grouped_gemm_forward_transposed_dual(*on(x, wt, x2, wt2), ms), both, what="input gradient, two terms")
     check_close(grouped_gemm_forward_transposed_lora(*on(x, wt, u, bt), ms, dy2=x2.to(DEV), w2=wt2.to(DEV)), both + term,
                 what="input gradient, two terms and the rank-r one")
+
+
+def test_gated_product_on_square_tiles_below_512_rows_per_expert():
+    # 60 experts, N = 504: one round of 256 x 256 tiles against two of 320 x 192; experts at the tile's borders, of two
+    # tiles and without rows, a last column slice that ends inside a tile
+    m_sizes = [255, 256, 257, 0, 31, 33, 300, 1, 128, 64] * 6
+    E, R, N, K, r = 60, sum(m_sizes), 504, 64, 8
+    g = gen(R)
+    sel = oracle.sel_from_m_sizes(np.array(m_sizes))
+    x, u = randn((R, K), g, 1.0, torch.bfloat16), randn((R, r), g, 1.0, torch.bfloat16)
+    w, w2 = (randn((E, N, K), g, 0.05, torch.bfloat16) for _ in range(2))
+    b, b2 = (randn((E, N, r), g, 0.05, torch.bfloat16) for _ in range(2))
+    e, g2, te, tg = (oracle.linear_fwd(to_np32(a), to_np32(v), sel).astype(np.float64)
+                     for a, v in ((x, w), (x, w2), (u, b), (u, b2)))
+    ms, on = torch.tensor(m_sizes).to(DEV), lambda *t: [v.to(DEV) for v in t]
+    h, pe, pg = grouped_glu_forward(*on(x, w, w2), ms, return_products=True)
+    check_close(pe, e, what="gate")
+    check_close(pg, g2, what="up")
+    assert torch.equal(h, silu_mul_forward(pe, pg))
+    h, pe, pg = grouped_glu_forward_lora(*on(x, w, w2, u, b, b2), ms)
+    check_close(pe, e + te, what="gate, rank-r term")
+    check_close(pg, g2 + tg, what="up, rank-r term")
+    assert torch.equal(h, silu_mul_forward(pe, pg))

@@ -37,6 +37,8 @@
 //   DX with two terms: the reduction runs over a second pair of operands after the first.
 // Memory hints: weights of the row-grouped products are copied non-temporal (each is read by one
 // workgroup), the output leaves with streaming stores.
+#include <cmath>
+
 #include "pipe_parts.h"
 
 namespace mfl {
@@ -1077,6 +1079,21 @@ constexpr int g_pipe_config = 0;
 
 namespace {
 
+// The gated product's tiles past the flat ones: 256 x 256 (128 columns of either matrix) or 320 x 192 (96).  A round of either
+// is a tile on every CU, of the same number of reduction steps: the square ones are taken where they have fewer rounds, and
+// from 512 rows per expert on.  An expert is counted with 1.5 standard deviations more rows than the average.  us at K =
+// 2048, 320 x 192 / 256 x 256, 128 experts, N = 768: 205 / 188, 203 / 195, 244 / 232, 266 / 257 at 64 / 128 / 188 / 232 rows per
+// expert (4 and 3 rounds), 273 / 298 at 256 (4 and 6), 447 / 409 at 400 (8 and 6); 160 experts, N = 1408: 500 / 440 at 188 (10
+// and 7); 60 experts, N = 768: 108 / 117 at 188 (2 and 2).  Skewed routing (Zipf 1.2), 128 experts: 255 / 209 at 64, 302 / 296
+// at 208.  (From 512 to 640 rows the tall ones are up to 6 % ahead when routing is even, and behind when it is not.)
+bool square_gated_tiles(int64_t R, int N, int E) {
+    if (R >= (int64_t)512 * E) return true;
+    const double mean = (double)R / E;
+    const int rows = (int)(mean + 1.5 * std::sqrt(mean)), cus = device_info().cu_count;
+    auto rounds = [&](int bm, int cols) { return ((int64_t)E * ceil_div(rows, bm) * ceil_div(N, cols) + cus - 1) / cus; };
+    return rounds(256, 128) < rounds(320, 96);
+}
+
 int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, int ms_i64, void *c, int64_t R, int N,
                   int K, int E, int out_dtype, float alpha, int accumulate, const Nf4Params *nf4,
                   const FwdFusion *fusion, hipStream_t stream) {
@@ -1104,11 +1121,15 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
                                                                                                         : 5;
     if (glu && (cfg == 0 || nf4 != nullptr)) {
         if (nf4 == nullptr)
-            cfg = R <= (int64_t)kFlatTileRowsPerExpert * E ? 15 : small_cfg ? small_cfg : R >= (int64_t)512 * E ? 8 : 3;
+            cfg = R <= (int64_t)kFlatTileRowsPerExpert * E ? 15 : small_cfg ? small_cfg : square_gated_tiles(R, N, E) ? 8 : 3;
         else
             // packed: 160 x 128 tiles (64 columns of either matrix) as long as they are all resident at once; 8 experts of
             // 512 rows, N = 768, K = 2048: 60 us against 68 (N = 1280, K = 2176, 672 tiles: 104 against 73)
-            cfg = (R / 160 + E) * (int64_t)ceil_div(N, 64) <= 2 * device_info().cu_count ? 5 : R >= (int64_t)512 * E ? 8 : 3;
+            // and past the streaming kernel's rows 256 x 256 (128 experts of 400 / 448 / 512 rows: 447 / 466 / 537 us against
+            // 525 / 516 / 633 on 320 x 192, 60 experts 191 / 207 / 261 against 229 / 232 / 282)
+            cfg = (R / 160 + E) * (int64_t)ceil_div(N, 64) <= 2 * device_info().cu_count ? 5
+                  : R > (int64_t)kNf4StreamGatedRowsPerExpert * E                         ? 8
+                                                                                          : 3;
     } else if (cfg == 0 || nf4 != nullptr) {
         if (mode == MODE_DW)
             cfg = (N <= 64 || K <= 64) ? 11 : 8;
