@@ -1,6 +1,9 @@
 """Shared helpers of the parity tests: seeded inputs, routing draws, error metrics."""
 from __future__ import annotations
 
+import re
+import warnings
+
 import numpy as np
 import torch
 
@@ -78,3 +81,45 @@ def unit_scale_atol(expect: np.ndarray, atol=BF16_ATOL) -> float:
 def oracle_rows(x: torch.Tensor, w: torch.Tensor, sel: np.ndarray, rows: np.ndarray) -> np.ndarray:
     """Oracle forward for a subset of rows (rows are independent)."""
     return oracle.linear_fwd(to_np32(x[rows]), to_np32(w), sel[rows])
+
+
+_TILED = re.compile(r"gemm_(pipe|wide)_kernel(I|<)(.*)")
+
+
+def tiles_of(fn):
+    """``(fn(), tiles)`` with the tiles that the pipelined and four-wave products launched by ``fn`` ran on, from the names
+    of their kernels: a set of ``(kernel, rows, columns, product, packed, fusion)``, kernel "pipe" or "wide", product 0
+    forward, 1 input gradient, 2 weight gradient, fusion as the pipelined kernel's template has it (0 none, 1 gated, 2 thin
+    last term, 3 both, 4 gated unit's backward).  None where the tracer gave no kernels at all (another tool may hold it)."""
+    from torch.profiler import ProfilerActivity, profile
+
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        out = fn()
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA]
+    if not names:
+        warnings.warn("no kernel names from the tracer: the tiles are not checked")
+        return out, None
+    found = set()
+    for name in names:
+        m = _TILED.search(name)
+        if m is None:
+            continue
+        if m[2] == "I":  # mangled: Li<number>E, Lb<0 or 1>E
+            args = [int(v) for v in re.findall(r"L[ib](\d+)E", m[3])]
+        else:
+            args = [int({"true": 1, "false": 0}.get(v, v)) for v in re.findall(r"true|false|\b\d+\b", m[3].split(">")[0])]
+        if m[1] == "pipe":
+            mb, nb, _, _, _, _, mode, packed, fuse = args[:9]
+        else:
+            mode, mb, nb, _, _, thin = args[:6]
+            packed, fuse = 0, 2 * thin
+        found.add((m[1], 32 * mb, 32 * nb, mode, bool(packed), fuse))
+    return out, found
+
+
+def check_tiles(fn, *expect):
+    """``fn()``, which has to run on exactly these tiles (see ``tiles_of``)."""
+    out, found = tiles_of(fn)
+    assert found is None or found == set(expect), f"ran on {sorted(found)}, expected {sorted(expect)}"
+    return out

@@ -1079,19 +1079,33 @@ constexpr int g_pipe_config = 0;
 
 namespace {
 
+// Rounds over the CUs of tiles of bm rows and bn columns, not rounded up, on average over even routings: an expert's rows
+// scatter around R / E with that variance, and every multiple of bm that they pass is one more row tile.
+double expected_rounds(int64_t R, int N, int E, int bm, int bn) {
+    const double mean = (double)R / E, sd = std::sqrt(mean);
+    double row_tiles = 1.0;
+    for (double edge = bm + 0.5; edge < mean + 6.0 * sd; edge += bm) row_tiles += 0.5 * std::erfc((edge - mean) / (sd * M_SQRT2));
+    return row_tiles * E * ceil_div(N, bn) / device_info().cu_count;
+}
+
 // The gated product's tiles past the flat ones: 256 x 256 (128 columns of either matrix) or 320 x 192 (96).  A round of either
-// is a tile on every CU, of the same number of reduction steps: the square ones are taken where they have fewer rounds, and
-// from 512 rows per expert on.  An expert is counted with 1.5 standard deviations more rows than the average.  us at K =
-// 2048, 320 x 192 / 256 x 256, 128 experts, N = 768: 205 / 188, 203 / 195, 244 / 232, 266 / 257 at 64 / 128 / 188 / 232 rows per
-// expert (4 and 3 rounds), 273 / 298 at 256 (4 and 6), 447 / 409 at 400 (8 and 6); 160 experts, N = 1408: 500 / 440 at 188 (10
-// and 7); 60 experts, N = 768: 108 / 117 at 188 (2 and 2).  Skewed routing (Zipf 1.2), 128 experts: 255 / 209 at 64, 302 / 296
-// at 208.  (From 512 to 640 rows the tall ones are up to 6 % ahead when routing is even, and behind when it is not.)
+// is a tile on every CU, of the same number of reduction steps, so the tiles of fewer rounds are ahead, and half a round more
+// is what the last one costs on average.  Square tiles: from 512 rows per expert on, at a fifth fewer rounds so counted, and at
+// an eighth fewer where the whole rounds are fewer too.  us at K = 2048, 320 x 192 / 256 x 256, 128 experts, N = 768: 205 / 188,
+// 203 / 195, 244 / 232 at 64 / 128 / 188 rows per expert (4 and 3 rounds), 312 / 350 and 323 / 353 at 300 and 307 (5 and 6),
+// 447 / 409 at 400 (8 and 6); 160 experts, N = 1408: 500 / 440 at 188 (10 and 7); 60 experts, N = 768: 108 / 117 at 188 (2 and
+// 2); 64 experts, N = 832, K = 2208: 211 / 253 at 304 (3 and 4).  Over 1416 shapes and routings (8 to 160 experts, N 256 to
+// 1536, K 512 to 4096, 49 to 511 rows per expert, Zipf 0 to 1.2) this is 1.9 % off the faster of the two on average (0.5 % where
+// routing is even), 320 x 192 alone 6.5 %, 256 x 256 alone 2.4 %, whole rounds of an expert 1.5 standard deviations above the
+// average, as before, 2.2 % (0.9 %).  Where it is off most: square tiles taken at 3 against 3.75 rounds (96 experts, N = 960, 60
+// rows: 59 against 52), and not taken around 300 rows where routing is skewed (64 experts, N = 448, Zipf 1.2: 93 against 68;
+// even: 68 against 61).  (From 512 to 640 rows the tall ones are up to 6 % ahead when routing is even, and behind when not.)
 bool square_gated_tiles(int64_t R, int N, int E) {
     if (R >= (int64_t)512 * E) return true;
-    const double mean = (double)R / E;
-    const int rows = (int)(mean + 1.5 * std::sqrt(mean)), cus = device_info().cu_count;
-    auto rounds = [&](int bm, int cols) { return ((int64_t)E * ceil_div(rows, bm) * ceil_div(N, cols) + cus - 1) / cus; };
-    return rounds(256, 128) < rounds(320, 96);
+    const double square = expected_rounds(R, N, E, 256, 128), tall = expected_rounds(R, N, E, 320, 96);
+    // (a round that a fiftieth of a tile a CU spills into is not counted)
+    const bool fewer = std::ceil(square - 0.02) < std::ceil(tall - 0.02);
+    return square + 0.5 < (fewer ? 0.88 : 0.8) * (tall + 0.5);
 }
 
 int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, int ms_i64, void *c, int64_t R, int N,
