@@ -251,9 +251,10 @@ from qwen3_moe_fused.grouped_gemm.forward_transposed import grouped_gemm_forward
 from qwen3_moe_fused.grouped_gemm.fused import grouped_gemm_forward_transposed_dual  # noqa: E402
 
 
-# dx (R, N) = dy1 (R, K) @ w1[e] + dy2 (R, K) @ w2[e], w (E, K, N)
+# dx (R, N) = dy1 (R, K) @ w1[e] + dy2 (R, K) @ w2[e], w (E, K, N); launches of few tiles (those of the large ones:
+# test_gpu_tiles.py, for this and the other fused products)
 @pytest.mark.parametrize("R,N,K,E", [(2048, 2048, 768, 8), (700, 200, 64, 5), (300, 72, 128, 3), (33, 8, 192, 40),
-                                     (5000, 392, 64, 2), (1000, 1024, 128, 8),   # 192 x 256 tiles
+                                     (5000, 392, 64, 2), (1000, 1024, 128, 8),
                                      (64, 24, 72, 4)])   # the last: K % 64 != 0, two plain products
 def test_two_term_input_gradient(R, N, K, E):
     g = gen(R + N)
@@ -285,7 +286,7 @@ from qwen3_moe_fused.kernels.silu_mul import silu_mul_backward  # noqa: E402
 # (N % 8 != 0; fp32) and run as two launches.
 @pytest.mark.parametrize("R,N,K,E,dtype", [(3000, 768, 2048, 8, torch.bfloat16), (700, 200, 64, 5, torch.bfloat16),
                                            (33, 8, 192, 40, torch.bfloat16), (5000, 392, 128, 2, torch.bfloat16),
-                                           (9000, 768, 256, 4, torch.bfloat16),   # 256 x 256 tiles
+                                           (9000, 768, 256, 4, torch.bfloat16),   # 160 x 128 tiles
                                            (64, 20, 72, 4, torch.bfloat16), (50, 24, 64, 3, torch.float32)])
 def test_input_gradient_with_silu_mul_backward_in_the_epilogue(R, N, K, E, dtype):
     gn = gen(R + N)
@@ -335,8 +336,8 @@ from qwen3_moe_fused.grouped_gemm.fused import (grouped_gemm_forward_lora,  # no
 
 # R, N, K, E, rank.  The rank-r term of a LoRA adapter in the reduction of the base product
 # (qwen3_moe_fused/lora.py:134): y = x w^T + xt wt^T.
-LORA_CASES = [(4096, 768, 2048, 16, 16),     # the 320 x 192 tiles of the expert shapes
-              (9000, 512, 256, 4, 32),       # more than 512 rows per expert: 256 x 256 tiles
+LORA_CASES = [(4096, 768, 2048, 16, 16),     # the expert shapes, 16 experts of them
+              (9000, 512, 256, 4, 32),       # more than 512 rows per expert
               (700, 200, 64, 5, 8),
               (300, 72, 128, 3, 24),         # rank not a multiple of 16
               (600, 136, 192, 6, 72),        # rank beyond one reduction step
@@ -512,8 +513,9 @@ def test_glu_with_lora_terms_equals_the_separate_products(R, N, K, E, r):
         assert torch.equal(h, silu_mul_forward(e, gg))
 
 
-# few experts or narrow outputs: 64 x 128 tiles, and 160 x 128 where those are too many to be resident at once (the
-# last three); borders of tiles and row blocks, experts without rows, columns that end inside a tile, odd numbers of steps
+# few experts or narrow outputs: 64 x 128 tiles, and 160 x 128 where those are too many to be resident at once (the fifth
+# and sixth, whose gated products have enough 256 x 256 tiles, and the gated product of the last); borders of tiles and row
+# blocks, experts without rows, columns that end inside a tile, odd numbers of steps
 @pytest.mark.parametrize("m_sizes,N,K", [([64, 65, 0, 63], 136, 64), ([0, 200, 50], 320, 192), ([49], 128, 320),
                                          ([321, 0], 256, 128), ([3900, 161], 1936, 64), ([2900, 1100, 7], 1920, 128),
                                          ([160, 159, 161, 0, 320] * 3, 760, 64)])

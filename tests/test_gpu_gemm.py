@@ -301,11 +301,11 @@ def test_dw_four_wave_kernel_matches_oracle(N, K, sizes, ms_dtype):
     assert torch.equal(grouped_gemm_backward_dw(xd, dyd, msd, torch.bfloat16), dw), "same bits from run to run"
 
 
-# the same kernel in the row-grouped products (forward and input gradient with more than 64 output columns, from 48
-# rows per expert on average): tiles of 320 x 192 up to 512 rows per expert, so N = 200, 520 and 2048 end in a partial
-# column tile; experts of 0, 1, 319, 320, 321 and 700 rows (no tile, one block, a full tile, a tile and one row,
-# several tiles); a reduction longer than the output is wide; 256 x 256 tiles from 512 rows per expert on (N = 520:
-# two tiles and eight columns).
+# The row-grouped products of the sizes that kernel takes (forward and input gradient with more than 64 output columns,
+# from 48 rows per expert on average), where its tiles are enough to occupy more than half of the CUs: 16 experts of 2048
+# columns and 70 experts here.  The others have too few large tiles and run on 64 x 128 or 160 x 128 ones; the borders of the
+# large tiles are in test_gpu_tiles.py.  N = 200 and 520 end in a partial column tile; experts of 0, 1, 319, 320, 321 and 700
+# rows; a reduction longer than the output is wide; 512 rows per expert and more.
 WIDE_ROW_CASES = [
     # N, K, m_sizes
     (200, 64, [300, 0, 1, 319, 320, 321, 700, 95]),
@@ -315,12 +315,12 @@ WIDE_ROW_CASES = [
     (768, 2048, [48, 60, 0, 130, 50, 49]),
     (520, 128, [1000, 0, 700]),
     (768, 256, [513, 2047, 256, 1300]),
-    # 192 x 256 tiles (outputs a multiple of 256 columns and at least 1024 wide, at most 152 rows per expert on
-    # average): experts of 0, 1, 191, 192 and 193 rows, one of two tiles, a reduction of one step
+    # outputs a multiple of 256 columns and at least 1024 wide, at most 152 rows per expert on average (the first: 192 x 256
+    # tiles of the four-wave kernel): experts of 0, 1, 191, 192 and 193 rows, a reduction of one step
     (2048, 768, [100 + 13 * (e % 7) for e in range(16)]),
     (1024, 128, [0, 193, 60, 192, 1, 150, 191, 120]),
     (1280, 64, [64] * 3 + [400, 48, 0, 97, 129]),
-    # the same widths between 152 and 232 rows per expert: 256 x 256 tiles (experts of 255, 256, 257 and 520 rows)
+    # the same widths between 152 and 232 rows per expert (experts of 255, 256, 257 and 520 rows)
     (1024, 192, [255, 256, 257, 0, 190, 520, 100, 180]),
 ]
 

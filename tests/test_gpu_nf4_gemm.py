@@ -28,10 +28,10 @@ def _quantised(E, N, K, blocksize, seed):
 
 @pytest.mark.parametrize("R,N,K,E,blocksize", [(1024, 768, 2048, 128, 256), (1024, 768, 2048, 128, 64),
                                                (128, 768, 2048, 128, 64), (300, 40, 72, 5, 8), (513, 136, 64, 3, 64),
-                                               # >= 32 rows per expert: the pipelined kernel, several row tiles
+                                               # many rows per expert: the pipelined kernel, several row tiles
                                                # per expert and many reduction steps
                                                (8192, 768, 2048, 16, 64), (4096, 200, 512, 4, 128),
-                                               # an output of 1024 columns at 200 rows per expert: 256 x 256 tiles
+                                               # an output of 1024 columns at 200 rows per expert
                                                (1600, 1024, 128, 8, 64),
                                                # small quantisation blocks on the pipelined kernel
                                                (2048, 64, 128, 2, 16), (1500, 72, 192, 3, 8),
@@ -306,7 +306,7 @@ from qwen3_moe_fused.grouped_gemm.forward_transposed import grouped_gemm_forward
 @pytest.mark.parametrize("R,N,K,E,blocksize", [(1024, 2048, 768, 128, 64), (4096, 768, 2048, 16, 64),
                                                (300, 64, 64, 5, 8), (513, 160, 128, 3, 32), (2000, 96, 192, 2, 16),
                                                (40, 32, 64, 7, 128), (5000, 416, 128, 3, 256),
-                                               (1600, 1024, 128, 8, 64)])   # 256 x 256 tiles at 200 rows per expert
+                                               (1600, 1024, 128, 8, 64)])
 def test_fused_nf4_input_gradient(R, N, K, E, blocksize):
     packed, state, w_deq = _quantised(E, K, N, blocksize, R + N)
     g = gen(R + 1)
