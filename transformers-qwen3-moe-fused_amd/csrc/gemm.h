@@ -42,14 +42,15 @@ inline int64_t expected_tiles(int64_t R, int N, int E, int BM, int BN) {
     return (row_tiles > E ? row_tiles : E) * ceil_div(N, BN);
 }
 
-// A row-grouped bf16 product (two: the gated unit's, half as many columns of each matrix in a tile) whose large tiles would
-// leave at least half of the CUs without one: with few experts, or narrow outputs, a launch then takes as long as one such
-// tile.  It runs on 64 x 128 tiles, or 160 x 128 where those are not all resident at once, two workgroups a CU either way
-// (the rule is in gemm_bf16_pipe.hip).  us at N x K = 768 x 2048 (8 experts of 64 / 128 / 256 / 512 rows, large tiles in brackets): forward 17 /
-// 19 / 20 / 33 (26 / 38 / 46 / 49), input gradient 11 / 16 / 17 / 26 (18 / 21 / 24 / 27; of two terms 18 / 27 / 29 / 41
-// against 33 / 36 / 39 / 43), gated 21 / 21 / 32 / 44 (37 / 40 / 51 / 57).  Where the large tiles occupy more than half of
-// the CUs they are ahead: 16 experts of 128 rows, 192 tiles: input gradient 28 against 34; 8 experts of 512 rows, 144 tiles:
-// 40 against 54.  The sums are the same bits on all of them.
+// A row-grouped bf16 product (gated: the two of the gated unit, half as many columns of each matrix in a tile) whose large
+// tiles would leave at least half of the CUs without one: with few experts, or narrow outputs, a launch then takes as long as
+// one such tile.  It runs on 64 x 128 tiles, or 160 x 128 where those are not all resident at once, two workgroups a CU either
+// way (the rule is in gemm_bf16_pipe.hip).  us, 8 experts of 64 / 128 / 256 / 512 rows, large tiles in brackets: forward, N =
+// 768, K = 2048, 19 / 19 / 20 / 33 (34 / 38 / 46 / 48), gated 21 / 22 / 34 / 49 (36 / 40 / 52 / 60); input gradient, N = 2048,
+// K = 768, 11 / 16 / 17 (19 / 22 / 25), of two terms 18 / 27 / 28 (33 / 36 / 39; at 512 rows 160 large tiles, which stay).
+// Past that line the 64 x 128 tiles are behind (input gradient, N = 2048, 16 experts of 128 rows, 144 large tiles: 25 against 24;
+// 8 of 512, 160 tiles: 34 against 27), the 160 x 128 ones ahead or behind by what the last round holds (the same two: 20 and
+// 25; 8 of 640, 192 tiles: 36 against 26; 60 of 128, 480 tiles: 51 against 50).  The sums are the same bits on all of them.
 inline bool few_large_tiles(int64_t R, int N, int E, bool gated) {
     int bm = 320, bn = 192;
     if (R >= (int64_t)512 * E)

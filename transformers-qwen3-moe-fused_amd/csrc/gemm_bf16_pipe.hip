@@ -83,22 +83,23 @@ struct FwdFusion {
     void *bw_de, *bw_dg, *bw_h;
 };
 
-// FUSE: 0 plain, 1 two weight matrices and the silu(gate) * up epilogue, 2 a thin last term in the reduction (built
-// as a kernel of its own: the test for it in every step cost the plain products 3-5 %), 3 both: each of the two
-// matrices with thin weights of its own, against one thin left operand; 4 the input gradient with the gated unit's
-// backward in its epilogue (a kernel of its own: its epilogue holds pieces of e and g in registers beside the
-// accumulators, which the plain input gradient has no room for).
-// Waves a SIMD has to hold: the workgroup's, and of two workgroups where two fit a CU's LDS (left to itself the compiler
-// gives a workgroup of four waves registers for itself alone: 267 in the packed 160 x 128 tile, one workgroup a CU).
 constexpr int lds_bytes(int MB, int NB, int BK, int S) {
     // stages | two NF4 code tables | three per-expert prefix tables
     return S * (MB + NB) * 32 * BK * 2 + 128 + 3 * (kMaxTableExperts + 1) * 4;
 }
 constexpr int workgroups_per_cu(int MB, int NB, int BK, int S) { return lds_bytes(MB, NB, BK, S) <= 80 * 1024 ? 2 : 1; }
+// Waves that a SIMD has to hold, asked of the compiler for workgroups of four waves only: left to itself it gives one registers
+// for itself alone (267 in the packed 160 x 128 tile, one workgroup a CU).  Eight waves are two a SIMD whatever is asked, and
+// the flat tiles, of which two workgroups fit, stay far below the 128 registers that four waves a SIMD leave (95).
 constexpr int min_waves(int MB, int NB, int BK, int S, int waves) {
     return waves == 4 ? workgroups_per_cu(MB, NB, BK, S) : 1;
 }
 
+// FUSE: 0 plain, 1 two weight matrices and the silu(gate) * up epilogue, 2 a thin last term in the reduction (built
+// as a kernel of its own: the test for it in every step cost the plain products 3-5 %), 3 both: each of the two
+// matrices with thin weights of its own, against one thin left operand; 4 the input gradient with the gated unit's
+// backward in its epilogue (a kernel of its own: its epilogue holds pieces of e and g in registers beside the
+// accumulators, which the plain input gradient has no room for).
 template <int MB, int NB, int BK, int S, int WGM, int WGN, int MODE, bool NF4, int FUSE, typename TO>
 __global__ __launch_bounds__(WGM *WGN * 64, min_waves(MB, NB, BK, S, WGM *WGN)) void gemm_pipe_kernel(const bf16_t *__restrict__ a,
                                                                   const bf16_t *__restrict__ b,
@@ -1150,16 +1151,22 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
         else {
             // packed weights with an output of 1024 columns and more that is a multiple of 256 wide, up to 232 rows per
             // expert: 256 x 256 tiles as well (8 column slices an expert instead of 11 of 192 columns)
-            const bool nf4_wide = nf4 != nullptr && N % 256 == 0 && N >= 1024 && R <= (int64_t)232 * E;
+            const bool nf4_wide = nf4 != nullptr && N % 256 == 0 && N >= 1024 && R <= (int64_t)kWideMidRowsPerExpert * E;
             // packed weights, up to 128 rows per expert on average (few experts then hold more than 160), or as long as the
             // smaller tiles are all resident at once (512 on 256 CUs): 160 x 128 tiles of four waves, two workgroups a CU.
             // A step with packed weights is a chain (copies land, codes are looked up, stage written, barrier) that one
             // workgroup a CU leaves the chip waiting on; two run theirs side by side.  us, 128 experts, N x K of the
             // weights, against the tiles below, with the thin last term, forward 768 x 2048: 83 / 87 / 98 against 108 /
-            // 96 / 105 at 48 / 96 / 128 rows per expert (142 against 113 at 160), 2048 x 768: 106 against 115 at 128;
-            // input gradient 96 against 109 and 91 against 95 at 128.  Skewed routing (Zipf 1.2) at 64 rows per expert
-            // 101 against 165 and 97 against 112.  8 experts of 512 rows 46 against 68, of 1024 rows 61 against 69; 16
-            // experts of 1024 rows (708 tiles) 102 against 75.  The sums are the same bits.
+            // 96 / 105 at 48 / 96 / 128 rows per expert, 2048 x 768: 106 against 115 at 128; input gradient 96 against 109
+            // and 91 against 95 at 128.  8 experts of 512 rows 46 against 68, of 1024 rows 61 against 69; 16 experts of
+            // 1024 rows (708 tiles) 102 against 75.  Past 128 rows, not resident: 0.90 of the time below up to 144 rows on
+            // average over shapes (0.69 to 1.16), 1.03 to 160, 1.28 at 193 to 200 (142 against 113 at 160 with 768 columns).
+            // What a routing costs is the row tiles that it makes, which the host does not know.  Where 160 x 128 has a third
+            // more columns a CU than one round of 320 x 192 (48 to 64 experts of 768 columns, 96 to 128 rows), it is behind
+            // if routing is even (50 against 57 at 60 experts of 128 rows) and far ahead if it is skewed (Zipf 0.4 to 1.2:
+            // 0.5 to 0.9 of the time); against one full round of 256 x 256, ahead but for light skew (Zipf 0.4: 28 against
+            // 22 at 60 experts, N = 1024).  The mean over routings is ahead for every number of rounds.  The sums are the
+            // same bits.
             const bool nf4_pair = nf4 != nullptr && (R <= (int64_t)128 * E ||
                                                      (R / 160 + E) * (int64_t)ceil_div(N, 128) <= 2 * device_info().cu_count);
             cfg = (N <= 64 && nf4 == nullptr) ? 10
@@ -1170,14 +1177,16 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
         }
     }
     switch (cfg) {
+#ifdef MFL_TUNING_BUILD
         case 1:
             return MFL_LAUNCH(4, 4, 64, 4, 2, 2, 7);
         case 2:
             return MFL_LAUNCH(8, 4, 64, 3, 4, 2, 7);
-        case 3:
-            return MFL_LAUNCH(10, 6, 64, 2, 4, 2, 31);
         case 4:
             return MFL_LAUNCH(10, 4, 64, 2, 4, 2, 7);
+#endif
+        case 3:
+            return MFL_LAUNCH(10, 6, 64, 2, 4, 2, 27);
         case 5:  // 160 x 128 tiles, two stages of 36 KiB, two workgroups of four waves a CU
             return MFL_LAUNCH(5, 4, 64, 2, 2, 2, 27);
         case 15:  // a few rows per expert (decode): the weights are all the traffic; flat 64 x 128 tiles,
