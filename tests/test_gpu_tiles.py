@@ -134,6 +134,29 @@ def test_products_with_a_thin_term(shape):
     check_close(dx, c.xw + c.ub, 1e-4, 1e-4, "input gradient, float32 result")
 
 
+# Parts of 96 columns: a wave's store starts in the middle of a row (store 1 in row 5 at column 32, 2 in row 10 at 64, 4 in
+# row 21 at 32, 5 in row 26 at 64).  Experts that end in just these rows, with 32 columns left to either wave, have stores
+# without a lane; one that was counted all the same let the next tile's second step be read before it had landed.
+@pytest.mark.parametrize("N", [224, 320])
+def test_last_rows_in_which_a_store_has_no_lane(N):
+    m_sizes = [54, 59, 38, 43, 70, 75, 22, 27, 86, 11, 6, 102] * 16
+    c = Case(m_sizes, N, 384)
+    tile = ("wide", 320, 192)
+    products = {
+        "forward": (lambda: grouped_gemm_forward(c.x, c.w, c.ms), c.xw, FWD, 0),
+        "input gradient": (lambda: grouped_gemm_forward_transposed(c.x, c.wt, c.ms), c.xw, DX, 0),
+        "forward, thin term": (lambda: grouped_gemm_forward_lora(c.x, c.w, c.u, c.b, c.ms), c.xw + c.ub, FWD, 2),
+        "input gradient, two terms and the thin one":
+            (lambda: grouped_gemm_forward_transposed_lora(c.x, c.wt, c.u, c.bt, c.ms, dy2=c.x2, w2=c.w2t),
+             c.xw + c.x2w2 + c.ub, DX, 2),
+    }
+    for what, (product, expect, mode, fusion) in products.items():
+        y = check_tiles(product, (*tile, mode, False, fusion))
+        check_close(y, expect, what=what)
+        for _ in range(20):
+            assert torch.equal(product(), y), f"{what}: the same bits from run to run"
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_products_of_the_pipelined_kernel(shape):
     c, tile = Case(*SHAPES[shape][:3]), SHAPES[shape][5]

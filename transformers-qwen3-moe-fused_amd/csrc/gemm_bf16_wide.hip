@@ -24,6 +24,7 @@
 // Shapes: bf16 in, bf16 out, no accumulation, no scaling; E <= 512; FWD/DX: N % 8 == 0, K % 64 == 0; DW: N % BM == 0,
 // K % BN == 0 (any number of rows per expert).  The caller falls back to gemm_bf16_pipe.hip otherwise.
 #include "pipe_parts.h"
+#include "store_lanes.h"
 
 namespace mfl {
 
@@ -851,9 +852,10 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
             const uint64_t c_part = c_tile + ((int64_t)t * (WGM * 32) * ldc + part * EPC) * 2;
 #pragma unroll
             for (int u = 0; u < NST; ++u) {
-                // a store whose rows all lie past the tile's last one, or whose columns all lie past N, is left
-                // out, and not counted
-                if (MODE != MODE_DW && (row_base + u * 64 / CPR >= ct.i_end || col0 >= N)) continue;
+                // a store without a lane inside the tile's rows and N's columns is left out (the branch around the
+                // statement below jumps over it), and must not be counted: a count too high makes the next wait
+                // one for a copy fewer than it needs
+                if (MODE != MODE_DW && !store_has_lane(u, CPR, ct.i_end - row_base, N - col0)) continue;
                 if (kNoStore) continue;
 #if defined(MFL_TUNING_BUILD) && defined(MFL_X_HALF_STORE)
                 if (p >= NP / 2) continue;
