@@ -1153,7 +1153,8 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
             // expert: 256 x 256 tiles as well (8 column slices an expert instead of 11 of 192 columns)
             const bool nf4_wide = nf4 != nullptr && N % 256 == 0 && N >= 1024 && R <= (int64_t)kWideMidRowsPerExpert * E;
             // packed weights, up to 128 rows per expert on average (few experts then hold more than 160), or as long as the
-            // smaller tiles are all resident at once (512 on 256 CUs): 160 x 128 tiles of four waves, two workgroups a CU.
+            // smaller tiles are all resident at once (512 on 256 CUs; R / 160 + E row tiles are the most that any routing
+            // makes, expected_tiles() counts those of an average one): 160 x 128 tiles of four waves, two workgroups a CU.
             // A step with packed weights is a chain (copies land, codes are looked up, stage written, barrier) that one
             // workgroup a CU leaves the chip waiting on; two run theirs side by side.  us, 128 experts, N x K of the
             // weights, against the tiles below, with the thin last term, forward 768 x 2048: 83 / 87 / 98 against 108 /
