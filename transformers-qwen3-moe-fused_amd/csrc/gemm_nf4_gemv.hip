@@ -102,6 +102,7 @@ constexpr int kGemvThreads = 1024;
 constexpr int kGemvTable = 65536;
 constexpr int kGemvScales = 2048;  // scales by 8-bit value, of either matrix (double-quantised matrices)
 
+__device__ __forceinline__ uint16_t bf16_bits(float v) { return __builtin_bit_cast(uint16_t, (bf16_t)v); }
 
 // The LDS address of the pair of packed byte `B` of w: 256 * byte + lane_copy (the lane's copy of the table, one
 // byte), put together by one byte permute.
@@ -134,38 +135,21 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
     int *const grp_e = (int *)(smem + kGemvTable + (NESTED ? kGemvScales : 0));          // expert | rows << 16
     int *const grp_r = grp_e + max_groups;                  // first row
     int *const n_groups_s = grp_r + max_groups;
-    int *const ms_s = n_groups_s + 1;                       // the E counts
+    uint16_t *const code_s = (uint16_t *)(n_groups_s + 1);  // the code values of either matrix as bf16
+    int *const ms_s = n_groups_s + 17;                      // the E counts
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     // the lookups address the table from LDS address 0: the kernel has no static LDS in front of the dynamic
     // (the launcher asks the runtime and does not launch a build that has)
-    // the counts, asked for first: their latency runs under the filling of the table
+    // the counts and the codes: one round trip
     int ms_own[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int e = tid + j * kGemvThreads;
         ms_own[j] = e < E ? load_msize(m_sizes, ms_i64, e) : 0;
     }
-    // ---- pair table: entry b = bf16(code[b >> 4]) in the low half (the first of the two weights is the high
-    // nibble), bf16(code[b & 15]) in the high half.  Entry b is the 256 bytes at 256 b: 32 copies for the first
-    // matrix, 32 for the second; thread t writes 64 of the bytes of entry t & 255.
-    {
-        const int b = tid & 255, part = tid >> 8;
-        if (part < 2 * CB) {
-            const float *const code = part < 2 ? w0.code16 : w1.code16;
-            union {
-                bf16_t e[2];
-                uint32_t u;
-            } pr;
-            pr.e[0] = (bf16_t)code[b >> 4];
-            pr.e[1] = (bf16_t)code[b & 15];
-            const uint4_t v = {pr.u, pr.u, pr.u, pr.u};
-            uint4_t *const dst = (uint4_t *)(table + b * 256 + part * 64);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) dst[j] = v;
-        }
-    }
+    if (tid < 16 * CB) code_s[tid] = bf16_bits((tid < 16 ? w0 : w1).code16[tid & 15]);
     if constexpr (NESTED)
         if (tid < 256 * CB) ((float *)(table + kGemvTable))[tid] = (tid < 256 ? w0 : w1).code256[tid & 255];
 #pragma unroll
@@ -196,6 +180,19 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
             grp_carry += wave_last(ginc);
         }
         if (lane == 0) *n_groups_s = grp_carry < max_groups ? grp_carry : max_groups;
+    } else {
+        // ---- pair table, filled by the other waves meanwhile: entry b = bf16(code[b >> 4]) in the low half (the first of
+        // the two weights is the high nibble), bf16(code[b & 15]) in the high half.  Entry b is the 256 bytes at 256 b: 32
+        // copies for the first matrix, 32 for the second.  Neighbouring threads write neighbouring 16 bytes: written 64
+        // bytes of an entry to a thread, the 64 lanes of a store met in the same four banks (3600 cycles of conflicts a CU,
+        // 1.7 us of the gated form's 14 at one token).
+        for (int p = tid - 64; p < 256 * 8 * CB; p += kGemvThreads - 64) {
+            const int b = p / (8 * CB), piece = p % (8 * CB);
+            const uint16_t *const code = code_s + (piece >> 3) * 16;
+            const uint32_t u = code[b >> 4] | (uint32_t)code[b & 15] << 16;
+            const uint4_t v = {u, u, u, u};
+            *(uint4_t *)(table + b * 256 + piece * 16) = v;
+        }
     }
     __syncthreads();
 
@@ -450,7 +447,7 @@ int launch_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf4M
                 const void *m_sizes, int ms_i64, TO *y, TO *e_out, TO *g_out, int64_t R, int N, int K, int E,
                 hipStream_t stream) {
     const int64_t max_groups = R / ROWS + (R < E ? R : E);  // upper bound on sum over experts of ceil(m / ROWS)
-    const int lds = kGemvTable + kGemvScales + (int)max_groups * 8 + 16 + E * 4;
+    const int lds = kGemvTable + kGemvScales + (int)max_groups * 8 + 80 + E * 4;
     auto *kernel = nf4_gemv_kernel<NL, ROWS, D, GLU, EXACT, HALF, NESTED, TO>;
     static PerDeviceOnce attr;
     // The table lookups take the dynamic LDS to start at address 0; static LDS in this kernel would move it, so
@@ -461,7 +458,7 @@ int launch_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf4M
         const hipError_t e1 = hipFuncGetAttributes(&fa, (const void *)kernel);
         if (e1 != hipSuccess) return e1;
         static_lds.store((int)fa.sharedSizeBytes, std::memory_order_release);
-        return hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kGemvTable + kGemvScales + 4096 * 8 + 16 + 2048 * 4);
+        return hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kGemvTable + kGemvScales + 4096 * 8 + 80 + 2048 * 4);
     });
     if (e != hipSuccess) return (int)e;
     if (static_lds.load(std::memory_order_acquire) != 0) return MFL_ERR_UNSUPPORTED;
