@@ -259,11 +259,18 @@ def test_tile_ordered_scales_shapes_without_a_copy():
     ([1, 2, 0, 1, 3, 0, 0, 1], 768, 2048, 64, torch.int64, torch.bfloat16),
     ([1, 1], 32, 1088, 64, torch.int32, torch.bfloat16),
     ([0, 0, 0, 4], 64, 1032, 8, torch.int32, torch.float32),
+    ([1, 0, 2, 0], 96, 1248, 32, torch.int32, torch.bfloat16),
     # 32 lanes to a column (K <= 1024, at most a row per expert on average) from here on
     ([1, 2, 0, 1, 0, 0, 0, 1], 2048, 768, 64, torch.int32, torch.bfloat16),
     ([2, 0, 0], 32, 1024, 128, torch.int64, torch.float32),
     ([1, 0, 1, 0, 0, 0, 3], 96, 264, 8, torch.int32, torch.bfloat16),
     ([0] * 66 + [1, 2], 64, 520, 8, torch.int32, torch.bfloat16),
+    ([1, 0, 2, 0], 96, 928, 32, torch.int32, torch.bfloat16),
+    # 16 lanes to a column: six dwords a lane, four, and lanes past the end of a row of either
+    ([2, 0, 1, 0, 0], 64, 768, 64, torch.int32, torch.float32),
+    ([1, 0, 0, 2, 0], 192, 576, 64, torch.int64, torch.bfloat16),
+    ([1, 1, 0], 128, 512, 32, torch.int32, torch.bfloat16),
+    ([3, 0, 0, 0], 64, 320, 64, torch.int32, torch.float32),
 ])
 def test_matrix_vector_decode_kernel_edges(m_sizes, N, K, blocksize, ms_dtype, out_dtype):
     E = len(m_sizes)

@@ -45,6 +45,9 @@ CASES = [
     ([1, 0, 1, 0, 0], 96, 768, 64),
     ([2, 1, 0, 2], 32, 1536, 64),
     ([1, 1, 0], 32, 1024, 128),
+    ([1, 0, 2, 1], 64, 768, 64),
+    ([1, 0, 1], 128, 576, 64),
+    ([2, 0, 1, 0], 64, 320, 64),
     ([5, 0, 3, 17], 200, 768, 64),
     ([40, 1, 33], 128, 384, 64),
     ([70, 0, 12], 72, 2048, 64),

@@ -3,11 +3,12 @@
 // With one or two rows per expert there is nothing for a matrix core to share: a 32-row MFMA tile would
 // be 3 to 6 % full, and what the launch has to do is pull every routed expert's packed weights through
 // the chip once.  So no tile and no LDS stage:
-//   * a wave owns two output columns at a time, 16 apart (one in the gated form, where the second matrix takes
-//     the registers).  Its 64 lanes lie along the reduction: load i of a column gives lane l the dword of 8
-//     packed weights k = (64 i + l) * 8 .., i.e. a wave reads 256 consecutive bytes per load and a column of
-//     K = 2048 in four.  The scale of those 8 weights is one float (blocks
-//     of at least 8 weights, K a multiple of the block size).
+//   * a wave owns two output columns at a time, 16 apart (one of both matrices in the gated form, where the second matrix
+//     takes the registers).  Its 64 lanes lie along the reduction, 32 weights in a row to a lane: one load of 16 bytes a
+//     lane takes a column of K = 2048, and the lane's weights lie under one scale.  (With the lanes' dwords 64 dwords
+//     apart a column took four loads of weights and four of scales, eight of 8-bit ones, which spilled: 16 tokens of 8
+//     experts out of 128, gated, N = 768, fp32 / 8-bit scales 40.8 / 51.2 -> 36.8 / 37.3 us; one token 8.2 / 12.0 -> 8.5 /
+//     9.2.  Rows that are no multiple of 32 elements still take that form.)
 //   * the rows of the group (up to two of one expert) stay in registers for all columns of the group: 16
 //     bytes per lane, load and row.
 //   * a byte of packed weights is two weights and one dword of bf16 pairs: a 256-entry table in LDS holds
@@ -16,19 +17,19 @@
 //     lookups of a wave meet no bank conflict, and the address 256 * byte + 4 * copy is ONE byte permute.
 //     One vector instruction per byte for the address, one per byte and row for the product; the scale goes
 //     onto the partial sum of the 8 weights in fp32.
-//   * the 64 partial sums of each of the two columns become 32 + 32 in one swap of half waves
-//     (v_permlane32_swap) and an add, and five data-parallel-primitive adds finish both at once; lanes 31 and
-//     63 store.
+//   * the 64 partial sums of each of the two columns (or of the two matrices' column) become 32 + 32 in one swap of half
+//     waves (v_permlane32_swap) and an add, and five data-parallel-primitive adds finish both at once.
 //   * one workgroup of 16 waves per CU, as many workgroups as CUs, and the (row group, 32 columns) units of
 //     the launch (16 columns in the gated form) dealt out in equal contiguous shares: no second round of
 //     workgroups, and a workgroup changes rows once or twice.  Each wave keeps the loads of four columns ahead
 //     in registers.
-//   * rows of at most 1024 elements: 32 lanes to a column, the wave's second column (16 further on) in lanes
-//     32..63, loads of 128 bytes per half wave, no swap before the five adds.
+//   * rows of at most 1024 elements: 32 lanes to a column, the wave's second column (16 further on) in lanes 32..63; up to
+//     512, and for 576 and 768: 16 lanes and four columns, four or six dwords to a lane.  No swap before the adds.
 //   What the loop is short of, with 16 waves to a CU, is issue slots, scalar ones first: addresses move by
 //   increments, the row count is branched on once per column, and the lookups of a dword wait once.
 //
-// The product is sum over 8-weight pieces of absmax * (x . bf16(code)), as in the streaming form.
+// The product is the sum over pieces of 32 weights (16 of six dwords a lane, 8 where the dwords lie apart or the blocks are
+// smaller) of absmax * (x . bf16(code)), as in the streaming form.
 #include <mutex>
 #include <type_traits>
 
@@ -65,13 +66,14 @@ __device__ __forceinline__ float two_sums_to_31_and_63(float a, float b) {
     return x;
 }
 
-// lanes 0..31 hold the partial sums of one column, lanes 32..63 of another: the sums in lanes 31 and 63
-__device__ __forceinline__ float half_sums_to_31_and_63(float x) {
+// each run of CL lanes (16 or 32) holds the partial sums of a column: the sums in the last lanes of the runs
+template <int CL>
+__device__ __forceinline__ float sums_to_last_lanes(float x) {
     x = dpp_fadd_step<0x111, 0xf>(x);  // row_shr 1
     x = dpp_fadd_step<0x112, 0xf>(x);  // row_shr 2
     x = dpp_fadd_step<0x114, 0xf>(x);  // row_shr 4
     x = dpp_fadd_step<0x118, 0xf>(x);  // row_shr 8
-    x = dpp_fadd_step<0x142, 0xa>(x);  // row_bcast 15 into rows 1 and 3
+    if constexpr (CL == 32) x = dpp_fadd_step<0x142, 0xa>(x);  // row_bcast 15 into rows 1 and 3
     return x;
 }
 
@@ -112,8 +114,9 @@ __device__ __forceinline__ uint32_t pair_address(uint32_t w, uint32_t lane_copy)
     return __builtin_amdgcn_perm(w, lane_copy, 0x0c0c0000u | ((4u + B) << 8));
 }
 
-// NL: loads per column (K <= 512 NL); ROWS: rows per group; D: columns whose loads a wave keeps in flight
-template <int NL, int ROWS, int D, bool GLU, bool EXACT, bool HALF, bool NESTED, typename TO>
+// CL: lanes per column; NL: dwords of a column per lane (K <= 8 CL NL); ROWS: rows per group; D: columns whose loads a wave
+// keeps in flight; WIDE: the dwords of a lane lie side by side (above), else CL dwords apart
+template <int CL, int NL, int ROWS, int D, bool GLU, bool WIDE, bool NESTED, typename TO>
 __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__restrict__ x,
                                                                 const int32_t *__restrict__ row_idx, int idx_div,
                                                                 Nf4Matrix w0, Nf4Matrix w1,
@@ -122,13 +125,19 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
                                                                 TO *__restrict__ g_out, int64_t R, int N, int K,
                                                                 int E, int units_n, int max_groups) {
     constexpr int CB = GLU ? 2 : 1;
-    // Columns per wave and unit: two, 16 apart, for the plain product (the loop's scalar work and the sum over the
-    // lanes are shared by both); one for the gated form, whose second matrix leaves no registers for a second column.
-    constexpr int COLS = (GLU || HALF) ? 1 : 2;
-    // HALF (rows of at most 1024 elements): 32 lanes to a column, the wave's second column (16 further on) in its
-    // upper 32 lanes instead of in registers of its own: a load serves both, and the sums need no swap.
-    constexpr int UCOLS = HALF ? 32 : 16 * COLS;  // columns of a unit per wave-column: 16 waves x UCOLS / 16
-    static_assert(!(HALF && EXACT), "");
+    // CL < 64: the wave's other columns (16 further on each) lie in its other lanes: a load serves all of them, and the sums
+    // need no swap.
+    constexpr int SUB = 64 / CL;
+    // Columns in registers of their own: two, 16 apart, for the plain product with all 64 lanes to a column (the loop's
+    // scalar work and the sum over the lanes are shared by both); one for the gated form, whose second matrix leaves no
+    // registers for a second column.
+    constexpr int COLS = (GLU || SUB > 1) ? 1 : 2;
+    constexpr int UCOLS = 16 * SUB * COLS;  // columns of a unit
+    // Scales of a column per lane: the 48 weights of six dwords lie under one or two blocks of 64, two neighbouring dwords
+    // always under one; the 32 of four dwords under one.
+    constexpr bool TWO = WIDE && NL == 6;
+    static_assert(!WIDE || NL == 4 || (CL == 16 && NL == 6), "");
+    constexpr int NS = TWO ? 2 : WIDE ? 1 : NL;
     static_assert(D % CB == 0, "the matrix of a ring slot is fixed");
     extern __shared__ __attribute__((aligned(256))) unsigned char smem[];
     unsigned char *const table = smem;                      // kGemvTable bytes
@@ -205,24 +214,23 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
     if (u_begin >= u_end) return;
     const int n_items = (int)(u_end - u_begin) * CB;  // (unit, matrix) pairs, matrix minor
 
-    // ---- what a lane reads of a column: dword (64 i + lane) of its packed row, if that is inside the row
-    // EXACT (K a multiple of 512): load i is inside the row for all lanes or for none, and the lane's offsets are
-    // lane * 8 plus constants; otherwise they are kept per load, clamped to 0 where the lane is past the row.
+    // ---- what a lane reads of a column: dword i of its NL, if that is inside the row (else it reads the row's first)
     uint32_t x_off[NL];
     bool inside[NL];
     const Nf4Matrix mat[2] = {w0, w1};
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
-        const int k = HALF ? (i * 32 + (lane & 31)) * 8 : (i * 64 + lane) * 8;
-        inside[i] = EXACT ? i * 512 < K : k < K;
-        x_off[i] = EXACT ? (uint32_t)(lane * 8 + (i * 512 < K ? i * 512 : 0)) : (uint32_t)(inside[i] ? k : 0);
+        const int l = lane % CL;
+        const int k = WIDE ? l * (8 * NL) : (i * CL + l) * 8;
+        inside[i] = k < K;
+        x_off[i] = (uint32_t)(inside[i] ? k : 0) + (WIDE ? 8 * i : 0);
     }
     const uint32_t copy_off = (lane & 31) * 4;  // + 128 for the second matrix
 
     // ---- the ring of columns ahead
     uint32_t ring_w[D][COLS][NL];  // a slot: the wave's columns of a unit
-    float ring_a[D][COLS][NL];     // the scale; double-quantised: its second-level factor,
-    uint32_t ring_q[NESTED ? D : 1][COLS][NL];  // and its 8-bit value
+    float ring_a[D][COLS][NS];     // the scale; double-quantised: its second-level factor,
+    uint32_t ring_q[NESTED ? D : 1][COLS][NS];  // and its 8-bit value
     float q_off[CB];
     if constexpr (NESTED) {
         q_off[0] = *w0.offset;
@@ -260,26 +268,37 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
     for (int cb = 0; cb < CB; ++cb) a_step[cb] = (16 * K) >> mat[cb].bs_shift;
     auto issue = [&](int d) {
         const int cb = d % CB;
+        auto weights = [&](uint32_t (&to)[NL], const uint32_t *from) {
+            if constexpr (SUB > 1) from += (lane / CL) * w_step;
+            if constexpr (WIDE) {
+                typedef uint4_t __attribute__((aligned(8))) piece_t;  // (24 bytes a lane)
+                const uint4_t v = *(const piece_t *)(from + (x_off[0] >> 3));
 #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const uint32_t w_idx = (x_off[i] >> 3) + (HALF ? (lane >> 5) * w_step : 0);
-            ring_w[d][0][i] = i_wp[cb][w_idx];
-            // (computed here: a register per load and matrix less)
-            const uint32_t a_off = (x_off[i] >> mat[cb].bs_shift) + (HALF ? (lane >> 5) * a_step[cb] : 0);
-            // (E N K / 64 scales: their numbers fit 32 bits, which the launcher checks)
-            if constexpr (NESTED) {
-                ring_q[d][0][i] = i_qp[cb][a_off];
-                ring_a[d][0][i] = mat[cb].absmax2[((uint32_t)i_b[cb] + a_off) >> mat[cb].bs2_shift];
+                for (int i = 0; i < 4; ++i) to[i] = v[i];
+                if constexpr (NL == 6) {
+                    const uint2_t u = *(const uint2_t *)(from + (x_off[0] >> 3) + 4);
+                    to[4] = u[0], to[5] = u[1];
+                }
             } else {
-                ring_a[d][0][i] = i_ap[cb][a_off];
+#pragma unroll
+                for (int i = 0; i < NL; ++i) to[i] = from[x_off[i] >> 3];
             }
-            if constexpr (COLS == 2) {
-                ring_w[d][1][i] = i_wp[cb][w_step + w_idx];
+        };
+        weights(ring_w[d][0], i_wp[cb]);
+        if constexpr (COLS == 2) weights(ring_w[d][1], i_wp[cb] + w_step);
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            // (computed here: a register per load and matrix less)
+            const uint32_t a_off = (x_off[i * (TWO ? NL - 1 : 1)] >> mat[cb].bs_shift) + (SUB > 1 ? (lane / CL) * a_step[cb] : 0);
+#pragma unroll
+            for (int c = 0; c < COLS; ++c) {
+                const uint32_t at = a_off + c * a_step[cb];
+                // (E N K / 64 scales: their numbers fit 32 bits, which the launcher checks)
                 if constexpr (NESTED) {
-                    ring_q[d][1][i] = i_qp[cb][a_step[cb] + a_off];
-                    ring_a[d][1][i] = mat[cb].absmax2[((uint32_t)i_b[cb] + a_step[cb] + a_off) >> mat[cb].bs2_shift];
+                    ring_q[d][c][i] = i_qp[cb][at];
+                    ring_a[d][c][i] = mat[cb].absmax2[((uint32_t)i_b[cb] + at) >> mat[cb].bs2_shift];
                 } else {
-                    ring_a[d][1][i] = i_ap[cb][a_step[cb] + a_off];
+                    ring_a[d][c][i] = i_ap[cb][at];
                 }
             }
         }
@@ -310,10 +329,10 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
     // ---- the loop over the columns
     uint4_t xr[ROWS][NL];
     int cg = ig0, cc = ic0;  // cursor of the arithmetic
-    int rows = 0, row0 = 0, o_col = cc * UCOLS;
+    int rows = 0, row0 = 0, o_col = cc * UCOLS, ge_now = 0;
     int64_t o_row[ROWS];  // where the wave's column of unit 0 is in the output, per row of the group
     bool fresh = true;
-    float first[ROWS];  // the gate projection's sums, until the up projection's are there
+    float first[ROWS];  // the gate projection's sums (of a lane, or finished), until the up projection's are there
     // One column: the arithmetic on ring slot d, then (in the loop) the loads of the column D further on into it.
     auto column = [&](const int d, const bool more) {
             const int cb = d % CB;
@@ -321,10 +340,12 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
                 fresh = false;
                 const int ge = __builtin_amdgcn_readfirstlane(grp_e[cg]);
                 rows = ge >> 16;
+                ge_now = ge;
                 row0 = __builtin_amdgcn_readfirstlane(grp_r[cg]);
 #pragma unroll
                 for (int r = 0; r < ROWS; ++r) {
-                    o_row[r] = (int64_t)(row0 + r) * N + wave + (UCOLS == 32 ? (lane >> 5) * 16 : 0);  // lanes 32..63 end up with the second column
+                    // (CL = 64: lanes 32..63 end up with the second column)
+                    o_row[r] = (int64_t)(row0 + r) * N + wave + (SUB > 1 ? lane / CL : COLS == 2 ? lane >> 5 : 0) * 16;
                     int64_t src_row = row0 + (r < rows ? r : rows - 1);
                     if (row_idx != nullptr) src_row = (uint32_t)row_idx[src_row] / (uint32_t)idx_div;
                     const bf16_t *const xp = x + src_row * K;
@@ -344,60 +365,89 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
             // the branches below they would land in different registers per branch, and the copy that reconciles
             // them would wait for the load just issued)
             // the arithmetic of the two columns for RN rows: one branch on the number of rows per unit, none inside
-            auto arithmetic = [&](auto RN) {
+            auto arithmetic = [&](auto RN, auto FINE) {
                 constexpr int rn = decltype(RN)::value;
+                constexpr bool fine = decltype(FINE)::value;  // a lane's dwords lie under more scales than the ring holds
                 float acc[COLS][rn];
 #pragma unroll
                 for (int c = 0; c < COLS; ++c)
 #pragma unroll
                     for (int r = 0; r < rn; ++r) acc[c][r] = 0.f;
+                float scale[COLS][NS], part[COLS][rn];
+                constexpr int RUN = fine || !WIDE ? 1 : TWO ? 2 : NL;  // dwords whose products are summed before they are scaled
 #pragma unroll
                 for (int i = 0; i < NL; ++i) {
 #pragma unroll
                     for (int c = 0; c < COLS; ++c) {
                         uint32_t pr[4];
                         const uint32_t w = ring_w[d][c][i];
-                        float scale = ring_a[d][c][i];
-                        if constexpr (NESTED) {
+                        if (NESTED && !fine && i < NS) {
                             float q;
                             lookup5(pr, q, pair_address<0>(w, lane_copy), pair_address<1>(w, lane_copy),
                                     pair_address<2>(w, lane_copy), pair_address<3>(w, lane_copy),
                                     ring_q[d][c][i] * 4 + (kGemvTable + cb * 1024));
-                            scale = q * scale + q_off[cb];
+                            scale[c][i] = q * ring_a[d][c][i] + q_off[cb];
                         } else {
                             lookup4(pr, pair_address<0>(w, lane_copy), pair_address<1>(w, lane_copy),
                                     pair_address<2>(w, lane_copy), pair_address<3>(w, lane_copy));
+                            if (!fine && i < NS) scale[c][i] = ring_a[d][c][i];
+                        }
+                        float under;
+                        if constexpr (fine) {
+                            const int64_t at = ((int64_t)(ge_now & 0xffff) * N + cc * UCOLS + wave + 16 * (SUB > 1 ? lane / CL : c)) * K + x_off[i];
+                            const int64_t b = at >> mat[cb].bs_shift;
+                            if constexpr (NESTED)
+                                under = ((const float *)(table + kGemvTable))[cb * 256 + mat[cb].absmax_u8[b]] * mat[cb].absmax2[b >> mat[cb].bs2_shift] + q_off[cb];
+                            else
+                                under = mat[cb].absmax[b];
+                        } else {
+                            under = TWO && i > 1 && ((x_off[i] ^ x_off[0]) >> 6) != 0 ? scale[c][NS - 1] : scale[c][WIDE ? 0 : i];
                         }
 #pragma unroll
                         for (int r = 0; r < rn; ++r) {
-                            float s = dot2_bf16(pr[0], xr[r][i][0], 0.f);
+                            float s = dot2_bf16(pr[0], xr[r][i][0], i % RUN == 0 ? 0.f : part[c][r]);
                             s = dot2_bf16(pr[1], xr[r][i][1], s);
                             s = dot2_bf16(pr[2], xr[r][i][2], s);
                             s = dot2_bf16(pr[3], xr[r][i][3], s);
-                            acc[c][r] = __builtin_fmaf(scale, s, acc[c][r]);
+                            part[c][r] = s;
+                            if (i % RUN == RUN - 1) acc[c][r] = RUN == NL ? under * s : __builtin_fmaf(under, s, acc[c][r]);
                         }
                     }
                 }
-                // the two columns' 64 partial sums each become 32 + 32 in one swap of half waves and one add, and
-                // five data-parallel-primitive adds finish both: the first column's sum in lane 31, the second's in 63
+                // the 64 partial sums of each of two columns (the gated form: of the same column of the two matrices) become
+                // 32 + 32 in one swap of half waves and one add, and five data-parallel-primitive adds finish both: the
+                // first one's sum in lane 31, the second's in 63
                 float tot[rn];
+                if constexpr (GLU && SUB == 1) {
+                    if (cb == 0) {
+#pragma unroll
+                        for (int r = 0; r < rn; ++r) first[r] = acc[0][r];
+                        return;
+                    }
+                }
 #pragma unroll
                 for (int r = 0; r < rn; ++r) {
-                    // (one column: summed in the same order as each of two, so that the gated form's products are
-                    // bit for bit those of the plain one; its sum is in lane 31 and in lane 63)
-                    if constexpr (HALF)
-                        tot[r] = half_sums_to_31_and_63(acc[0][r]);
+                    if constexpr (SUB > 1)
+                        tot[r] = sums_to_last_lanes<CL>(acc[0][r]);
                     else
-                        tot[r] = two_sums_to_31_and_63(acc[0][r], acc[COLS - 1][r]);
+                        tot[r] = two_sums_to_31_and_63(GLU ? first[r] : acc[0][r], acc[COLS - 1][r]);
                 }
-                if (GLU && cb == 0) {
+                if constexpr (GLU && SUB > 1) {
+                    if (cb == 0) {
 #pragma unroll
-                    for (int r = 0; r < rn; ++r) first[r] = tot[r];
-                    return;
+                        for (int r = 0; r < rn; ++r) first[r] = tot[r];
+                        return;
+                    }
                 }
-                if (UCOLS == 32 ? (lane & 31) == 31 : lane == 63) {  // one lane per column
+                if constexpr (GLU && SUB == 1) {
+#pragma unroll
+                    for (int r = 0; r < rn; ++r)
+                        first[r] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, tot[r]), 31));
+                }
+                if (SUB > 1 ? lane % CL == CL - 1 : COLS == 2 ? (lane & 31) == 31 : lane == 63) {  // one lane per column
 #pragma unroll
                     for (int r = 0; r < rn; ++r) {
+                        if (fine && r >= rows) continue;
                         const int64_t o = o_row[r] + o_col;
                         if constexpr (GLU) {
                             const bf16_t pe = (bf16_t)first[r], pg = (bf16_t)tot[r];
@@ -410,14 +460,14 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
                     }
                 }
             };
-            if (rows == 1)
-                arithmetic(std::integral_constant<int, 1>());
-            else if (ROWS == 2 || rows == 2)
-                arithmetic(std::integral_constant<int, 2>());
-            else if (ROWS == 4 && rows == 3)
-                arithmetic(std::integral_constant<int, (ROWS > 2 ? 3 : 1)>());
+            static_assert(ROWS == 2, "");
+            typedef std::integral_constant<bool, false> ring_scales;
+            if (WIDE && mat[cb].bs_shift < (TWO ? 6 : 5))
+                arithmetic(std::integral_constant<int, 2>(), std::integral_constant<bool, WIDE>());
+            else if (rows == 1)
+                arithmetic(std::integral_constant<int, 1>(), ring_scales());
             else
-                arithmetic(std::integral_constant<int, ROWS>());
+                arithmetic(std::integral_constant<int, 2>(), ring_scales());
             if (more) issue(d);
             if (cb == CB - 1) {
                 o_col += UCOLS;
@@ -442,13 +492,13 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
         if (d < rest) column(d, false);
 }
 
-template <int NL, int ROWS, int D, bool GLU, bool EXACT, bool HALF, bool NESTED, typename TO>
+template <int CL, int NL, int ROWS, int D, bool GLU, bool WIDE, bool NESTED, typename TO>
 int launch_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf4Matrix &w0, const Nf4Matrix &w1,
                 const void *m_sizes, int ms_i64, TO *y, TO *e_out, TO *g_out, int64_t R, int N, int K, int E,
                 hipStream_t stream) {
     const int64_t max_groups = R / ROWS + (R < E ? R : E);  // upper bound on sum over experts of ceil(m / ROWS)
     const int lds = kGemvTable + kGemvScales + (int)max_groups * 8 + 80 + E * 4;
-    auto *kernel = nf4_gemv_kernel<NL, ROWS, D, GLU, EXACT, HALF, NESTED, TO>;
+    auto *kernel = nf4_gemv_kernel<CL, NL, ROWS, D, GLU, WIDE, NESTED, TO>;
     static PerDeviceOnce attr;
     // The table lookups take the dynamic LDS to start at address 0; static LDS in this kernel would move it, so
     // such a build is left to the kernels that decode in registers.
@@ -464,28 +514,22 @@ int launch_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf4M
     if (static_lds.load(std::memory_order_acquire) != 0) return MFL_ERR_UNSUPPORTED;
     kernel<<<(unsigned)device_info().cu_count, kGemvThreads, lds, stream>>>(x, row_idx, idx_div, w0, w1, m_sizes, ms_i64,
                                                                             y, e_out, g_out, R, N, K, E,
-                                                                            N / ((GLU && !HALF) ? 16 : 32), (int)max_groups);
+                                                                            N / (CL < 64 ? 1024 / CL : GLU ? 16 : 32), (int)max_groups);
     return launch_status();
 }
 
-template <int NL, int ROWS, bool HALF>
+template <int CL, int NL, int ROWS, bool WIDE>
 int dispatch_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf4Matrix &w0, const Nf4Matrix &w1,
                   bool glu, const void *m_sizes, int ms_i64, void *y, void *e_out, void *g_out, int64_t R, int N,
                   int K, int E, int out_dtype, hipStream_t stream) {
-    const bool exact = !HALF && K % 512 == 0;
-#define MFL_GEMV(GLU, EXACT, TO, Y, EO, GO)                                                                         \
-    (w0.nested() ? launch_gemv<NL, ROWS, ((GLU || HALF) ? 4 : 2), GLU, (EXACT && !HALF), HALF, true, TO>(              \
+#define MFL_GEMV(GLU, TO, Y, EO, GO)                                                                               \
+    (w0.nested() ? launch_gemv<CL, NL, ROWS, ((NL <= 4 && (GLU || CL < 64)) ? 4 : 2), GLU, WIDE, true, TO>(                        \
                        x, row_idx, idx_div, w0, w1, m_sizes, ms_i64, Y, EO, GO, R, N, K, E, stream)                 \
-                 : launch_gemv<NL, ROWS, ((GLU || HALF) ? 4 : 2), GLU, (EXACT && !HALF), HALF, false, TO>(             \
+                 : launch_gemv<CL, NL, ROWS, ((NL <= 4 && (GLU || CL < 64)) ? 4 : 2), GLU, WIDE, false, TO>(                       \
                        x, row_idx, idx_div, w0, w1, m_sizes, ms_i64, Y, EO, GO, R, N, K, E, stream))
-    if (glu)
-        return exact ? MFL_GEMV(true, true, bf16_t, (bf16_t *)y, (bf16_t *)e_out, (bf16_t *)g_out)
-                     : MFL_GEMV(true, false, bf16_t, (bf16_t *)y, (bf16_t *)e_out, (bf16_t *)g_out);
-    if (out_dtype == MFL_BF16)
-        return exact ? MFL_GEMV(false, true, bf16_t, (bf16_t *)y, nullptr, nullptr)
-                     : MFL_GEMV(false, false, bf16_t, (bf16_t *)y, nullptr, nullptr);
-    return exact ? MFL_GEMV(false, true, float, (float *)y, nullptr, nullptr)
-                 : MFL_GEMV(false, false, float, (float *)y, nullptr, nullptr);
+    if (glu) return MFL_GEMV(true, bf16_t, (bf16_t *)y, (bf16_t *)e_out, (bf16_t *)g_out);
+    if (out_dtype == MFL_BF16) return MFL_GEMV(false, bf16_t, (bf16_t *)y, nullptr, nullptr);
+    return MFL_GEMV(false, float, (float *)y, nullptr, nullptr);
 #undef MFL_GEMV
 }
 
@@ -495,10 +539,16 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
                   bool glu, const void *m_sizes, int ms_i64, void *y, void *e_out, void *g_out, int64_t R, int N,
                   int K, int E, int out_dtype, hipStream_t stream) {
     if (R <= 0 || R > 2 * (int64_t)E || E > 2048) return MFL_ERR_UNSUPPORTED;  // a few rows per expert only
-    const bool half = K <= 1024;  // 32 lanes to a column
-    // (short rows: ahead of the streaming form only up to a row per expert: 23.5 against 25.5 us at 16 tokens of 8
-    // experts each for K = 768, N = 2048, 35.0 against 30.4 us at 32 tokens)
-    if (half && R > E) return MFL_ERR_UNSUPPORTED;
+    const bool half = K <= 1024;
+    // (by the sizes alone: the gated form's products are the same bits as the plain one's, whatever either matrix's blocks)
+    const bool wide = K % 32 == 0;
+    // Ahead of the streaming form, or even, up to two rows per expert of long reductions and 1.5 of short ones (128 experts,
+    // gated / plain us, H = 2048, I = 768, fp32 scales: 48 / 26 against 57 / 27 at 1.5 rows, 58 / 31 against 58 / 31 at 2; I
+    // = 512: 32 / 18 against 39 / 20 at 1.5, 39 / 22 against 40 / 20 at 2; 8-bit ones, whose sums are the same bits and the
+    // line therefore the same: 53 / 30 against 54 / 28 at 1.75, 59 / 32 against 55 / 30 at 2; I = 512: 34 / 19 against 37 /
+    // 20 at 1.5, 41 / 23 against 38 / 20 at 2).  Short reductions whose lanes take their dwords apart: up to a row per
+    // expert (35.0 against 30.4 at 2).
+    if (2 * R > (int64_t)E * (!half ? 4 : wide ? 3 : 2)) return MFL_ERR_UNSUPPORTED;
     if (K % 8 != 0 || K > 2048 || K <= 256) return MFL_ERR_UNSUPPORTED;
     // whole units (32 columns; 16 in the gated form with 64 lanes to a column); fewer than 2^31 units in all
     if (N % ((glu && !half) ? 16 : 32) != 0 || N > (1 << 18)) return MFL_ERR_UNSUPPORTED;
@@ -507,15 +557,22 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
         const Nf4Matrix &m = *mats[cb];
         // a lane's 8 weights under one scale, and every column starts a quantisation block
         if (m.bs_shift < 3 || (K & ((1 << m.bs_shift) - 1)) != 0) return MFL_ERR_UNSUPPORTED;
-        if (!aligned(m.absmax, 4) || !aligned(m.wq, 4)) return MFL_ERR_UNSUPPORTED;
+        if (!aligned(m.absmax, 4) || !aligned(m.wq, 16)) return MFL_ERR_UNSUPPORTED;
         if (m.nested() != w0.nested() || (m.nested() && (((int64_t)E * N * K) >> m.bs_shift) > 0x7fffffff))
             return MFL_ERR_UNSUPPORTED;
     }
     if (!aligned(x, 16)) return MFL_ERR_UNSUPPORTED;
-#define MFL_GEMV_D(NL, ROWS, HALF) \
-    dispatch_gemv<NL, ROWS, HALF>(x, row_idx, idx_div, w0, w1, glu, m_sizes, ms_i64, y, e_out, g_out, R, N, K, E, out_dtype, stream)
-    if (!half) return MFL_GEMV_D(4, 2, false);
-    return K <= 768 ? MFL_GEMV_D(3, 2, true) : MFL_GEMV_D(4, 2, true);
+#define MFL_GEMV_D(CL, NL, ROWS, WIDE) \
+    dispatch_gemv<CL, NL, ROWS, WIDE>(x, row_idx, idx_div, w0, w1, glu, m_sizes, ms_i64, y, e_out, g_out, R, N, K, E, out_dtype, stream)
+    if (!half) return wide ? MFL_GEMV_D(64, 4, 2, true) : MFL_GEMV_D(64, 4, 2, false);
+    // (16 lanes: plain product, N = 2048, 16 tokens of 8 experts each, fp32 / 8-bit scales: K = 768 22.1 / 25.6 -> 19.9 / 20.2
+    // us, K = 512 21.4 / 25.1 -> 15.8 / 16.8.  K = 1024 with eight dwords a lane spills: 25.8 -> 30.9.)
+    if (wide && N % 64 == 0) {
+        if (K > 512 && K % 192 == 0) return MFL_GEMV_D(16, 6, 2, true);
+        if (K <= 512) return MFL_GEMV_D(16, 4, 2, true);
+    }
+    if (K <= 768) return MFL_GEMV_D(32, 3, 2, false);
+    return wide ? MFL_GEMV_D(32, 4, 2, true) : MFL_GEMV_D(32, 4, 2, false);
 #undef MFL_GEMV_D
 }
 
