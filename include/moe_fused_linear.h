@@ -293,6 +293,10 @@ MFL_API int mfl_nf4_dequant(const uint8_t *wq, const float *code16, const float 
 MFL_API int mfl_dequant_blockwise_u8(const uint8_t *v, const float *code256, const float *absmax2,
                              int blocksize2, float offset, float *out, int64_t n, void *stream);
 
+/* The fp32 scales of up to four double-quantised matrices in one launch: out[i] gets the n[i] scales of w[i] (its
+ * absmax_u8, code256, absmax2, offset, blocksize2), as mfl_nf4_unnest_absmax writes them. */
+MFL_API int mfl_nf4_write_out_scales(const mfl_nf4_weight *w, const int64_t *n, float *const *out, int count, void *stream);
+
 /* The same with the offset read on the device (offset: one float) and blocksize2 a power of two. */
 MFL_API int mfl_nf4_unnest_absmax(const uint8_t *v, const float *code256, const float *absmax2, int blocksize2,
                           const float *offset, float *out, int64_t n, void *stream);

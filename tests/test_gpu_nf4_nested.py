@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 from qwen3_moe_fused.grouped_gemm.forward_4bit import grouped_gemm_forward_4bit  # noqa: E402
 from qwen3_moe_fused.grouped_gemm.fused import grouped_gemm_forward_4bit_gathered, grouped_glu_forward_4bit  # noqa: E402
-from qwen3_moe_fused.quantize.nf4 import Nf4QuantState, quantize_nf4, resolve_absmax  # noqa: E402
+from qwen3_moe_fused.quantize.nf4 import Nf4QuantState, _quantize_absmax, quantize_nf4, resolve_absmax  # noqa: E402
+from qwen3_moe_fused.quantize.nf4 import write_out_scales  # noqa: E402
 
 
 def _weights(e, n, k, blocksize, seed):
@@ -109,3 +110,19 @@ def test_second_level_blocks_of_any_size(blocksize2):
     outs = [moe_block_4bit(x, logits, *(Nf4Params(p, quant_state=s) for p, s in zip((g, u, d), which)), 2, True)[0]
             for which in ((g8, u8, d8), (g32, u32, d32))]
     assert torch.equal(*outs)
+
+
+# several matrices' scales in one launch: sizes that differ, one that four does not divide, a plain state and none between them
+def test_scales_of_several_matrices_written_out_at_once():
+    states = []
+    for n, blocksize2 in ((3 * 8 * 64, 256), (1 * 7 * 64, 8), (2 * 96 * 192, 256)):
+        _, nested, _ = _weights(1, n // 64, 64, 64, n)
+        if blocksize2 != 256:
+            scales = resolve_absmax(nested)
+            nested.absmax, nested.state2, nested.offset = _quantize_absmax(scales, blocksize2)
+        states.append(nested)
+    plain = _weights(1, 8, 64, 64, 5)[2]
+    got = write_out_scales(states[0], plain, None, states[1], states[2])
+    assert got[1] is plain and got[2] is None
+    for state, out in zip(states, (got[0], got[3], got[4])):
+        assert not out.nested and torch.equal(out.absmax, resolve_absmax(state))

@@ -514,7 +514,20 @@ int mfl_nf4_unnest_absmax(const uint8_t *v, const float *code256, const float *a
                           const float *offset, float *out, int64_t n, void *stream) {
     if (n < 0 || !blocksize_ok(blocksize2)) return MFL_ERR_SHAPE;
     if (n > 0 && (!v || !code256 || !absmax2 || !offset || !out)) return MFL_ERR_NULL;
-    return nf4_unnest_absmax(v, code256, absmax2, blocksize2, offset, out, n, (hipStream_t)stream);
+    const UnnestScales one = {v, code256, absmax2, offset, blocksize2, out, n};
+    return nf4_unnest_absmax(&one, 1, (hipStream_t)stream);
+}
+
+int mfl_nf4_write_out_scales(const mfl_nf4_weight *w, const int64_t *n, float *const *out, int count, void *stream) {
+    if (count < 0 || count > kMaxUnnest) return MFL_ERR_LIMIT;
+    if (count > 0 && (!w || !n || !out)) return MFL_ERR_NULL;
+    UnnestScales s[kMaxUnnest];
+    for (int i = 0; i < count; ++i) {
+        if (n[i] < 0 || !blocksize_ok(w[i].blocksize2)) return MFL_ERR_SHAPE;
+        if (n[i] > 0 && (!w[i].absmax_u8 || !w[i].code256 || !w[i].absmax2 || !w[i].offset || !out[i])) return MFL_ERR_NULL;
+        s[i] = {w[i].absmax_u8, w[i].code256, w[i].absmax2, w[i].offset, w[i].blocksize2, out[i], n[i]};
+    }
+    return nf4_unnest_absmax(s, count, (hipStream_t)stream);
 }
 
 int mfl_nf4_quant(const void *w, int w_dtype, int64_t n, int blocksize, const float *code16, uint8_t *wq, float *absmax,

@@ -4,6 +4,8 @@
 // decode sizes the block is a chain of five kernels of 5 to 40 us, and preparing each from the caller's language
 // (a tensor per output, an autograd node per step) took longer than the kernels run: 118 us of host time against
 // 95 us of kernels at 16 tokens on packed weights, 690 us for a training step of a toy block whose kernels take 120.
+#include <initializer_list>
+
 #include "common.h"
 #include "gemm.h"
 
@@ -96,15 +98,28 @@ int spread_rows(const mfl_moe_block &b, const void *src, const char *ws, const L
     return mfl_gather_rows(src, (const int32_t *)(ws + l.sort), 1, scale, dst, b.T, b.H, b.dtype, stream);
 }
 
-// A double-quantised matrix with its scales written out to `out`; others as they are
-int write_out_scales(const mfl_moe_block &b, const mfl_nf4_weight *w, float *out, mfl_nf4_weight &plain, void *stream) {
-    plain = *w;
-    if (w->absmax_u8 == nullptr) return MFL_OK;
-    plain.absmax = out;
-    plain.absmax_tiled = nullptr;
-    plain.absmax_u8 = nullptr;
-    return mfl_nf4_unnest_absmax(w->absmax_u8, w->code256, w->absmax2, w->blocksize2, w->offset, out,
-                                 (int64_t)b.E * b.H * b.I / w->blocksize, stream);
+// The matrices with the scales of double-quantised ones written out, matrix i's from out + i * scale_bytes on; others as
+// they are
+int write_out_scales(const mfl_moe_block &b, std::initializer_list<const mfl_nf4_weight *> from, mfl_nf4_weight *plain,
+                     char *out, size_t scale_bytes, void *stream) {
+    mfl_nf4_weight nested[2];
+    int64_t n[2];
+    float *to[2];
+    int count = 0, i = 0;
+    for (const mfl_nf4_weight *w : from) {
+        plain[i] = *w;
+        if (w->absmax_u8 != nullptr) {
+            nested[count] = *w;
+            n[count] = (int64_t)b.E * b.H * b.I / w->blocksize;
+            to[count] = (float *)(out + i * scale_bytes);
+            plain[i].absmax = to[count];
+            plain[i].absmax_tiled = nullptr;
+            plain[i].absmax_u8 = nullptr;
+            ++count;
+        }
+        ++i;
+    }
+    return mfl_nf4_write_out_scales(nested, n, to, count, stream);
 }
 
 #define MFL_TRY(call)                \
@@ -121,10 +136,9 @@ int front(const mfl_moe_block &b, char *ws, const Layout &l, void *stream) {
         int rc = mfl_glu_fwd_nf4_packed(b.tokens, b.T, sort, b.k, b.q_gate, b.q_up, ms, MFL_I32, h, e, g, R, b.I, b.H, b.E,
                                         b.dtype, stream);
         if (rc == MFL_ERR_UNSUPPORTED && (b.q_gate->absmax_u8 != nullptr || b.q_up->absmax_u8 != nullptr) && l.scale_slots == 2) {
-            mfl_nf4_weight gate, up;
-            MFL_TRY(write_out_scales(b, b.q_gate, (float *)(ws + l.scales), gate, stream));
-            MFL_TRY(write_out_scales(b, b.q_up, (float *)(ws + l.scales + l.scale_bytes), up, stream));
-            rc = mfl_glu_fwd_nf4_packed(b.tokens, b.T, sort, b.k, &gate, &up, ms, MFL_I32, h, e, g, R, b.I, b.H, b.E, b.dtype,
+            mfl_nf4_weight w[2];
+            MFL_TRY(write_out_scales(b, {b.q_gate, b.q_up}, w, ws + l.scales, l.scale_bytes, stream));
+            rc = mfl_glu_fwd_nf4_packed(b.tokens, b.T, sort, b.k, &w[0], &w[1], ms, MFL_I32, h, e, g, R, b.I, b.H, b.E, b.dtype,
                                         stream);
         }
         return rc;
@@ -150,7 +164,7 @@ int down(const mfl_moe_block &b, char *ws, const Layout &l, void *stream) {
                                      b.dtype, stream);
     if (rc == MFL_ERR_UNSUPPORTED && b.q_down->absmax_u8 != nullptr && l.scale_slots != 0) {
         mfl_nf4_weight w;
-        MFL_TRY(write_out_scales(b, b.q_down, (float *)(ws + l.scales), w, stream));
+        MFL_TRY(write_out_scales(b, {b.q_down}, &w, ws + l.scales, l.scale_bytes, stream));
         rc = mfl_gemm_fwd_nf4_packed(ws + l.h, 0, nullptr, 1, &w, ms, MFL_I32, ws + l.y, R, b.H, b.I, b.E, b.dtype, b.dtype,
                                      stream);
     }

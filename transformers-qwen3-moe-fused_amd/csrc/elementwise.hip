@@ -403,12 +403,25 @@ __global__ __launch_bounds__(256) void dequant_u8_kernel(const uint8_t *__restri
         out[i] = code[v[i]] * absmax2[i / blocksize2] + offset;
 }
 
-// The fp32 scales of a double-quantised matrix, offset included.  3.1 M scales: two launches of a byte per lane each
+struct UnnestJobs {
+    const uint8_t *v[kMaxUnnest];
+    const float *code256[kMaxUnnest], *absmax2[kMaxUnnest], *offset[kMaxUnnest];
+    float *out[kMaxUnnest];
+    int64_t n[kMaxUnnest];
+    int bs2_shift[kMaxUnnest], vec_ok[kMaxUnnest];
+};
+
+// The fp32 scales of double-quantised matrices (one per blockIdx.y), offset included.  3.1 M scales: two launches of a byte per lane each
 // (scales, then the offset) took 10.0 + 6.6 us, 16 bytes in and 64 out per lane 8.3 us (a store touched every line).
-__global__ __launch_bounds__(256) void nf4_unnest_kernel(const uint8_t *__restrict__ v, const float *__restrict__ code256,
-                                                         const float *__restrict__ absmax2, int bs2_shift,
-                                                         const float *__restrict__ offset, float *__restrict__ out,
-                                                         int64_t n, int vec_ok) {
+__global__ __launch_bounds__(256) void nf4_unnest_kernel(UnnestJobs jobs) {
+    const int job = blockIdx.y;
+    const uint8_t *__restrict__ const v = jobs.v[job];
+    const float *__restrict__ const code256 = jobs.code256[job];
+    const float *__restrict__ const absmax2 = jobs.absmax2[job];
+    const float *__restrict__ const offset = jobs.offset[job];
+    float *__restrict__ const out = jobs.out[job];
+    const int64_t n = jobs.n[job];
+    const int bs2_shift = jobs.bs2_shift[job], vec_ok = jobs.vec_ok[job];
     __shared__ float code[256];
     code[threadIdx.x] = code256[threadIdx.x];
     const float off = *offset;
@@ -599,13 +612,22 @@ int dequant_blockwise_u8(const uint8_t *v, const float *code256, const float *ab
     return launch_status();
 }
 
-int nf4_unnest_absmax(const uint8_t *v, const float *code256, const float *absmax2, int blocksize2, const float *offset,
-                      float *out, int64_t n, hipStream_t stream) {
-    if (n == 0) return MFL_OK;
-    const int shift = log2_exact(blocksize2);
-    const int vec_ok = aligned(v, 4) && aligned(out, 16) && blocksize2 >= 4;
-    nf4_unnest_kernel<<<stream_grid(vec_ok ? n / 16 + 1 : n), 256, 0, stream>>>(v, code256, absmax2, shift, offset, out, n,
-                                                                                vec_ok);
+int nf4_unnest_absmax(const UnnestScales *s, int count, hipStream_t stream) {
+    UnnestJobs jobs = {};
+    unsigned grid = 0;
+    int used = 0;
+    for (int i = 0; i < count; ++i) {
+        if (s[i].n == 0) continue;
+        const int vec_ok = aligned(s[i].v, 4) && aligned(s[i].out, 16) && s[i].blocksize2 >= 4;
+        jobs.v[used] = s[i].v, jobs.code256[used] = s[i].code256, jobs.absmax2[used] = s[i].absmax2;
+        jobs.offset[used] = s[i].offset, jobs.out[used] = s[i].out, jobs.n[used] = s[i].n;
+        jobs.bs2_shift[used] = log2_exact(s[i].blocksize2), jobs.vec_ok[used] = vec_ok;
+        const unsigned g = stream_grid(vec_ok ? s[i].n / 16 + 1 : s[i].n);
+        grid = g > grid ? g : grid;
+        ++used;
+    }
+    if (used == 0) return MFL_OK;
+    nf4_unnest_kernel<<<dim3(grid, used), 256, 0, stream>>>(jobs);
     return launch_status();
 }
 

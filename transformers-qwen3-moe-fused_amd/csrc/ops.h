@@ -20,8 +20,16 @@ int nf4_dequant(const uint8_t *wq, const float *code16, const float *absmax, int
                 int out_dtype, hipStream_t stream);
 int dequant_blockwise_u8(const uint8_t *v, const float *code256, const float *absmax2, int blocksize2, float offset,
                          float *out, int64_t n, hipStream_t stream);
-int nf4_unnest_absmax(const uint8_t *v, const float *code256, const float *absmax2, int blocksize2, const float *offset,
-                      float *out, int64_t n, hipStream_t stream);
+// The scales of up to kMaxUnnest double-quantised matrices, written out in one launch.
+constexpr int kMaxUnnest = 4;
+struct UnnestScales {
+    const uint8_t *v;
+    const float *code256, *absmax2, *offset;
+    int blocksize2;
+    float *out;
+    int64_t n;
+};
+int nf4_unnest_absmax(const UnnestScales *s, int count, hipStream_t stream);
 int nf4_quant(const void *w, int w_dtype, int64_t n, int blocksize, const float *code16, uint8_t *wq, float *absmax,
               hipStream_t stream);
 

@@ -90,6 +90,7 @@ _SIGNATURES = {
     "mfl_nf4_dequant": (_i, [_vp, _vp, _vp, _i, _vp, _i64, _i, _vp]),
     "mfl_dequant_blockwise_u8": (_i, [_vp, _vp, _vp, _i, _f, _vp, _i64, _vp]),
     "mfl_nf4_unnest_absmax": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _i64, _vp]),
+    "mfl_nf4_write_out_scales": (_i, [_nf4p, ctypes.POINTER(_i64), ctypes.POINTER(_vp), _i, _vp]),
     "mfl_nf4_quant": (_i, [_vp, _i, _i64, _i, _vp, _vp, _vp, _vp]),
     "mfl_router_fwd": (_i, [_vp, _vp, _vp, _i64, _i, _i, _i, _vp]),
     "mfl_router_dw_workspace": (_sz, [_i64, _i, _i]),

@@ -31,7 +31,7 @@ from ..grouped_gemm.fused import grouped_gemm_forward_lora as _fwd_lora
 from ..grouped_gemm.fused import grouped_glu_forward_lora as _glu_lora
 from ..grouped_gemm.fused import grouped_gemm_forward_transposed_4bit_lora as _dx4_lora
 from ..grouped_gemm.fused import grouped_gemm_forward_transposed_lora as _dx_lora
-from ..quantize.nf4 import dequantize_nf4
+from ..quantize.nf4 import dequantize_nf4, write_out_scales
 from .silu_mul import silu_mul_backward_inplace, silu_mul_forward
 
 
@@ -158,6 +158,8 @@ class FastLora(torch.autograd.Function):
         dt = x.dtype
         x = x.contiguous()
         Ag, Bg, Au, Bu, Aw, Bw = (p.to(dt).contiguous() for p in (Ag, Bg, Au, Bu, Aw, Bw))
+        frozen_states = (Gqs, Uqs, Wqs)
+        Gqs, Uqs, Wqs = write_out_scales(Gqs, Uqs, Wqs)
         ug = uu = ucat = None
         if Sg == Su and Ag.shape == Au.shape and x.shape[0] >= _WIDE_ROWS:
             # one pass over x for both adapters' rank-r activations
@@ -182,6 +184,7 @@ class FastLora(torch.autograd.Function):
             g, uu = _proj_fwd(x, Uq, Uqs, Au, Bu, Su, m_sizes, uu)
             h = silu_mul_forward(e, g)
         y, uw = _proj_fwd(h, Wq, Wqs, Aw, Bw, Sw, m_sizes)
+        Gqs, Uqs, Wqs = frozen_states  # (the scales are written out again: 6 MB a matrix less held between the passes)
         ctx.frozen = (Gq, Gqs, Sg, Uq, Uqs, Su, Wq, Wqs, Sw, m_sizes)
         ctx.save_for_backward(x, Ag, Bg, Au, Bu, Aw, Bw, e, g, ug, uu, uw)
         return y
@@ -192,6 +195,8 @@ class FastLora(torch.autograd.Function):
         x, Ag, Bg, Au, Bu, Aw, Bw, e, g, ug, uu, uw = ctx.saved_tensors
         dt = x.dtype
         dy = dy.contiguous()
+        if ctx.needs_input_grad[0]:
+            Gqs, Uqs, Wqs = write_out_scales(Gqs, Uqs, Wqs)
 
         # The rank-r activations carry the adapter's scaling (ug, uu, uw from the forward pass; tw, tu, tg here),
         # so every product below takes them as they are.

@@ -9,6 +9,7 @@ reads: quant_type, blocksize, code, absmax, nested, state2, offset, shape, dtype
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 from typing import Any, Optional, Tuple
 
@@ -195,6 +196,41 @@ def resolve_absmax(quant_state) -> torch.Tensor:
         return out
     assert absmax.dtype == torch.float32
     return absmax.contiguous()
+
+
+class _WrittenOut:
+    """A double-quantised state with its fp32 scales, for the calls of one pass."""
+
+    __slots__ = ("absmax", "shape", "code", "blocksize", "quant_type", "dtype", "_mfl_absmax_tiled")
+    nested = False
+
+    def __init__(self, state, absmax: torch.Tensor) -> None:
+        self.absmax = absmax
+        self.shape, self.code, self.blocksize = state.shape, state.code, state.blocksize
+        self.quant_type, self.dtype = state.quant_type, state.dtype
+        self._mfl_absmax_tiled = (absmax, absmax._version, -1, None)  # (no tile-ordered copy for one pass)
+
+
+def write_out_scales(*states):
+    """The states with the scales of the double-quantised ones (four at most) written out, all in one launch (three
+    matrices of 128 x 768 x 2048: 18.6 -> 9 us); others, and None, as they are."""
+    nested = [s for s in states if s is not None and getattr(s, "nested", False) and _is_shift(int(s.state2.blocksize))]
+    if not nested or len({s.absmax.device for s in nested}) != 1:
+        return states
+    out, keep = {}, []
+    weights = (_lib.Nf4Weight * len(nested))()
+    counts, ptrs = (ctypes.c_int64 * len(nested))(), (ctypes.c_void_p * len(nested))()
+    for i, s in enumerate(nested):
+        absmax, code2, absmax2, blocksize2, offset = parts = _second_level(s)
+        scales = torch.empty(absmax.numel(), device=absmax.device, dtype=torch.float32)
+        keep.append(parts)
+        weights[i].absmax_u8, weights[i].code256, weights[i].absmax2 = absmax.data_ptr(), code2.data_ptr(), absmax2.data_ptr()
+        weights[i].offset, weights[i].blocksize2 = offset.data_ptr(), blocksize2
+        counts[i], ptrs[i] = absmax.numel(), scales.data_ptr()
+        out[id(s)] = _WrittenOut(s, scales)
+    rc = _lib.lib().mfl_nf4_write_out_scales(weights, counts, ptrs, len(nested), _lib.stream())
+    _lib.check(rc, "mfl_nf4_write_out_scales")
+    return tuple(out.get(id(s), s) for s in states)
 
 
 def packed_weight(w_quant: torch.Tensor, quant_state, rows: int, unnested: bool = False):
