@@ -280,6 +280,17 @@ MFL_API int mfl_glu_fwd_nf4_packed(const void *x, int64_t src_rows, const int32_
                            int m_sizes_dtype, void *h, void *e_out, void *g_out, int64_t R, int N, int K, int E,
                            int dtype, void *stream);
 
+/* mfl_glu_fwd_lora over packed base weights with fp32 scales, and the input gradient of the two projections with both
+ * rank-r terms in one reduction: dx = dy1 w1 + dy2 w2 + xt wt, dy1, dy2 (R,K), w1, w2 (E,K,N), xt (R,KT), wt (E,KT,N).
+ * MFL_ERR_UNSUPPORTED, with nothing enqueued, as for mfl_gemm_fwd_nf4_lora / mfl_gemm_dx_nf4_lora and for
+ * double-quantised weights. */
+MFL_API int mfl_glu_fwd_nf4_lora(const void *x, const mfl_nf4_weight *w_gate, const mfl_nf4_weight *w_up, const void *xt,
+                         const void *wt_gate, const void *wt_up, int KT, const void *m_sizes, int m_sizes_dtype,
+                         void *h, void *e_out, void *g_out, int64_t R, int N, int K, int E, int dtype, void *stream);
+MFL_API int mfl_gemm_dx_nf4_dual_lora(const void *dy1, const mfl_nf4_weight *w1, const void *dy2, const mfl_nf4_weight *w2,
+                              const void *xt, const void *wt, int KT, const void *m_sizes, int m_sizes_dtype, void *dx,
+                              int64_t R, int N, int K, int E, int in_dtype, int out_dtype, void *stream);
+
 /* ---- NF4 / blockwise dequantisation ----------------------------------------------- */
 
 /* out[i] = code16[nibble(i)] * absmax[i / blocksize], i < n (n even).  Stands in for the

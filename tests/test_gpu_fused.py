@@ -513,6 +513,49 @@ def test_glu_with_lora_terms_equals_the_separate_products(R, N, K, E, r):
         assert torch.equal(h, silu_mul_forward(e, gg))
 
 
+from qwen3_moe_fused.grouped_gemm.fused import (grouped_glu_forward_4bit_lora,  # noqa: E402
+                                                grouped_gemm_forward_transposed_4bit_dual_lora)
+
+
+# rows per expert, inner width (out of gate and up), hidden, rank, block sizes of the two matrices: 160 x 128 tiles all resident,
+# the same not resident, 256 x 256 tiles; experts without rows, row tiles and column tiles that end inside, a rank of more than
+# a reduction step, blocks under 32, widths that the kernels leave to the separate products
+@pytest.mark.parametrize("m_sizes,M,H,r,bs", [([160, 0, 161, 31, 33], 160, 192, 8, (64, 64)), ([100] * 20, 2048, 64, 16, (64, 16)),
+                                              ([150, 0, 300, 257, 1, 255] * 2, 1984, 128, 72, (32, 64)), ([5, 9], 72, 40, 8, (8, 8)),
+                                              ([300, 20], 64, 2048, 24, (64, 64))])
+def test_packed_gate_and_up_with_lora_terms(m_sizes, M, H, r, bs):
+    """Forward: the bits of the two products and the SiLU-mul; input gradient: one rounding of the sum of both terms and the
+    rank-r ones, against 64 bits and against the two products that round twice."""
+    E, R = len(m_sizes), sum(m_sizes)
+    g = gen(R + M + r)
+    ms = torch.tensor(m_sizes)
+    sel = oracle.sel_from_m_sizes(ms.numpy())
+    ms = ms.to(DEV)
+    (gq, gs), (uq, us) = (quantize_nf4(randn((E, M, H), g, 0.05, torch.bfloat16).to(DEV), b) for b in bs)
+    x, ug, uu = (randn((R, n), g, 1.0, torch.bfloat16).to(DEV) for n in (H, r, r))
+    bg, bu = (randn((E, M, r), g, 0.2, torch.bfloat16).to(DEV) for _ in range(2))
+    zeros = torch.zeros_like(bg)
+    h, e, g2 = grouped_glu_forward_4bit_lora(x, gq, gs, uq, us, torch.cat([ug, uu], 1).contiguous(),
+                                             torch.cat([bg, zeros], 2).contiguous(), torch.cat([zeros, bu], 2).contiguous(), ms)
+    assert torch.equal(e, grouped_gemm_forward_4bit_lora(x, gq, gs, ug, bg, ms))
+    assert torch.equal(g2, grouped_gemm_forward_4bit_lora(x, uq, us, uu, bu, ms))
+    assert torch.equal(h, silu_mul_forward(e, g2))
+
+    from qwen3_moe_fused.quantize.nf4 import dequantize_nf4
+    de, dg, t = (randn((R, n), g, 1.0, torch.bfloat16).to(DEV) for n in (M, M, 2 * r))
+    a = randn((E, 2 * r, H), g, 0.2, torch.bfloat16).to(DEV)
+    dx = grouped_gemm_forward_transposed_4bit_dual_lora(de, gq, gs, dg, uq, us, t, a, ms)
+    ref = sum(oracle.linear_bwd_input(to_np32(d), w, sel).astype(np.float64)
+              for d, w in ((de, to_np32(dequantize_nf4(gq, gs, torch.bfloat16))), (dg, to_np32(dequantize_nf4(uq, us, torch.bfloat16))),
+                           (t, to_np32(a))))
+    # (separate products round three times: a bf16 half-ulp, 2^-9 of the value, each)
+    kw = {} if M % 64 == 0 and H % 32 == 0 else {"atol": unit_scale_atol(ref, 2e-2)}
+    check_close(dx, ref, what="input gradient of both packed matrices with rank-r terms vs oracle", **kw)
+    two = grouped_gemm_forward_transposed_4bit_lora(de, gq, gs, t, a, ms)
+    grouped_gemm_forward_transposed_4bit(dg, uq, us, ms, out=two, accumulate=True)
+    check_close(dx, to_np32(two), atol=unit_scale_atol(to_np32(two), 2e-2), what="one reduction vs two products")
+
+
 # few experts or narrow outputs: 64 x 128 tiles, and 160 x 128 where those are too many to be resident at once (the fifth
 # and sixth, whose gated products have enough 256 x 256 tiles, and the gated product of the last); borders of tiles and row
 # blocks, experts without rows, columns that end inside a tile, odd numbers of steps

@@ -372,6 +372,27 @@ int mfl_gemm_dx_nf4_lora(const void *dy, const uint8_t *wq, const float *code16,
                             out_dtype, 1.0f, 0, (hipStream_t)stream, &fu);
 }
 
+int mfl_gemm_dx_nf4_dual_lora(const void *dy1, const mfl_nf4_weight *w1, const void *dy2, const mfl_nf4_weight *w2,
+                              const void *xt, const void *wt, int KT, const void *m_sizes, int m_sizes_dtype, void *dx,
+                              int64_t R, int N, int K, int E, int in_dtype, int out_dtype, void *stream) {
+    if (N <= 0 || K <= 0 || E <= 0) return MFL_ERR_SHAPE;
+    Nf4Matrix m1, m2;
+    int rc = nf4_matrix_of(w1, K, N, E, m1);
+    if (!rc) rc = nf4_matrix_of(w2, K, N, E, m2);
+    if (rc) return rc;
+    if (m1.nested() || m2.nested()) return MFL_ERR_UNSUPPORTED;
+    rc = check_nf4_lora(dy1, m1.wq, m1.code16, m1.absmax, 1 << m1.bs_shift, xt, wt, KT, m_sizes, m_sizes_dtype, dx, R, N, K, E,
+                        in_dtype, out_dtype);
+    if (rc) return rc;
+    if (R == 0) return MFL_OK;
+    if (!dy2) return MFL_ERR_NULL;
+    if (in_dtype != MFL_BF16) return MFL_ERR_UNSUPPORTED;
+    GemmFusion fu = {nullptr, 1, 0, m2.wq, m2.code16, m2.absmax, 1 << m2.bs_shift, nullptr, nullptr, dy2};
+    fu.xt = xt, fu.wt = wt, fu.kt = KT;
+    return gemm_nf4_pipe_dx(dy1, m1.wq, m1.code16, m1.absmax, 1 << m1.bs_shift, m_sizes, m_sizes_dtype == MFL_I64, dx, R, N, K,
+                            E, out_dtype, 1.0f, 0, (hipStream_t)stream, &fu);
+}
+
 /* ---- forward products fused with their neighbours in the sparse MLP block ---- */
 
 namespace {
@@ -438,6 +459,25 @@ int mfl_glu_fwd_lora(const void *x, const void *w_gate, const void *w_up, const 
     fu.xt = xt, fu.wt = wt_gate, fu.kt = KT, fu.wt2 = wt_up;
     return gemm_bf16_pipe(MODE_FWD, x, w_gate, m_sizes, m_sizes_dtype == MFL_I64, h, R, N, K, E, MFL_BF16, 1.0f, 0,
                           (hipStream_t)stream, &fu);
+}
+
+int mfl_glu_fwd_nf4_lora(const void *x, const mfl_nf4_weight *w_gate, const mfl_nf4_weight *w_up, const void *xt,
+                         const void *wt_gate, const void *wt_up, int KT, const void *m_sizes, int m_sizes_dtype, void *h,
+                         void *e_out, void *g_out, int64_t R, int N, int K, int E, int dtype, void *stream) {
+    int rc = check_fused(0, nullptr, 1, m_sizes, m_sizes_dtype, R, N, K, E, dtype, dtype);
+    if (rc) return rc;
+    if (KT <= 0) return MFL_ERR_SHAPE;
+    Nf4Matrix gate, up;
+    rc = nf4_matrix_of(w_gate, N, K, E, gate);
+    if (!rc) rc = nf4_matrix_of(w_up, N, K, E, up);
+    if (rc) return rc;
+    if (R > 0 && (!x || !h || !xt || !wt_gate || !wt_up)) return MFL_ERR_NULL;
+    if (R == 0) return MFL_OK;
+    if (dtype != MFL_BF16 || gate.nested() || up.nested()) return MFL_ERR_UNSUPPORTED;
+    GemmFusion fu = {nullptr, 1, 0, up.wq, up.code16, up.absmax, 1 << up.bs_shift, e_out, g_out, nullptr};
+    fu.xt = xt, fu.wt = wt_gate, fu.kt = KT, fu.wt2 = wt_up;
+    return gemm_nf4_pipe(x, gate.wq, gate.code16, gate.absmax, 1 << gate.bs_shift, m_sizes, m_sizes_dtype == MFL_I64, h, R, N,
+                         K, E, MFL_BF16, (hipStream_t)stream, &fu);
 }
 
 static int glu_fwd_nf4(const void *x, int64_t src_rows, const int32_t *row_idx, int idx_div, const Nf4Matrix &gate,

@@ -99,7 +99,8 @@ constexpr int min_waves(int MB, int NB, int BK, int S, int waves) {
 // as a kernel of its own: the test for it in every step cost the plain products 3-5 %), 3 both: each of the two
 // matrices with thin weights of its own, against one thin left operand; 4 the input gradient with the gated unit's
 // backward in its epilogue (a kernel of its own: its epilogue holds pieces of e and g in registers beside the
-// accumulators, which the plain input gradient has no room for).
+// accumulators, which the plain input gradient has no room for); 5 the input gradient of two packed matrices, one term behind
+// the other, and a thin last term.
 template <int MB, int NB, int BK, int S, int WGM, int WGN, int MODE, bool NF4, int FUSE, typename TO>
 __global__ __launch_bounds__(WGM *WGN * 64, min_waves(MB, NB, BK, S, WGM *WGN)) void gemm_pipe_kernel(const bf16_t *__restrict__ a,
                                                                   const bf16_t *__restrict__ b,
@@ -107,7 +108,9 @@ __global__ __launch_bounds__(WGM *WGN * 64, min_waves(MB, NB, BK, S, WGM *WGN)) 
                                                                   TO *__restrict__ c, int64_t R, int N, int K, int E,
                                                                   float alpha, int accumulate, Nf4Params nf4,
                                                                   FwdFusion fu) {
-    constexpr bool GLU = FUSE == 1 || FUSE == 3, THIN = FUSE == 2 || FUSE == 3, BWG = FUSE == 4;
+    constexpr bool GLU = FUSE == 1 || FUSE == 3, THIN = FUSE == 2 || FUSE == 3 || FUSE == 5, BWG = FUSE == 4;
+    constexpr bool DUAL4 = FUSE == 5;
+    static_assert(!DUAL4 || (NF4 && MODE == MODE_DX), "two packed terms: input gradient");
     static_assert(!BWG || (MODE == MODE_DX && sizeof(TO) == 2), "the gated unit's backward: input gradient, bf16");
     static_assert(!THIN || MODE != MODE_DW, "the thin last term belongs to the row-grouped products");
     static_assert(!NF4 || (MODE != MODE_DW && S == 2 && BK == 64), "NF4 weights: row-grouped products, two stages");
@@ -660,6 +663,12 @@ __global__ __launch_bounds__(WGM *WGN * 64, min_waves(MB, NB, BK, S, WGM *WGN)) 
         };
         auto nf4_load = [&](int kt, Nf4Regs &r) {
             if (!nf4_on) return;
+            // the matrix of the step's term (wave-uniform)
+            const bool term2 = DUAL4 && kt >= KT1;
+            const unsigned char *const w = term2 ? (const unsigned char *)fu.b2 : nf4_w;
+            const float *const am = term2 ? fu.nf4_2.absmax : nf4_am;
+            const int shift = term2 ? fu.nf4_2.bs_shift : nf4_shift;
+            if (term2) kt -= KT1;
             int64_t el;
             if (B_RC) {
                 int row = GLU ? glu_col(nf4_row) : nf4_row;
@@ -670,23 +679,25 @@ __global__ __launch_bounds__(WGM *WGN * 64, min_waves(MB, NB, BK, S, WGM *WGN)) 
                 if (col >= j_lim) col = j_lim - 32;
                 el = nf4_base + (int64_t)(kt * BK + nf4_row) * N + col;
             }
-            r.w = *(const uint4_t *)(nf4_w + (el >> 1));
-            if (nf4_shift >= 5) {
-                r.am[0] = nf4_am[el >> nf4_shift];
+            r.w = *(const uint4_t *)(w + (el >> 1));
+            if (shift >= 5) {
+                r.am[0] = am[el >> shift];
             } else {
 #pragma unroll
-                for (int u = 0; u < 4; ++u) r.am[u] = nf4_am[(el + 8 * u) >> nf4_shift];
+                for (int u = 0; u < 4; ++u) r.am[u] = am[(el + 8 * u) >> shift];
             }
         };
         // one packed dword (8 weights, one 16-byte chunk of the stage) of the thread's 32
         auto nf4_decode_part = [&](int kt, const Nf4Regs &r, int u) {
             unsigned char *sb = smem + (kt % S) * STAGE_BYTES + SA::kBytes + nf4_row * SB::kRowBytes;
-            const float am = nf4_shift >= 5 ? r.am[0] : r.am[u];
+            const bool term2 = DUAL4 && kt >= KT1;
+            const float am = (term2 ? fu.nf4_2.bs_shift : nf4_shift) >= 5 ? r.am[0] : r.am[u];
+            const float *const codes = nf4_lut + (term2 ? 16 : 0);
             bf16x8 v;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const uint32_t nib = (r.w[u] >> (8 * (j >> 1) + ((j & 1) ? 0 : 4))) & 15u;
-                v[j] = (bf16_t)(nf4_lut[nib] * am);
+                v[j] = (bf16_t)(codes[nib] * am);
             }
             *(bf16x8 *)(sb + SB::swz(nf4_row, nf4_half * 4 + u) * 16) = v;
         };
@@ -699,7 +710,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, min_waves(MB, NB, BK, S, WGM *WGN)) 
             constexpr int TA = decltype(ta_tag)::value;
             Nf4Regs r0, r1;
             if (tid < 16) lut[tid] = nf4.code16[tid];
-            if (GLU && tid >= 16 && tid < 32) lut[tid] = fu.nf4_2.code16[tid - 16];
+            if ((GLU || DUAL4) && tid >= 16 && tid < 32) lut[tid] = fu.nf4_2.code16[tid - 16];
             // steps from KT_thin on (a thin last term) copy bf16 weights: nothing to load or decode for them
             if (KT_thin > 0) nf4_load(0, r0);
             if (KT_thin > 1) nf4_load(1, r1);
@@ -990,8 +1001,8 @@ int launch_pipe(int mode, const void *a, const void *b, const void *m_sizes, int
     const FwdFusion fu = fusion ? *fusion : no_fusion;
     const bool glu = fu.b2 != nullptr && fu.a2 == nullptr;
     if ((glu || fu.row_idx) && mode != MODE_FWD) return MFL_ERR_UNSUPPORTED;
-    if (fu.a2 != nullptr && (mode != MODE_DX || nf4 != nullptr || fu.b2 == nullptr)) return MFL_ERR_UNSUPPORTED;
-    if (fu.at != nullptr && (mode == MODE_DW || fu.bt == nullptr || (glu && (fu.bt2 == nullptr || nf4 != nullptr)))) return MFL_ERR_UNSUPPORTED;
+    if (fu.a2 != nullptr && (mode != MODE_DX || (nf4 != nullptr && fu.at == nullptr) || fu.b2 == nullptr)) return MFL_ERR_UNSUPPORTED;
+    if (fu.at != nullptr && (mode == MODE_DW || fu.bt == nullptr || (glu && fu.bt2 == nullptr))) return MFL_ERR_UNSUPPORTED;
 #define MFL_PIPE(MODE, NF4, GLU)                                                                                \
     {                                                                                                           \
         auto kern = gemm_pipe_kernel<MB, NB, BK, S, WGM, WGN, MODE, NF4, GLU, TO>;                              \
@@ -1007,8 +1018,16 @@ int launch_pipe(int mode, const void *a, const void *b, const void *m_sizes, int
     // MODES bit 3: the configuration is also built with the GLU epilogue (bf16 output only)
     constexpr bool GLU_OK = (MODES & 8) && WGN % 2 == 0 && sizeof(TO) == 2 && BK == 64;
     if (glu && fu.at != nullptr) {
-        if constexpr (GLU_OK && (MODES & 16) != 0) MFL_PIPE(MODE_FWD, false, 3)
-        else return MFL_ERR_UNSUPPORTED;
+        if constexpr (GLU_OK && (MODES & 16) != 0) {
+            if (nf4 == nullptr) {
+                MFL_PIPE(MODE_FWD, false, 3)
+            } else {
+                if constexpr (S == 2 && NB * 64 <= NT) MFL_PIPE(MODE_FWD, true, 3)
+                else return MFL_ERR_UNSUPPORTED;
+            }
+        } else {
+            return MFL_ERR_UNSUPPORTED;
+        }
     } else if (glu) {
         if constexpr (GLU_OK) {
             if (nf4 != nullptr) {
@@ -1026,6 +1045,7 @@ int launch_pipe(int mode, const void *a, const void *b, const void *m_sizes, int
             if (nf4 != nullptr) {
                 if constexpr (S == 2 && BK == 64 && NB * 64 <= NT) {
                     if (mode == MODE_FWD) MFL_PIPE(MODE_FWD, true, 2)
+                    else if (fu.a2 != nullptr) MFL_PIPE(MODE_DX, true, 5)
                     else MFL_PIPE(MODE_DX, true, 2)
                 } else {
                     return MFL_ERR_UNSUPPORTED;
@@ -1145,6 +1165,11 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
             cfg = (R / 160 + E) * (int64_t)ceil_div(N, 64) <= 2 * device_info().cu_count ? 5
                   : R > (int64_t)kNf4StreamGatedRowsPerExpert * E                         ? 8
                                                                                           : 3;
+        // with rank-r terms, which the streaming kernel does not take: 160 x 128 tiles up to 128 rows per expert, as the plain
+        // products do, then 256 x 256 (N = 768, K = 2048, 128 experts, us on 320 x 192 / 160 x 128 / 256 x 256 and for the two
+        // products and the SiLU-mul by themselves: 257 / 211 / 225, 255 at 128 rows; 273 / 266 / 252, 255 at 160; 556 / 405 /
+        // 357, 339 at 256, under Zipf(1.2) routing 686 / 422 / 383, 521; 970 / 726 / 570, 624 at 512)
+        if (nf4 != nullptr && fusion->at != nullptr && cfg != 5) cfg = R <= (int64_t)128 * E ? 5 : 8;
     } else if (cfg == 0 || nf4 != nullptr) {
         if (mode == MODE_DW)
             cfg = (N <= 64 || K <= 64) ? 11 : 8;
@@ -1211,6 +1236,15 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
 
 namespace {
 
+// The quantisation state of a second packed matrix.
+int second_packed(const GemmFusion *f, FwdFusion *out) {
+    int shift = 0;
+    while ((1 << shift) < f->blocksize_2) ++shift;
+    if (f->blocksize_2 < 8 || f->code16_2 == nullptr || f->absmax_2 == nullptr) return MFL_ERR_UNSUPPORTED;
+    out->nf4_2 = Nf4Params{f->code16_2, f->absmax_2, shift};
+    return MFL_OK;
+}
+
 // Checks the fusion request of a forward product and translates it for the kernel.
 // Returns MFL_ERR_UNSUPPORTED for what the pipelined kernels do not take.
 int make_fusion(const GemmFusion *f, int K, bool nf4, FwdFusion *out) {
@@ -1228,7 +1262,7 @@ int make_fusion(const GemmFusion *f, int K, bool nf4, FwdFusion *out) {
         // for that matrix too
         const bool glu_thin = f->w2 != nullptr && f->x2 == nullptr;
         if (f->wt == nullptr || f->kt < 8 || f->kt % 8 != 0 || !aligned(f->xt, 16) || !aligned(f->wt, 16) ||
-            f->row_idx != nullptr || (glu_thin && (nf4 || f->wt2 == nullptr || !aligned(f->wt2, 16))))
+            f->row_idx != nullptr || (glu_thin && (f->wt2 == nullptr || !aligned(f->wt2, 16))))
             return MFL_ERR_UNSUPPORTED;
         out->at = f->xt;
         out->bt = f->wt;
@@ -1247,25 +1281,20 @@ int make_fusion(const GemmFusion *f, int K, bool nf4, FwdFusion *out) {
         out->bw_h = f->bw_h;
     }
     if (f->x2 != nullptr) {
-        // two-term input gradient: whole reduction steps only, bf16 weights
-        if (nf4 || f->w2 == nullptr || K % 64 != 0 || !aligned(f->x2, 16) || !aligned(f->w2, 16) ||
+        // two-term input gradient: whole reduction steps only; packed weights with a thin last term only
+        if ((nf4 && f->xt == nullptr) || f->w2 == nullptr || K % 64 != 0 || !aligned(f->x2, 16) || !aligned(f->w2, 16) ||
             f->row_idx != nullptr)
             return MFL_ERR_UNSUPPORTED;
         out->a2 = f->x2;
         out->b2 = f->w2;
-        return MFL_OK;
+        return nf4 ? second_packed(f, out) : MFL_OK;
     }
     if (f->w2 != nullptr) {
         out->b2 = f->w2;
         out->c_e = f->e_out;
         out->c_g = f->g_out;
         if (!aligned(f->w2, nf4 ? 4 : 16) || !aligned(f->e_out, 16) || !aligned(f->g_out, 16)) return MFL_ERR_UNSUPPORTED;
-        if (nf4) {
-            int shift = 0;
-            while ((1 << shift) < f->blocksize_2) ++shift;
-            if (f->blocksize_2 < 8 || f->code16_2 == nullptr || f->absmax_2 == nullptr) return MFL_ERR_UNSUPPORTED;
-            out->nf4_2 = Nf4Params{f->code16_2, f->absmax_2, shift};
-        }
+        if (nf4) return second_packed(f, out);
     }
     return MFL_OK;
 }
@@ -1336,8 +1365,8 @@ int gemm_nf4_pipe_dx(const void *dy, const uint8_t *wq, const float *code16, con
     if (out_dtype != MFL_BF16 && out_dtype != MFL_F32) return MFL_ERR_UNSUPPORTED;
     FwdFusion fu;
     if (fusion != nullptr) {
-        // only the thin last term
-        if (fusion->xt == nullptr || fusion->x2 != nullptr || fusion->w2 != nullptr || fusion->row_idx != nullptr ||
+        // the thin last term, behind one packed term or two
+        if (fusion->xt == nullptr || (fusion->x2 == nullptr) != (fusion->w2 == nullptr) || fusion->row_idx != nullptr ||
             accumulate || alpha != 1.0f)
             return MFL_ERR_UNSUPPORTED;
         const int rc = make_fusion(fusion, K, true, &fu);

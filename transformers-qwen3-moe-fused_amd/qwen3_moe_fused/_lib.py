@@ -87,6 +87,8 @@ _SIGNATURES = {
                                    _vp, _vp, _i64, _i, _i, _i, _i, _vp]),
     "mfl_gemm_fwd_nf4_packed": (_i, [_vp, _i64, _vp, _i, _nf4p, _vp, _i, _vp, _i64, _i, _i, _i, _i, _i, _vp]),
     "mfl_glu_fwd_nf4_packed": (_i, [_vp, _i64, _vp, _i, _nf4p, _nf4p, _vp, _i, _vp, _vp, _vp, _i64, _i, _i, _i, _i, _vp]),
+    "mfl_glu_fwd_nf4_lora": (_i, [_vp, _nf4p, _nf4p, _vp, _vp, _vp, _i, _vp, _i, _vp, _vp, _vp, _i64, _i, _i, _i, _i, _vp]),
+    "mfl_gemm_dx_nf4_dual_lora": (_i, [_vp, _nf4p, _vp, _nf4p, _vp, _vp, _i, _vp, _i, _vp, _i64, _i, _i, _i, _i, _i, _vp]),
     "mfl_nf4_dequant": (_i, [_vp, _vp, _vp, _i, _vp, _i64, _i, _vp]),
     "mfl_dequant_blockwise_u8": (_i, [_vp, _vp, _vp, _i, _f, _vp, _i64, _vp]),
     "mfl_nf4_unnest_absmax": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _i64, _vp]),

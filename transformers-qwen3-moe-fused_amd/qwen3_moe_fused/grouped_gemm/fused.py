@@ -321,6 +321,69 @@ def grouped_gemm_forward_transposed_4bit_lora(dy: torch.Tensor, w_quant: torch.T
     return dx
 
 
+def _written_out(w_quant: torch.Tensor, state, absmax: torch.Tensor) -> "_lib.Nf4Weight":
+    return _lib.Nf4Weight(w_quant.data_ptr(), state.code.data_ptr(), absmax.data_ptr(), None, None, None, None, None,
+                          int(state.blocksize), 0)
+
+
+def grouped_gemm_forward_transposed_4bit_dual_lora(dy1: torch.Tensor, w1_quant: torch.Tensor, w1_state, dy2: torch.Tensor,
+                                                   w2_quant: torch.Tensor, w2_state, xt: torch.Tensor, wt: torch.Tensor,
+                                                   m_sizes: torch.Tensor) -> torch.Tensor:
+    """``dy1 @ W1[e] + dy2 @ W2[e] + xt @ wt[e]`` over two packed base weights of one shape (E, out, in) in one kernel: the
+    input gradient of the gate and up projections with both adapters' rank-r terms side by side, rounded once
+    (qwen3_moe_fused/kernels/fast_lora.py:127-131,151-152)."""
+    from .forward_4bit import grouped_gemm_forward_transposed_4bit
+
+    for dy, w_quant, state in ((dy1, w1_quant, w1_state), (dy2, w2_quant, w2_state)):
+        assert dy.is_cuda and dy.ndim == 2 and dy.is_contiguous() and m_sizes.is_contiguous() and is_int_tensor(m_sizes)
+        assert state.quant_type in ("nf4", "fp4") and is_int_tensor(w_quant) and w_quant.is_contiguous()
+    experts, k, n = w1_state.shape
+    rows, r = dy1.shape[0], xt.shape[1]
+    assert tuple(w2_state.shape) == tuple(w1_state.shape) and dy2.shape == dy1.shape and dy2.dtype == dy1.dtype
+    assert dy1.shape[1] == k and m_sizes.numel() == experts and xt.shape == (rows, r) and wt.shape == (experts, r, n)
+    assert xt.is_contiguous() and wt.is_contiguous() and xt.dtype == dy1.dtype and wt.dtype == dy1.dtype
+    absmax1, absmax2 = resolve_absmax(w1_state), resolve_absmax(w2_state)
+    dx = torch.empty((rows, n), device=dy1.device, dtype=dy1.dtype)
+    ms = _lib.as_index_tensor(m_sizes)
+    rc = _lib.lib().mfl_gemm_dx_nf4_dual_lora(dy1.data_ptr(), _written_out(w1_quant, w1_state, absmax1), dy2.data_ptr(),
+                                              _written_out(w2_quant, w2_state, absmax2), xt.data_ptr(), wt.data_ptr(), r,
+                                              ms.data_ptr(), _lib.itype_code(ms.dtype), dx.data_ptr(), rows, n, k, experts,
+                                              _lib.dtype_code(dy1.dtype), _lib.dtype_code(dx.dtype), _lib.stream())
+    if rc == UNSUPPORTED:
+        dx = grouped_gemm_forward_transposed_4bit_lora(dy1, w1_quant, w1_state, xt, wt, m_sizes)
+        return grouped_gemm_forward_transposed_4bit(dy2, w2_quant, w2_state, m_sizes, out=dx, accumulate=True)
+    _lib.check(rc, "mfl_gemm_dx_nf4_dual_lora")
+    return dx
+
+
+def grouped_glu_forward_4bit_lora(x: torch.Tensor, gate_quant: torch.Tensor, gate_state, up_quant: torch.Tensor, up_state,
+                                  xt: torch.Tensor, wt_gate: torch.Tensor, wt_up: torch.Tensor, m_sizes: torch.Tensor):
+    """``grouped_glu_forward_lora`` over packed base weights."""
+    assert x.is_cuda and x.ndim == 2 and x.is_contiguous() and m_sizes.is_contiguous() and is_int_tensor(m_sizes)
+    rows, k = x.shape
+    experts, n = check_packed(x, gate_quant, gate_state, k)
+    assert check_packed(x, up_quant, up_state, k) == (experts, n)
+    kt = xt.shape[1]
+    assert m_sizes.numel() == experts and xt.shape[0] == rows
+    assert wt_gate.shape == (experts, n, kt) and wt_up.shape == (experts, n, kt)
+    assert all(t.is_contiguous() and t.dtype == x.dtype for t in (xt, wt_gate, wt_up))
+    absmax_gate, absmax_up = resolve_absmax(gate_state), resolve_absmax(up_state)
+    h = torch.empty((rows, n), device=x.device, dtype=x.dtype)
+    e, g = torch.empty_like(h), torch.empty_like(h)
+    ms = _lib.as_index_tensor(m_sizes)
+    rc = _lib.lib().mfl_glu_fwd_nf4_lora(x.data_ptr(), _written_out(gate_quant, gate_state, absmax_gate),
+                                         _written_out(up_quant, up_state, absmax_up), xt.data_ptr(), wt_gate.data_ptr(),
+                                         wt_up.data_ptr(), kt, ms.data_ptr(), _lib.itype_code(ms.dtype), h.data_ptr(),
+                                         e.data_ptr(), g.data_ptr(), rows, n, k, experts, _lib.dtype_code(x.dtype),
+                                         _lib.stream())
+    if rc == UNSUPPORTED:
+        e = grouped_gemm_forward_4bit_lora(x, gate_quant, gate_state, xt, wt_gate, m_sizes)
+        g = grouped_gemm_forward_4bit_lora(x, up_quant, up_state, xt, wt_up, m_sizes)
+        return silu_mul_forward(e, g), e, g
+    _lib.check(rc, "mfl_glu_fwd_nf4_lora")
+    return h, e, g
+
+
 def grouped_glu_forward_lora(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, xt: torch.Tensor,
                              wt_gate: torch.Tensor, wt_up: torch.Tensor, m_sizes: torch.Tensor):
     """``(h, e, g)`` with ``e = x w_gate^T + xt wt_gate^T``, ``g = x w_up^T + xt wt_up^T``, ``h = silu(e) * g`` in

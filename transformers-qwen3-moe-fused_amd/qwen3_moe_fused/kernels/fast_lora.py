@@ -28,11 +28,19 @@ from ..grouped_gemm.forward_4bit import grouped_gemm_forward_transposed_4bit as 
 from ..grouped_gemm.forward_transposed import grouped_gemm_forward_transposed as _dx
 from ..grouped_gemm.fused import grouped_gemm_forward_4bit_lora as _fwd4_lora
 from ..grouped_gemm.fused import grouped_gemm_forward_lora as _fwd_lora
+from ..grouped_gemm.fused import grouped_glu_forward_4bit_lora as _glu4_lora
 from ..grouped_gemm.fused import grouped_glu_forward_lora as _glu_lora
+from ..grouped_gemm.fused import grouped_gemm_forward_transposed_4bit_dual_lora as _dx4_dual_lora
 from ..grouped_gemm.fused import grouped_gemm_forward_transposed_4bit_lora as _dx4_lora
 from ..grouped_gemm.fused import grouped_gemm_forward_transposed_lora as _dx_lora
 from ..quantize.nf4 import dequantize_nf4, write_out_scales
 from .silu_mul import silu_mul_backward_inplace, silu_mul_forward
+
+
+def _packed_pair(x, Gqs, Uqs):
+    """Whether the gate and up projections are packed matrices that one kernel takes for rows like ``x``."""
+    return (Gqs is not None and Uqs is not None and x.dtype == torch.bfloat16 and x.shape[1] % 8 == 0
+            and int(Gqs.blocksize) >= 8 and int(Uqs.blocksize) >= 8 and tuple(Gqs.shape) == tuple(Uqs.shape))
 
 
 def _base_fwd(x, wq, wqs, m_sizes):
@@ -167,8 +175,9 @@ class FastLora(torch.autograd.Function):
             assert x.is_cuda and all(t.device == x.device for t in (Ag, Bg, Au, Bu))  # (the copies come before the products)
             pieces = []
             acat = _joined(Ag, Au, 1, pieces)
-            one_launch = (Gqs is None and Uqs is None and dt == torch.bfloat16 and Gq.dtype == dt and Uq.dtype == dt
-                          and Bg.shape == Bu.shape)
+            packed = _packed_pair(x, Gqs, Uqs)
+            one_launch = Bg.shape == Bu.shape and (packed or (Gqs is None and Uqs is None and dt == torch.bfloat16
+                                                              and Gq.dtype == dt and Uq.dtype == dt))
             if one_launch:
                 # each matrix's thin weights are its adapter's B over its own columns of ucat and zeros over the other's
                 assert Bg.shape[2] == r, "an adapter's A and B have one rank"
@@ -178,7 +187,10 @@ class FastLora(torch.autograd.Function):
             ug, uu = _halves(ucat, 1, r)
         if ucat is not None and one_launch:
             # gate, up, both rank-r terms and the SiLU-mul in one launch
-            h, e, g = _glu_lora(x, Gq, Uq, ucat, bg, bu, m_sizes)
+            if packed:
+                h, e, g = _glu4_lora(x, Gq, Gqs, Uq, Uqs, ucat, bg, bu, m_sizes)
+            else:
+                h, e, g = _glu_lora(x, Gq, Uq, ucat, bg, bu, m_sizes)
         else:
             e, ug = _proj_fwd(x, Gq, Gqs, Ag, Bg, Sg, m_sizes, ug)
             g, uu = _proj_fwd(x, Uq, Uqs, Au, Bu, Su, m_sizes, uu)
@@ -231,6 +243,8 @@ class FastLora(torch.autograd.Function):
             if Gqs is None and Uqs is None and dt == torch.bfloat16 and Gq.dtype == dt and Uq.dtype == dt:
                 # both base terms and both rank-r terms (side by side as one term of rank 2 r) in one reduction
                 dx = _dx_lora(de, Gq, tcat, acat, m_sizes, dy2=dg, w2=Uq)
+            elif _packed_pair(de, Gqs, Uqs):
+                dx = _dx4_dual_lora(de, Gq, Gqs, dg, Uq, Uqs, tcat, acat, m_sizes)
             else:
                 # both rank-r terms with the first base product, the second base product accumulates
                 dx = _proj_bwd_input(de, tcat, Gq, Gqs, acat, m_sizes)
