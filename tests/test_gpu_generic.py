@@ -124,3 +124,20 @@ def test_outputs_of_more_column_tiles_than_a_grid_has_rows(n):
             exact += term
             bound += term.abs()
         assert ((got - exact).abs() <= k * 2.0 ** -24 * bound + 2.0 ** -23 * exact.abs()).all()
+
+
+# Matrices larger than the last cache, rows of whole lines: the weights are loaded, a weight gradient is stored past the
+# caches.  Tiles of 16 and of 32 rows, experts without rows, one with a second tile, output tiles that end inside both ways.
+@pytest.mark.parametrize("sizes", [[8, 0, 17, 1] * 8 + [16], [20, 33, 0, 24] * 8 + [31]])
+def test_matrices_larger_than_the_caches(sizes):
+    e, n, k, rows = len(sizes), 1056, 2080, sum(sizes)
+    assert e * n * k * 4 > 256 << 20
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x, dy = (torch.randn((rows, c), device="cuda", generator=g) for c in (k, n))
+    w = torch.randn((e, n, k), device="cuda", generator=g)
+    ms = torch.tensor(sizes, dtype=torch.int32).cuda()
+    got = (grouped_gemm_forward(x, w, ms), grouped_gemm_forward_transposed(dy, w, ms), grouped_gemm_backward_dw(x, dy, ms, torch.float32))
+    for y, exact, bound, length, what in zip(got, _products(x, w, dy, sizes), _products(x.abs(), w.abs(), dy.abs(), sizes),
+                                             (k, n, max(sizes)), ("forward", "dx", "dw")):
+        room = length * 2.0 ** -24 * bound + 2 * ULP[torch.float32] * exact.abs()
+        assert torch.isfinite(y).all() and ((y.double() - exact).abs() <= room + 1e-30).all(), what

@@ -24,7 +24,7 @@ constexpr int kPad = 4;  // floats: rows stay 16-byte aligned and 16 consecutive
 // An operand tile of BI rows (output side) by BK reduction elements.
 //   RC (reduction-contiguous): element (i, r) at base[i * ld + r], in LDS at [i][r]
 //   RS (reduction-strided):    element (i, r) at base[r * ld + i], in LDS at [r][i]
-template <typename TI, int BI, int BK, bool RC, int VEC>
+template <typename TI, int BI, int BK, bool RC, int VEC, bool NT = false>
 struct Operand {
     static constexpr int kRow = RC ? BK : BI;                  // contiguous elements of a tile row
     static constexpr int kStride = kRow + kPad;                // floats
@@ -45,7 +45,7 @@ struct Operand {
             if constexpr (VEC == 4) {  // the contiguous dimension is a multiple of four: a group is inside or outside
                 if (i < i_end && r < r_end) {
                     typedef __attribute__((ext_vector_type(4))) TI vec_t;
-                    const vec_t t = *(const vec_t *)p;
+                    const vec_t t = NT ? __builtin_nontemporal_load((const vec_t *)p) : *(const vec_t *)p;
 #pragma unroll
                     for (int u = 0; u < 4; ++u) v[q][u] = to_f32(t[u]);
                 }
@@ -107,8 +107,9 @@ __device__ __forceinline__ int rows_before_expert(const void *m_sizes, int ms_i6
     return wave_last(wave_inclusive_scan(m));
 }
 
+// NT: the weights are read, a weight gradient is written past the caches (non-temporal; where, is at the launch).
 // WM x WN waves over the tile; WK > 1: the waves share the tile and split the reduction (partial sums meet in LDS).
-template <typename TI, typename TO, int MODE, int BM, int BN, int WM, int WN, int WK, int BK, int VEC>
+template <typename TI, typename TO, int MODE, int BM, int BN, int WM, int WN, int WK, int BK, int VEC, bool NT>
 __global__ __launch_bounds__(kThreads) void gemm_generic_kernel(const TI *__restrict__ a, const TI *__restrict__ b,
                                                                 const void *__restrict__ m_sizes, int ms_i64, TO *c,
                                                                 int64_t R, int N, int K, int E, float alpha,
@@ -119,10 +120,15 @@ __global__ __launch_bounds__(kThreads) void gemm_generic_kernel(const TI *__rest
     // (consecutive lanes then store consecutive single elements, where rows are not aligned)
     constexpr bool kRowLanes = VEC == 4;
     typedef Operand<TI, BM, BK, MODE != MODE_DW, VEC> OpA;
-    typedef Operand<TI, BN, BK, MODE == MODE_FWD, VEC> OpB;
+    typedef Operand<TI, BN, BK, MODE == MODE_FWD, VEC, NT && MODE != MODE_DW> OpB;
     constexpr int kPartFloats = WM * WN * TM * TN * (WK - 1) * 4 * kWave;  // partial sums of the waves that share a tile
     static_assert(kPartFloats <= OpA::kFloats + OpB::kFloats, "partial sums go where the stage was");
-    __shared__ __align__(16) float smem[OpA::kFloats + OpB::kFloats];
+    // weight gradients in fp32 leave by way of LDS, 16 rows of a wave at a time
+    constexpr bool kStaged = MODE == MODE_DW && kRowLanes && WK == 1 && TN >= 2 && sizeof(TO) == 4;
+    constexpr int kOutRow = TN * 16 + kPad;
+    constexpr int kOutFloats = kStaged ? WM * WN * 16 * kOutRow : 0;
+    constexpr int kStageFloats = OpA::kFloats + OpB::kFloats;
+    __shared__ __align__(16) float smem[kStageFloats > kOutFloats ? kStageFloats : kOutFloats];
     float *As = smem, *Bs = smem + OpA::kFloats;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wk = wave % WK, wn = wave / WK % WN, wm = wave / WK / WN;
@@ -209,6 +215,38 @@ __global__ __launch_bounds__(kThreads) void gemm_generic_kernel(const TI *__rest
                     acc[t / TN][t % TN] += *(const floatx4 *)(part + (t * (WK - 1) + s) * kWave * 4);
     }
 
+    if constexpr (kStaged) {
+        if (vec_out && !accumulate) {
+            // A lane's four columns of 16 rows are 64 bytes of each row to a store; put together in LDS a store takes 128 to
+            // 256 bytes a row, whole lines, and may pass the caches by where the output is larger than they are.
+            __syncthreads();  // the last step's fragments have been read
+            float *const st = smem + wave * (16 * kOutRow);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    floatx4 o;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) o[u] = alpha * acc[i][j][u];
+                    *(floatx4 *)(st + (lane & 15) * kOutRow + j * 16 + (lane >> 4) * 4) = o;
+                }
+                // (the same wave reads back what it wrote: LDS operations of one wave complete in order)
+#pragma unroll
+                for (int q = lane; q < 16 * TN * 4; q += kWave) {
+                    const int row_l = q / (TN * 4), col_l = (q % (TN * 4)) * 4;
+                    const int row = i0 + (wm * TM + i) * 16 + row_l, col = j0 + wn * TN * 16 + col_l;
+                    const floatx4 o = *(const floatx4 *)(st + row_l * kOutRow + col_l);
+                    if (row >= i_end || col >= j_end) continue;
+                    floatx4 *const p = (floatx4 *)(c_base + (int64_t)row * ldc + col);
+                    if constexpr (NT)
+                        __builtin_nontemporal_store(o, p);
+                    else
+                        *p = o;
+                }
+            }
+            return;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -264,23 +302,38 @@ int launch_tile(const Args &g) {
         if (slots > 0x7fffffff || ceil_div(g.N, BN) > 65535) return MFL_ERR_UNSUPPORTED;
         grid = dim3((unsigned)slots, ceil_div(g.N, BN), 1);
     }
-    gemm_generic_kernel<TI, TO, MODE, BM, BN, WM, WN, WK, BK, VEC><<<grid, kThreads, 0, g.stream>>>(
-        (const TI *)g.a, (const TI *)g.b, g.m_sizes, g.ms_i64, (TO *)g.c, g.R, g.N, g.K, g.E, g.alpha, g.accumulate,
-        g.vec_out);
+    // Past the caches: matrices larger than the 256 MB of the last one.  A weight gradient, because its own writes, written
+    // back behind it, cost the kernels after it more than it gained; the weights where nearly every expert's rows are one
+    // tile and each weight is read once.  Rows of whole lines only: a line that two stores fill, or two loads take, moves
+    // twice.  fp32, 128 experts of 8 rows, 768 x 2048 (805 MB), forward / input gradient / weight gradient and the three in
+    // turn: 154 / 159 / 177, 559 us; with the gradient's rows put together in LDS 154 / 159 / 147, 507; that past the caches
+    // 154 / 159 / 126, 446; the weights too 145 / 147 / 126, 411.  64 experts (403 MB) 293 -> 230.  Rows of 6048 bytes: weight
+    // gradient 61 -> 96, input gradient 76 -> 83.  Experts with a second tile: input gradient at 16 rows per expert 187 ->
+    // 248, at 32 (32-row tiles) 231 -> 269.
+    constexpr bool kNt = VEC == 4 && sizeof(TI) == 4 && (MODE == MODE_DW || BM <= 32);
+    [[maybe_unused]] const void *const streamed = MODE == MODE_DW ? g.c : g.b;
+    [[maybe_unused]] const bool nt = (int64_t)g.E * g.N * g.K * 4 > ((int64_t)256 << 20) && aligned(streamed, 128) &&
+                                     (MODE == MODE_DX ? g.N : g.K) % 32 == 0 &&
+                                     (MODE == MODE_DW || 4 * g.R <= (int64_t)3 * BM * g.E);
+    auto *kernel = gemm_generic_kernel<TI, TO, MODE, BM, BN, WM, WN, WK, BK, VEC, false>;
+    if constexpr (kNt)
+        if (nt) kernel = gemm_generic_kernel<TI, TO, MODE, BM, BN, WM, WN, WK, BK, VEC, true>;
+    kernel<<<grid, kThreads, 0, g.stream>>>((const TI *)g.a, (const TI *)g.b, g.m_sizes, g.ms_i64, (TO *)g.c, g.R, g.N, g.K,
+                                            g.E, g.alpha, g.accumulate, g.vec_out);
     return launch_status();
 }
 
 // Tiles, with fp32 times at 128 experts, K = 2048, N = 768 (us; the plain FMA kernel that stood here in brackets):
 // * up to 16 rows per expert the product streams the weights: 16-row tiles whose waves split the reduction, so that a
-//   step asks for 512 consecutive bytes of every weight row and 24 KiB workgroups keep 96 KiB a CU in flight: 150 us
-//   forward at 8 rows per expert = 5.4 TB/s (712), 168 dX (533); 64 x 64 tiles with the waves side by side: 285.
+//   step asks for 512 consecutive bytes of every weight row and 24 KiB workgroups keep 96 KiB a CU in flight: 145 us
+//   forward at 8 rows per expert = 5.6 TB/s (712), 147 dX (533); 64 x 64 tiles with the waves side by side: 285.
 // * up to 48, and where 64-row tiles would leave CUs without a second and third workgroup, 32 x 64 tiles: 191 us
 //   forward at 24 rows per expert (746; 64 x 64 tiles 275, 16-row tiles 295), 154 us at 8 experts of 512 rows (518;
 //   64 x 64 166).
 // * beyond, 64 x 64 tiles: 373 us at 64 rows per expert (1584; 128 x 128 tiles 392, whose 64 accumulators and 32
 //   registers in transit leave two workgroups a CU).
 // * the weight gradient writes more than it reads up to about 100 rows per expert: 64 x 128 tiles and 16-row steps,
-//   182 us at 8 rows per expert = 4.5 TB/s (294; with 32-row steps 225, the zeros of a half-empty stage cost as much
+//   126 us at 8 rows per expert = 6.4 TB/s (294; before its rows left as whole lines 177, with 32-row steps 225, the zeros of a half-empty stage cost as much
 //   as rows do); outputs of at most 16 rows per expert (N: the rank in the gradient of an adapter's A) take
 //   16-row tiles.
 // * short reductions (adapter ranks, toy sizes) leave most of a 64- or 128-wide step empty: 16-wide steps.  16000 rows of 8
