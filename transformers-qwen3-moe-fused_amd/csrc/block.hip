@@ -171,6 +171,26 @@ int down(const mfl_moe_block &b, char *ws, const Layout &l, void *stream) {
     return rc;
 }
 
+// The down projection and the sum over each token's selections as one launch, where there is a kernel for it
+int down_and_combine(const mfl_moe_block &b, const char *ws, const Layout &l, void *out, void *stream) {
+    if (b.q_down == nullptr || !b.q_down->packed || !b.q_down->code16 || (b.q_down->blocksize & (b.q_down->blocksize - 1)) != 0)
+        return MFL_ERR_UNSUPPORTED;
+    const mfl_nf4_weight &w = *b.q_down;
+    auto log2_of = [](int v) { return 31 - __builtin_clz((unsigned)v); };
+    Nf4Matrix m = {w.packed, w.code16, w.absmax, log2_of(w.blocksize)};
+    if (w.absmax_u8 != nullptr) {
+        if (!w.code256 || !w.absmax2 || !w.offset || w.blocksize2 < 2 || (w.blocksize2 & (w.blocksize2 - 1)) != 0)
+            return MFL_ERR_UNSUPPORTED;
+        m.absmax = nullptr;
+        m.absmax_u8 = w.absmax_u8, m.code256 = w.code256, m.absmax2 = w.absmax2, m.offset = w.offset;
+        m.bs2_shift = log2_of(w.blocksize2);
+    } else if (!w.absmax) {
+        return MFL_ERR_UNSUPPORTED;
+    }
+    return gemm_nf4_down_combine((const bf16_t *)(ws + l.h), (const int32_t *)(ws + l.inv), (const int64_t *)(ws + l.idx),
+                                 (const bf16_t *)(ws + l.weights), m, (bf16_t *)out, b.T, b.k, b.H, b.I, b.E, (hipStream_t)stream);
+}
+
 // What the backward needs besides the forward's buffer: the output gradient's rows (then, in their place, the input
 // gradient's), the tokens' rows, dh, de and dg
 struct BackLayout {
@@ -237,6 +257,8 @@ int mfl_moe_block_fwd(const mfl_moe_block *b, void *out, void *workspace, size_t
                            b->dtype, (int64_t *)(ws + l.idx), (int32_t *)(ws + l.counts), (int32_t *)(ws + l.sort),
                            (int32_t *)(ws + l.inv), ws + l.route, l.route_bytes, stream));
     MFL_TRY(front(*b, ws, l, stream));
+    const int rc = down_and_combine(*b, ws, l, out, stream);
+    if (rc != MFL_ERR_UNSUPPORTED) return rc;
     MFL_TRY(down(*b, ws, l, stream));
     return mfl_combine_rows(ws + l.y, (const int32_t *)(ws + l.inv), ws + l.weights, out, b->T, b->k, b->H, b->dtype, stream);
 }

@@ -155,6 +155,12 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
                   bool glu, const void *m_sizes, int ms_i64, void *y, void *e_out, void *g_out, int64_t R, int N,
                   int K, int E, int out_dtype, hipStream_t stream);
 
+// The down projection of a few selections and the routing-weighted sum over each token's: out (T, N) = sum over j of
+// weights[t, j] * (h[inv[t, j]] w[idx[t, j]]^T), with the roundings of the product and the combine kernel by themselves.  h
+// (T k, K) in the order of the experts, inv the selections' rows in it.  MFL_ERR_UNSUPPORTED but for the smallest batches.
+int gemm_nf4_down_combine(const bf16_t *h, const int32_t *inv, const int64_t *idx, const bf16_t *weights, const Nf4Matrix &w,
+                          bf16_t *out, int64_t T, int k, int N, int K, int E, hipStream_t stream);
+
 // Forward with NF4 weights for decode-sized batches: the matrix-vector, streaming or register-decoding kernel.  glu:
 // w0 is the gate and w1 the up projection (else w1 is not read).  A double-quantised matrix is taken by the first two.
 int gemm_nf4_decode(const void *x, const int32_t *row_idx, int idx_div, const Nf4Matrix &w0, const Nf4Matrix &w1, bool glu,
