@@ -325,9 +325,48 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
     const int xcd = blockIdx.x % kXcd;
     const int per_xcd = gridDim.x / kXcd;
     const int chunk = ceil_div(total, kXcd);
-    const int L_first = xcd * chunk + blockIdx.x / kXcd;
+    int L_first = xcd * chunk + blockIdx.x / kXcd;
     int L_end = (xcd + 1) * chunk;
     if (L_end > total) L_end = total;
+
+    // DW: the time of a tile is that of its expert's rows.  The experts are ranked by their rows and dealt out to the
+    // XCDs to and fro (0..7, 7..0, ...), and an XCD goes through its experts from the largest to the smallest, so
+    // that skewed routing leaves no XCD with the work of many popular experts and no late long tile.
+    // Where: an expert of more than 1.5 times the mean (even routing gains nothing: 181.7 against 177.6 us at 128
+    // experts x 768 x 2048, 256 rows each); at least four experts an XCD (16 experts: 94 against 89); at least 96 rows
+    // per expert on average (at 64 the time is that of the weights: 105 / 200 us against 101 / 210 at 128 / 256
+    // experts); and whole experts an XCD make no more rounds under even routing than runs of equal numbers.
+    // 32768 rows over 128 experts x 768 x 2048, largest expert 11 / 15 / 16 times the mean: 209 / 222 / 208 us
+    // against 235 / 273 / 285; 16384 rows 140 against 160; 8000 rows over 60 experts x 1536 x 2048 138 against 157.
+    bool by_size = MODE == MODE_DW && E >= 4 * kXcd &&
+                   ceil_div(ceil_div(E, kXcd) * per_expert, per_xcd) <= ceil_div(chunk, per_xcd);
+    if (by_size) {
+        const int64_t rows = tab_rows[E];
+        uint64_t hits = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + lane < E ? e0 + lane : E - 1;
+            hits |= __ballot((int64_t)(tab_rows[e + 1] - tab_rows[e]) * 2 * E > 3 * rows);
+        }
+        by_size = hits != 0 && rows >= (int64_t)96 * E;
+    }
+    uint16_t *tab_rank = (uint16_t *)(tab_tiles + (kMaxTableExperts + 1));
+    if (by_size) {
+        for (int e = threadIdx.x; e < E; e += 256) {
+            const int m = tab_rows[e + 1] - tab_rows[e];
+            int rank = 0, before = 0;
+            for (int o = 0; o < E; ++o) {  // equal sizes in the experts' order
+                const int after = tab_rows[o + 1], mo = after - before;
+                rank += mo > m || (mo == m && o < e);
+                before = after;
+            }
+            tab_rank[rank] = (uint16_t)e;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        const int last = E / kXcd, place = last % 2 ? kXcd - 1 - xcd : xcd;
+        L_first = blockIdx.x / kXcd;
+        L_end = (last + (place < E % kXcd ? 1 : 0)) * per_expert;
+    }
 
     // ---- what a cursor knows about a tile; every field wave-uniform
     // DX with a second term (a2, b2 shaped like a, b): the tile's reduction runs over (a, b) and goes on over
@@ -345,7 +384,10 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
     };
     auto tile_at = [&](int L, Tile &t) {
         if (MODE == MODE_DW) {
-            const int e = L / per_expert, local = L % per_expert;
+            const int slot = L / per_expert, local = L % per_expert;
+            const int e = by_size ? __builtin_amdgcn_readfirstlane(
+                                        tab_rank[slot * kXcd + (slot % 2 ? kXcd - 1 - xcd : xcd)])
+                                  : slot;
             t.i0 = (local / tiles_n) * BM;
             t.i_end = t.i0 + BM;
             t.j0 = (local % tiles_n) * BN;
@@ -923,7 +965,8 @@ int launch_wide(const void *a, const void *b, const void *m_sizes, int ms_i64, v
 #if defined(MFL_TUNING_BUILD) && defined(MFL_X_TRACE)
     constexpr int LDS_BYTES = 160 * 1024;
 #else
-    constexpr int LDS_BYTES = SR * STAGE_BYTES + 4 * 32 * EP_ROWB + 2 * (kMaxTableExperts + 1) * 4;
+    constexpr int LDS_BYTES = SR * STAGE_BYTES + 4 * 32 * EP_ROWB + 2 * (kMaxTableExperts + 1) * 4 +
+                              (MODE == MODE_DW ? kMaxTableExperts * 2 : 0);
 #endif
     static_assert(LDS_BYTES <= 160 * 1024, "LDS capacity of a CDNA4 compute unit");
     auto kern = gemm_wide_kernel<MODE, MB, NB, BK, SR, THIN, bf16_t>;
