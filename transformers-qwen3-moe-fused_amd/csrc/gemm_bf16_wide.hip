@@ -292,9 +292,11 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
     fo_a.init(wm * 32, WGM * 32, lane);
     fo_b.init(wn * WTN, 32, lane);
 
-    // ---- per-expert prefix tables in LDS behind the ring and the staging area: rows and tiles before expert e
+    // ---- per-expert prefix tables in LDS behind the ring and the staging area: rows and tiles before expert e; DW: first
+    // row, end of the rows and number of the expert in place e
     int *tab_rows = (int *)(smem + RING_BYTES + NW * EP_WAVE);
     int *tab_tiles = tab_rows + (kMaxTableExperts + 1);
+    uint16_t *tab_expert = (uint16_t *)(tab_tiles + (kMaxTableExperts + 1));
     const int tiles_n = MODE == MODE_DW ? K / BN : ceil_div(N, BN);  // row-grouped products: the last may be partial
     const int per_expert = MODE == MODE_DW ? (N / BM) * tiles_n : 0;
     {
@@ -302,11 +304,12 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
         for (int e0 = 0; e0 < E; e0 += 64) {
             const int e = e0 + lane;
             const int m = e < E ? load_msize(m_sizes, ms_i64, e) : 0;
-            const int t = e >= E ? 0 : MODE == MODE_DW ? per_expert : m_tiles_of<BM>(m) * tiles_n;
+            const int t = e >= E || MODE == MODE_DW ? 0 : m_tiles_of<BM>(m) * tiles_n;
             const int minc = wave_inclusive_scan(m), tinc = wave_inclusive_scan(t);
             if (wave == 0 && e <= E) {
                 tab_rows[e] = row_carry + minc - m;
-                tab_tiles[e] = tile_carry + tinc - t;
+                tab_tiles[e] = MODE == MODE_DW ? row_carry + minc : tile_carry + tinc - t;
+                if (MODE == MODE_DW && e < E) tab_expert[e] = (uint16_t)e;
             }
             row_carry += wave_last(minc);
             tile_carry += wave_last(tinc);
@@ -318,7 +321,7 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
     }
-    const int total = __builtin_amdgcn_readfirstlane(tab_tiles[E]);
+    const int total = MODE == MODE_DW ? E * per_expert : __builtin_amdgcn_readfirstlane(tab_tiles[E]);
 
     // ---- tile range of this workgroup: XCD x owns a contiguous run of logical tiles (the tiles of an expert meet
     // in one L2), dealt out with a stride inside the run
@@ -341,31 +344,52 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
     bool by_size = MODE == MODE_DW && E >= 4 * kXcd &&
                    ceil_div(ceil_div(E, kXcd) * per_expert, per_xcd) <= ceil_div(chunk, per_xcd);
     if (by_size) {
-        const int64_t rows = tab_rows[E];
+        const int64_t rows = __builtin_amdgcn_readfirstlane(tab_rows[E]);
         uint64_t hits = 0;
         for (int e0 = 0; e0 < E; e0 += 64) {
             const int e = e0 + lane < E ? e0 + lane : E - 1;
-            hits |= __ballot((int64_t)(tab_rows[e + 1] - tab_rows[e]) * 2 * E > 3 * rows);
+            hits |= __ballot((int64_t)(tab_tiles[e] - tab_rows[e]) * 2 * E > 3 * rows);
         }
         by_size = hits != 0 && rows >= (int64_t)96 * E;
     }
-    uint16_t *tab_rank = (uint16_t *)(tab_tiles + (kMaxTableExperts + 1));
     if (by_size) {
-        for (int e = threadIdx.x; e < E; e += 256) {
-            const int m = tab_rows[e + 1] - tab_rows[e];
-            int rank = 0, before = 0;
+        // XCD x's experts take the places from first_place(x) on
+        const int whole = E / kXcd, rest = E % kXcd;
+        auto dealt = [&](int q, int j) { return q % 2 ? kXcd - 1 - j : j; };
+        auto first_place = [&](int x) {
+            const int skip = whole % 2 ? x - (kXcd - rest) : x < rest ? x : rest;
+            return x * whole + (skip > 0 ? skip : 0);
+        };
+        constexpr int PER_THREAD = kMaxTableExperts / 256;
+        int begin[PER_THREAD], end[PER_THREAD], place[PER_THREAD];
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+            const int e = threadIdx.x + 256 * i;
+            if (e >= E) continue;
+            begin[i] = tab_rows[e], end[i] = tab_tiles[e];
+            const int m = end[i] - begin[i];
+            int rank = 0;
             for (int o = 0; o < E; ++o) {  // equal sizes in the experts' order
-                const int after = tab_rows[o + 1], mo = after - before;
+                const int mo = tab_tiles[o] - tab_rows[o];
                 rank += mo > m || (mo == m && o < e);
-                before = after;
             }
-            tab_rank[rank] = (uint16_t)e;
+            place[i] = first_place(dealt(rank / kXcd, rank % kXcd)) + rank / kXcd;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();  // every size is read
+#pragma unroll
+        for (int i = 0; i < PER_THREAD; ++i) {
+            const int e = threadIdx.x + 256 * i;
+            if (e >= E) continue;
+            tab_rows[place[i]] = begin[i];
+            tab_tiles[place[i]] = end[i];
+            tab_expert[place[i]] = (uint16_t)e;
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
-        const int last = E / kXcd, place = last % 2 ? kXcd - 1 - xcd : xcd;
-        L_first = blockIdx.x / kXcd;
-        L_end = (last + (place < E % kXcd ? 1 : 0)) * per_expert;
+        const int first = first_place(xcd);
+        L_first = first * per_expert + blockIdx.x / kXcd;
+        L_end = (first + whole + (dealt(whole, xcd) < rest ? 1 : 0)) * per_expert;
     }
 
     // ---- what a cursor knows about a tile; every field wave-uniform
@@ -384,15 +408,13 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
     };
     auto tile_at = [&](int L, Tile &t) {
         if (MODE == MODE_DW) {
-            const int slot = L / per_expert, local = L % per_expert;
-            const int e = by_size ? __builtin_amdgcn_readfirstlane(
-                                        tab_rank[slot * kXcd + (slot % 2 ? kXcd - 1 - xcd : xcd)])
-                                  : slot;
+            const int place = L / per_expert, local = L % per_expert;
+            const int e = __builtin_amdgcn_readfirstlane(tab_expert[place]);
             t.i0 = (local / tiles_n) * BM;
             t.i_end = t.i0 + BM;
             t.j0 = (local % tiles_n) * BN;
-            int rb = __builtin_amdgcn_readfirstlane(tab_rows[e]);
-            int re = __builtin_amdgcn_readfirstlane(tab_rows[e + 1]);
+            int rb = __builtin_amdgcn_readfirstlane(tab_rows[place]);
+            int re = __builtin_amdgcn_readfirstlane(tab_tiles[place]);
             if ((int64_t)re > R) re = (int)R;
             if (rb > re) rb = re;
             t.red = re - rb;
