@@ -1,0 +1,42 @@
+"""Which elements of the reduction the lanes of the packed matrix-vector kernel take, for every size that it is given."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "transformers-qwen3-moe-fused_amd", "csrc")
+
+PROGRAM = r"""
+#include <cstdio>
+#include <vector>
+#include "gemv_layout.h"
+int main() {
+    int wrong = 0;
+    for (int K = 320; K <= 2048; K += 64)
+        for (int N = 64; N <= 4096; N *= 2) {
+            const mfl::GemvLayout l = mfl::gemv_layout(K, N);
+            std::vector<int> taken(K);
+            bool whole = true;  // a lane's dwords are inside the row together or not at all where they lie side by side
+            for (int lane = 0; lane < l.lanes; ++lane)
+                for (int i = 0; i < l.dwords; ++i) {
+                    const int k = l.side_by_side ? (lane * l.dwords + i) * 8 : (i * l.lanes + lane) * 8;
+                    if (l.side_by_side && (lane * l.dwords * 8 < K) != (k < K)) whole = false;
+                    for (int u = 0; u < 8 && k < K; ++u) ++taken[k + u];
+                }
+            bool ok = whole && l.reach() >= K;
+            for (int t : taken) ok = ok && t == 1;
+            if (!ok && wrong++ < 8) std::printf("K = %d, N = %d: %d lanes of %d dwords\n", K, N, l.lanes, l.dwords);
+        }
+    return wrong ? 1 : 0;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
+def test_every_element_of_a_reduction_is_taken_once(tmp_path):
+    src, exe = tmp_path / "gemv_layout.cpp", tmp_path / "gemv_layout"
+    src.write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    run = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert run.returncode == 0, run.stdout

@@ -305,6 +305,40 @@ def test_matrix_vector_decode_kernel_edges(m_sizes, N, K, blocksize, ms_dtype, o
         assert torch.equal(y3[:R_short], y[:R_short]) and torch.all(y3[R_short] == 7.0)
 
 
+# A reduction of 960 is a multiple of 192, as 576 and 768 are, but longer than 16 lanes of six dwords reach: up to one and a half
+# rows per expert, on scales of either kind, plain, gated, and in the block at one token (hidden and inner size 960).
+@pytest.mark.parametrize("nested", [False, True])
+@pytest.mark.parametrize("m_sizes", [[1, 0, 2, 1], [0, 2, 1, 3]])
+def test_reductions_of_960(m_sizes, nested):
+    from qwen3_moe_fused.fused_mlp import moe_block_4bit
+    from qwen3_moe_fused.grouped_gemm.fused import grouped_glu_forward_4bit
+    from qwen3_moe_fused.quantize.layer import Nf4Params
+    from qwen3_moe_fused.quantize.nf4 import dequantize_nf4, quantize_nf4
+
+    E, R, K = len(m_sizes), sum(m_sizes), 960
+    ws = []
+    for s, shape in enumerate(((E, K, K), (E, K, K), (E, K, K))):
+        w = randn(shape, gen(s), K ** -0.5, torch.bfloat16).to(DEV)
+        packed, state = quantize_nf4(w, 64, compress_statistics=nested)
+        ws.append((packed, state, dequantize_nf4(packed, state, torch.float32).cpu().double()))
+    (g, gs, wg), (u, us, wu), (d, ds, wd) = ws
+    x = randn((R, K), gen(9), 1.0, torch.bfloat16)
+    ms, expert = torch.tensor(m_sizes, dtype=torch.int32).to(DEV), torch.arange(E).repeat_interleave(torch.tensor(m_sizes))
+    eg, eu = ((x.double()[:, None] @ w[expert].transpose(1, 2))[:, 0] for w in (wg, wu))
+    check_close(grouped_gemm_forward_4bit(x.to(DEV), g, gs, ms), eg.numpy(), atol=2e-2, what="plain")
+    for got, want in zip(grouped_glu_forward_4bit(x.to(DEV), g, gs, u, us, ms, return_products=True),
+                         (torch.nn.functional.silu(eg) * eu, eg, eu)):
+        check_close(got, want.numpy(), atol=2e-2, what="gated")
+    logits = torch.zeros((1, E))
+    logits[0, 2] = 4.0  # one expert of weight 1
+    with torch.no_grad():
+        out = moe_block_4bit(x[:1].to(DEV), logits.to(torch.bfloat16).to(DEV),
+                             *(Nf4Params(p, quant_state=s) for p, s in ((g, gs), (u, us), (d, ds))), 1, True)[0]
+    xs = x[0].double()
+    want = wd[2] @ (torch.nn.functional.silu(wg[2] @ xs) * (wu[2] @ xs))
+    check_close(out, want[None].numpy(), atol=2e-2, what="block at one token")
+
+
 from qwen3_moe_fused.grouped_gemm.forward_4bit import grouped_gemm_forward_transposed_4bit  # noqa: E402
 from qwen3_moe_fused.grouped_gemm.forward_transposed import grouped_gemm_forward_transposed  # noqa: E402
 

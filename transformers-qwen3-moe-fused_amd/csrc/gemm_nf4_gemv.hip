@@ -35,6 +35,7 @@
 
 #include "common.h"
 #include "gemm.h"
+#include "gemv_layout.h"
 
 namespace mfl {
 
@@ -496,6 +497,7 @@ template <int CL, int NL, int ROWS, int D, bool GLU, bool WIDE, bool NESTED, typ
 int launch_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf4Matrix &w0, const Nf4Matrix &w1,
                 const void *m_sizes, int ms_i64, TO *y, TO *e_out, TO *g_out, int64_t R, int N, int K, int E,
                 hipStream_t stream) {
+    if (K > 8 * CL * NL) return MFL_ERR_UNSUPPORTED;  // the lanes would leave the end of the reduction out
     const int64_t max_groups = R / ROWS + (R < E ? R : E);  // upper bound on sum over experts of ceil(m / ROWS)
     const int lds = kGemvTable + kGemvScales + (int)max_groups * 8 + 80 + E * 4;
     auto *kernel = nf4_gemv_kernel<CL, NL, ROWS, D, GLU, WIDE, NESTED, TO>;
@@ -679,7 +681,6 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
                   int K, int E, int out_dtype, hipStream_t stream) {
     if (R <= 0 || R > 2 * (int64_t)E || E > 2048) return MFL_ERR_UNSUPPORTED;  // a few rows per expert only
     const bool half = K <= 1024;
-    // (by the sizes alone: the gated form's products are the same bits as the plain one's, whatever either matrix's blocks)
     const bool wide = K % 32 == 0;
     // Ahead of the streaming form, or even, up to two rows per expert of long reductions and 1.5 of short ones (128 experts,
     // gated / plain us, H = 2048, I = 768, fp32 scales: 48 / 26 against 57 / 27 at 1.5 rows, 58 / 31 against 58 / 31 at 2; I
@@ -688,7 +689,7 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
     // 20 at 1.5, 41 / 23 against 38 / 20 at 2).  Short reductions whose lanes take their dwords apart: up to a row per
     // expert (35.0 against 30.4 at 2).
     if (2 * R > (int64_t)E * (!half ? 4 : wide ? 3 : 2)) return MFL_ERR_UNSUPPORTED;
-    if (K % 8 != 0 || K > 2048 || K <= 256) return MFL_ERR_UNSUPPORTED;
+    if (K % 32 != 0 || K > 2048 || K <= 256) return MFL_ERR_UNSUPPORTED;
     // whole units (32 columns; 16 in the gated form with 64 lanes to a column); fewer than 2^31 units in all
     if (N % ((glu && !half) ? 16 : 32) != 0 || N > (1 << 18)) return MFL_ERR_UNSUPPORTED;
     const Nf4Matrix *mats[2] = {&w0, &w1};
@@ -703,15 +704,10 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
     if (!aligned(x, 16)) return MFL_ERR_UNSUPPORTED;
 #define MFL_GEMV_D(CL, NL, ROWS, WIDE) \
     dispatch_gemv<CL, NL, ROWS, WIDE>(x, row_idx, idx_div, w0, w1, glu, m_sizes, ms_i64, y, e_out, g_out, R, N, K, E, out_dtype, stream)
-    if (!half) return wide ? MFL_GEMV_D(64, 4, 2, true) : MFL_GEMV_D(64, 4, 2, false);
-    // (16 lanes: plain product, N = 2048, 16 tokens of 8 experts each, fp32 / 8-bit scales: K = 768 22.1 / 25.6 -> 19.9 / 20.2
-    // us, K = 512 21.4 / 25.1 -> 15.8 / 16.8.  K = 1024 with eight dwords a lane spills: 25.8 -> 30.9.)
-    if (wide && N % 64 == 0) {
-        if (K > 512 && K % 192 == 0) return MFL_GEMV_D(16, 6, 2, true);
-        if (K <= 512) return MFL_GEMV_D(16, 4, 2, true);
-    }
-    if (K <= 768) return MFL_GEMV_D(32, 3, 2, false);
-    return wide ? MFL_GEMV_D(32, 4, 2, true) : MFL_GEMV_D(32, 4, 2, false);
+    const GemvLayout l = gemv_layout(K, N);
+    if (l.lanes == 64) return MFL_GEMV_D(64, 4, 2, true);
+    if (l.lanes == 16) return l.dwords == 6 ? MFL_GEMV_D(16, 6, 2, true) : MFL_GEMV_D(16, 4, 2, true);
+    return l.dwords == 3 ? MFL_GEMV_D(32, 3, 2, false) : MFL_GEMV_D(32, 4, 2, true);
 #undef MFL_GEMV_D
 }
 
