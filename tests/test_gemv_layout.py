@@ -1,4 +1,5 @@
-"""Which elements of the reduction the lanes of the packed matrix-vector kernel take, for every size that it is given."""
+"""Which elements of the reduction the lanes of the packed matrix-vector kernel take, and under how many scales they lie, for
+every size and block size that it is given."""
 import os
 import shutil
 import subprocess
@@ -14,8 +15,9 @@ PROGRAM = r"""
 int main() {
     int wrong = 0;
     for (int K = 320; K <= 2048; K += 64)
-        for (int N = 64; N <= 4096; N *= 2) {
-            const mfl::GemvLayout l = mfl::gemv_layout(K, N);
+        for (int at = 0; at < 4 * 6; ++at) {
+            const int N = 32 << at % 4, bs_shift = 3 + at / 4;
+            const mfl::GemvLayout l = mfl::gemv_layout(K, N, bs_shift);
             std::vector<int> taken(K);
             bool whole = true;  // a lane's dwords are inside the row together or not at all where they lie side by side
             for (int lane = 0; lane < l.lanes; ++lane)
@@ -24,9 +26,17 @@ int main() {
                     if (l.side_by_side && (lane * l.dwords * 8 < K) != (k < K)) whole = false;
                     for (int u = 0; u < 8 && k < K; ++u) ++taken[k + u];
                 }
+            // side by side, the kernel loads one scale for a lane's four dwords and two for six, of which the second is that of
+            // the dwords past a multiple of 64
+            if (l.side_by_side)
+                for (int lane = 0; lane < l.lanes; ++lane)
+                    for (int k = lane * l.dwords * 8, first = k; k < first + l.dwords * 8; ++k) {
+                        const int loaded = l.dwords == 6 && (k ^ first) >> 6 != 0 ? first + 40 : first;
+                        if (k < K && k >> bs_shift != loaded >> bs_shift) whole = false;
+                    }
             bool ok = whole && l.reach() >= K;
             for (int t : taken) ok = ok && t == 1;
-            if (!ok && wrong++ < 8) std::printf("K = %d, N = %d: %d lanes of %d dwords\n", K, N, l.lanes, l.dwords);
+            if (!ok && wrong++ < 8) std::printf("K = %d, N = %d, blocks of %d: %d lanes of %d dwords\n", K, N, 1 << bs_shift, l.lanes, l.dwords);
         }
     return wrong ? 1 : 0;
 }
@@ -34,7 +44,7 @@ int main() {
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
-def test_every_element_of_a_reduction_is_taken_once(tmp_path):
+def test_every_element_of_a_reduction_is_taken_once_and_under_its_scale(tmp_path):
     src, exe = tmp_path / "gemv_layout.cpp", tmp_path / "gemv_layout"
     src.write_text(PROGRAM)
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC, str(src), "-o", str(exe)], check=True)

@@ -247,10 +247,10 @@ def test_tile_ordered_scales_shapes_without_a_copy():
     check_close(y, oracle.linear_fwd(to_np32(x), w_deq, oracle.sel_from_m_sizes(ms.numpy())), what="ignored copy")
 
 
-# The matrix-vector kernel (at most two rows per expert on average, 256 < K <= 2048, K a multiple of the block
-# size, N a multiple of 32; up to K = 1024 with 32 lanes to a column): lanes past the end of a row (K not a multiple of 512), experts of one to five rows
-# (up to three row groups), empty experts, more than 64 experts, more units than workgroups and fewer, one
-# block per row, 64-bit counts, fp32 output, rows past sum(m_sizes).
+# The matrix-vector kernel (at most two rows per expert on average, 1.5 up to K = 1024; 256 < K <= 2048, K a multiple of 64 and of
+# the block size, N a multiple of 32): lanes past the end of a row, experts of one to five rows (up to three row groups), empty
+# experts, more than 64 experts, more units than workgroups and fewer, one block per row, 64-bit counts, fp32 output, rows
+# past sum(m_sizes); blocks smaller than a lane's run, whose lanes take their dwords apart.
 @pytest.mark.parametrize("m_sizes,N,K,blocksize,ms_dtype,out_dtype", [
     ([1, 0, 2, 1], 32, 2048, 64, torch.int32, torch.bfloat16),
     ([5, 0, 0, 0, 1, 0, 0, 0], 96, 1280, 128, torch.int64, torch.bfloat16),
@@ -258,11 +258,27 @@ def test_tile_ordered_scales_shapes_without_a_copy():
     ([2, 1, 0, 1, 0, 0], 288, 1536, 512, torch.int32, torch.bfloat16),
     ([1, 2, 0, 1, 3, 0, 0, 1], 768, 2048, 64, torch.int64, torch.bfloat16),
     ([1, 1], 32, 1088, 64, torch.int32, torch.bfloat16),
-    ([0, 0, 0, 4], 64, 1032, 8, torch.int32, torch.float32),
-    ([1, 0, 2, 0], 96, 1248, 32, torch.int32, torch.bfloat16),
-    # 32 lanes to a column (K <= 1024, at most a row per expert on average) from here on
+    ([1, 0, 2, 0], 96, 1344, 32, torch.int32, torch.bfloat16),
+    ([1, 0, 2, 0], 96, 1088, 16, torch.int32, torch.bfloat16),
+    ([0, 2, 1, 0, 0], 64, 2048, 8, torch.int64, torch.float32),
+    # 32 lanes to a column (768 < K <= 1024, or N no multiple of 64) from here on
     ([1, 2, 0, 1, 0, 0, 0, 1], 2048, 768, 64, torch.int32, torch.bfloat16),
     ([2, 0, 0], 32, 1024, 128, torch.int64, torch.float32),
+    ([1, 0, 2, 0, 3, 0], 96, 896, 64, torch.int32, torch.bfloat16),
+    ([1, 0, 2, 0], 96, 960, 32, torch.int32, torch.bfloat16),
+    ([0] * 66 + [1, 2], 64, 832, 8, torch.int32, torch.bfloat16),
+    ([1, 2, 0, 1], 64, 1024, 16, torch.int32, torch.bfloat16),
+    # the same three dwords a lane
+    ([1, 0, 2, 0], 96, 640, 128, torch.int32, torch.bfloat16),
+    ([1, 2, 0, 2, 1, 0], 64, 704, 64, torch.int32, torch.float32),
+    ([2, 1, 0, 2, 1, 0], 64, 768, 32, torch.int32, torch.bfloat16),
+    ([1, 0, 1, 0], 128, 768, 8, torch.int32, torch.bfloat16),
+    ([1, 2, 0, 0], 64, 576, 16, torch.int32, torch.float32),
+    ([1, 0, 2, 1], 64, 512, 16, torch.int32, torch.bfloat16),
+    ([1, 0, 1, 0, 0, 0, 3], 96, 320, 8, torch.int32, torch.bfloat16),
+    # rows of another length run elsewhere
+    ([0, 0, 0, 4], 64, 1032, 8, torch.int32, torch.float32),
+    ([1, 0, 2, 0], 96, 1248, 32, torch.int32, torch.bfloat16),
     ([1, 0, 1, 0, 0, 0, 3], 96, 264, 8, torch.int32, torch.bfloat16),
     ([0] * 66 + [1, 2], 64, 520, 8, torch.int32, torch.bfloat16),
     ([1, 0, 2, 0], 96, 928, 32, torch.int32, torch.bfloat16),
@@ -271,13 +287,15 @@ def test_tile_ordered_scales_shapes_without_a_copy():
     ([1, 0, 0, 2, 0], 192, 576, 64, torch.int64, torch.bfloat16),
     ([1, 1, 0], 128, 512, 32, torch.int32, torch.bfloat16),
     ([3, 0, 0, 0], 64, 320, 64, torch.int32, torch.float32),
+    ([1, 2, 0, 3, 0, 0], 64, 576, 64, torch.int32, torch.bfloat16),
+    ([1, 0, 2, 3], 64, 384, 32, torch.int32, torch.bfloat16),
 ])
 def test_matrix_vector_decode_kernel_edges(m_sizes, N, K, blocksize, ms_dtype, out_dtype):
     E = len(m_sizes)
     ms = torch.tensor(m_sizes, dtype=ms_dtype)
-    pad = min(3, (2 * E if K > 1024 else E) - int(ms.sum()))   # rows past the last expert: not written
+    pad = min(3, (4 * E if K > 1024 else 3 * E) // 2 - int(ms.sum()))   # rows past the last expert: not written
     R = int(ms.sum()) + pad
-    assert R <= (2 * E if K > 1024 else E) and 256 < K <= 2048 and K % blocksize == 0 and N % 32 == 0
+    assert pad >= 0 and 256 < K <= 2048 and K % blocksize == 0 and N % 32 == 0
     packed, state, w_deq = _quantised(E, N, K, blocksize, N + K)
     x = randn((R, K), gen(K), 1.0, torch.bfloat16)
     sel = oracle.sel_from_m_sizes(np.asarray(m_sizes))
@@ -303,6 +321,35 @@ def test_matrix_vector_decode_kernel_edges(m_sizes, N, K, blocksize, ms_dtype, o
                                          E, _lib.dtype_code(torch.bfloat16), _lib.dtype_code(out_dtype), _lib.stream())
         _lib.check(rc, "mfl_gemm_fwd_nf4")
         assert torch.equal(y3[:R_short], y[:R_short]) and torch.all(y3[R_short] == 7.0)
+
+
+# Gated products in small blocks and in blocks that differ between the matrices: blocks smaller than a lane's run of either
+# matrix take the lanes of both apart.  Against the oracle on the gate's and up's products, which equal blocks give the bits of
+# the plain ones.
+@pytest.mark.parametrize("m_sizes,N,K,blocks", [
+    ([1, 0, 2, 1], 64, 2048, (16, 16)), ([1, 0, 2, 0], 64, 1088, (64, 8)), ([2, 1, 0, 0], 96, 1024, (8, 8)),
+    ([1, 0, 2, 3], 64, 832, (16, 64)), ([1, 0, 1, 0], 64, 768, (32, 32)), ([1, 2, 0, 0], 64, 768, (64, 32)),
+    ([2, 0, 1, 3], 64, 576, (8, 64)), ([1, 2, 0, 1], 64, 512, (16, 16)), ([1, 0, 2, 3], 64, 512, (32, 64)),
+    ([1, 0, 2, 0], 64, 320, (64, 16))])
+@pytest.mark.parametrize("nested", [False, True])
+def test_gated_matrix_vector_kernel_in_small_and_unequal_blocks(m_sizes, N, K, blocks, nested):
+    from qwen3_moe_fused.grouped_gemm.fused import grouped_glu_forward_4bit
+    from qwen3_moe_fused.kernels.silu_mul import silu_mul_forward
+    from qwen3_moe_fused.quantize.nf4 import dequantize_nf4, quantize_nf4
+
+    E, R = len(m_sizes), sum(m_sizes)
+    ws = [quantize_nf4(randn((E, N, K), gen(s), K ** -0.5, torch.bfloat16).to(DEV), b, compress_statistics=nested)
+          for s, b in enumerate(blocks)]
+    x = randn((R, K), gen(K + N), 1.0, torch.bfloat16)
+    ms = torch.tensor(m_sizes, dtype=torch.int32).to(DEV)
+    h, e, g = grouped_glu_forward_4bit(x.to(DEV), *ws[0], *ws[1], ms, return_products=True)
+    for got, (packed, state) in zip((e, g), ws):
+        ref = oracle.linear_fwd(to_np32(x), to_np32(dequantize_nf4(packed, state, torch.float32)),
+                                oracle.sel_from_m_sizes(np.asarray(m_sizes)))
+        check_close(got, ref, atol=2e-2, what=f"K={K} blocks={blocks}")
+        if blocks[0] == blocks[1]:
+            assert torch.equal(got, grouped_gemm_forward_4bit(x.to(DEV), packed, state, ms))
+    assert torch.equal(h, silu_mul_forward(e, g))
 
 
 # A reduction of 960 is a multiple of 192, as 576 and 768 are, but longer than 16 lanes of six dwords reach: up to one and a half

@@ -8,7 +8,7 @@
 //     lane takes a column of K = 2048, and the lane's weights lie under one scale.  (With the lanes' dwords 64 dwords
 //     apart a column took four loads of weights and four of scales, eight of 8-bit ones, which spilled: 16 tokens of 8
 //     experts out of 128, gated, N = 768, fp32 / 8-bit scales 40.8 / 51.2 -> 36.8 / 37.3 us; one token 8.2 / 12.0 -> 8.5 /
-//     9.2.  Rows that are no multiple of 32 elements still take that form.)
+//     9.2.  Blocks of fewer weights than a lane's run still take that form.)
 //   * the rows of the group (up to two of one expert) stay in registers for all columns of the group: 16
 //     bytes per lane, load and row.
 //   * a byte of packed weights is two weights and one dword of bf16 pairs: a 256-entry table in LDS holds
@@ -28,8 +28,7 @@
 //   What the loop is short of, with 16 waves to a CU, is issue slots, scalar ones first: addresses move by
 //   increments, the row count is branched on once per column, and the lookups of a dword wait once.
 //
-// The product is the sum over pieces of 32 weights (16 of six dwords a lane, 8 where the dwords lie apart or the blocks are
-// smaller) of absmax * (x . bf16(code)), as in the streaming form.
+// The product is the sum over pieces of 32 weights (16 of six dwords a lane, 8 where the dwords lie apart) of absmax * (x . bf16(code)), as in the streaming form.
 #include <mutex>
 #include <type_traits>
 
@@ -330,7 +329,7 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
     // ---- the loop over the columns
     uint4_t xr[ROWS][NL];
     int cg = ig0, cc = ic0;  // cursor of the arithmetic
-    int rows = 0, row0 = 0, o_col = cc * UCOLS, ge_now = 0;
+    int rows = 0, row0 = 0, o_col = cc * UCOLS;
     int64_t o_row[ROWS];  // where the wave's column of unit 0 is in the output, per row of the group
     bool fresh = true;
     float first[ROWS];  // the gate projection's sums (of a lane, or finished), until the up projection's are there
@@ -341,7 +340,6 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
                 fresh = false;
                 const int ge = __builtin_amdgcn_readfirstlane(grp_e[cg]);
                 rows = ge >> 16;
-                ge_now = ge;
                 row0 = __builtin_amdgcn_readfirstlane(grp_r[cg]);
 #pragma unroll
                 for (int r = 0; r < ROWS; ++r) {
@@ -366,23 +364,22 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
             // the branches below they would land in different registers per branch, and the copy that reconciles
             // them would wait for the load just issued)
             // the arithmetic of the two columns for RN rows: one branch on the number of rows per unit, none inside
-            auto arithmetic = [&](auto RN, auto FINE) {
+            auto arithmetic = [&](auto RN) {
                 constexpr int rn = decltype(RN)::value;
-                constexpr bool fine = decltype(FINE)::value;  // a lane's dwords lie under more scales than the ring holds
                 float acc[COLS][rn];
 #pragma unroll
                 for (int c = 0; c < COLS; ++c)
 #pragma unroll
                     for (int r = 0; r < rn; ++r) acc[c][r] = 0.f;
                 float scale[COLS][NS], part[COLS][rn];
-                constexpr int RUN = fine || !WIDE ? 1 : TWO ? 2 : NL;  // dwords whose products are summed before they are scaled
+                constexpr int RUN = TWO ? 2 : WIDE ? NL : 1;  // dwords whose products are summed before they are scaled
 #pragma unroll
                 for (int i = 0; i < NL; ++i) {
 #pragma unroll
                     for (int c = 0; c < COLS; ++c) {
                         uint32_t pr[4];
                         const uint32_t w = ring_w[d][c][i];
-                        if (NESTED && !fine && i < NS) {
+                        if (NESTED && i < NS) {
                             float q;
                             lookup5(pr, q, pair_address<0>(w, lane_copy), pair_address<1>(w, lane_copy),
                                     pair_address<2>(w, lane_copy), pair_address<3>(w, lane_copy),
@@ -391,19 +388,9 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
                         } else {
                             lookup4(pr, pair_address<0>(w, lane_copy), pair_address<1>(w, lane_copy),
                                     pair_address<2>(w, lane_copy), pair_address<3>(w, lane_copy));
-                            if (!fine && i < NS) scale[c][i] = ring_a[d][c][i];
+                            if (i < NS) scale[c][i] = ring_a[d][c][i];
                         }
-                        float under;
-                        if constexpr (fine) {
-                            const int64_t at = ((int64_t)(ge_now & 0xffff) * N + cc * UCOLS + wave + 16 * (SUB > 1 ? lane / CL : c)) * K + x_off[i];
-                            const int64_t b = at >> mat[cb].bs_shift;
-                            if constexpr (NESTED)
-                                under = ((const float *)(table + kGemvTable))[cb * 256 + mat[cb].absmax_u8[b]] * mat[cb].absmax2[b >> mat[cb].bs2_shift] + q_off[cb];
-                            else
-                                under = mat[cb].absmax[b];
-                        } else {
-                            under = TWO && i > 1 && ((x_off[i] ^ x_off[0]) >> 6) != 0 ? scale[c][NS - 1] : scale[c][WIDE ? 0 : i];
-                        }
+                        const float under = TWO && i > 1 && ((x_off[i] ^ x_off[0]) >> 6) != 0 ? scale[c][NS - 1] : scale[c][WIDE ? 0 : i];
 #pragma unroll
                         for (int r = 0; r < rn; ++r) {
                             float s = dot2_bf16(pr[0], xr[r][i][0], i % RUN == 0 ? 0.f : part[c][r]);
@@ -448,7 +435,6 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
                 if (SUB > 1 ? lane % CL == CL - 1 : COLS == 2 ? (lane & 31) == 31 : lane == 63) {  // one lane per column
 #pragma unroll
                     for (int r = 0; r < rn; ++r) {
-                        if (fine && r >= rows) continue;
                         const int64_t o = o_row[r] + o_col;
                         if constexpr (GLU) {
                             const bf16_t pe = (bf16_t)first[r], pg = (bf16_t)tot[r];
@@ -462,13 +448,10 @@ __global__ __launch_bounds__(kGemvThreads) void nf4_gemv_kernel(const bf16_t *__
                 }
             };
             static_assert(ROWS == 2, "");
-            typedef std::integral_constant<bool, false> ring_scales;
-            if (WIDE && mat[cb].bs_shift < (TWO ? 6 : 5))
-                arithmetic(std::integral_constant<int, 2>(), std::integral_constant<bool, WIDE>());
-            else if (rows == 1)
-                arithmetic(std::integral_constant<int, 1>(), ring_scales());
+            if (rows == 1)
+                arithmetic(std::integral_constant<int, 1>());
             else
-                arithmetic(std::integral_constant<int, 2>(), ring_scales());
+                arithmetic(std::integral_constant<int, 2>());
             if (more) issue(d);
             if (cb == CB - 1) {
                 o_col += UCOLS;
@@ -663,8 +646,9 @@ template <int CL, int NL, int ROWS, bool WIDE>
 int dispatch_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf4Matrix &w0, const Nf4Matrix &w1,
                   bool glu, const void *m_sizes, int ms_i64, void *y, void *e_out, void *g_out, int64_t R, int N,
                   int K, int E, int out_dtype, hipStream_t stream) {
+// (four scales a column of 8-bit values and factors: two columns ahead, four spill: 128 rows, K = 1024, gated 84 -> 62 us)
 #define MFL_GEMV(GLU, TO, Y, EO, GO)                                                                               \
-    (w0.nested() ? launch_gemv<CL, NL, ROWS, ((NL <= 4 && (GLU || CL < 64)) ? 4 : 2), GLU, WIDE, true, TO>(                        \
+    (w0.nested() ? launch_gemv<CL, NL, ROWS, ((NL <= (WIDE ? 4 : 3) && (GLU || CL < 64)) ? 4 : 2), GLU, WIDE, true, TO>( \
                        x, row_idx, idx_div, w0, w1, m_sizes, ms_i64, Y, EO, GO, R, N, K, E, stream)                 \
                  : launch_gemv<CL, NL, ROWS, ((NL <= 4 && (GLU || CL < 64)) ? 4 : 2), GLU, WIDE, false, TO>(                       \
                        x, row_idx, idx_div, w0, w1, m_sizes, ms_i64, Y, EO, GO, R, N, K, E, stream))
@@ -681,14 +665,15 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
                   int K, int E, int out_dtype, hipStream_t stream) {
     if (R <= 0 || R > 2 * (int64_t)E || E > 2048) return MFL_ERR_UNSUPPORTED;  // a few rows per expert only
     const bool half = K <= 1024;
-    const bool wide = K % 32 == 0;
+    const int smallest = glu && w1.bs_shift < w0.bs_shift ? w1.bs_shift : w0.bs_shift;
+    const GemvLayout l = gemv_layout(K, N, smallest);
     // Ahead of the streaming form, or even, up to two rows per expert of long reductions and 1.5 of short ones (128 experts,
     // gated / plain us, H = 2048, I = 768, fp32 scales: 48 / 26 against 57 / 27 at 1.5 rows, 58 / 31 against 58 / 31 at 2; I
     // = 512: 32 / 18 against 39 / 20 at 1.5, 39 / 22 against 40 / 20 at 2; 8-bit ones, whose sums are the same bits and the
     // line therefore the same: 53 / 30 against 54 / 28 at 1.75, 59 / 32 against 55 / 30 at 2; I = 512: 34 / 19 against 37 /
     // 20 at 1.5, 41 / 23 against 38 / 20 at 2).  Short reductions whose lanes take their dwords apart: up to a row per
     // expert (35.0 against 30.4 at 2).
-    if (2 * R > (int64_t)E * (!half ? 4 : wide ? 3 : 2)) return MFL_ERR_UNSUPPORTED;
+    if (2 * R > (int64_t)E * (!half ? 4 : 3)) return MFL_ERR_UNSUPPORTED;
     if (K % 32 != 0 || K > 2048 || K <= 256) return MFL_ERR_UNSUPPORTED;
     // whole units (32 columns; 16 in the gated form with 64 lanes to a column); fewer than 2^31 units in all
     if (N % ((glu && !half) ? 16 : 32) != 0 || N > (1 << 18)) return MFL_ERR_UNSUPPORTED;
@@ -702,12 +687,12 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
             return MFL_ERR_UNSUPPORTED;
     }
     if (!aligned(x, 16)) return MFL_ERR_UNSUPPORTED;
-#define MFL_GEMV_D(CL, NL, ROWS, WIDE) \
-    dispatch_gemv<CL, NL, ROWS, WIDE>(x, row_idx, idx_div, w0, w1, glu, m_sizes, ms_i64, y, e_out, g_out, R, N, K, E, out_dtype, stream)
-    const GemvLayout l = gemv_layout(K, N);
-    if (l.lanes == 64) return MFL_GEMV_D(64, 4, 2, true);
-    if (l.lanes == 16) return l.dwords == 6 ? MFL_GEMV_D(16, 6, 2, true) : MFL_GEMV_D(16, 4, 2, true);
-    return l.dwords == 3 ? MFL_GEMV_D(32, 3, 2, false) : MFL_GEMV_D(32, 4, 2, true);
+#define MFL_GEMV_D(CL, NL, WIDE) \
+    dispatch_gemv<CL, NL, 2, WIDE>(x, row_idx, idx_div, w0, w1, glu, m_sizes, ms_i64, y, e_out, g_out, R, N, K, E, out_dtype, stream)
+    if (l.lanes == 64) return l.side_by_side ? MFL_GEMV_D(64, 4, true) : MFL_GEMV_D(64, 4, false);
+    if (l.lanes == 16) return l.dwords == 6 ? MFL_GEMV_D(16, 6, true) : MFL_GEMV_D(16, 4, true);
+    if (l.dwords == 3) return MFL_GEMV_D(32, 3, false);
+    return l.side_by_side ? MFL_GEMV_D(32, 4, true) : MFL_GEMV_D(32, 4, false);
 #undef MFL_GEMV_D
 }
 

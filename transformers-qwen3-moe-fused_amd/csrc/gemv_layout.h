@@ -10,23 +10,32 @@ struct GemvLayout {
     constexpr int reach() const { return 8 * lanes * dwords; }  // longest reduction that it covers
 };
 
-// By the sizes alone (256 < K <= 2048, K % 32 == 0, N % 32 == 0): the gated form's products are the same bits as the plain one's.
-constexpr GemvLayout gemv_layout(int K, int N) {
-    if (K > 1024) return {64, 4, true};
+// 256 < K <= 2048, K % 32 == 0, N % 32 == 0; 1 << bs_shift: the smaller of the blocks of the one matrix or two.  A lane's run lies
+// under one scale (two, in blocks of 64, with six dwords), which is loaded once.  Smaller blocks take their dwords apart, where
+// neighbouring lanes load neighbouring scales: with the scales of a run each loaded where it is used, 128 experts and rows, blocks of
+// 8 / 16, us: K = 2048, N = 768 plain 41 / 30, gated 67 / 53, against 30 / 24 and 53 / 43 apart; K = 768, N = 2048 39 / 33 and 72 / 57
+// against 30 / 26 and 53 / 45, blocks of 32 30 and 52 against 24 and 42.  (With a run's scales in registers ahead 35 / 29 and 61 /
+// 51 at K = 2048: the lanes' loads of a scale lie in as many lines as there are lanes.  K = 512 in blocks of 16 alone is behind
+// apart, gated, 42 against 35.)  The gated form's products are the same bits as the plain one's where both matrices' blocks are
+// equal.
+constexpr GemvLayout gemv_layout(int K, int N, int bs_shift) {
+    const bool runs = bs_shift >= 5;
+    if (K > 1024) return {64, 4, runs};
     // (16 lanes: plain product, N = 2048, 16 tokens of 8 experts each, fp32 / 8-bit scales: K = 768 22.1 / 25.6 -> 19.9 / 20.2
     // us, K = 512 21.4 / 25.1 -> 15.8 / 16.8.  K = 1024 with eight dwords a lane spills: 25.8 -> 30.9.)
     if (N % 64 == 0) {
-        if (K <= 512) return {16, 4, true};
-        if (K <= 768 && K % 192 == 0) return {16, 6, true};
+        if (K <= 512 && runs) return {16, 4, true};
+        if (K > 512 && K <= 768 && K % 192 == 0 && bs_shift >= 6) return {16, 6, true};
     }
     if (K <= 768) return {32, 3, false};
-    return {32, 4, true};
+    return {32, 4, runs};
 }
 
 constexpr bool gemv_layouts_reach() {
     for (int K = 288; K <= 2048; K += 32)
         for (int N = 32; N <= 64; N += 32)
-            if (gemv_layout(K, N).reach() < K) return false;
+            for (int bs_shift = 3; bs_shift <= 6; ++bs_shift)
+                if (gemv_layout(K, N, bs_shift).reach() < K) return false;
     return true;
 }
 static_assert(gemv_layouts_reach(), "a layout leaves elements of the reduction out");
