@@ -36,6 +36,10 @@ int main() {
                     }
             bool ok = whole && l.reach() >= K;
             for (int t : taken) ok = ok && t == 1;
+            // with the dwords of a short reduction apart, past a row per expert the streaming kernel takes what it can
+            const int half_rows = mfl::gemv_half_rows(K, l, bs_shift);
+            const bool left = K <= 1024 && !l.side_by_side && K % 128 == 0 && bs_shift >= 6;
+            ok = ok && half_rows == (K > 1024 ? 4 : left ? 2 : 3);
             if (!ok && wrong++ < 8) std::printf("K = %d, N = %d, blocks of %d: %d lanes of %d dwords\n", K, N, 1 << bs_shift, l.lanes, l.dwords);
         }
     return wrong ? 1 : 0;

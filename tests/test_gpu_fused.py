@@ -39,11 +39,11 @@ def _quantised(E, N, K, blocksize, seed):
 
 def _nf4_atol(ref, K, *blocksizes, rows=None, experts=None):
     """The decode-size kernels that scale partial sums (see unit_scale_atol) take K % 128 == 0 with blocks of at
-    least 64 weights, and, with at most two rows per expert (one up to K = 1024), 256 < K <= 2048 with any block size that
+    least 64 weights, and, with at most two rows per expert (1.5 up to K = 1024), 256 < K <= 2048 with any block size that
     divides K:
     two percent of the output scale there, one percent of unit scale elsewhere."""
     streaming = K % 128 == 0 and min(blocksizes) >= 64
-    matrix_vector = (rows is not None and rows <= (2 if K > 1024 else 1) * experts and 256 < K <= 2048
+    matrix_vector = (rows is not None and rows <= (2 if K > 1024 else 1.5) * experts and 256 < K <= 2048
                      and all(K % b == 0 for b in blocksizes))
     if streaming or matrix_vector:
         return unit_scale_atol(ref, 2e-2)

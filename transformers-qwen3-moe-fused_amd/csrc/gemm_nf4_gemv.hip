@@ -667,13 +667,7 @@ int gemm_nf4_gemv(const bf16_t *x, const int32_t *row_idx, int idx_div, const Nf
     const bool half = K <= 1024;
     const int smallest = glu && w1.bs_shift < w0.bs_shift ? w1.bs_shift : w0.bs_shift;
     const GemvLayout l = gemv_layout(K, N, smallest);
-    // Ahead of the streaming form, or even, up to two rows per expert of long reductions and 1.5 of short ones (128 experts,
-    // gated / plain us, H = 2048, I = 768, fp32 scales: 48 / 26 against 57 / 27 at 1.5 rows, 58 / 31 against 58 / 31 at 2; I
-    // = 512: 32 / 18 against 39 / 20 at 1.5, 39 / 22 against 40 / 20 at 2; 8-bit ones, whose sums are the same bits and the
-    // line therefore the same: 53 / 30 against 54 / 28 at 1.75, 59 / 32 against 55 / 30 at 2; I = 512: 34 / 19 against 37 /
-    // 20 at 1.5, 41 / 23 against 38 / 20 at 2).  Short reductions whose lanes take their dwords apart: up to a row per
-    // expert (35.0 against 30.4 at 2).
-    if (2 * R > (int64_t)E * (!half ? 4 : 3)) return MFL_ERR_UNSUPPORTED;
+    if (2 * R > (int64_t)E * gemv_half_rows(K, l, smallest)) return MFL_ERR_UNSUPPORTED;
     if (K % 32 != 0 || K > 2048 || K <= 256) return MFL_ERR_UNSUPPORTED;
     // whole units (32 columns; 16 in the gated form with 64 lanes to a column); fewer than 2^31 units in all
     if (N % ((glu && !half) ? 16 : 32) != 0 || N > (1 << 18)) return MFL_ERR_UNSUPPORTED;

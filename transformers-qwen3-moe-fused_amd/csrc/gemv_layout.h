@@ -31,6 +31,20 @@ constexpr GemvLayout gemv_layout(int K, int N, int bs_shift) {
     return {32, 4, runs};
 }
 
+// Halves of a row per expert up to which the kernel is taken: where it is ahead of the one that would follow, or even.
+// Against the streaming kernel (K % 128 == 0, blocks of 64 and more), 128 experts, gated / plain us, H = 2048, I = 768, fp32
+// scales: 48 / 26 against 57 / 27 at 1.5 rows, 58 / 31 against 58 / 31 at 2; I = 512: 32 / 18 against 39 / 20 at 1.5, 39 / 22
+// against 40 / 20 at 2; K = 896: 59 / 32 against 59 / 33 at 1.5; 8-bit ones, whose sums are the same bits and the line
+// therefore the same: 53 / 30 against 54 / 28 at 1.75, 59 / 32 against 55 / 30 at 2; I = 512: 34 / 19 against 37 / 20 at 1.5,
+// 41 / 23 against 38 / 20 at 2.  Short reductions with the dwords apart are behind it past a row: K = 640, 1.125 rows 47 / 25
+// against 41 / 23, 1.5 rows 54 / 28 against 42 / 24, 8-bit scales 64 / 33 against 41 / 23.  What the streaming kernel does not take
+// goes to the register-decoding one, which is further behind: K = 704, 1.5 rows 54 / 29 against 61 / 33; K = 768 in blocks
+// of 32 58 / 31 against 78 / 41, of 16 60 / 33 against 127 / 69.
+constexpr int gemv_half_rows(int K, GemvLayout l, int bs_shift) {
+    const bool streams = K % 128 == 0 && bs_shift >= 6;
+    return K > 1024 ? 4 : streams && !l.side_by_side ? 2 : 3;
+}
+
 constexpr bool gemv_layouts_reach() {
     for (int K = 288; K <= 2048; K += 32)
         for (int N = 32; N <= 64; N += 32)
