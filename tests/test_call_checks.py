@@ -253,6 +253,35 @@ def test_thin_matrices_on_another_device_never_reach_the_copies(monkeypatch, els
     assert not lib.seen
 
 
+def _double_quantised(device, numel=4 * 16 * 16 // 64, blocksize2=4):
+    from qwen3_moe_fused.quantize.nf4 import BlockwiseState, Nf4QuantState, code_of
+
+    return Nf4QuantState(absmax=torch.ones(numel, dtype=torch.uint8, device=device), shape=(2, 16, 16),
+                         code=code_of("nf4", device), blocksize=64, quant_type="nf4", dtype=torch.bfloat16,
+                         offset=torch.zeros((), device=device),
+                         state2=BlockwiseState(absmax=torch.ones(-(-numel // blocksize2), device=device),
+                                               code=torch.zeros(256, device=device), blocksize=blocksize2))
+
+
+@pytest.mark.parametrize("states_on,rows_on_gpu", [("cpu", False), ("meta", False), ("meta", True)])
+def test_scales_on_another_device_than_the_rows_are_not_written_out(monkeypatch, states_on, rows_on_gpu):
+    """The scales are written out before the products, whose checks refuse weights that are not on the rows' GPU: with states
+    elsewhere (an offloaded layer), or with everything on the host, no kernel sees an address."""
+    from qwen3_moe_fused.kernels.fast_lora import fast_lora
+
+    if rows_on_gpu:
+        monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    lib = _Recorder({})
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    args = _lora_args(rows=64)
+    for i in (1, 6, 11):
+        args[i], args[i + 1] = torch.zeros((2 * 16 * 16 // 2, 1), dtype=torch.uint8), _double_quantised(states_on, 2 * 16 * 16 // 64)
+    with pytest.raises((AssertionError, RuntimeError)):
+        fast_lora(*args)
+    assert not any(name in ("mfl_nf4_write_out_scales", "mfl_nf4_unnest_absmax") for name, _ in lib.seen)
+
+
 def _router_and_rows():
     from qwen3_moe_fused.modular_qwen3_moe_fused import Qwen3MoeFusedRouter
 

@@ -122,7 +122,7 @@ def test_scales_of_several_matrices_written_out_at_once():
             nested.absmax, nested.state2, nested.offset = _quantize_absmax(scales, blocksize2)
         states.append(nested)
     plain = _weights(1, 8, 64, 64, 5)[2]
-    got = write_out_scales(states[0], plain, None, states[1], states[2])
+    got = write_out_scales(states[0].absmax, states[0], plain, None, states[1], states[2])
     assert got[1] is plain and got[2] is None
     for state, out in zip(states, (got[0], got[3], got[4])):
         assert not out.nested and torch.equal(out.absmax, resolve_absmax(state))

@@ -167,7 +167,7 @@ class FastLora(torch.autograd.Function):
         x = x.contiguous()
         Ag, Bg, Au, Bu, Aw, Bw = (p.to(dt).contiguous() for p in (Ag, Bg, Au, Bu, Aw, Bw))
         frozen_states = (Gqs, Uqs, Wqs)
-        Gqs, Uqs, Wqs = write_out_scales(Gqs, Uqs, Wqs)
+        Gqs, Uqs, Wqs = write_out_scales(x, Gqs, Uqs, Wqs)
         ug = uu = ucat = None
         if Sg == Su and Ag.shape == Au.shape and x.shape[0] >= _WIDE_ROWS:
             # one pass over x for both adapters' rank-r activations
@@ -208,7 +208,7 @@ class FastLora(torch.autograd.Function):
         dt = x.dtype
         dy = dy.contiguous()
         if ctx.needs_input_grad[0]:
-            Gqs, Uqs, Wqs = write_out_scales(Gqs, Uqs, Wqs)
+            Gqs, Uqs, Wqs = write_out_scales(dy, Gqs, Uqs, Wqs)
 
         # The rank-r activations carry the adapter's scaling (ug, uu, uw from the forward pass; tw, tu, tg here),
         # so every product below takes them as they are.

@@ -211,11 +211,12 @@ class _WrittenOut:
         self._mfl_absmax_tiled = (absmax, absmax._version, -1, None)  # (no tile-ordered copy for one pass)
 
 
-def write_out_scales(*states):
+def write_out_scales(rows: torch.Tensor, *states):
     """The states with the scales of the double-quantised ones (four at most) written out, all in one launch (three
-    matrices of 128 x 768 x 2048: 18.6 -> 11.6 us); others, and None, as they are."""
+    matrices of 128 x 768 x 2048: 18.6 -> 11.6 us); others, and None, as they are.  With scales that are not on the GPU of
+    ``rows`` all are left as they are: the products refuse them."""
     nested = [s for s in states if s is not None and getattr(s, "nested", False) and _is_shift(int(s.state2.blocksize))]
-    if not nested or len({s.absmax.device for s in nested}) != 1:
+    if not nested or not rows.is_cuda or any(s.absmax.device != rows.device for s in nested):
         return states
     out, keep = {}, []
     weights = (_lib.Nf4Weight * len(nested))()
