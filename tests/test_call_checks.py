@@ -282,6 +282,22 @@ def test_scales_on_another_device_than_the_rows_are_not_written_out(monkeypatch,
     assert not any(name in ("mfl_nf4_write_out_scales", "mfl_nf4_unnest_absmax") for name, _ in lib.seen)
 
 
+def test_scales_are_written_out_under_inference_mode(monkeypatch):
+    """A tensor made under inference mode has no version to ask for."""
+    from qwen3_moe_fused.quantize.nf4 import tiled_absmax, write_out_scales
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    lib = _Recorder({})
+    monkeypatch.setattr(_lib, "lib", lambda: lib)
+    state = _double_quantised("cpu", 2 * 16 * 16 // 64)
+    for mode in (torch.no_grad, torch.inference_mode):
+        with mode():
+            out, = write_out_scales(torch.zeros(2, 16), state)
+            assert out is not state and not out.nested and tiled_absmax(out, out.absmax, 2) is None
+    assert [name for name, _ in lib.seen] == ["mfl_nf4_write_out_scales"] * 2
+
+
 def _router_and_rows():
     from qwen3_moe_fused.modular_qwen3_moe_fused import Qwen3MoeFusedRouter
 

@@ -201,14 +201,13 @@ def resolve_absmax(quant_state) -> torch.Tensor:
 class _WrittenOut:
     """A double-quantised state with its fp32 scales, for the calls of one pass."""
 
-    __slots__ = ("absmax", "shape", "code", "blocksize", "quant_type", "dtype", "_mfl_absmax_tiled")
+    __slots__ = ("absmax", "shape", "code", "blocksize", "quant_type", "dtype")
     nested = False
 
     def __init__(self, state, absmax: torch.Tensor) -> None:
         self.absmax = absmax
         self.shape, self.code, self.blocksize = state.shape, state.code, state.blocksize
         self.quant_type, self.dtype = state.quant_type, state.dtype
-        self._mfl_absmax_tiled = (absmax, absmax._version, -1, None)  # (no tile-ordered copy for one pass)
 
 
 def write_out_scales(rows: torch.Tensor, *states):
@@ -259,6 +258,8 @@ def tiled_absmax(quant_state, absmax: torch.Tensor, rows: int):
     them (``mfl_nf4_tile_absmax``), built on the first decode-sized call and kept on the quant state; ``None``
     where it does not apply (a larger batch, a double-quantised state whose fp32 scales are rebuilt per call,
     a shape without such a copy).  Costs as many bytes again as ``absmax`` (3 % of the packed weights)."""
+    if isinstance(quant_state, _WrittenOut):  # (no copy for one pass)
+        return None
     cached = getattr(quant_state, "_mfl_absmax_tiled", None)
     if cached is not None and cached[0] is absmax and cached[1] == absmax._version:
         return cached[3] if rows <= cached[2] else None  # the path of every call but the first
