@@ -298,6 +298,28 @@ def test_scales_are_written_out_under_inference_mode(monkeypatch):
     assert [name for name, _ in lib.seen] == ["mfl_nf4_write_out_scales"] * 2
 
 
+def test_a_state_that_several_matrices_share_is_written_out_once(monkeypatch):
+    """The room for a state's scales is kept until the launch: a second piece for the same state would replace the first one,
+    whose memory the next state could get while the kernel still writes both."""
+    from qwen3_moe_fused.quantize.nf4 import write_out_scales
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    jobs = []
+
+    class Library:
+        def mfl_nf4_write_out_scales(self, weights, counts, ptrs, n, stream):
+            jobs.append([(counts[i], ptrs[i]) for i in range(n)])
+            return 0
+
+    monkeypatch.setattr(_lib, "lib", lambda: Library())
+    a, b = _double_quantised("cpu", 4096), _double_quantised("cpu", 4096)
+    outs = write_out_scales(torch.zeros(2, 16), a, a, b)
+    assert outs[0] is outs[1] and outs[2] is not outs[0]
+    assert jobs == [[(4096, outs[0].absmax.data_ptr()), (4096, outs[2].absmax.data_ptr())]]
+    assert outs[0].absmax.data_ptr() != outs[2].absmax.data_ptr()
+
+
 def _router_and_rows():
     from qwen3_moe_fused.modular_qwen3_moe_fused import Qwen3MoeFusedRouter
 

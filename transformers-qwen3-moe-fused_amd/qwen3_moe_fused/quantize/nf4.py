@@ -215,6 +215,7 @@ def write_out_scales(rows: torch.Tensor, *states):
     matrices of 128 x 768 x 2048: 18.6 -> 11.6 us); others, and None, as they are.  With scales that are not on the GPU of
     ``rows`` all are left as they are: the products refuse them."""
     nested = [s for s in states if s is not None and getattr(s, "nested", False) and _is_shift(int(s.state2.blocksize))]
+    nested = list({id(s): s for s in nested}.values())  # (a state that several matrices share: once)
     if not nested or not rows.is_cuda or any(s.absmax.device != rows.device for s in nested):
         return states
     out, keep = {}, []
