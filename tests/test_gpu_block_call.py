@@ -86,6 +86,28 @@ def test_block_call_on_packed_weights(t, e, k, h, i, kind):
     assert float((out[0] - out[1]).abs().max()) <= 2e-2 * float(out[1].abs().max())
 
 
+# blocks of 32: an inner size that is no multiple of 64 has another down projection, and its sum over the selections by itself
+@pytest.mark.parametrize("i", [288, 480, 320, 512])
+@pytest.mark.parametrize("kind", ["nf4", "nf4dq"])
+def test_block_call_on_packed_weights_in_blocks_of_32(i, kind):
+    from qwen3_moe_fused.quantize.layer import Nf4Params
+    from qwen3_moe_fused.quantize.nf4 import quantize_nf4
+
+    blk, dtype = _block(8, 2, 128, i, kind, 1)
+    for seed, name in enumerate(PROJ):
+        proj = getattr(blk, name)
+        w = torch.randn((8, proj.out_features, proj.in_features), generator=gen(seed)) * proj.in_features ** -0.5
+        packed, state = quantize_nf4(w.to(dtype).cuda(), 32, compress_statistics=kind == "nf4dq")
+        proj._parameters["weight"] = Nf4Params(packed, quant_state=state)
+    hidden = torch.randn((2, 1, 128), generator=gen(i)).to(dtype).cuda()
+    out = []
+    for fused in (True, False):
+        blk.fuse_front = fused
+        with torch.no_grad():
+            out.append(blk(hidden)[0])
+    assert torch.isfinite(out[0]).all() and torch.equal(out[0], out[1])
+
+
 def test_block_call_on_two_streams_and_with_a_hook():
     blk, _ = _block(8, 2, 64, 64, "bf16", 3)
     xs = [torch.randn((1, 40, 64), generator=gen(s)).to(torch.bfloat16).cuda() for s in range(2)]

@@ -55,8 +55,9 @@ def _close(a, b, tol):
     assert float((a.float() - b.float()).abs().max()) <= tol * max(1e-3, float(b.float().abs().max()))
 
 
-# one row per expert and more, one selection per token and more; the packed weights' three kernels
-@pytest.mark.parametrize("t,e,k,h,i", [(1, 8, 2, 64, 32), (3, 16, 4, 512, 128), (65, 16, 1, 128, 64), (300, 8, 8, 256, 96)])
+# one row per expert and more, one selection per token and more; the packed weights' three kernels, and (the third and fourth) the
+# down projection with the sum over the selections in one launch
+@pytest.mark.parametrize("t,e,k,h,i", [(1, 8, 2, 64, 32), (3, 16, 4, 512, 128), (1, 8, 2, 64, 512), (3, 16, 5, 512, 768), (65, 16, 1, 128, 64), (300, 8, 8, 256, 96)])
 @pytest.mark.parametrize("kind", ["bf16", "fp32", "nf4", "nf4dq"])
 @pytest.mark.parametrize("one_call", [True, False])
 def test_block_with_a_nan_token(t, e, k, h, i, kind, one_call):
