@@ -230,7 +230,11 @@ __global__ __launch_bounds__(kThreads) void gemm_generic_kernel(const TI *__rest
                     for (int u = 0; u < 4; ++u) o[u] = alpha * acc[i][j][u];
                     *(floatx4 *)(st + (lane & 15) * kOutRow + j * 16 + (lane >> 4) * 4) = o;
                 }
-                // (the same wave reads back what it wrote: LDS operations of one wave complete in order)
+                // The same wave reads back what it wrote, and its LDS operations complete in order; that lanes read what other
+                // lanes wrote, and overwrite what others read, has to be said (no instructions)
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
                 for (int q = lane; q < 16 * TN * 4; q += kWave) {
                     const int row_l = q / (TN * 4), col_l = (q % (TN * 4)) * 4;
@@ -243,6 +247,9 @@ __global__ __launch_bounds__(kThreads) void gemm_generic_kernel(const TI *__rest
                     else
                         *p = o;
                 }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             }
             return;
         }
