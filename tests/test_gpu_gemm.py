@@ -275,11 +275,15 @@ WIDE_DW_CASES = [
     (512, 256, [0, 0, 517, 0, 15, 16, 17, 480, 0]),
     (768, 256, [96] * 7 + [0] + [1000]),
     (256, 768, [70 + (3 * e) % 11 for e in range(130)]),
-    # skewed sizes over 32 experts and more (dealt out to the XCDs by size): full and partial last rounds of experts,
-    # equal sizes, experts without rows, several tiles a workgroup; then the same with too few rows, and just even enough
+    # skewed sizes over 32 experts and more (dealt out to the XCDs by size, the first four): rounds of tiles that end inside, to and
+    # fro, equal sizes, experts without rows; then outputs, sizes and numbers of experts that are left as they are
+    (512, 768, [1500 if e == 7 else 90 + e % 5 for e in range(48)]),
+    (1024, 512, [0 if e % 7 == 3 else 4200 // (e + 1) for e in range(43)]),
+    (768, 512, [900, 800, 0] + [97] * 98),
     (256, 256, [3200 if e == 5 else 33 * (e % 3) for e in range(32)]),
     (512, 256, [4000 // (e + 1) for e in range(37)] + [0, 0, 700, 700]),
     (768, 2048, [2500 if e == 32 else 90 - e for e in range(33)]),
+    (768, 512, [2000 if e == 200 else 95 for e in range(257)]),
     (256, 256, [2000 if e == 200 else 95 for e in range(201)]),
     (256, 256, [400] + [80] * 39),
     (256, 256, [150] + [100] * 39),

@@ -331,17 +331,28 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
     int L_first = xcd * chunk + blockIdx.x / kXcd;
     int L_end = (xcd + 1) * chunk;
     if (L_end > total) L_end = total;
+    int L_step = per_xcd;  // to a workgroup's next tile, then 2 * per_xcd - L_step to the one after it, and so on
+    auto next_tile = [&](int &L, int &step) {
+        L += step;
+        if (MODE == MODE_DW) step = 2 * per_xcd - step;
+    };
 
     // DW: the time of a tile is that of its expert's rows.  The experts are ranked by their rows and dealt out to the
-    // XCDs to and fro (0..7, 7..0, ...), and an XCD goes through its experts from the largest to the smallest, so
-    // that skewed routing leaves no XCD with the work of many popular experts and no late long tile.
+    // XCDs to and fro (0..7, 7..0, ...), an XCD goes through its experts from the largest to the smallest, and its workgroups
+    // take the tiles of a round to and fro as well, so that skewed routing leaves no XCD with the work of many popular
+    // experts, no workgroup with the larger tile of every round and no late long tile.
     // Where: an expert of more than 1.5 times the mean (even routing gains nothing: 181.7 against 177.6 us at 128
-    // experts x 768 x 2048, 256 rows each); at least four experts an XCD (16 experts: 94 against 89); at least 96 rows
-    // per expert on average (at 64 the time is that of the weights: 105 / 200 us against 101 / 210 at 128 / 256
-    // experts); and whole experts an XCD make no more rounds under even routing than runs of equal numbers.
-    // 32768 rows over 128 experts x 768 x 2048, largest expert 11 / 15 / 16 times the mean: 209 / 222 / 208 us
-    // against 235 / 273 / 285; 16384 rows 140 against 160; 8000 rows over 60 experts x 1536 x 2048 138 against 157.
-    bool by_size = MODE == MODE_DW && E >= 4 * kXcd &&
+    // experts x 768 x 2048, 256 rows each); more than one round of tiles (with one the ranking's time is lost: 160 experts x 256
+    // x 256, 16384 rows, 37.5 -> 43.5) of more than 512 x 512 an expert (512 x 512: 96 to 256 experts 0.96 to 1.2 times
+    // as long, the long tiles all wait for memory at once); 32 to 256 experts (16: 94 against 89; the ranking compares all with
+    // all, 512 experts of 256 x 256 123 -> 158); at least 96 rows per expert on average (at 64 the time is that of the
+    // weights: 105 / 200 us against 101 / 210 at 128 / 256 experts); and whole experts an XCD make no more rounds under even
+    // routing than runs of equal numbers.
+    // us before / with the experts ranked / and the tiles to and fro, 32768 rows, Zipf over the top 8: 128 experts x 768 x 2048,
+    // largest 11 / 16 times the mean, 239 / 211 / 208 and 292 / 213 / 207; 64 experts x 1024 x 2048 240 / 204 / 200; 48 experts x
+    // 512 x 768, 16384 rows, 45 / 52 / 46.  512 x 1024 of 160 and 192 experts is 3 to 9 % behind, of 48 to 128 and 256 5 to 25 %
+    // ahead.
+    bool by_size = MODE == MODE_DW && E >= 4 * kXcd && E <= 256 && chunk > per_xcd && per_expert > 4 &&
                    ceil_div(ceil_div(E, kXcd) * per_expert, per_xcd) <= ceil_div(chunk, per_xcd);
     if (by_size) {
         const int64_t rows = __builtin_amdgcn_readfirstlane(tab_rows[E]);
@@ -360,36 +371,32 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
             const int skip = whole % 2 ? x - (kXcd - rest) : x < rest ? x : rest;
             return x * whole + (skip > 0 ? skip : 0);
         };
-        constexpr int PER_THREAD = kMaxTableExperts / 256;
-        int begin[PER_THREAD], end[PER_THREAD], place[PER_THREAD];
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
-            const int e = threadIdx.x + 256 * i;
-            if (e >= E) continue;
-            begin[i] = tab_rows[e], end[i] = tab_tiles[e];
-            const int m = end[i] - begin[i];
+        const int e = threadIdx.x;
+        int begin = 0, end = 0, place = 0;
+        if (e < E) {
+            begin = tab_rows[e], end = tab_tiles[e];
+            const int m = end - begin;
             int rank = 0;
+#pragma unroll 8
             for (int o = 0; o < E; ++o) {  // equal sizes in the experts' order
                 const int mo = tab_tiles[o] - tab_rows[o];
                 rank += mo > m || (mo == m && o < e);
             }
-            place[i] = first_place(dealt(rank / kXcd, rank % kXcd)) + rank / kXcd;
+            place = first_place(dealt(rank / kXcd, rank % kXcd)) + rank / kXcd;
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();  // every size is read
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
-            const int e = threadIdx.x + 256 * i;
-            if (e >= E) continue;
-            tab_rows[place[i]] = begin[i];
-            tab_tiles[place[i]] = end[i];
-            tab_expert[place[i]] = (uint16_t)e;
+        if (e < E) {
+            tab_rows[place] = begin;
+            tab_tiles[place] = end;
+            tab_expert[place] = (uint16_t)e;
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         const int first = first_place(xcd);
         L_first = first * per_expert + blockIdx.x / kXcd;
         L_end = (first + whole + (dealt(whole, xcd) < rest ? 1 : 0)) * per_expert;
+        L_step = 2 * (per_xcd - (int)blockIdx.x / kXcd) - 1;
     }
 
     // ---- what a cursor knows about a tile; every field wave-uniform
@@ -482,7 +489,7 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
     constexpr bool SPLIT = NG >= 2 && (SR >= 3 || MB * NB >= 64);
     constexpr int NG1 = SPLIT ? (NG + 1) / 2 : NG;  // groups in the sub-step after point P
     Tile pt;
-    int pL = L_first, pk = 0, p_full = 0;  // p_full: steps of the producer's tile that are whole
+    int pL = L_first, p_step = L_step, pk = 0, p_full = 0;  // p_full: steps of the producer's tile that are whole
     // Row-grouped products: copy groups of A whose stage rows all lie past the tile's last row are left out (nothing
     // that is stored reads them): bit j of p_amask says that this wave issues group j, p_copies how many copies
     // a step of the producer's tile comes to for this wave.
@@ -525,7 +532,7 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
                 if (MODE != MODE_DW) prod_offsets();
                 break;
             }
-            pL += per_xcd;
+            next_tile(pL, p_step);
         }
         pk = 0;
         p_full = MODE == MODE_DW ? pt.red / BK : pt.KT - thin_steps;
@@ -656,7 +663,7 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
         pa_cur += step_a;
         pb_cur += step_b;
         if (++pk == pt.KT) {
-            pL += per_xcd;
+            next_tile(pL, p_step);
             prod_seek();
         } else if (MODE == MODE_DX && two_term && pk == K / BK) {
             // the second term starts at the beginning of its own operands
@@ -679,7 +686,7 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
 
     // ---- consumer
     Tile ct;
-    int cL = L_first;
+    int cL = L_first, c_step = L_step;
     unsigned g = 0;  // steps multiplied so far (of the whole workgroup)
     bf16x8 fa[2][TM], fb[2][TN];  // carried from step to step, across tiles
     // The fragment offsets carry the ring slot they read: moved on by one stage at point P.
@@ -733,7 +740,7 @@ __global__ __launch_bounds__(256) void gemm_wide_kernel(const bf16_t *__restrict
     constexpr int PPT = WTN / EPC;  // parts (32 rows x EPC columns) per row block
 
 #pragma unroll 1
-    for (; cL < L_end; cL += per_xcd) {
+    for (; cL < L_end; next_tile(cL, c_step)) {
         tile_at(cL, ct);
         const int i_lim = ct.i_end - ct.i0 < BM ? ct.i_end - ct.i0 : BM;
         const int n_blocks = ceil_div(i_lim, 32);
