@@ -320,10 +320,13 @@ int launch_tile(const Args &g) {
     // turn: 154 / 159 / 177, 559 us; with the gradient's rows put together in LDS 154 / 159 / 147, 507; that past the caches
     // 154 / 159 / 126, 446; the weights too 145 / 147 / 126, 411.  64 experts (403 MB) 293 -> 230.  Rows of 6048 bytes: weight
     // gradient 61 -> 96, input gradient 76 -> 83.  Experts with a second tile: input gradient at 16 rows per expert 187 ->
-    // 248, at 32 (32-row tiles) 231 -> 269.
+    // 248, at 32 (32-row tiles) 231 -> 269; at 8 under Zipf(1) routing 155 -> 171, the three in turn 549 -> 474.  Of the weights
+    // what counts is what is read, at most an expert's a row: 64 rows over 160 experts of 544 x 1056, which fit, 27 -> 29 past the
+    // caches.
     constexpr bool kNt = VEC == 4 && sizeof(TI) == 4 && (MODE == MODE_DW || BM <= 32);
     [[maybe_unused]] const void *const streamed = MODE == MODE_DW ? g.c : g.b;
-    [[maybe_unused]] const bool nt = (int64_t)g.E * g.N * g.K * 4 > ((int64_t)256 << 20) && aligned(streamed, 128) &&
+    const int64_t matrices = MODE != MODE_DW && g.R < g.E ? g.R : g.E;
+    [[maybe_unused]] const bool nt = matrices * g.N * g.K * 4 > ((int64_t)256 << 20) && aligned(streamed, 128) &&
                                      (MODE == MODE_DX ? g.N : g.K) % 32 == 0 &&
                                      (MODE == MODE_DW || 4 * g.R <= (int64_t)3 * BM * g.E);
     auto *kernel = gemm_generic_kernel<TI, TO, MODE, BM, BN, WM, WN, WK, BK, VEC, false>;
