@@ -556,6 +556,38 @@ def test_packed_gate_and_up_with_lora_terms(m_sizes, M, H, r, bs):
     check_close(dx, to_np32(two), atol=unit_scale_atol(to_np32(two), 2e-2), what="one reduction vs two products")
 
 
+# Both adapters' activations lie side by side against weights that are zero over the other's columns, and 0 x inf is NaN: an
+# infinite activation of one adapter makes the other matrix's product NaN in its row.  What leaves the unit is not finite in
+# that row either way, and no other row feels it.
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("column", [1, 9])
+def test_an_infinite_activation_of_an_adapter_stays_in_its_row(packed, column):
+    from qwen3_moe_fused.quantize.nf4 import dequantize_nf4
+
+    sizes, M, H, r, bad = [70, 0, 130], 128, 192, 8, 75
+    g = gen(M + column)
+    ms = torch.tensor(sizes, dtype=torch.int32).to(DEV)
+    ws = [quantize_nf4(randn((3, M, H), g, 0.05, torch.bfloat16).to(DEV), 64) for _ in range(2)]
+    x, u = (randn((200, n), g, 1.0, torch.bfloat16).to(DEV) for n in (H, 2 * r))
+    bg, bu = (randn((3, M, r), g, 0.2, torch.bfloat16).to(DEV) for _ in range(2))
+    zeros = torch.zeros_like(bg)
+    wide = [torch.cat(p, 2).contiguous() for p in ((bg, zeros), (zeros, bu))]
+
+    def both(u):
+        if packed:
+            return grouped_glu_forward_4bit_lora(x, *ws[0], *ws[1], u, *wide, ms)
+        return grouped_glu_forward_lora(x, *(dequantize_nf4(*w, torch.bfloat16) for w in ws), u, *wide, ms)
+
+    clean = both(u)
+    u[bad, column] = float("inf")
+    got = both(u)
+    rows = torch.arange(200, device=DEV) != bad
+    for a, b in zip(got, clean):
+        assert torch.isfinite(b).all() and torch.equal(a[rows], b[rows])
+    h, products = got[0][bad], got[1:]
+    assert not torch.isfinite(h).any() and not torch.isfinite(products[column >= r][bad]).any()
+
+
 # few experts or narrow outputs: 64 x 128 tiles, and 160 x 128 where those are too many to be resident at once (the fifth
 # and sixth, whose gated products have enough 256 x 256 tiles, and the gated product of the last); borders of tiles and row
 # blocks, experts without rows, columns that end inside a tile, odd numbers of steps

@@ -1,7 +1,8 @@
 // The sparse MoE block after its router projection, forward and backward, as one call each: the launches of
 // api.hip's entry points one behind the other, with every intermediate in one buffer of the caller's.  The kernels
 // and their results are those of the separate calls.  What it saves is the host's time between the launches: at
-// decode sizes the block is a chain of five kernels of 5 to 40 us, and preparing each from the caller's language
+// decode sizes the block is a chain of five kernels of 5 to 40 us (on packed weights four up to 16 selections, the down projection
+// with the sum over them in one), and preparing each from the caller's language
 // (a tensor per output, an autograd node per step) took longer than the kernels run: 118 us of host time against
 // 95 us of kernels at 16 tokens on packed weights, 690 us for a training step of a toy block whose kernels take 120.
 #include <initializer_list>
@@ -98,8 +99,8 @@ int spread_rows(const mfl_moe_block &b, const void *src, const char *ws, const L
     return mfl_gather_rows(src, (const int32_t *)(ws + l.sort), 1, scale, dst, b.T, b.H, b.dtype, stream);
 }
 
-// The matrices with the scales of double-quantised ones written out, matrix i's from out + i * scale_bytes on; others as
-// they are
+// The matrices (two at most) with the scales of double-quantised ones written out in one launch, matrix i's from out + i *
+// scale_bytes on; others as they are
 int write_out_scales(const mfl_moe_block &b, std::initializer_list<const mfl_nf4_weight *> from, mfl_nf4_weight *plain,
                      char *out, size_t scale_bytes, void *stream) {
     mfl_nf4_weight nested[2];

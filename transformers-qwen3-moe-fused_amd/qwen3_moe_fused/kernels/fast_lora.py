@@ -179,7 +179,8 @@ class FastLora(torch.autograd.Function):
             one_launch = Bg.shape == Bu.shape and (packed or (Gqs is None and Uqs is None and dt == torch.bfloat16
                                                               and Gq.dtype == dt and Uq.dtype == dt))
             if one_launch:
-                # each matrix's thin weights are its adapter's B over its own columns of ucat and zeros over the other's
+                # each matrix's thin weights are its adapter's B over its own columns of ucat and zeros over the other's (an
+                # infinite activation of one adapter, whose row is not finite anyway, makes the other's product NaN there)
                 assert Bg.shape[2] == r, "an adapter's A and B have one rank"
                 bg, bu = _padded(Bg, 2, 0, 2 * r, pieces), _padded(Bu, 2, r, 2 * r, pieces)
             _copy_pieces(pieces, True)
@@ -196,7 +197,7 @@ class FastLora(torch.autograd.Function):
             g, uu = _proj_fwd(x, Uq, Uqs, Au, Bu, Su, m_sizes, uu)
             h = silu_mul_forward(e, g)
         y, uw = _proj_fwd(h, Wq, Wqs, Aw, Bw, Sw, m_sizes)
-        Gqs, Uqs, Wqs = frozen_states  # (the scales are written out again: 6 MB a matrix less held between the passes)
+        Gqs, Uqs, Wqs = frozen_states  # (the scales are written out again: 4 E N K / blocksize bytes each, 12.6 MB at 128 x 768 x 2048, not held between the passes)
         ctx.frozen = (Gq, Gqs, Sg, Uq, Uqs, Su, Wq, Wqs, Sw, m_sizes)
         ctx.save_for_backward(x, Ag, Bg, Au, Bu, Aw, Bw, e, g, ug, uu, uw)
         return y
