@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import oracle
-from util import check_close, gen, m_sizes_uniform, randn, to_np32, unit_scale_atol
+from util import check_close, check_tiles, gen, m_sizes_uniform, randn, to_np32, unit_scale_atol
 
 pytestmark = pytest.mark.gpu
 
@@ -554,6 +554,27 @@ def test_packed_gate_and_up_with_lora_terms(m_sizes, M, H, r, bs):
     two = grouped_gemm_forward_transposed_4bit_lora(de, gq, gs, t, a, ms)
     grouped_gemm_forward_transposed_4bit(dg, uq, us, ms, out=two, accumulate=True)
     check_close(dx, to_np32(two), atol=unit_scale_atol(to_np32(two), 2e-2), what="one reduction vs two products")
+
+
+# with rank-r terms past 128 rows per expert: one launch of 256 x 256 tiles, unless they spill into a second round while each
+# product's 160 x 128 tiles are all resident
+@pytest.mark.parametrize("R,E,M,one_launch", [(4096, 16, 1536, False), (6144, 16, 1536, True), (8192, 8, 768, True),
+                                              (12288, 8, 768, False), (16384, 8, 768, True)])
+def test_packed_gate_and_up_with_lora_terms_in_one_launch_or_two(R, E, M, one_launch):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the rule counts rounds of 256 compute units")
+    g = gen(R + M)
+    ms = m_sizes_uniform(R, E, g).to(DEV)
+    (gq, gs), (uq, us) = (quantize_nf4(randn((E, M, 64), g, 0.05, torch.bfloat16).to(DEV), 64) for _ in range(2))
+    x, ug, uu = (randn((R, n), g, 1.0, torch.bfloat16).to(DEV) for n in (64, 8, 8))
+    bg, bu = (randn((E, M, 8), g, 0.2, torch.bfloat16).to(DEV) for _ in range(2))
+    z = torch.zeros_like(bg)
+    u, *wide = (torch.cat(p, d).contiguous() for p, d in (((ug, uu), 1), ((bg, z), 2), ((z, bu), 2)))
+    h, e, g2 = check_tiles(lambda: grouped_glu_forward_4bit_lora(x, gq, gs, uq, us, u, *wide, ms),
+                           ("pipe", 256, 256, 0, True, 3) if one_launch else ("pipe", 160, 128, 0, True, 2))
+    assert torch.equal(e, grouped_gemm_forward_4bit_lora(x, gq, gs, ug, bg, ms))
+    assert torch.equal(g2, grouped_gemm_forward_4bit_lora(x, uq, us, uu, bu, ms))
+    assert torch.equal(h, silu_mul_forward(e, g2))
 
 
 # Both adapters' activations lie side by side against weights that are zero over the other's columns, and 0 x inf is NaN: an

@@ -1169,7 +1169,15 @@ int dispatch_pipe(int mode, const void *a, const void *b, const void *m_sizes, i
         // products do, then 256 x 256 (N = 768, K = 2048, 128 experts, us on 320 x 192 / 160 x 128 / 256 x 256 and for the two
         // products and the SiLU-mul by themselves: 257 / 211 / 225, 255 at 128 rows; 273 / 266 / 252, 255 at 160; 556 / 405 /
         // 357, 339 at 256, under Zipf(1.2) routing 686 / 422 / 383, 521; 970 / 726 / 570, 624 at 512)
-        if (nf4 != nullptr && fusion->at != nullptr && cfg != 5) cfg = R <= (int64_t)128 * E ? 5 : 8;
+        // But where either product by itself has all its 160 x 128 tiles resident at once and the 256 x 256 tiles of both spill
+        // into a second round, the separate products are ahead (16 experts, N = 1536, K = 4096, 4096 rows 222 against 262 us; 8
+        // experts, N = 768, K = 2048, 12288 rows 137 against 148, with 8192, one round, 127 against 78).
+        if (nf4 != nullptr && fusion->at != nullptr && cfg != 5) {
+            cfg = R <= (int64_t)128 * E ? 5 : 8;
+            if (cfg == 8 && (R / 160 + E) * (int64_t)ceil_div(N, 128) <= 2 * device_info().cu_count &&
+                expected_rounds(R, N, E, 256, 128) > 1.02)
+                return MFL_ERR_UNSUPPORTED;
+        }
     } else if (cfg == 0 || nf4 != nullptr) {
         if (mode == MODE_DW)
             cfg = (N <= 64 || K <= 64) ? 11 : 8;
