@@ -320,6 +320,37 @@ def test_a_state_that_several_matrices_share_is_written_out_once(monkeypatch):
     assert outs[0].absmax.data_ptr() != outs[2].absmax.data_ptr()
 
 
+@pytest.mark.parametrize("h", [64, 96, 192, 224])
+def test_packed_gate_and_up_in_one_launch_for_whole_reduction_steps(monkeypatch, h):
+    """For other hidden sizes there is no such kernel, and the separate products take each adapter's own rank."""
+    from qwen3_moe_fused.kernels.fast_lora import fast_lora
+    from qwen3_moe_fused.quantize.nf4 import Nf4QuantState, code_of
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(_lib, "stream", lambda: 0)
+    names, ranks = [], []
+
+    class Library:
+        def __getattr__(self, name):
+            def call(*args):
+                names.append(name)
+                if name == "mfl_gemm_fwd_nf4_lora":
+                    ranks.append(args[7])
+                return 0
+
+            return call
+
+    monkeypatch.setattr(_lib, "lib", lambda: Library())
+    args = _lora_args(h=h, m=64, r=8)
+    for i, shape in ((1, (2, 64, h)), (6, (2, 64, h)), (11, (2, h, 64))):
+        args[i] = torch.zeros((2 * 64 * h // 2, 1), dtype=torch.uint8)
+        args[i + 1] = Nf4QuantState(absmax=torch.ones(2 * 64 * h // 32), shape=shape, code=code_of("nf4", "cpu"), blocksize=32,
+                                    quant_type="nf4", dtype=torch.bfloat16)
+    fast_lora(*args)
+    assert names.count("mfl_glu_fwd_nf4_lora") == (h % 64 == 0)
+    assert names.count("mfl_gemm_fwd_nf4_lora") == (1 if h % 64 == 0 else 3) and set(ranks) == {8}
+
+
 def _router_and_rows():
     from qwen3_moe_fused.modular_qwen3_moe_fused import Qwen3MoeFusedRouter
 
