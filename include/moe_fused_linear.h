@@ -282,8 +282,8 @@ MFL_API int mfl_glu_fwd_nf4_packed(const void *x, int64_t src_rows, const int32_
 
 /* mfl_glu_fwd_lora over packed base weights with fp32 scales, and the input gradient of the two projections with both
  * rank-r terms in one reduction: dx = dy1 w1 + dy2 w2 + xt wt, dy1, dy2 (R,K), w1, w2 (E,K,N), xt (R,KT), wt (E,KT,N).
- * MFL_ERR_UNSUPPORTED, with nothing enqueued, as for mfl_gemm_fwd_nf4_lora / mfl_gemm_dx_nf4_lora and for
- * double-quantised weights. */
+ * MFL_ERR_UNSUPPORTED, with nothing enqueued, as for mfl_gemm_fwd_nf4_lora / mfl_gemm_dx_nf4_lora, for
+ * double-quantised weights, and for sizes at which the two products by themselves are ahead. */
 MFL_API int mfl_glu_fwd_nf4_lora(const void *x, const mfl_nf4_weight *w_gate, const mfl_nf4_weight *w_up, const void *xt,
                          const void *wt_gate, const void *wt_up, int KT, const void *m_sizes, int m_sizes_dtype,
                          void *h, void *e_out, void *g_out, int64_t R, int N, int K, int E, int dtype, void *stream);

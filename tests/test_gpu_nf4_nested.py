@@ -49,6 +49,12 @@ CASES = [
     ([1, 0, 2, 1], 64, 768, 64),
     ([1, 0, 1], 128, 576, 64),
     ([2, 0, 1, 0], 64, 320, 64),
+    ([1, 2, 0, 3], 64, 960, 64),
+    # blocks smaller than a lane's run
+    ([1, 0, 2, 1], 64, 2048, 8),
+    ([1, 0, 2, 1], 64, 1024, 16),
+    ([1, 2, 0, 1], 64, 768, 32),
+    ([1, 0, 2, 1], 64, 512, 16),
     ([5, 0, 3, 17], 200, 768, 64),
     ([40, 1, 33], 128, 384, 64),
     ([70, 0, 12], 72, 2048, 64),

@@ -411,8 +411,9 @@ struct UnnestJobs {
     int bs2_shift[kMaxUnnest], vec_ok[kMaxUnnest];
 };
 
-// The fp32 scales of double-quantised matrices (one per blockIdx.y), offset included.  3.1 M scales: two launches of a byte per lane each
-// (scales, then the offset) took 10.0 + 6.6 us, 16 bytes in and 64 out per lane 8.3 us (a store touched every line).
+// The fp32 scales of double-quantised matrices (one per blockIdx.y), offset included.  3.1 M scales: two launches of a byte
+// per lane each (scales, then the offset) took 10.0 + 6.6 us, 16 bytes in and 64 out per lane 8.3 us (a store touched
+// every line).
 __global__ __launch_bounds__(256) void nf4_unnest_kernel(UnnestJobs jobs) {
     const int job = blockIdx.y;
     const uint8_t *__restrict__ const v = jobs.v[job];

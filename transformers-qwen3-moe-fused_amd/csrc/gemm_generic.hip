@@ -347,8 +347,8 @@ int launch_tile(const Args &g) {
 // * beyond, 64 x 64 tiles: 373 us at 64 rows per expert (1584; 128 x 128 tiles 392, whose 64 accumulators and 32
 //   registers in transit leave two workgroups a CU).
 // * the weight gradient writes more than it reads up to about 100 rows per expert: 64 x 128 tiles and 16-row steps,
-//   126 us at 8 rows per expert = 6.4 TB/s (294; before its rows left as whole lines 177, with 32-row steps 225, the zeros of a half-empty stage cost as much
-//   as rows do); outputs of at most 16 rows per expert (N: the rank in the gradient of an adapter's A) take
+//   126 us at 8 rows per expert = 6.4 TB/s (294; before its rows left as whole lines 177, with 32-row steps 225, the zeros
+//   of a half-empty stage cost as much as rows do); outputs of at most 16 rows per expert (N: the rank in the gradient of an adapter's A) take
 //   16-row tiles.
 // * short reductions (adapter ranks, toy sizes) leave most of a 64- or 128-wide step empty: 16-wide steps.  16000 rows of 8
 //   experts, 1500 outputs, reduction 8 / 32 / 64 / 128: 64 x 64 tiles 22.0 / 31.0 / 46 / 75 us (64-wide steps 34.9 / 44.5 / 54 /

@@ -24,7 +24,8 @@
 //     workgroups, and a workgroup changes rows once or twice.  Each wave keeps the loads of four columns ahead
 //     in registers.
 //   * rows of at most 1024 elements: 32 lanes to a column, the wave's second column (16 further on) in lanes 32..63; up to
-//     512, and for 576 and 768: 16 lanes and four columns, four or six dwords to a lane.  No swap before the adds.
+//     512, and for 576 and 768: 16 lanes and four columns, four or six dwords to a lane (gemv_layout.h).  No swap before
+//     the adds.
 //   What the loop is short of, with 16 waves to a CU, is issue slots, scalar ones first: addresses move by
 //   increments, the row count is branched on once per column, and the lookups of a dword wait once.
 //
