@@ -36,9 +36,11 @@ int main() {
                     }
             bool ok = whole && l.reach() >= K;
             for (int t : taken) ok = ok && t == 1;
-            // with the dwords of a short reduction apart, past a row per expert the streaming kernel takes what it can
+            // with the dwords of a short reduction apart, past a row per expert the streaming kernel takes what it can, and the
+            // register-decoding one the shortest
             const int half_rows = mfl::gemv_half_rows(K, l, bs_shift);
-            const bool left = K <= 1024 && !l.side_by_side && K % 128 == 0 && bs_shift >= 6;
+            const bool left = K <= 1024 && ((K % 128 == 0 && bs_shift >= 6 && (K == 384 || !l.side_by_side)) ||
+                                            (K < 512 && bs_shift >= 5 && !l.side_by_side));
             ok = ok && half_rows == (K > 1024 ? 4 : left ? 2 : 3);
             if (!ok && wrong++ < 8) std::printf("K = %d, N = %d, blocks of %d: %d lanes of %d dwords\n", K, N, 1 << bs_shift, l.lanes, l.dwords);
         }

@@ -69,7 +69,7 @@ def test_block_call_both_ways(t, e, k, h, i, kind):
 
 # (two times t tokens; the first five: the down projection and the sum over the selections in one launch, up to 16 selections)
 @pytest.mark.parametrize("t,e,k,h,i", [(1, 8, 2, 256, 512), (1, 16, 8, 128, 768), (1, 32, 8, 192, 576), (4, 24, 2, 128, 768),
-                                       (1, 16, 5, 64, 320), (9, 16, 4, 512, 128), (200, 8, 4, 128, 96), (1500, 6, 2, 128, 256)])
+                                       (1, 16, 5, 64, 320), (3, 8, 2, 128, 384), (9, 16, 4, 512, 128), (200, 8, 4, 128, 96), (1500, 6, 2, 128, 256)])
 @pytest.mark.parametrize("kind", ["nf4", "nf4dq"])
 def test_block_call_on_packed_weights(t, e, k, h, i, kind):
     blk, dtype = _block(e, k, h, i, kind, t)

@@ -697,10 +697,11 @@ int gemm_nf4_down_combine(const bf16_t *h, const int32_t *inv, const int64_t *id
     // kernels at every number of selections: a block of 128 experts, 2048 x 768, 1 / 4 / 8 / 12 / 16 of them, fp32 scales, all
     // its kernels: 17.5 / 20.1 / 24.8 / 26.8 / 28.6 -> 13.4 / 15.1 / 19.2 / 22.2 / 23.6 us; 16 of one token 32.7 -> 24.8)
     const int64_t R = T * k;
-    if (R <= 0 || R > kDownRows || 2 * R > 3 * (int64_t)E || N % 64 != 0 || N > (1 << 18)) return MFL_ERR_UNSUPPORTED;
+    if (R <= 0 || R > kDownRows || N % 64 != 0 || N > (1 << 18)) return MFL_ERR_UNSUPPORTED;
     if (K <= 256 || K > 768 || K % 64 != 0) return MFL_ERR_UNSUPPORTED;
     const GemvLayout l = gemv_layout(K, N, w.bs_shift);
     if (l.lanes != 16 || !l.side_by_side || (K & ((1 << w.bs_shift) - 1)) != 0) return MFL_ERR_UNSUPPORTED;
+    if (2 * R > (int64_t)E * gemv_half_rows(K, l, w.bs_shift)) return MFL_ERR_UNSUPPORTED;
     if (!aligned(h, 16) || !aligned(w.wq, 16) || !aligned(w.absmax, 4) || !aligned(out, 2)) return MFL_ERR_UNSUPPORTED;
 #define MFL_DOWN(NL, NESTED) \
     launch_down_combine<NL, NESTED>(h, inv, idx, weights, w, out, (int)R, k, N, K, E, stream)

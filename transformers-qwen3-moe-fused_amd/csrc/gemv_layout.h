@@ -37,12 +37,18 @@ constexpr GemvLayout gemv_layout(int K, int N, int bs_shift) {
 // against 40 / 20 at 2; K = 896: 59 / 32 against 59 / 33 at 1.5; 8-bit ones, whose sums are the same bits and the line
 // therefore the same: 53 / 30 against 54 / 28 at 1.75, 59 / 32 against 55 / 30 at 2; I = 512: 34 / 19 against 37 / 20 at 1.5,
 // 41 / 23 against 38 / 20 at 2.  Short reductions with the dwords apart are behind it past a row: K = 640, 1.125 rows 47 / 25
-// against 41 / 23, 1.5 rows 54 / 28 against 42 / 24, 8-bit scales 64 / 33 against 41 / 23.  What the streaming kernel does not take
+// against 41 / 23, 1.5 rows 54 / 28 against 42 / 24, 8-bit scales 64 / 33 against 41 / 23; K = 384 is in either layout (side by
+// side, 1.25 rows, N = 448 / 1280 / 2048, plain 9.7 / 13.7 / 16.7 against 7.4 / 12.2 / 16.2, with 8-bit scales gated 13.5 / 22.2 /
+// 29.8 against 11.8 / 19.8 / 26.4; N = 4096 27.7 against 31.1 and 52.6 against 54.0).  What the streaming kernel does not take
 // goes to the register-decoding one, which is further behind: K = 704, 1.5 rows 54 / 29 against 61 / 33; K = 768 in blocks
-// of 32 58 / 31 against 78 / 41, of 16 60 / 33 against 127 / 69.
+// of 32 58 / 31 against 78 / 41, of 16 60 / 33 against 127 / 69; but below 512 in blocks of 32 and more it is ahead there: 60
+// experts, K = 320, N = 992, 1.5 rows 17 / 10 against 13 / 7; 64 experts, K = 448, N = 1376, blocks of 32, 1.1 rows 19 / 12
+// against 18 / 10.
 constexpr int gemv_half_rows(int K, GemvLayout l, int bs_shift) {
     const bool streams = K % 128 == 0 && bs_shift >= 6;
-    return K > 1024 ? 4 : streams && !l.side_by_side ? 2 : 3;
+    const bool decodes = K < 512 && bs_shift >= 5;
+    if (streams && K < 512) return 2;
+    return K > 1024 ? 4 : (streams || decodes) && !l.side_by_side ? 2 : 3;
 }
 
 constexpr bool gemv_layouts_reach() {
