@@ -222,9 +222,10 @@ __global__ __launch_bounds__(kThreads) void gemm_generic_kernel(const TI *__rest
             __syncthreads();  // the last step's fragments have been read
             float *const st = smem + wave * (16 * kOutRow);
             // (asked for again here: what follows from the lane's number otherwise takes two registers through the reduction, which
-            // leave room for five workgroups a CU instead of six: 8 experts x 768 x 2048, 1536 tiles, 4096 rows 133 against 119 us)
+            // leave room for five workgroups a CU instead of six: 8 experts x 768 x 2048, 1536 tiles, 4096 rows 133 against 119 us.
+            // Past the caches, where the write rate is what counts, five are ahead: 128 experts, 1024 rows 134 against 136.)
             int ln = tid & 63;
-            asm volatile("" : "+v"(ln));
+            if constexpr (!NT) asm volatile("" : "+v"(ln));
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
 #pragma unroll
